@@ -45,6 +45,18 @@ def _is_symbolic(value: Any) -> bool:
     return isinstance(value, torch.SymInt)
 
 
+def _record_use(value: Any, stream: Any) -> None:
+    """Register every device tensor of a launch's input with the allocator for ``stream``.  An operator with several
+    results reaches the next sub-graph as the tuple it returned when the cut lies in front of the node that unpacks
+    it, so tuples and lists are walked."""
+    if isinstance(value, torch.Tensor):
+        if value.is_cuda:
+            value.record_stream(stream)
+    elif isinstance(value, (tuple, list)):
+        for item in value:
+            _record_use(item, stream)
+
+
 class _SharedOutput:
     """Rows of one output buffer handed to the operator that ends each nano-batch (``ops.offer_output_rows``).
 
@@ -448,8 +460,7 @@ class DynaFlowEngine:
                 if device.is_gpu:
                     current = device.current_stream()
                     for value in pos:
-                        if isinstance(value, torch.Tensor) and value.is_cuda:
-                            value.record_stream(current)
+                        _record_use(value, current)
                 call_pos.append(pos)
                 call_kw.append(kw)
 

@@ -313,6 +313,39 @@ def test_fp8_layer_with_fused_gate_up_epilogue_through_the_manager():
     assert torch.equal(y, plain.forward_schedule(xg, split.split_indices))
 
 
+@pytest.mark.parametrize("tokens", [24, 600])
+def test_fp8_fused_sub_graph_result_survives_until_the_other_stream_has_read_it(tokens):
+    """The fused fp8 operator's two results reach the down projection as one tuple on another stream, while the next
+    nano-batch's first sub-graph already allocates on the stream they were made on: the memory must stay theirs until
+    the down projection has run (at 600 tokens the activation codes were overwritten and the result was NaN)."""
+    from dynaflow_amd.backend import make_backend
+    from dynaflow_amd.config import CUDAGraphConfig, DynaFlowConfig, InductorConfig
+    from dynaflow_amd.fp8_mlp import Fp8SwiGLU
+    from dynaflow_amd.manager import DynaFlowManager
+
+    gen = torch.Generator(device="cuda").manual_seed(tokens)
+    hidden, inter = 8192, 28672
+    weights = [(torch.randn(s, generator=gen, device="cuda") * 0.02).bfloat16()
+               for s in ((inter, hidden), (inter, hidden), (hidden, inter))]
+    layer = Fp8SwiGLU.from_weights(*weights, fuse_gate_up=True)
+    x = torch.randn(tokens, hidden, generator=gen, device="cuda").bfloat16()
+    cfg = DynaFlowConfig("dynaflow_amd.schedulers:MLPOverlapScheduler", 2, InductorConfig(enabled=True),
+                         CUDAGraphConfig(enabled=False, capture_sizes=[tokens]),
+                         {"min_nano_split_tokens": 1, "num_nano_batches": 2, "dump_graph": False,
+                          "fuse_silu_epilogue": True, "whole_graph": True, "streams": "by_kind"})
+    manager = DynaFlowManager()
+    torch._dynamo.reset()
+    torch._dynamo.mark_dynamic(x, 0)
+    compiled = torch.compile(layer, backend=make_backend(manager, cfg), fullgraph=True)
+    with torch.no_grad():
+        manager.prepare(tokens, [tokens])
+        compiled(x)
+        want = layer.forward_schedule(x, [0, tokens // 2, tokens])
+        for graph in (False, True, True):
+            manager.prepare(tokens, [tokens], use_cudagraph=graph)
+            assert torch.equal(compiled(x), want), f"graph={graph}"
+
+
 def test_piecewise_graphs_capture_in_dryrun_and_replay():
     """Per-sub-graph hipGraphs as in the reference: captured for every (size, nano-batch index) during a
     dry-run over fake nano-batches, replayed by the scheduled forward against per-nano-batch static buffers."""
