@@ -57,6 +57,13 @@ DFHIP_DEVICE uint32_t pack2_bf16(float lo, float hi) {
 DFHIP_DEVICE float bf16_lo_to_f32(uint32_t pair) { return __uint_as_float(pair << 16); }
 DFHIP_DEVICE float bf16_hi_to_f32(uint32_t pair) { return __uint_as_float(pair & 0xffff0000u); }
 
+// bf16(x + r) on packed pairs: the product is rounded to bf16 first (x is such a rounded value), the
+// sum is rounded again - the roundings of a GEMM followed by a separate bf16 addition.
+DFHIP_DEVICE uint32_t add2_bf16(uint32_t x, uint32_t r) {
+  return pack2_bf16(bf16_lo_to_f32(x) + bf16_lo_to_f32(r),
+                    bf16_hi_to_f32(x) + bf16_hi_to_f32(r));
+}
+
 // silu(g) = g / (1 + e^-g) on the hardware exponential and reciprocal (a few fp32 ulp; the bf16 paths
 // round the result to 8 bits of mantissa right after).  -inf gives NaN like the exact quotient.
 DFHIP_DEVICE float silu_fast(float g) {
@@ -118,5 +125,22 @@ template <int N>
 DFHIP_DEVICE void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// 16-byte store / load that is coherent across the XCDs (sc1: written through to, and read
+// from, the memory side instead of the XCD-private L2).  Used for split-K partial blocks so
+// that no L2-wide write-back or invalidate is needed to hand them from one XCD to another.
+// A store of more than 8 bytes reads its data registers for a few cycles after issue and the compiler
+// cannot see that this statement is one: the wait states keep the next write to those registers away.
+DFHIP_DEVICE void store_f32x4_device_coherent(f32x4* p, f32x4 v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+DFHIP_DEVICE f32x4 load_f32x4_device_coherent(const f32x4* p) {
+  f32x4 v;
+  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
+  return v;
+}
+// The loads above are invisible to the compiler's own wait-count bookkeeping: a value may only
+// be used after this, which ties the wait to the register so that the use cannot move above it.
+DFHIP_DEVICE void wait_loaded(f32x4& v) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(v)::"memory"); }
+
 DFHIP_DEVICE void workgroup_barrier() { asm volatile("s_barrier" ::: "memory"); }
 #define DFHIP_PIN __builtin_amdgcn_sched_barrier(0)

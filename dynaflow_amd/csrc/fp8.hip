@@ -13,7 +13,7 @@
 //                       XOR-swizzled 128-byte rows, one LDS read or DMA issue behind every
 //                       MFMA, barrier between the two column halves of a slab, staged epilogue.
 // gemm_fp8_nt_kernel    register-staged double buffer for small shapes.
-#include "dfhip_common.h"
+#include "dfhip_stream.h"
 
 namespace {
 
@@ -695,6 +695,10 @@ int launch_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, 
   return dfhip_check_launch();
 }
 
+// Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip); with 16 rows and more from K = 4096
+// on, as for bf16 rows of the same bytes.
+bool stream_planned(int M, int N, int K) { return dfhip_stream_fits(M, N, K, 1) && (M < 16 || K >= 4096); }
+
 int check_q(const void* x, int64_t ld, int M, int D) {
   if (!x) return DFHIP_ERR_NULL_POINTER;
   if (M < 1 || D < 8 || D % 8 != 0 || (int64_t)M * (D / 8) >= (int64_t)1 << 31) return DFHIP_ERR_BAD_SHAPE;
@@ -760,6 +764,8 @@ extern "C" int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void*
       !dfhip_aligned16(w_scale))
     return DFHIP_ERR_BAD_ALIGNMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (variant < 0 && stream_planned(M, N, K))
+    return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
   if (variant < 0) {   // the planned kernel
     const int64_t big_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     variant = 1;
@@ -787,6 +793,9 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, co
       !dfhip_aligned16(W_up) || !dfhip_aligned16(act) || !dfhip_aligned16(w_gate_scale) ||
       !dfhip_aligned16(w_up_scale))
     return DFHIP_ERR_BAD_ALIGNMENT;
+  if (stream_planned(M, I, K))
+    return dfhip_stream_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I,
+                                    K, static_cast<hipStream_t>(stream));
   return launch_fp8_ring_fused(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I,
                                K, static_cast<hipStream_t>(stream));
 }

@@ -39,7 +39,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "dfhip_common.h"
+#include "dfhip_stream.h"
 
 // Split-K scratch of dfhip_gemm_bf16_nt_splitk_static: arrival counters followed by fp32 partial blocks,
 // laid out like a caller's workspace.  One copy per GPU, held until the process ends.  In host code this
@@ -66,13 +66,6 @@ struct Shape {
   static_assert(BM % (WAVES_M * 32) == 0 && BN % (WAVES_N * 32) == 0, "wave tile must be MFMA blocks");
   static_assert((BM * CHUNKS) % THREADS == 0 && (BN * CHUNKS) % THREADS == 0, "loads must divide evenly");
 };
-
-// bf16(x + r) on packed pairs: the product is rounded to bf16 first (x is such a rounded value), the
-// sum is rounded again - the roundings of a GEMM followed by a separate bf16 addition.
-DFHIP_DEVICE uint32_t add2_bf16(uint32_t x, uint32_t r) {
-  return pack2_bf16(bf16_bits_to_f32(x & 0xffffu) + bf16_bits_to_f32(r & 0xffffu),
-                    __uint_as_float(x & 0xffff0000u) + __uint_as_float(r & 0xffff0000u));
-}
 
 // R (may be null): residual [M, N] with the leading dimension of C, added in the epilogue.
 template <int BM, int BN, int WAVES_M, int WAVES_N>
@@ -229,23 +222,6 @@ constexpr int GROUP_M = 4;   // tiles of one XCD are walked in panels of GROUP_M
 constexpr int EROW = 272;    // padded row of the epilogue staging area (bytes)
 // Split-K: the bound of the last part's wait for the others (sleeps of about a microsecond: a second).
 constexpr int SPLITK_SPIN_LIMIT = 1 << 20;
-
-// 16-byte store / load that is coherent across the XCDs (sc1: written through to, and read
-// from, the memory side instead of the XCD-private L2).  Used for split-K partial blocks so
-// that no L2-wide write-back or invalidate is needed to hand them from one XCD to another.
-// A store of more than 8 bytes reads its data registers for a few cycles after issue and the compiler
-// cannot see that this statement is one: the wait states keep the next write to those registers away.
-DFHIP_DEVICE void store_f32x4_device_coherent(f32x4* p, f32x4 v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
-}
-DFHIP_DEVICE f32x4 load_f32x4_device_coherent(const f32x4* p) {
-  f32x4 v;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
-  return v;
-}
-// The loads above are invisible to the compiler's own wait-count bookkeeping: a value may only
-// be used after this, which ties the wait to the register so that the use cannot move above it.
-DFHIP_DEVICE void wait_loaded(f32x4& v) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(v)::"memory"); }
 
 // Split-K workspaces start with the arrival counters.  Both split-K kernels use the same size of
 // counter area for a workspace (at least 4 KiB), so that the fp32 blocks one of them leaves behind
@@ -1567,6 +1543,13 @@ int launch_skinny(const void* A, int64_t lda, const void* W, const void* W2, int
   return dfhip_check_launch();
 }
 
+// The few-rows kernel with K cut into parts: arrival counters and fp32 blocks of the workspace as in launch_skinny.
+int launch_stream(const void* A, int64_t lda, const void* W, const void* R, int64_t ldw, void* C, int64_t ldc, int M,
+                  int N, int K, int split_k, void* workspace, hipStream_t stream) {
+  void* partials = split_k > 1 ? static_cast<uint8_t*>(workspace) + skinny_counter_bytes(M, N) : nullptr;
+  return dfhip_stream_bf16(A, lda, W, ldw, R, C, ldc, M, N, K, split_k, partials, static_cast<int*>(workspace), stream);
+}
+
 int launch_skinny_wide(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                        int M, int N, int K, hipStream_t stream) {
   if (M > SK_MAX_M || K / BK < 2) return DFHIP_ERR_BAD_SHAPE;
@@ -1607,6 +1590,18 @@ double round_fill(int M, int N, int tile_n, int share = 1) {
   return (double)M * N * share / ((double)rounds * 256 * RBM * tile_n);
 }
 
+// Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip), whatever runs beside it.
+// With 16 rows and more a K below 2048 keeps the 128-row tiles.  Weights of more than 2^27 elements keep them too: there
+// a row has the same bits in a launch of few rows and of many, which is worth more than the gain (2 x 28672 x 8192 with
+// SiLU*mul, us: 154 against 186 at 1 .. 16 rows, but 193 against 182 at 64, where the re-read activations weigh more).
+// From 33 rows on two such launches side by side cost what they cost one after the other - the re-read activation rows
+// bound them - where the 128-row tiles of a pair share what they read (8B layer, 2 x 48 rows: 167 against 136 us; 2 x 20
+// rows in a decode step: 161 against 190 us a layer).
+bool stream_planned(int M, int N, int K) {
+  return M <= 32 && dfhip_stream_fits(M, N, (int64_t)K * 2, 1) && (M < 16 || K >= 2048) &&
+         (int64_t)N * K <= (int64_t)1 << 27;
+}
+
 int check_args(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
                int K) {
   if (!A || !W || !C) return DFHIP_ERR_NULL_POINTER;
@@ -1634,6 +1629,9 @@ extern "C" int dfhip_gemm_bf16_nt_variant(const void* A, int64_t lda, const void
     case 5: return launch_ring224<false>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, s);
     case 7: return launch_ring224<false, 128>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, s);
     case 6: return launch_skinny<false>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, 1, nullptr, s);
+    case 8:
+      if (!dfhip_stream_fits(M, N, (int64_t)K * 2, 1)) return DFHIP_ERR_BAD_SHAPE;
+      return dfhip_stream_bf16(A, lda, W, ldw, nullptr, C, ldc, M, N, K, 1, nullptr, nullptr, s);
     default: return DFHIP_ERR_BAD_ARGUMENT;
   }
 }
@@ -1652,6 +1650,11 @@ extern "C" int dfhip_gemm_bf16_plan_shared(int M, int N, int K, int share, int* 
   const int64_t big_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
   *variant = 2;
   *split_k = 1;
+  if (stream_planned(M, N, K)) {
+    *variant = 8;
+    *split_k = dfhip_stream_split(M, N, (int64_t)K * 2);
+    return DFHIP_OK;
+  }
   // decode-sized activations: up to 128 rows always, up to 512 rows (1024 with K <= 8192: with a longer K the
   // 256 x 256 tiles with K split win) while the 128 x 128 tiles fit one round of 256 workgroups; beyond that
   // the 256 x 256 tiles below move fewer bytes through LDS per flop
@@ -1717,7 +1720,9 @@ extern "C" int dfhip_gemm_bf16_nt_splitk(const void* A, int64_t lda, const void*
   }
   int variant = 0, planned = 1;
   dfhip_gemm_bf16_plan(M, N, K, &variant, &planned);
-  if (variant == 6)
+  if (variant == 8 && dfhip_stream_fits(M, N, (int64_t)K * 2, split_k))
+    return launch_stream(A, lda, W, nullptr, ldw, C, ldc, M, N, K, split_k, workspace, static_cast<hipStream_t>(stream));
+  if (variant == 6 || variant == 8)
     return launch_skinny<false>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, split_k, workspace,
                                 static_cast<hipStream_t>(stream));
   if (split_k > 8) return DFHIP_ERR_BAD_ARGUMENT;
@@ -1746,6 +1751,8 @@ extern "C" int dfhip_gemm_bf16_gate_up_silu_shared(const void* A, int64_t lda, c
   if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
   if (int rc = check_args(A, lda, W_gate, ldw, Out, ldo, M, I, K)) return rc;
   if (!dfhip_aligned16(W_up)) return DFHIP_ERR_BAD_ALIGNMENT;
+  if (stream_planned(M, I, K))
+    return dfhip_stream_bf16_gate_up(A, lda, W_gate, W_up, ldw, Out, ldo, M, I, K, static_cast<hipStream_t>(stream));
   if (M <= 2 * SK_BM && I >= 1024 && K >= 1024) {   // decode-sized activations: stream both weights once
     // 128 outputs per workgroup when the launches that run side by side, or the two row tiles of 129 .. 256
     // rows, then still give every compute unit a workgroup's worth of the round; 64 outputs otherwise
@@ -1784,7 +1791,7 @@ extern "C" int dfhip_gemm_bf16_nt_add(const void* A, int64_t lda, const void* W,
   if (int rc = dfhip_gemm_bf16_plan(M, N, K, &variant, &planned)) return rc;
   if (split_k < 1 || split_k > 16 || K / BK < split_k) return DFHIP_ERR_BAD_ARGUMENT;
   if (split_k > 1) {
-    if (variant != 0 && variant != 6) return DFHIP_ERR_BAD_ARGUMENT;   // the planned kernel does not split K
+    if (variant != 0 && variant != 6 && variant != 8) return DFHIP_ERR_BAD_ARGUMENT;   // the planned kernel does not split K
     if (variant == 0 && split_k > 8) return DFHIP_ERR_BAD_ARGUMENT;
     if (!workspace) return DFHIP_ERR_NULL_POINTER;
     if (!dfhip_aligned16(workspace)) return DFHIP_ERR_BAD_ALIGNMENT;
@@ -1796,6 +1803,10 @@ extern "C" int dfhip_gemm_bf16_nt_add(const void* A, int64_t lda, const void* W,
     case 5: return launch_ring224<false>(A, lda, W, R, ldw, C, ldc, M, N, K, s);
     case 7: return launch_ring224<false, 128>(A, lda, W, R, ldw, C, ldc, M, N, K, s);
     case 6: return launch_skinny<false>(A, lda, W, R, ldw, C, ldc, M, N, K, split_k, workspace, s);
+    case 8:
+      if (!dfhip_stream_fits(M, N, (int64_t)K * 2, split_k))
+        return launch_skinny<false>(A, lda, W, R, ldw, C, ldc, M, N, K, split_k, workspace, s);
+      return launch_stream(A, lda, W, R, ldw, C, ldc, M, N, K, split_k, workspace, s);
     default: return launch<128, 128, 2, 2>(A, lda, W, ldw, C, ldc, M, N, K, s, R);
   }
 }

@@ -93,6 +93,10 @@ int dfhip_gemm_bf16_nt(const void* A, int64_t lda, const void* W, int64_t ldw, v
  *              while the tiles fit one round of 256 workgroups;
  *          7 = 256x128 tile, LDS-DMA ring (chosen instead of a split along K when the
  *              256x256 tiling has few tiles and K <= 8192);
+ *          8 = up to 64 rows: W streamed from memory to registers past LDS, K optionally in
+ *          parts that meet as with variant 6 (needs K >= 1024 and K / split_k >= 1024; the
+ *          plan picks it up to 32 rows for K >= 2048, below 16 rows for every such K, and
+ *          weights of at most 2^27 elements);
  *          register-staged tiles: 1 = 256x256 / 8 waves, 2 = 128x128 / 4 waves,
  *          3 = 256x128 / 4 waves, 4 = 256x256 / 4 waves. */
 int dfhip_gemm_bf16_nt_variant(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
@@ -123,13 +127,13 @@ int dfhip_gemm_bf16_plan_shared(int M, int N, int K, int share, int* variant, in
  * the highest launch index of its tile for every tile count and whoever it waits
  * for was dispatched before it.  The wait is bounded (about a second); a tile
  * whose parts never arrived is written as NaN.  With the weight-streaming kernel
- * (variant 6) every part leaves a block and the part that arrives last adds them
+ * (variants 6 and 8) every part leaves a block and the part that arrives last adds them
  * up; nobody waits.  `workspace` (device memory, 16-byte aligned,
  * at least dfhip_gemm_bf16_splitk_workspace_bytes(M, N, split_k) bytes) starts
  * with the per-tile arrival counters, which must be ZERO before the first use
  * and are left zero by every launch; launches that may overlap in time need
- * workspaces of their own.  1 <= split_k <= 8 (16 where the plan picks the
- * weight-streaming kernel, variant 6), split_k <= K / 64. */
+ * workspaces of their own.  1 <= split_k <= 8 (16 where the plan picks a
+ * weight-streaming kernel, variant 6 or 8), split_k <= K / 64. */
 size_t dfhip_gemm_bf16_splitk_workspace_bytes(int M, int N, int split_k);
 int dfhip_gemm_bf16_nt_splitk(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
                               int64_t ldc, int M, int N, int K, int split_k, void* workspace,
