@@ -37,6 +37,15 @@ struct KVFrags {
   bf16x8 v[8];      // [dim block]
 };
 
+// Four dims of a head of the output: item `it` is head it / 32, dims 4 (it % 32) .. + 3.
+DFHIP_DEVICE void store_row(uint16_t* out_row, int it, f32x4 num, float den) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) out_row[4 * it + e] = static_cast<uint16_t>(f32_to_bf16_bits(num[e] / den));
+}
+
+// 16-byte words of a part's block in the workspace: the sums of `group` heads, then one word (maximum, sum) per head.
+__host__ __device__ constexpr int part_block(int group) { return group * (HD / 4 + 1); }
+
 // One workgroup per (token, kv head).  Wave w takes the chunks w, w+4, ... of 32 positions.
 // MFMA row i of a score tile is mapped to position 8*(i/4) + i%4 (+4 for the second tile of the
 // chunk), so that after the two tiles lane (head = lane%16, g = lane/16) holds the scores of its
@@ -49,27 +58,36 @@ struct KVFrags {
 // fragments of that position, which it patches when it gets there (no read of what was just written and no
 // barrier: the wave that wrote the LDS words is the one that reads them; the other three waves only rotate their
 // copies of the query heads).
-template <bool APPEND>
+//
+// SPLIT: a (token, kv head) pair has `parts` workgroups, each with its share of the token's chunks, for launches with too
+// few pairs to fill the chip (attention_parts says when).  A part leaves its unnormalised sums, maximum and sum of exponentials in `partials`
+// ([pair][part][part_block(group)] words of 16 bytes), counts itself in and is done; the part that arrives last combines
+// them, in the same order whoever that is.
+template <bool APPEND, bool SPLIT>
 __global__ void __launch_bounds__(DEC_THREADS)
 decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* __restrict__ kc,
                         uint16_t* __restrict__ vc, const int32_t* __restrict__ slots,
                         const int32_t* __restrict__ lengths, uint16_t* __restrict__ out, int64_t ld_out,
                         int kv_heads, int group, int num_slots, int capacity, float scale_log2,
-                        const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table_rows) {
+                        const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table_rows, int parts,
+                        float* __restrict__ partials, int* __restrict__ arrivals) {
   // partial results of the four waves, sized by the launch for the real group (a workgroup that asks for
   // little LDS leaves room for a GEMM workgroup of the other nano-batch on the same CU)
   extern __shared__ __attribute__((aligned(16))) float combine_lds[];
   float* const o_lds = combine_lds;                       // [4][group][HD]
   float* const m_lds = combine_lds + 4 * group * HD;      // [4][group]
   float* const l_lds = m_lds + 4 * group;                 // [4][group]
-  const int t = blockIdx.x / kv_heads, kvh = blockIdx.x - t * kv_heads;
+  const int pair = SPLIT ? blockIdx.x / parts : blockIdx.x;
+  const int part = SPLIT ? blockIdx.x - pair * parts : 0;
+  const int t = pair / kv_heads, kvh = pair - t * kv_heads;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hq = lane & 15, g = lane >> 4;
   const int slot = slots[t];
   int len = lengths[t];
   uint16_t* out_row = out + (int64_t)t * ld_out + (int64_t)kvh * group * HD;
   if (slot < 0 || slot >= num_slots || len < 1) {   // nothing to attend to: defined output, no access
-    for (int idx = tid; idx < group * HD; idx += DEC_THREADS) out_row[idx] = 0;
+    if (part == 0)
+      for (int idx = tid; idx < group * HD; idx += DEC_THREADS) out_row[idx] = 0;
     return;
   }
   const int pos = len - 1;                     // APPEND: the new token's position (before the clamp below)
@@ -191,9 +209,11 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
   };
 
   // two fragment sets in turn: the loads of the next chunk are in flight while one is multiplied
-  const int chunks = (len + CHUNK - 1) / CHUNK;
+  const int all_chunks = (len + CHUNK - 1) / CHUNK;
+  const int chunk0 = SPLIT ? (int)((int64_t)all_chunks * part / parts) : 0;
+  const int chunks = SPLIT ? (int)((int64_t)all_chunks * (part + 1) / parts) : all_chunks;   // end of this part's
   KVFrags fa, fb;
-  if (wave < chunks) load(fa, wave);
+  if (chunk0 + wave < chunks) load(fa, chunk0 + wave);
   // (the first chunk's loads are on their way while the query heads are rotated)
   if (APPEND) {
     // the lane's fragments ks and ks + 2 hold the two halves of the pairs i = 32 ks + 8 g + e, ks = 0, 1
@@ -211,7 +231,8 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
     // The wave whose chunks include the new position appends: lane i rotates the pair (i, i + 64) of the new key
     // and copies two elements of the new value - to the caches for the later steps, to LDS for this wave's own
     // fragments of that position (the same wave writes and reads them: no barrier).
-    if (append && wave == (pos / CHUNK) % 4) {
+    const int pos_chunk = pos / CHUNK;
+    if (append && pos_chunk >= chunk0 && pos_chunk < chunks && wave == (pos_chunk - chunk0) % 4) {
       const int q_heads = kv_heads * group;
       const uint16_t* k_in = token_row + (int64_t)(q_heads + kvh) * HD;
       const uint16_t* v_in = token_row + (int64_t)(q_heads + kv_heads + kvh) * HD;
@@ -230,7 +251,7 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
       }
     }
   }
-  for (int c = wave; c < chunks; c += 8) {
+  for (int c = chunk0 + wave; c < chunks; c += 8) {
     if (c + 4 < chunks) load(fb, c + 4);
     step(fa, c);
     if (c + 4 < chunks) {
@@ -253,19 +274,101 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
     l_lds[wave * group + hq] = l;
   }
   __syncthreads();
-  for (int idx = tid; idx < group * HD; idx += DEC_THREADS) {
-    const int h = idx >> 7, dim = idx & (HD - 1);
+  // a thread combines four dims of a head: items (head, dims 4 d .. 4 d + 3)
+  const int items = group * (HD / 4);
+  f32x4* const blocks = SPLIT ? reinterpret_cast<f32x4*>(partials) + (int64_t)pair * parts * part_block(group) : nullptr;
+  for (int it = tid; it < items; it += DEC_THREADS) {
+    const int h = it >> 5;
     float mm = m_lds[h];
 #pragma unroll
     for (int w = 1; w < 4; ++w) mm = fmaxf(mm, m_lds[w * group + h]);
-    float num = 0.0f, den = 0.0f;
+    f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
+    float den = 0.0f;
+    if (!SPLIT || mm > -INFINITY) {                         // (a part can be without a chunk, a token cannot)
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float f = exp2f(m_lds[w * group + h] - mm);   // 0 for a wave that had no chunk (m = -inf)
-      num += o_lds[(w * group + h) * HD + dim] * f;
-      den += l_lds[w * group + h] * f;
+      for (int w = 0; w < 4; ++w) {
+        const float f = exp2f(m_lds[w * group + h] - mm);   // 0 for a wave that had no chunk (m = -inf)
+        const f32x4 v = reinterpret_cast<const f32x4*>(o_lds)[w * items + it];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) num[e] += v[e] * f;
+        den += l_lds[w * group + h] * f;
+      }
     }
-    out_row[idx] = static_cast<uint16_t>(f32_to_bf16_bits(num / den));
+    if constexpr (SPLIT) {
+      f32x4* const mine = blocks + part * part_block(group);
+      store_f32x4_device_coherent(mine + it, num);
+      if ((it & 31) == 0) store_f32x4_device_coherent(mine + items + h, f32x4{mm, den, 0.0f, 0.0f});
+    } else {
+      store_row(out_row, it, num, den);
+    }
+  }
+  if constexpr (SPLIT) {
+    wait_vmcnt<0>();
+    __syncthreads();
+    int* const ticket_cell = reinterpret_cast<int*>(combine_lds);
+    if (tid == 0) *ticket_cell = atomicAdd(arrivals + pair, 1);
+    __syncthreads();
+    const int ticket = *ticket_cell;
+    __syncthreads();
+    if (ticket != parts - 1) return;
+    if (tid == 0) atomicExch(arrivals + pair, 0);
+    // Two threads share an item's parts (part q: thread q % 2) where there are threads enough; their sums meet in LDS,
+    // in the room of the waves' partial results.
+    const int lanes = 2 * items <= DEC_THREADS ? 2 : 1;
+    const int share = lanes > 1 ? tid / items : 0;
+    const int it0 = lanes > 1 ? tid - share * items : tid;
+    f32x4* const sums = reinterpret_cast<f32x4*>(combine_lds);          // [lanes][items] sums, then [lanes][items] (m, l)
+    if (share < lanes)
+      for (int it = it0; it < items; it += lanes > 1 ? items : DEC_THREADS) {
+        f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
+        float mm = -INFINITY, den = 0.0f;
+        for (int q0 = share; q0 < parts; q0 += 4 * lanes) {
+          f32x4 v[4], ml[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int q = q0 + c * lanes < parts ? q0 + c * lanes : q0;
+            v[c] = load_f32x4_device_coherent(blocks + q * part_block(group) + it);
+            ml[c] = load_f32x4_device_coherent(blocks + q * part_block(group) + items + (it >> 5));
+          }
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            wait_loaded(v[c]);
+            wait_loaded(ml[c]);
+          }
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            if (q0 + c * lanes >= parts || ml[c][0] == -INFINITY) continue;
+            const float m_new = fmaxf(mm, ml[c][0]);
+            const float keep = exp2f(mm - m_new), add = exp2f(ml[c][0] - m_new);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) num[e] = num[e] * keep + v[c][e] * add;
+            den = den * keep + ml[c][1] * add;
+            mm = m_new;
+          }
+        }
+        if (lanes > 1) {
+          sums[share * items + it] = num;
+          sums[(lanes + share) * items + it] = f32x4{mm, den, 0.0f, 0.0f};
+        } else {
+          store_row(out_row, it, num, den);
+        }
+      }
+    if (lanes > 1) {
+      __syncthreads();
+      if (tid < items) {
+        float mm = -INFINITY, den = 0.0f;
+        for (int c = 0; c < lanes; ++c) mm = fmaxf(mm, sums[(lanes + c) * items + tid][0]);
+        f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int c = 0; c < lanes; ++c) {
+          const f32x4 v = sums[c * items + tid], ml = sums[(lanes + c) * items + tid];
+          const float f = exp2f(ml[0] - mm);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) num[e] += v[e] * f;
+          den += ml[1] * f;
+        }
+        store_row(out_row, tid, num, den);
+      }
+    }
   }
 }
 
@@ -342,20 +445,36 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
   const float scale_log2 = scale * 1.4426950408889634f;
   const int group = q_heads / kv_heads;
   const size_t combine_bytes = (size_t)4 * group * (HD + 2) * sizeof(float);
-  hipLaunchKernelGGL(decode_attention_kernel<false>, dim3(T * kv_heads), dim3(DEC_THREADS), combine_bytes,
+  hipLaunchKernelGGL((decode_attention_kernel<false, false>), dim3(T * kv_heads), dim3(DEC_THREADS), combine_bytes,
                      static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(q), ld_q,
                      static_cast<uint16_t*>(const_cast<void*>(k_cache)), static_cast<uint16_t*>(const_cast<void*>(v_cache)),
                      slots, lengths, static_cast<uint16_t*>(out), ld_out, kv_heads, group, num_slots, capacity,
-                     scale_log2, nullptr, nullptr, 1);
+                     scale_log2, nullptr, nullptr, 1, 1, nullptr, nullptr);
   return dfhip_check_launch();
 }
 
-extern "C" int dfhip_decode_attention_append_bf16(const void* qkv, int64_t ld_qkv, void* k_cache, void* v_cache,
-                                                  const int32_t* slots, const int32_t* lengths,
-                                                  const float* cos_table, const float* sin_table, void* out,
-                                                  int64_t ld_out, int T, int q_heads, int kv_heads, int head_dim,
-                                                  int num_slots, int capacity, int table_rows, float scale,
-                                                  dfhip_stream_t stream) {
+// Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), with at least 256 positions of
+// a full cache each (two chunks per wave).  From 257 pairs on nothing is cut: the meeting of the parts costs about 10 us
+// of latency and an uncut launch fills the chip.  [us, uncut -> cut: 2 sequences of up to 8192 positions 111 -> 18
+// (their bytes at 6.7 TB/s: 8), 8 of 2048 33 -> 18 (10), 20 of up to 4096 68 -> 48 (32), 20 of 4096 74 -> 62 (50); 40 of
+// up to 1024 30 -> 30, 64 of 2048 87 -> 95, so those stay whole.]  The lengths are on the device: a short sequence in a
+// large cache is cut too finely rather than not at all, its parts without a chunk cost their start.
+static int attention_parts(int T, int kv_heads, int capacity) {
+  const int64_t pairs = (int64_t)T * kv_heads;
+  int64_t parts = 512 / pairs;
+  if (parts > capacity / 256) parts = capacity / 256;
+  if (parts > 32) parts = 32;
+  return parts < 1 ? 1 : (int)parts;
+}
+// The arrival counters at the start of the workspace: a launch that splits has at most 256 pairs, and the area is the same
+// for every shape, so that no launch's partial sums lie where another's counters are expected to be zero.
+constexpr size_t ATTENTION_COUNTER_BYTES = 4096;
+
+static int decode_attention_append(const void* qkv, int64_t ld_qkv, void* k_cache, void* v_cache, const int32_t* slots,
+                                   const int32_t* lengths, const float* cos_table, const float* sin_table, void* out,
+                                   int64_t ld_out, int T, int q_heads, int kv_heads, int head_dim, int num_slots,
+                                   int capacity, int table_rows, float scale, int parts, void* workspace,
+                                   dfhip_stream_t stream) {
   if (!qkv || !k_cache || !v_cache || !slots || !lengths || !cos_table || !sin_table || !out)
     return DFHIP_ERR_NULL_POINTER;
   if (T < 1 || q_heads < 1 || kv_heads < 1 || q_heads % kv_heads != 0 || q_heads / kv_heads > MAX_GROUP ||
@@ -367,10 +486,48 @@ extern "C" int dfhip_decode_attention_append_bf16(const void* qkv, int64_t ld_qk
     return DFHIP_ERR_BAD_ALIGNMENT;
   const int group = q_heads / kv_heads;
   const size_t lds_bytes = (size_t)4 * group * (HD + 2) * sizeof(float) + 2 * HD * sizeof(uint16_t);
-  hipLaunchKernelGGL(decode_attention_kernel<true>, dim3(T * kv_heads), dim3(DEC_THREADS), lds_bytes,
+  const auto kernel = parts > 1 ? decode_attention_kernel<true, true> : decode_attention_kernel<true, false>;
+  float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + ATTENTION_COUNTER_BYTES);
+  hipLaunchKernelGGL(kernel, dim3(T * kv_heads * parts), dim3(DEC_THREADS), lds_bytes,
                      static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(qkv), ld_qkv,
                      static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), slots, lengths,
                      static_cast<uint16_t*>(out), ld_out, kv_heads, group, num_slots, capacity,
-                     scale * 1.4426950408889634f, cos_table, sin_table, table_rows);
+                     scale * 1.4426950408889634f, cos_table, sin_table, table_rows, parts,
+                     parts > 1 ? partials : nullptr, static_cast<int*>(workspace));
   return dfhip_check_launch();
+}
+
+extern "C" int dfhip_decode_attention_append_bf16(const void* qkv, int64_t ld_qkv, void* k_cache, void* v_cache,
+                                                  const int32_t* slots, const int32_t* lengths,
+                                                  const float* cos_table, const float* sin_table, void* out,
+                                                  int64_t ld_out, int T, int q_heads, int kv_heads, int head_dim,
+                                                  int num_slots, int capacity, int table_rows, float scale,
+                                                  dfhip_stream_t stream) {
+  return decode_attention_append(qkv, ld_qkv, k_cache, v_cache, slots, lengths, cos_table, sin_table, out, ld_out, T,
+                                 q_heads, kv_heads, head_dim, num_slots, capacity, table_rows, scale, 1, nullptr, stream);
+}
+
+extern "C" size_t dfhip_decode_attention_workspace_bytes(int T, int q_heads, int kv_heads, int capacity) {
+  if (T < 1 || kv_heads < 1 || q_heads < kv_heads || capacity < 1) return 0;
+  const int parts = attention_parts(T, kv_heads, capacity);
+  if (parts < 2) return 0;
+  return ATTENTION_COUNTER_BYTES +
+         (size_t)T * kv_heads * parts * part_block(q_heads / kv_heads) * 16;
+}
+
+extern "C" int dfhip_decode_attention_append_split_bf16(
+    const void* qkv, int64_t ld_qkv, void* k_cache, void* v_cache, const int32_t* slots, const int32_t* lengths,
+    const float* cos_table, const float* sin_table, void* out, int64_t ld_out, int T, int q_heads, int kv_heads,
+    int head_dim, int num_slots, int capacity, int table_rows, float scale, void* workspace, size_t workspace_bytes,
+    dfhip_stream_t stream) {
+  const size_t need = dfhip_decode_attention_workspace_bytes(T, q_heads, kv_heads, capacity);
+  if (need > 0) {
+    if (!workspace) return DFHIP_ERR_NULL_POINTER;
+    if (!dfhip_aligned16(workspace)) return DFHIP_ERR_BAD_ALIGNMENT;
+    if (workspace_bytes < need) return DFHIP_ERR_BAD_ARGUMENT;
+  }
+  const int parts = need > 0 ? attention_parts(T, kv_heads, capacity) : 1;
+  return decode_attention_append(qkv, ld_qkv, k_cache, v_cache, slots, lengths, cos_table, sin_table, out, ld_out, T,
+                                 q_heads, kv_heads, head_dim, num_slots, capacity, table_rows, scale, parts, workspace,
+                                 stream);
 }

@@ -142,5 +142,12 @@ DFHIP_DEVICE f32x4 load_f32x4_device_coherent(const f32x4* p) {
 // be used after this, which ties the wait to the register so that the use cannot move above it.
 DFHIP_DEVICE void wait_loaded(f32x4& v) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(v)::"memory"); }
 
+// one float, coherent across the XCDs
+DFHIP_DEVICE void store_device_coherent(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+DFHIP_DEVICE float load_device_coherent(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 DFHIP_DEVICE void workgroup_barrier() { asm volatile("s_barrier" ::: "memory"); }
 #define DFHIP_PIN __builtin_amdgcn_sched_barrier(0)

@@ -619,6 +619,10 @@ torch.library.register_fake("dynaflow_hip::causal_attention", lambda q, k, v: to
 
 
 # ------------------------------------------------------- decode attention
+#: partial sums and arrival counters of attention launches whose positions are cut, kept like the split-K workspaces
+_attention_workspaces: dict[tuple, torch.Tensor] = {}
+
+
 def _decode_attention_impl(qkv, k_cache, v_cache, slots, lengths, cos, sin, q_heads: int, kv_heads: int):
     """RoPE + cache append + attention of one new token per sequence (see ``dynaflow_amd.decode``).
 
@@ -645,13 +649,17 @@ def _decode_attention_impl(qkv, k_cache, v_cache, slots, lengths, cos, sin, q_he
     slots, lengths, cos, sin = slots.contiguous(), lengths.contiguous(), cos.contiguous(), sin.contiguous()
     out = torch.empty((T, q_heads * d), dtype=qkv.dtype, device=qkv.device)
     if T > 0:
-        # rotation, cache append and attention in one launch
-        rc = lib.dfhip_decode_attention_append_bf16(
+        # rotation, cache append and attention in one launch; few sequences: several workgroups per head
+        stream = _stream()
+        nbytes = lib.dfhip_decode_attention_workspace_bytes(T, q_heads, kv_heads, capacity)
+        ws = _zeroed_workspace(_attention_workspaces, qkv.device, stream, nbytes) if nbytes else None
+        rc = lib.dfhip_decode_attention_append_split_bf16(
             qkv.data_ptr(), qkv.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), slots.data_ptr(),
             lengths.data_ptr(), cos.data_ptr(), sin.data_ptr(), out.data_ptr(), q_heads * d, T, q_heads, kv_heads, d,
-            num_slots, capacity, cos.shape[0], 1.0 / math.sqrt(d), _stream(),
+            num_slots, capacity, cos.shape[0], 1.0 / math.sqrt(d), ws.data_ptr() if nbytes else None,
+            ws.numel() if nbytes else 0, stream,
         )
-        _cabi.check("dfhip_decode_attention_append_bf16", rc)
+        _cabi.check("dfhip_decode_attention_append_split_bf16", rc)
     return out
 
 

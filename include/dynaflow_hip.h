@@ -341,6 +341,21 @@ int dfhip_decode_attention_append_bf16(const void* qkv, int64_t ld_qkv, void* k_
                                        int kv_heads, int head_dim, int num_slots, int capacity, int table_rows,
                                        float scale, dfhip_stream_t stream);
 
+/* dfhip_decode_attention_append_bf16 for a step with few sequences: where T * kv_heads is too small to fill the chip, the
+ * positions of a sequence are cut into parts (as many as T, kv_heads and capacity give) whose partial sums meet in
+ * `workspace` (device memory, 16-byte aligned, at least dfhip_decode_attention_workspace_bytes; that is 0, and the
+ * workspace may be null, where nothing is cut).  The workspace starts with arrival counters that must be zero before the
+ * first use and are left zero; launches that may overlap in time need workspaces of their own.  The parts are combined
+ * in a fixed order: the same bits in every run, but for a cut launch not those of the uncut one.  (The same node of the
+ * host framework as above, examples/ae/scheduler/vllm/nanoflow.py:89-95.) */
+size_t dfhip_decode_attention_workspace_bytes(int T, int q_heads, int kv_heads, int capacity);
+int dfhip_decode_attention_append_split_bf16(const void* qkv, int64_t ld_qkv, void* k_cache, void* v_cache,
+                                             const int32_t* slots, const int32_t* lengths, const float* cos_table,
+                                             const float* sin_table, void* out, int64_t ld_out, int T, int q_heads,
+                                             int kv_heads, int head_dim, int num_slots, int capacity, int table_rows,
+                                             float scale, void* workspace, size_t workspace_bytes,
+                                             dfhip_stream_t stream);
+
 /* out[N,K] = in[K,N]^T for bf16 matrices: packs a weight kept as [in, out]
  * (x @ W convention) into the [out, in] layout the GEMMs read.  K, N % 8 == 0.  No counterpart in the
  * reference (torch.nn.functional.linear takes [out, in] weights as they are): a set-up helper. */

@@ -163,6 +163,49 @@ def test_one_launch_decode_attention_has_the_bits_of_the_two_launches(heads, kv_
     assert torch.isfinite(out_one.float()).all()
 
 
+@pytest.mark.parametrize("heads,kv_heads,capacity,lengths", [
+    (32, 8, 512, [1, 512, 33, 256]),                 # two parts: one position, the cut on and beside a chunk's edge
+    (4, 1, 8192, [8192, 1, 300]),                    # 32 parts, most of them without a chunk for the short ones
+    (16, 1, 4096, [4095, 2049, 7, 65]),              # 16 query heads on one kv head
+    (3, 3, 1024, [1024, 31, 513] * 7),               # no grouping
+    (32, 8, 2048, [2048 - 31 * i for i in range(32)]),   # the most pairs that are still cut
+])
+def test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, lengths):
+    """Few (token, kv head) pairs: several workgroups share a token's positions and the last to arrive combines them.
+    Against the uncut launch of the same inputs (which the tests above hold to the oracle; two bf16 roundings of the
+    output apart: 2^-7 of the largest value), the same caches, the same bits in every run and counters left at zero."""
+    import math
+
+    from dynaflow_amd import _cabi
+    from dynaflow_amd.decoder import rope_tables
+
+    lib = _cabi.load()
+    T, slots_n = len(lengths), len(lengths) + 1
+    assert lib.dfhip_decode_attention_workspace_bytes(T, heads, kv_heads, capacity) > 0
+    g = torch.Generator(device="cuda").manual_seed(capacity)
+    qkv = torch.randn(T, (heads + 2 * kv_heads) * D, generator=g, device="cuda").bfloat16()
+    slots = torch.randperm(slots_n, generator=g, device="cuda")[:T].int()
+    lens = torch.tensor(lengths, dtype=torch.int32, device="cuda")
+    cos, sin = (t.cuda() for t in rope_tables(capacity, D, 500000.0))
+    k0 = torch.randn(slots_n, kv_heads, capacity, D, generator=g, device="cuda").bfloat16()
+    v0 = torch.randn(slots_n, kv_heads, capacity // 8, D, 8, generator=g, device="cuda").bfloat16()
+    k1, v1 = k0.clone(), v0.clone()
+    want = torch.empty(T, heads * D, dtype=torch.bfloat16, device="cuda")
+    _cabi.check("append", lib.dfhip_decode_attention_append_bf16(
+        qkv.data_ptr(), qkv.stride(0), k1.data_ptr(), v1.data_ptr(), slots.data_ptr(), lens.data_ptr(), cos.data_ptr(),
+        sin.data_ptr(), want.data_ptr(), heads * D, T, heads, kv_heads, D, slots_n, capacity, capacity,
+        1.0 / math.sqrt(D), torch.cuda.current_stream().cuda_stream))
+    outs = []
+    for _ in range(3):
+        k2, v2 = k0.clone(), v0.clone()
+        outs.append(ops.decode_attention(qkv, k2, v2, slots, lens, cos, sin, heads, kv_heads))
+        assert torch.equal(k2, k1) and torch.equal(v2, v1)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert rel_err(outs[0], want) < 2 ** -7
+    for ws in ops._attention_workspaces.values():
+        assert int(ws[:4096].view(torch.int32).abs().sum()) == 0
+
+
 def test_decode_attention_ignores_what_lies_past_the_length(ops):
     """Caches are usually allocated uninitialised or hold recycled slots: NaN and Inf patterns in positions
     from lengths[t] on (keys and values) must not reach the output, and the result is the one a cache with
