@@ -1,10 +1,12 @@
-// fp32 GEMM for gfx950:  C[M,N] = A[M,K] * W[N,K]^T with v_mfma_f32_32x32x2_f32.
+// fp32 GEMM for gfx950:  C[M,N] = A[M,K] * W[N,K]^T.
 //
-// Serves the small fp32 configuration, where agreement with an fp32 host
-// result to 1e-5 matters and speed does not: a 128x128 tile per workgroup,
-// K walked in slabs of 16 through one LDS buffer.  LDS rows hold 16 floats
-// padded to 17 so that the 32 lanes of a fragment read (one float each, rows
-// 17 words apart) hit 32 different banks.
+// gemm_f32_split_kernel (v_mfma_f32_16x16x4_f32, the kernel of the small fp32 configuration): a few 16 x 16 blocks of C
+//   per workgroup so that a small product still has a workgroup for every compute unit; its four waves share the blocks
+//   and take the 128-byte slabs of K in turn, operands go straight from memory (L2) to registers, and the four partial
+//   sums meet in LDS.  Bound by the matrix pipes' fp32 rate and, at these sizes, by how evenly the blocks fall.
+// gemm_f32_nt_kernel (v_mfma_f32_32x32x2_f32, any K that is a multiple of 4): a 128x128 tile per workgroup, K walked in
+//   slabs of 16 through one LDS buffer.  LDS rows hold 16 floats padded to 17 so that the 32 lanes of a fragment read
+//   (one float each, rows 17 words apart) hit 32 different banks.
 #include "dfhip_common.h"
 
 namespace {
@@ -84,6 +86,161 @@ gemm_f32_nt_kernel(const float* __restrict__ A, const float* __restrict__ W, flo
   }
 }
 
+// A tile of MB x NB blocks of 16 x 16.  A lane loads 16 bytes of a row, k = 4 (lane / 16) + e of the 16 floats of half a
+// slab; the e-th MFMA takes element e of both operands, so four MFMAs cover the 16 floats (each sums its own quarter of
+// them: the same order of k for both operands is all that matters).
+constexpr int SWAVES = 4;
+
+template <int MB, int NB, int SDEPTH>
+__global__ void __launch_bounds__(SWAVES * 64)
+gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
+                      int slabs, int64_t lda, int64_t ldw, int64_t ldc, int tiles_m) {
+  __shared__ f32x4 sums[SWAVES * MB * NB * 64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = lane & 15, quad = lane >> 4;
+  const int m0 = (int)(blockIdx.x % tiles_m) * (16 * MB), n0 = (int)(blockIdx.x / tiles_m) * (16 * NB);
+  const float* a_ptr[MB];
+  const float* w_ptr[NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    int m = m0 + 16 * i + row; m = m < M ? m : M - 1;        // rows past the edge re-read the last one; never stored
+    a_ptr[i] = A + (int64_t)m * lda + wave * 32 + quad * 4;
+  }
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    int n = n0 + 16 * j + row; n = n < N ? n : N - 1;
+    w_ptr[j] = W + (int64_t)n * ldw + wave * 32 + quad * 4;
+  }
+  const int n_slabs = (slabs - wave + SWAVES - 1) / SWAVES;   // >= SDEPTH (checked by the launch)
+
+  f32x4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 af[SDEPTH][MB][2], wf[SDEPTH][NB][2];
+  auto load = [&](int d, int s) {
+    const int off = s * (SWAVES * 32);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) af[d][i][h] = *reinterpret_cast<const f32x4*>(a_ptr[i] + off + h * 16);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) wf[d][j][h] = *reinterpret_cast<const f32x4*>(w_ptr[j] + off + h * 16);
+    }
+  };
+  auto multiply = [&](int d) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[d][j][h][e], af[d][i][h][e], acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int d = 0; d < SDEPTH; ++d) load(d, d);
+  int s = 0;
+  for (; s + 2 * SDEPTH <= n_slabs; s += SDEPTH) {
+#pragma unroll
+    for (int d = 0; d < SDEPTH; ++d) {
+      multiply(d);
+      load(d, s + SDEPTH + d);
+      DFHIP_PIN;
+    }
+  }
+  const int rest = n_slabs - s - SDEPTH;                      // 0 .. SDEPTH - 1
+#pragma unroll
+  for (int d = 0; d < SDEPTH; ++d) {
+    multiply(d);
+    if (d < rest) load(d, s + SDEPTH + d);
+  }
+#pragma unroll
+  for (int d = 0; d < SDEPTH - 1; ++d)
+    if (d < rest) multiply(d);
+
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) sums[((wave * MB + i) * NB + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  // W was the first operand: item (i, j, l) is row 16 i + l % 16, columns 16 j + 4 (l / 16) .. + 3
+  const bool whole = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
+  for (int item = tid; item < MB * NB * 64; item += SWAVES * 64) {
+    f32x4 v = sums[item];
+#pragma unroll
+    for (int w = 1; w < SWAVES; ++w) v += sums[w * (MB * NB * 64) + item];
+    const int l = item & 63, i = (item >> 6) / NB, j = (item >> 6) % NB;
+    const int m = m0 + 16 * i + (l & 15), n = n0 + 16 * j + 4 * (l >> 4);
+    if (m >= M) continue;
+    float* c = C + (int64_t)m * ldc + n;
+    if (whole && n + 4 <= N) {
+      *reinterpret_cast<f32x4*>(c) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) c[e] = v[e];
+    }
+  }
+}
+
+struct F32Args {
+  const float *A, *W;
+  float* C;
+  int M, N, K;
+  int64_t lda, ldw, ldc;
+};
+
+int64_t split_tiles(const F32Args& p, int mb, int nb) {
+  return (int64_t)((p.M + 16 * mb - 1) / (16 * mb)) * ((p.N + 16 * nb - 1) / (16 * nb));
+}
+
+template <int MB, int NB, int DEPTH>
+int launch_split(const F32Args& p, hipStream_t stream) {
+  hipLaunchKernelGGL((gemm_f32_split_kernel<MB, NB, DEPTH>), dim3((unsigned)split_tiles(p, MB, NB)), dim3(SWAVES * 64), 0,
+                     stream, p.A, p.W, p.C, p.M, p.N, p.K / 32, p.lda, p.ldw, p.ldc, (p.M + 16 * MB - 1) / (16 * MB));
+  return dfhip_check_launch();
+}
+// Two slabs in flight per wave while the tiles fit one round of workgroups, four beyond that (several workgroups follow
+// each other on a compute unit and their loads cost more than their registers: 256 x 5632 x 2048 77 -> 62 us, 1024 x 2048
+// x 5632 264 -> 178, but 256 x 2816 x 1024, one round, 18 -> 20).
+template <int MB, int NB>
+int launch_deep(const F32Args& p, hipStream_t stream) {
+  if (p.K >= 512 && split_tiles(p, MB, NB) > 256) return launch_split<MB, NB, 4>(p, stream);
+  return launch_split<MB, NB, 2>(p, stream);
+}
+
+// Smallest tile for which a wave's share of K has two slabs in flight.
+constexpr int SPLIT_MIN_K = 32 * SWAVES * 2;
+
+// The tile whose rounds of 256 workgroups take the least: a round costs its blocks and about 1.5 blocks' worth of start,
+// loads and meeting.  [us at [128 x 1024] x [2816 x 1024]^T / [128 x 2816] x [1024 x 2816]^T, with the workgroups in
+// parentheses: 2 x 3 blocks 12.4 (236) / 27.5 (88), 4 x 2 14.9 (176) / 32.7 (64), 2 x 2 17.2 (352) / 22.2 (128), 2 x 1
+// 18.4 (704) / 16.9 (256); the 128 x 128 tiles used before 105 (22) / 274 (8).  Floor at the fp32 rate: 4.9.]
+int launch_f32(const F32Args& p, hipStream_t stream) {
+  constexpr int SHAPES[8][2] = {{4, 4}, {4, 3}, {4, 2}, {2, 3}, {2, 2}, {2, 1}, {1, 2}, {1, 1}};
+  int best = 0;
+  double least = 0.0;
+  for (int i = 0; i < 8; ++i) {
+    const int64_t rounds = (split_tiles(p, SHAPES[i][0], SHAPES[i][1]) + 255) / 256;
+    const double cost = (double)rounds * (SHAPES[i][0] * SHAPES[i][1] + 1.5);
+    if (i == 0 || cost < least) { best = i; least = cost; }
+  }
+  switch (best) {
+    case 0: return launch_deep<4, 4>(p, stream);
+    case 1: return launch_deep<4, 3>(p, stream);
+    case 2: return launch_deep<4, 2>(p, stream);
+    case 3: return launch_split<2, 3, 2>(p, stream);
+    case 4: return launch_split<2, 2, 2>(p, stream);
+    case 5: return launch_split<2, 1, 2>(p, stream);
+    case 6: return launch_split<1, 2, 2>(p, stream);
+    default: return launch_split<1, 1, 2>(p, stream);
+  }
+}
+
 }  // namespace
 
 extern "C" int dfhip_gemm_f32_nt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
@@ -94,6 +251,9 @@ extern "C" int dfhip_gemm_f32_nt(const void* A, int64_t lda, const void* W, int6
   if (lda % 4 || ldw % 4 || !dfhip_aligned16(A) || !dfhip_aligned16(W) ||
       (reinterpret_cast<uintptr_t>(C) & 3u))
     return DFHIP_ERR_BAD_ALIGNMENT;
+  if (K % 32 == 0 && K >= SPLIT_MIN_K)
+    return launch_f32({static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N, K, lda,
+                       ldw, ldc}, static_cast<hipStream_t>(stream));
   dim3 grid((N + FBN - 1) / FBN, (M + FBM - 1) / FBM);
   hipLaunchKernelGGL(gemm_f32_nt_kernel, grid, dim3(FTHREADS), 0, static_cast<hipStream_t>(stream),
                      static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N,

@@ -1,0 +1,25 @@
+"""The fp32 GEMM over its tile shapes, through the operator."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# one shape or more for each tile the cost rule picks (1 x 1 .. 4 x 4 blocks, one round of workgroups and several), ragged
+# rows and columns, outputs whose rows are not 16-byte aligned (N = 7, 2815), K at the edges of the split kernel's range:
+# 224 (below it), 252 and 260 (no whole slabs), 256 (two slabs a wave), 288 and 544 (an uneven share)
+@pytest.mark.parametrize("M,N,K", [(1, 1, 256), (5, 7, 288), (16, 2816, 256), (17, 33, 544), (50, 2815, 1024),
+                                   (128, 1024, 2816), (128, 2816, 1024), (131, 2816, 512), (128, 5632, 288),
+                                   (256, 5632, 512), (300, 2000, 544), (1000, 2047, 256), (1024, 5632, 512),
+                                   (64, 64, 224), (64, 64, 252), (70, 65, 260)])
+def test_gemm_f32_tiles(M, N, K):
+    """|error| <= K 2^-24 (|A| |W|^T) element by element: what any order of K fp32 products and sums stays within."""
+    from dynaflow_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda")
+    got = ops.linear(a, w)
+    bound = K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
+    assert bool(((got.double() - a.double() @ w.double().t()).abs() <= bound).all())
+    assert torch.equal(ops.linear(a, w), got)
