@@ -24,6 +24,7 @@ import asyncio
 from abc import ABC, abstractmethod
 from collections.abc import Callable
 from dataclasses import dataclass
+from typing import Any
 
 from dynaflow_amd.matching import MatchingRule
 
@@ -108,17 +109,20 @@ class OperatorHandle:
 
 
 class ExecutionContext:
-    """The two queues a scheduler talks to the engine through."""
+    """What a scheduler talks to the engine through: a forward that it drives directly (``forward``, an object with
+    ``next_operator`` and ``launch``), or two queues with an engine coroutine at their other end."""
 
     def __init__(
         self,
         split_config: SplitConfig,
-        op_queue: dict[int, asyncio.Queue],
-        execute_queue: asyncio.Queue,
+        op_queue: dict[int, asyncio.Queue] | None = None,
+        execute_queue: asyncio.Queue | None = None,
+        forward: Any = None,
     ) -> None:
         self._split_config = split_config
         self._op_queue = op_queue
         self._execute_queue = execute_queue
+        self._forward = forward
 
     @property
     def split_config(self) -> SplitConfig:
@@ -126,6 +130,8 @@ class ExecutionContext:
 
     async def pop(self, batch_idx: int) -> OperatorHandle | None:
         """Next ready operator of ``batch_idx``; ``None`` when it is finished."""
+        if self._forward is not None:
+            return await self._forward.next_operator(batch_idx)
         return await self._op_queue[batch_idx].get()
 
     async def execute(
@@ -140,6 +146,9 @@ class ExecutionContext:
         sub-graph would.  The reference's callers always pass a 1-tuple
         (dynaflow/runtime/engine.py:296-299); a bare handle is accepted too.
         """
+        if self._forward is not None:
+            self._forward.launch(operator, func)
+            return
         if isinstance(operator, OperatorHandle):
             operator = (operator,)
         finished = asyncio.Event()

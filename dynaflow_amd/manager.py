@@ -6,10 +6,10 @@
 ``prepare`` / ``override_split_config`` (manager.py:114-159)  store the
                 ``SplitConfig`` of the *next* forward; every forward consumes it.
 ``get_callable`` (manager.py:161-190) the synchronous forward: one nano-batch
-                takes the scheduler-free fast path, otherwise engine and
-                scheduler coroutines run side by side in a fresh event loop,
-                the caller's stream waits for every nano-batch's tail event and
-                the per-nano-batch outputs are concatenated on dim 0
+                takes the scheduler-free fast path, otherwise the scheduler
+                coroutine runs in this thread's event loop and drives the
+                forward, the caller's stream waits for every nano-batch's tail
+                event and the per-nano-batch outputs are concatenated on dim 0
                 (manager.py:192-261).
 
 On top of that, ``additional_config["whole_graph"]`` turns on whole-schedule
@@ -21,7 +21,6 @@ scheduler and all launches.
 """
 from __future__ import annotations
 
-import asyncio
 import logging
 import os
 import tempfile
@@ -38,6 +37,7 @@ from dynaflow_amd.matching import split_graph, tag_graph
 from dynaflow_amd.runtime import capture_plan
 from dynaflow_amd.runtime.device import get_device, stream_key
 from dynaflow_amd.runtime.engine import DynaFlowEngine
+from dynaflow_amd.runtime.loop import run_coroutine
 
 log = logging.getLogger("dynaflow")
 if os.environ.get("DYNAFLOW_VERBOSE"):
@@ -220,32 +220,26 @@ class DynaFlowManager:
                     return self.engine.execute_single_batch(split, args, kwargs)
                 if self._wants_whole_graph(split):
                     return self._forward_whole_graph(split, args, kwargs)
-                return asyncio.run(self._forward_async(args, kwargs))
+                return run_coroutine(self._forward_async(args, kwargs, split))
             finally:
                 self.cached_config = None
 
         return _forward
 
     async def _forward_async(self, args: tuple, kwargs: dict, split: SplitConfig | None = None) -> Any:
-        """Engine and scheduler side by side; join and concatenate at the end."""
+        """A forward under the scheduler's control; join and concatenate at the end."""
         split = split if split is not None else self.cached_config
         assert self.initialized and self.engine is not None and self.scheduler is not None
         assert split is not None
-        lanes = split.num_nano_batches
-        op_queue = {b: asyncio.Queue(maxsize=10) for b in range(lanes)}
-        execute_queue: asyncio.Queue = asyncio.Queue()
-        context = ExecutionContext(split, op_queue, execute_queue)
-
         from dynaflow_amd import ops
 
         with ops.launch_options(side_by_side=self.launches_side_by_side(split)):
             if split.is_dryrun:
                 results, events = self.engine.dryrun(args, kwargs, split)
             else:
-                (results, events), _ = await asyncio.gather(
-                    self.engine.execute(args, kwargs, op_queue, execute_queue, split),
-                    self.scheduler.schedule(context),
-                )
+                forward = self.engine.begin(args, split)
+                await self.scheduler.schedule(ExecutionContext(split, forward=forward))
+                results, events = await forward.completed()
         # the caller's stream continues only after every nano-batch's last launch
         for event in events:
             event.wait()
@@ -327,7 +321,7 @@ class DynaFlowManager:
             device = get_device()
             device.trace = []
             try:
-                asyncio.run(self._forward_async(args, kwargs, eager_split))
+                run_coroutine(self._forward_async(args, kwargs, eager_split))
             finally:
                 event_log, device.trace = device.trace, None
             caller = stream_key(torch.cuda.current_stream())
@@ -344,7 +338,7 @@ class DynaFlowManager:
             # stream of the schedule that the others meet at
             capture_on = {} if origin == caller else {"stream": device.streams_seen[origin]}
             with torch.cuda.graph(graph, **capture_on):
-                output = asyncio.run(self._forward_async(args, kwargs, eager_split))
+                output = run_coroutine(self._forward_async(args, kwargs, eager_split))
             self.capture_origins[key] = "caller" if origin == caller else "schedule"
             entry = _ScheduleGraph(graph, list(args), self._token_shaped_flags(args), output)
             self._schedule_graphs[key] = entry

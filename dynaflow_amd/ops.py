@@ -29,6 +29,9 @@ import threading
 import torch
 
 from dynaflow_amd import _cabi
+from dynaflow_amd.interface import OperatorHandle
+from dynaflow_amd.runtime.device import current_stream, current_stream_key
+from dynaflow_amd.runtime.env import peek_op_handle
 
 _lib = torch.library.Library("dynaflow_hip", "DEF")
 
@@ -65,7 +68,7 @@ FP8_MAX = 448.0
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return current_stream_key()[1]
 
 
 def _rows(t: torch.Tensor) -> tuple[torch.Tensor, int, int, int]:
@@ -132,9 +135,6 @@ def _zeroed_workspace(cache: dict, device: torch.device, stream: int, nbytes: in
     eager launch (the warm-up that precedes every capture) serves the captured launches of the same
     nano-batch as it is: no allocation and no clearing inside the graph.
     """
-    from dynaflow_amd.interface import OperatorHandle
-    from dynaflow_amd.runtime.env import peek_op_handle
-
     handle = peek_op_handle()
     if isinstance(handle, OperatorHandle):
         key = (device.index or 0, "nano-batch", handle._owner, handle.batch_idx)
@@ -157,7 +157,7 @@ def _zeroed_workspace(cache: dict, device: torch.device, stream: int, nbytes: in
         if ws.data_ptr() in _captured_workspaces:
             _retired_workspaces.append(ws)
         else:
-            ws.record_stream(torch.cuda.current_stream())   # launches already queued on this stream still use it
+            ws.record_stream(current_stream())   # launches already queued on this stream still use it
     ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
     cache[key] = ws
     return ws

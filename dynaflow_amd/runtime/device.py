@@ -104,6 +104,54 @@ def stream_key(stream: "torch.cuda.Stream") -> tuple[int, int]:
     return (stream.device_index, stream.cuda_stream)
 
 
+def current_stream_key() -> tuple[int, int]:
+    """``stream_key(torch.cuda.current_stream())`` without making a stream object (a launch asks several times)."""
+    index = torch._C._cuda_getDevice()
+    return (index, torch._C._cuda_getCurrentRawStream(index))
+
+
+#: one stream object per stream that has been current here; the object only names the stream
+_stream_objects: dict[tuple[int, int], "torch.cuda.Stream"] = {}
+
+
+def current_stream() -> "torch.cuda.Stream":
+    key = current_stream_key()
+    stream = _stream_objects.get(key)
+    if stream is None:
+        stream = _stream_objects[key] = torch.cuda.current_stream()
+    return stream
+
+
+class _CurrentStream:
+    """``torch.cuda.stream`` for a stream of the current device."""
+
+    __slots__ = ("_stream", "_previous")
+
+    def __init__(self, stream: "torch.cuda.Stream") -> None:
+        self._stream = stream
+
+    def __enter__(self) -> "torch.cuda.Stream":
+        self._previous = current_stream()
+        torch.cuda.set_stream(self._stream)
+        return self._stream
+
+    def __exit__(self, *exc) -> None:
+        torch.cuda.set_stream(self._previous)
+
+
+class _Range:
+    __slots__ = ("_name",)
+
+    def __init__(self, name: str) -> None:
+        self._name = name
+
+    def __enter__(self) -> None:
+        torch.cuda.nvtx.range_push(self._name)
+
+    def __exit__(self, *exc) -> None:
+        torch.cuda.nvtx.range_pop()
+
+
 class HipEvent:
     """A HIP event that knows the stream it was recorded on.
 
@@ -123,18 +171,18 @@ class HipEvent:
         self._recorded_on: tuple[int, int] | None = None
 
     def record(self, stream: "torch.cuda.Stream | None" = None) -> None:
-        stream = stream if stream is not None else torch.cuda.current_stream()
+        stream = stream if stream is not None else current_stream()
         self._recorded_on = stream_key(stream)
         self._owner.note(("record", self.uid, self._recorded_on), stream)
         self._event.record(stream)
 
     def wait(self, stream: "torch.cuda.Stream | None" = None) -> None:
-        stream = stream if stream is not None else torch.cuda.current_stream()
-        key = stream_key(stream)
-        self._owner.note(("wait", self.uid, key), stream)
+        key = stream_key(stream) if stream is not None else current_stream_key()
+        if self._owner.trace is not None:
+            self._owner.note(("wait", self.uid, key), stream if stream is not None else current_stream())
         if self._recorded_on is None or key == self._recorded_on:
             return
-        self._event.wait(stream)
+        self._event.wait(stream if stream is not None else current_stream())
 
     def synchronize(self) -> None:
         self._event.synchronize()
@@ -203,18 +251,15 @@ class HipDevice:
         return torch.cuda.ExternalStream(_masked_stream(cu_mask))
 
     def current_stream(self) -> "torch.cuda.Stream":
-        return torch.cuda.current_stream()
+        return current_stream()
 
     def stream(self, stream: "torch.cuda.Stream"):
-        return torch.cuda.stream(stream)
+        if stream.device_index != torch._C._cuda_getDevice():
+            return torch.cuda.stream(stream)
+        return _CurrentStream(stream)
 
-    @contextlib.contextmanager
     def range(self, name: str):
-        torch.cuda.nvtx.range_push(name)
-        try:
-            yield
-        finally:
-            torch.cuda.nvtx.range_pop()
+        return _Range(name)
 
 
 _device: HostDevice | HipDevice | None = None

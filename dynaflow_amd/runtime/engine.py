@@ -68,6 +68,7 @@ class _SharedOutput:
     def __init__(self, module_name: str, split_config: SplitConfig, device: Any) -> None:
         self.module_name = module_name
         self.split = split_config
+        self.device = device
         self.origin_stream = device.current_stream()
         self.buffer: torch.Tensor | None = None
 
@@ -85,12 +86,12 @@ class _SharedOutput:
                 return None
             per_token = rows // tokens
             if self.buffer is None:
-                with torch.cuda.stream(self.origin_stream):
+                with self.device.stream(self.origin_stream):
                     self.buffer = torch.empty((per_token * total, cols), dtype=dtype, device=dev)
             buf = self.buffer
             if buf.shape[1] != cols or buf.dtype != dtype or buf.shape[0] != per_token * total:
                 return None
-            buf.record_stream(torch.cuda.current_stream())
+            buf.record_stream(self.device.current_stream())
             return buf[per_token * first: per_token * first + rows]
 
         ops.offer_output_rows(provider)
@@ -247,18 +248,10 @@ class DynaFlowEngine:
             _owner=id(self),
         )
 
-    def _shared_output_for(self, split_config: SplitConfig, device: Any) -> "_SharedOutput | None":
-        """One buffer for the model output of all nano-batches, when the graph allows it: the graph returns the
-        result of its last sub-graph call as it is, that result is token-shaped, and no per-sub-graph graph or
-        capture-size padding stands between the operator and its output."""
-        if not device.is_gpu or split_config.is_dryrun or split_config.use_cudagraph:
-            return None
-        if not self.config.knob("shared_output", True):
-            return None
-        if list(split_config.num_tokens_padded) != list(split_config.num_tokens):
-            return None
-        output = self.nodes[-1]
-        if output.op != "output":
+    def _output_module(self) -> str | None:
+        """The sub-graph whose result the graph returns as it is, if that result is a token-shaped tensor."""
+        output = self.nodes[-1] if self.nodes else None
+        if output is None or output.op != "output":
             return None
         producer = output.args[0]
         if isinstance(producer, (tuple, list)) and len(producer) == 1:
@@ -276,7 +269,19 @@ class DynaFlowEngine:
         example = returned.meta.get("example_value", None)
         if not isinstance(example, torch.Tensor) or example.dim() < 1 or not _is_symbolic(example.shape[0]):
             return None
-        return _SharedOutput(producer.target, split_config, device)
+        return producer.target
+
+    def _shared_output_for(self, split_config: SplitConfig, device: Any) -> "_SharedOutput | None":
+        """One buffer for the model output of all nano-batches, when the graph allows it (``_output_module``) and no
+        per-sub-graph graph or capture-size padding stands between the operator and its output."""
+        if not device.is_gpu or split_config.is_dryrun or split_config.use_cudagraph:
+            return None
+        if not self.config.knob("shared_output", True):
+            return None
+        if list(split_config.num_tokens_padded) != list(split_config.num_tokens):
+            return None
+        module = self._output_module()
+        return None if module is None else _SharedOutput(module, split_config, device)
 
     # ------------------------------------------------------------------ dry-run
     def dryrun(
@@ -375,6 +380,10 @@ class DynaFlowEngine:
             return self.graph_module(*call_args, **kwargs)
 
     # ---------------------------------------------------------- scheduled path
+    def begin(self, args: tuple, split_config: SplitConfig) -> "ScheduledForward":
+        """Start a forward that a scheduler drives; inputs are bound on the stream that is current now."""
+        return ScheduledForward(self, args, split_config)
+
     async def execute(
         self,
         args: tuple,
@@ -383,123 +392,174 @@ class DynaFlowEngine:
         execute_queue: asyncio.Queue,
         split_config: SplitConfig,
     ) -> tuple[dict[int, Any], list[Any]]:
-        """Producer coroutine of one forward; runs beside ``scheduler.schedule``.
+        """A forward as a coroutine that talks to the scheduler through queues (engine.py:222-424), for callers that
+        run the two side by side themselves; the manager drives a ``ScheduledForward`` without them.
 
         Returns the per-nano-batch results and each nano-batch's tail event,
         which the caller must wait on before touching the results.
         """
-        device = get_device()
-        lanes = split_config.num_nano_batches
-        env = ExecutionEnvironment(lanes)
-        self.last_env = env
-        self.issue_trace = []
-        results: dict[int, Any] = {}
-        tail_events = [device.new_event() for _ in range(lanes)]
-        todo: dict[int, deque[torch.fx.Node]] = {b: deque(self.nodes) for b in range(lanes)}
-        # operators handed to the scheduler and not yet executed, per nano-batch
-        outstanding: dict[int, deque[OperatorHandle]] = {b: deque() for b in range(lanes)}
+        forward = self.begin(args, split_config)
+        lanes = range(split_config.num_nano_batches)
 
-        async def run_inline_until_op(b: int) -> None:
-            """Run inline nodes of ``b`` up to its next sub-graph call / the end."""
-            queue = todo[b]
-            while queue:
-                node = queue[0]
-                if node.op == "call_module":
-                    return
-                if node.op == "output":
-                    results[b] = self._collect_output(node, b, env)
-                    queue.popleft()
+        async def hand_over() -> None:
+            for b in lanes:
+                while forward.ready[b] and not op_queue[b].full():
+                    await op_queue[b].put(forward.ready[b].popleft())
+                if forward.finished[b] and not told[b]:
+                    told[b] = True
                     await op_queue[b].put(None)
-                    return
-                self._execute_non_module(node, b, args, env, split_config)
-                queue.popleft()
 
-        shared_output = self._shared_output_for(split_config, device)
+        told = [False] * split_config.num_nano_batches
+        await hand_over()
+        while not all(forward.finished):
+            operators, func, finished = await execute_queue.get()
+            forward.launch(operators, func)
+            await hand_over()
+            finished.set()
+        return await forward.completed()
 
+
+class ScheduledForward:
+    """One forward under a scheduler's control: which operators are ready, and what launching one does.
+
+    Every nano-batch walks the top-level node list.  ``ready[b]`` holds the sub-graph calls that nano-batch ``b`` has
+    reached and nobody has taken yet; consecutive calls are ready together, inline nodes behind a call run once it has
+    been launched.  ``launch`` enqueues an operator on the stream that is current and moves every nano-batch on.
+    """
+
+    #: most operators of a nano-batch that wait to be taken
+    MOST_READY = 10
+
+    def __init__(self, engine: DynaFlowEngine, args: tuple, split_config: SplitConfig) -> None:
+        self.engine = engine
+        self.split = split_config
+        self.args = args
+        self.device = get_device()
+        lanes = split_config.num_nano_batches
+        self.env = ExecutionEnvironment(lanes)
+        engine.last_env = self.env
+        engine.issue_trace = []
+        self.results: dict[int, Any] = {}
+        self.tail_events = [self.device.new_event() for _ in range(lanes)]
+        self.finished = [False] * lanes
+        self.ready: list[deque[OperatorHandle]] = [deque() for _ in range(lanes)]
+        # operators handed out and not yet executed, per nano-batch
+        self._outstanding: list[deque[OperatorHandle]] = [deque() for _ in range(lanes)]
+        self._next = [0] * lanes                       # index of each nano-batch's next node
+        self._waiting: list[asyncio.Event] = []        # of coroutines that wait for an operator
+        self.shared_output = engine._shared_output_for(split_config, self.device)
         # Inputs of every nano-batch are bound up front, on the caller's stream.
         for b in range(lanes):
-            queue = todo[b]
-            while queue and queue[0].op not in ("call_module", "output"):
-                self._execute_non_module(queue[0], b, args, env, split_config)
-                queue.popleft()
-            tail_events[b].record()
+            self._run_inline(b)
+            self.tail_events[b].record()
+        for b in range(lanes):
+            self._advance(b)
 
-        while any(todo.values()):
-            # publish every sub-graph call that heads a nano-batch's list
-            for b in range(lanes):
-                queue = todo[b]
-                while queue and queue[0].op == "call_module" and not op_queue[b].full():
-                    handle = self._handle_for(
-                        queue[0], b, split_config.num_tokens_padded[b], split_config
-                    )
-                    await op_queue[b].put(handle)
-                    outstanding[b].append(handle)
-                    queue.popleft()
+    def _run_inline(self, b: int) -> None:
+        """Run the nodes of ``b`` up to its next sub-graph call or the output node."""
+        nodes, i = self.engine.nodes, self._next[b]
+        while i < len(nodes) and nodes[i].op not in ("call_module", "output"):
+            self.engine._execute_non_module(nodes[i], b, self.args, self.env, self.split)
+            i += 1
+        self._next[b] = i
 
-            if not any(outstanding.values()):
-                # nothing for the scheduler to ask for: only inline work is left
-                for b in range(lanes):
-                    await run_inline_until_op(b)
-                continue
+    def _advance(self, b: int) -> None:
+        """Publish what ``b`` has reached: its next sub-graph calls, or its result."""
+        nodes = self.engine.nodes
+        if not self._outstanding[b]:
+            self._run_inline(b)
+        i = self._next[b]
+        while i < len(nodes) and nodes[i].op == "call_module" and len(self.ready[b]) < self.MOST_READY:
+            handle = self.engine._handle_for(nodes[i], b, self.split.num_tokens_padded[b], self.split)
+            self.ready[b].append(handle)
+            self._outstanding[b].append(handle)
+            i += 1
+        self._next[b] = i
+        if i < len(nodes) and nodes[i].op == "output" and not self._outstanding[b]:
+            self.results[b] = self.engine._collect_output(nodes[i], b, self.env)
+            self._next[b] = i = len(nodes)
+        if i == len(nodes) and not self._outstanding[b]:
+            self.finished[b] = True
 
-            operators, func, finished = await execute_queue.get()
-            if isinstance(operators, OperatorHandle):
-                operators = (operators,)
+    async def next_operator(self, b: int) -> OperatorHandle | None:
+        """The next ready operator of nano-batch ``b``, ``None`` once it has produced its output; waits while another
+        coroutine holds the operators that have to be launched first."""
+        while not self.ready[b]:
+            if self.finished[b]:
+                return None
+            await self._moved()
+        return self.ready[b].popleft()
 
-            call_pos: list[list[Any]] = []
-            call_kw: list[dict[str, Any]] = []
-            for op in operators:
-                b = op.batch_idx
-                node = self.module_name_to_node[op.module_name]
-                # chain: this launch starts after the nano-batch's previous work
-                tail_events[b].wait()
-                tail_events[b] = device.new_event()
-                # only node-valued positional inputs are forwarded (engine.py:304-310)
-                pos = [env.get(b, a) for a in node.args if isinstance(a, torch.fx.Node)]
-                kw = {k: self._load(env, b, v) for k, v in node.kwargs.items()}
-                if device.is_gpu:
-                    current = device.current_stream()
-                    for value in pos:
-                        _record_use(value, current)
-                call_pos.append(pos)
-                call_kw.append(kw)
+    async def _moved(self) -> None:
+        """Wait for another coroutine's launch."""
+        moved = asyncio.Event()
+        self._waiting.append(moved)
+        await moved.wait()
 
-            outputs: list[Any] = []
-            if func is not None:
-                if len(operators) != 1:
-                    raise NotImplementedError("Operator batching is not implemented")
-                with set_op_handle(operators[0]):
-                    outputs.append(func(*call_pos[0], **call_kw[0]))
-            elif len(operators) != 1 and all(
-                op.module_name == operators[0].module_name for op in operators
-            ):
+    def launch(self, operators: "OperatorHandle | tuple[OperatorHandle, ...]", func: Callable | None = None) -> None:
+        """Enqueue operators on the current stream, behind the previous work of their nano-batches."""
+        if isinstance(operators, OperatorHandle):
+            operators = (operators,)
+        engine, device, env = self.engine, self.device, self.env
+        call_pos: list[list[Any]] = []
+        call_kw: list[dict[str, Any]] = []
+        for op in operators:
+            b = op.batch_idx
+            node = engine.module_name_to_node[op.module_name]
+            # chain: this launch starts after the nano-batch's previous work
+            self.tail_events[b].wait()
+            self.tail_events[b] = device.new_event()
+            # only node-valued positional inputs are forwarded (engine.py:304-310)
+            pos = [env.get(b, a) for a in node.args if isinstance(a, torch.fx.Node)]
+            kw = {k: engine._load(env, b, v) for k, v in node.kwargs.items()}
+            if device.is_gpu:
+                current = device.current_stream()
+                for value in pos:
+                    _record_use(value, current)
+            call_pos.append(pos)
+            call_kw.append(kw)
+
+        outputs: list[Any] = []
+        if func is not None:
+            if len(operators) != 1:
                 raise NotImplementedError("Operator batching is not implemented")
-            else:
-                for i, op in enumerate(operators):
-                    with device.range(f"op_{op.module_name}_{op.batch_idx}"), set_op_handle(op):
-                        module = getattr(self.graph_module, op.module_name)
-                        offered = shared_output.offer(op) if shared_output is not None else False
-                        try:
-                            outputs.append(module(*call_pos[i], **call_kw[i]))
-                        finally:
-                            if offered:
-                                shared_output.withdraw()
+            with set_op_handle(operators[0]):
+                outputs.append(func(*call_pos[0], **call_kw[0]))
+        elif len(operators) != 1 and all(op.module_name == operators[0].module_name for op in operators):
+            raise NotImplementedError("Operator batching is not implemented")
+        else:
+            for i, op in enumerate(operators):
+                with device.range(f"op_{op.module_name}_{op.batch_idx}"), set_op_handle(op):
+                    module = getattr(engine.graph_module, op.module_name)
+                    offered = self.shared_output.offer(op) if self.shared_output is not None else False
+                    try:
+                        outputs.append(module(*call_pos[i], **call_kw[i]))
+                    finally:
+                        if offered:
+                            self.shared_output.withdraw()
 
-            for op, value in zip(operators, outputs):
-                b = op.batch_idx
-                tail_events[b].record()
-                env.put(b, self.module_name_to_node[op.module_name], value)
-                # per-nano-batch FIFO: the executed handle is the oldest published one
-                assert outstanding[b] and op is outstanding[b][0], (
-                    f"{op.module_name} of nano-batch {b} executed out of order"
-                )
-                outstanding[b].popleft()
-                self.issue_trace.append((op.module_name, b))
+        for op, value in zip(operators, outputs):
+            b = op.batch_idx
+            self.tail_events[b].record()
+            env.put(b, engine.module_name_to_node[op.module_name], value)
+            # per-nano-batch FIFO: the executed handle is the oldest published one
+            assert self._outstanding[b] and op is self._outstanding[b][0], (
+                f"{op.module_name} of nano-batch {b} executed out of order"
+            )
+            self._outstanding[b].popleft()
+            engine.issue_trace.append((op.module_name, b))
 
-            for b in range(lanes):
-                if not outstanding[b]:
-                    await run_inline_until_op(b)
-            finished.set()
+        for b in range(len(self.finished)):
+            if not self.finished[b]:
+                self._advance(b)
+        waiting, self._waiting = self._waiting, []
+        for moved in waiting:
+            moved.set()
 
-        self.shared_output_buffer = shared_output.buffer if shared_output is not None else None
-        return results, tail_events
+    async def completed(self) -> tuple[dict[int, Any], list[Any]]:
+        """The per-nano-batch results and tail events once every nano-batch has produced its output (tasks that the
+        scheduler has started may still be launching operators)."""
+        while not all(self.finished):
+            await self._moved()
+        self.engine.shared_output_buffer = self.shared_output.buffer if self.shared_output is not None else None
+        return self.results, self.tail_events

@@ -101,7 +101,7 @@ def equal_n_way(
         n = max(1, batch_size // min_nano_split_tokens)
         chunk = batch_size // n if n > 1 else batch_size
     per_request = list(input_info.num_tokens)
-    uniform = len(per_request) != batch_size or all(t == 1 for t in per_request)
+    uniform = len(per_request) != batch_size or per_request.count(1) == batch_size
     if n <= 1:
         total = batch_size if uniform else sum(per_request)
         return _single(batch_size, total, total, use_cudagraph)

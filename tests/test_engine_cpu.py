@@ -470,3 +470,42 @@ def test_a_side_by_side_override_that_contradicts_the_schedule_is_refused(host_d
     manager.prepare(96, [96])
     with torch.no_grad(), pytest.raises(ValueError, match="side_by_side"):
         compiled(x)
+
+
+def test_engine_coroutine_behind_queues_issues_what_the_manager_issues(host_device):
+    """``engine.execute`` with a context of two queues - for callers that run engine and scheduler side by side
+    themselves - against the manager's own forward: the same launches, events and result."""
+    cfg = make_config(2)
+    model, manager, compiled, x = compile_mlp(cfg)
+    split = manager.prepare(64, [64])
+    args = (model.gate_proj.weight, 64, x, model.up_proj.weight, model.down_proj.weight)
+
+    def log_of(forward):
+        host_device.log.clear()
+        with torch.no_grad():
+            y = asyncio.run(forward())
+        first = min(e[1] for e in host_device.log if e[0] == "record")     # events are numbered process-wide
+        return y, [(kind, n - first, where) if kind != "range" else (kind, n, where) for kind, n, where in host_device.log]
+
+    async def queues():
+        op_queue = {b: asyncio.Queue(maxsize=10) for b in range(2)}
+        execute_queue = asyncio.Queue()
+        (results, events), _ = await asyncio.gather(
+            manager.engine.execute(args, {}, op_queue, execute_queue, split),
+            manager.scheduler.schedule(ExecutionContext(split, op_queue, execute_queue)))
+        for event in events:
+            event.wait()
+        return torch.cat([results[0], results[1]]) if isinstance(results[0], torch.Tensor) else results
+
+    async def direct():
+        return await manager._forward_async(args, {}, split)
+
+    y_direct, log_direct = log_of(direct)
+    trace = list(manager.engine.issue_trace)
+    y_queues, log_queues = log_of(queues)
+    assert manager.engine.issue_trace == trace and log_queues == log_direct
+    if isinstance(y_queues, dict):
+        y_queues = tuple(torch.cat([y_queues[0][i], y_queues[1][i]]) for i in range(len(y_queues[0])))
+    for got, want in zip(y_queues if isinstance(y_queues, tuple) else (y_queues,),
+                         y_direct if isinstance(y_direct, tuple) else (y_direct,)):
+        assert torch.equal(got, want)
