@@ -37,6 +37,14 @@ static inline int dfhip_check_launch() {
   return hipGetLastError() == hipSuccess ? DFHIP_OK : DFHIP_ERR_LAUNCH;
 }
 
+// Split-K workspaces start with the arrival counters.  All split-K kernels, bf16 and fp8, use the same size of
+// counter area for a workspace (at least 4 KiB), so that the fp32 blocks one of them leaves behind
+// never lie where another expects counters that are zero.
+static inline size_t dfhip_counter_area(size_t tiles) {
+  const size_t need = ((tiles * sizeof(int)) + 255) & ~(size_t)255;
+  return need > 4096 ? need : 4096;
+}
+
 // bf16 <-> fp32 on raw 16-bit storage
 DFHIP_DEVICE float bf16_bits_to_f32(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
 

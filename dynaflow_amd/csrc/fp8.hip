@@ -12,7 +12,10 @@
 //                       bf16 ring kernel: five 32 KiB LDS units, 1.5 slabs in flight,
 //                       XOR-swizzled 128-byte rows, one LDS read or DMA issue behind every
 //                       MFMA, barrier between the two column halves of a slab, staged epilogue.
-// gemm_fp8_nt_kernel    register-staged double buffer for small shapes.
+//                       Forms with 192 and 128 rows for launches of few rows (TM: 16-row blocks per wave), and
+//                       with K cut into parts for few tiles: [350 x 28672] x [8192 x 28672]^T ran on 64 workgroups
+//                       (230 us, 0.71 PFLOP/s), with 192 rows and four parts it takes 96.
+// gemm_fp8_nt_kernel    register-staged double buffer, 128 x 128: an independent second kernel, by variant only.
 #include "dfhip_stream.h"
 
 namespace {
@@ -247,49 +250,61 @@ constexpr int F8_GROUP_M = 4, F8_EROW = 272;
 // then is 256 x 128 outputs, N counts those, and the epilogue writes act = bf16(silu(bf16 g) * bf16 u) -
 // the roundings of the separate GEMMs and of silu_mul_absmax_kernel, so the same bits - and folds
 // max |act| into amax[0].
-template <bool FUSED>
+template <bool FUSED, int TM, bool SPLIT>
 __global__ void __launch_bounds__(256)
 gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ W, const uint8_t* __restrict__ W2,
                      uint16_t* __restrict__ C, const float* __restrict__ a_scale, const float* __restrict__ w_scale,
                      const float* __restrict__ w2_scale, float* __restrict__ amax, int M, int N, int K, int64_t lda,
-                     int64_t ldw, int64_t ldc, int tiles_m, int tiles_n) {
+                     int64_t ldw, int64_t ldc, int tiles_m, int tiles_n, int split_k, float* __restrict__ partials,
+                     int* __restrict__ arrivals) {
+  static_assert(!(FUSED && SPLIT), "the fused form keeps K whole");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave_m = wave & 1, wave_n = wave >> 1;
+  constexpr int TILE_M = 32 * TM;              // rows of a tile: two wave rows of TM blocks of 16
   constexpr int TILE_N = FUSED ? 128 : 256;    // output columns of a tile
+  constexpr int MQ = 4 * TM;                   // MFMAs of a column half
 
-  const int tile = remap_xcd(blockIdx.x, tiles_m * tiles_n);
+  int tile, part = 0;
+  if (SPLIT) splitk_work_of(blockIdx.x, tiles_m * tiles_n, tile, part);
+  else tile = remap_xcd(blockIdx.x, tiles_m * tiles_n);
   const int per_panel = F8_GROUP_M * tiles_n;
   const int first_m = (tile / per_panel) * F8_GROUP_M;
   const int rows_in_panel = (tiles_m - first_m) < F8_GROUP_M ? (tiles_m - first_m) : F8_GROUP_M;
   const int in_panel = tile % per_panel;
-  const int m0 = (first_m + in_panel % rows_in_panel) * 256;
+  const int m0 = (first_m + in_panel % rows_in_panel) * TILE_M;
   const int n0 = (in_panel / rows_in_panel) * TILE_N;
-  const int KT = K / FBK;
+  const int slabs = K / FBK;
+  const int slab0 = SPLIT ? (int)((int64_t)slabs * part / split_k) : 0;
+  const int KT = SPLIT ? (int)((int64_t)slabs * (part + 1) / split_k) - slab0 : slabs;
 
   // DMA addresses: a wave-uniform tile base (scalar registers, advanced per slab) plus a 32-bit byte
   // offset per lane.  FUSED: rows 0..127 of the W half come from W (waves 0, 1), rows 128..255 from W2.
-  uint32_t a_off[8], w_off[8];
+  uint32_t a_off[TM], w_off[8];
+#pragma unroll
+  for (int t = 0; t < TM; ++t) {
+    const int row = (wave * TM + t) * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
+    int ar = m0 + row; ar = ar < M ? ar : M - 1;
+    a_off[t] = (uint32_t)((int64_t)(ar - m0) * lda + chunk * 16);
+  }
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
     const int row = (wave * 8 + t) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-    int ar = m0 + row; ar = ar < M ? ar : M - 1;
-    a_off[t] = (uint32_t)((int64_t)(ar - m0) * lda + chunk * 16);
     int wr = n0 + (FUSED ? (row & 127) : row); wr = wr < N ? wr : N - 1;
     w_off[t] = (uint32_t)((int64_t)(wr - n0) * ldw + chunk * 16);
   }
-  const uint8_t* const a_tile = A + (int64_t)m0 * lda;
-  const uint8_t* const w_tile = ((FUSED && wave >= 2) ? W2 : W) + (int64_t)n0 * ldw;
-  const uint32_t wave_lds = wave * 8 * 1024;
+  const uint8_t* const a_tile = A + (int64_t)m0 * lda + (int64_t)slab0 * FBK;
+  const uint8_t* const w_tile = ((FUSED && wave >= 2) ? W2 : W) + (int64_t)n0 * ldw + (int64_t)slab0 * FBK;
   auto dma_a = [&](int t, int slab, int unit) {
     const int s = slab < KT ? slab : KT - 1;
-    dma16_base(unit * F8_UNIT + wave_lds + t * 1024, a_tile + (int64_t)s * FBK, a_off[t]);
+    dma16_base(unit * F8_UNIT + (wave * TM + t) * 1024, a_tile + (int64_t)s * FBK, a_off[t]);
   };
   auto dma_w = [&](int t, int slab, int unit) {
     const int s = slab < KT ? slab : KT - 1;
-    dma16_base(unit * F8_UNIT + wave_lds + t * 1024, w_tile + (int64_t)s * FBK, w_off[t]);
+    dma16_base(unit * F8_UNIT + (wave * 8 + t) * 1024, w_tile + (int64_t)s * FBK, w_off[t]);
   };
 
   // v_mfma_scale_f32_16x16x128_f8f6f4: one instruction covers the 128 bytes of k of a slab.  A fragment of a
@@ -300,31 +315,31 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
   int koff[2];
 #pragma unroll
   for (int part = 0; part < 2; ++part) koff[part] = ((2 * fquad + part) ^ fswz) * 16;
-  const int a_lane = (wave_m * 128 + frow) * 128, w_lane = (wave_n * 128 + frow) * 128;
+  const int a_lane = (wave_m * (16 * TM) + frow) * 128, w_lane = (wave_n * 128 + frow) * 128;
 
-  f32x4 acc[8][8];
+  f32x4 acc[TM][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
 #pragma unroll
-  for (int t = 0; t < 8; ++t) dma_a(t, 0, 0);
+  for (int t = 0; t < TM; ++t) dma_a(t, 0, 0);
 #pragma unroll
   for (int t = 0; t < 8; ++t) dma_w(t, 0, 1);
 #pragma unroll
-  for (int t = 0; t < 8; ++t) dma_a(t, 1, 2);
+  for (int t = 0; t < TM; ++t) dma_a(t, 1, 2);
 #pragma unroll
   for (int t = 0; t < 8; ++t) dma_w(t, 1, 3);
-  wait_vmcnt<16>();
+  wait_vmcnt<8 + TM>();
   workgroup_barrier();
 
   // A whole slab of fragments is 128 registers per operand; both operands double-buffered would not fit.
   // The slab is multiplied in two column halves instead: W blocks 0..3 (fwa), then W blocks 4..7 (fwb), both
-  // against all eight A blocks.  The A blocks are double-buffered across slabs, each W half is read while the
+  // against all TM A blocks.  The A blocks are double-buffered across slabs, each W half is read while the
   // other one is in use.
-  u32x4 fa[2][8][2], fwa[4][2], fwb[4][2];   // [..][block][low / high 16 bytes]
-  auto read_a = [&](int half_idx, int slot, int unit_a) {   // half_idx 0..15: block half_idx/2, low / high half
+  u32x4 fa[2][TM][2], fwa[4][2], fwb[4][2];   // [..][block][low / high 16 bytes]
+  auto read_a = [&](int half_idx, int slot, int unit_a) {   // half_idx 0..2 TM - 1: block half_idx/2, low / high half
     const int blk = half_idx >> 1, part = half_idx & 1;
     fa[slot][blk][part] = *reinterpret_cast<const u32x4*>(smem + unit_a * F8_UNIT + a_lane + koff[part] + blk * 2048);
   };
@@ -334,7 +349,7 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
     if (second) fwb[blk][part] = v; else fwa[blk][part] = v;
   };
   const int unit_scale = 0x7f7f7f7f;   // e8m0 scales 2^0
-  auto mfma = [&](int q, int slot, bool second) {   // snake over 8 A blocks x 4 W blocks
+  auto mfma = [&](int q, int slot, bool second) {   // snake over TM A blocks x 4 W blocks
     const int i = q >> 2, jj = (i & 1) ? 3 - (q & 3) : (q & 3);
     const u32x4 (&w)[2] = second ? fwb[jj] : fwa[jj];
     const i32x8 av = {(int)fa[slot][i][0][0], (int)fa[slot][i][0][1], (int)fa[slot][i][0][2], (int)fa[slot][i][0][3],
@@ -344,41 +359,47 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
     asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %3 op_sel_hi:[0,0,0]"
                  : "+a"(acc[i][second ? 4 + jj : jj]) : "v"(wv), "v"(av), "v"(unit_scale));
   };
-  // reads of the next slab in the order its first MFMAs need them: W block 0, A block 0, W blocks 1..3, A 1..7
-  auto read_next = [&](int pos, int slot, int unit_a, int unit_w) {   // pos 0..23 (fragment halves)
+  // reads of the next slab in the order its first MFMAs need them: W block 0, A block 0, W blocks 1..3, then the other A blocks
+  auto read_next = [&](int pos, int slot, int unit_a, int unit_w) {   // pos 0..READS - 1 (fragment halves)
     if (pos < 2) read_w(pos, false, unit_w);
     else if (pos < 4) read_a(pos - 2, slot, unit_a);
     else if (pos < 10) read_w(pos - 2, false, unit_w);
     else read_a(pos - 8, slot, unit_a);
   };
 
+  constexpr int READS = 8 + 2 * TM;
   int ua = 0, uw = 1, ia = 4, iw = 0;
 #pragma unroll
-  for (int pos = 0; pos < 24; ++pos) read_next(pos, 0, ua, uw);
+  for (int pos = 0; pos < READS; ++pos) read_next(pos, 0, ua, uw);
   // one slab; `sl` (0 / 1, a constant at each call) is the A fragment buffer this slab multiplies from
   auto slab = [&](int kt, int sl) {
     // first column half: the fragments of W blocks 4..7 behind MFMAs 0..7, the DMA of A(kt+2) behind every
     // other MFMA after that
 #pragma unroll
-    for (int q = 0; q < 32; ++q) {
+    for (int q = 0; q < MQ; ++q) {
       mfma(q, sl, false);
       if (q < 8) read_w(q, true, uw);
-      else if (q % 2 == 0 && q < 24) dma_a((q - 8) / 2, kt + 2, ia);
+      else if (q % 2 == 0 && q < 8 + 2 * TM) dma_a((q - 8) / 2, kt + 2, ia);
       DFHIP_PIN;
     }
     // every LDS read of slab kt has been issued; slab kt+1 must have landed, only A(kt+2) may be in flight
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wait_vmcnt<8>();
+    wait_vmcnt<TM>();
     workgroup_barrier();
     int na = ua + 2; if (na >= F8_NUNITS) na -= F8_NUNITS;
     int nw = uw + 2; if (nw >= F8_NUNITS) nw -= F8_NUNITS;
-    // second column half: the DMA of W(kt+2) behind every other MFMA, the 24 fragment halves of slab kt+1
-    // (all of A, W blocks 0..3) behind the others
+    // second column half: the DMA of W(kt+2) behind every other MFMA, the fragment halves of slab kt+1 (all of A,
+    // W blocks 0..3) behind the others.  256 rows: one operation behind every MFMA; shorter tiles have fewer MFMAs
+    // than operations and some carry two.
+    constexpr int OPS = 8 + READS;
 #pragma unroll
-    for (int q = 0; q < 32; ++q) {
+    for (int q = 0; q < MQ; ++q) {
       mfma(q, sl, true);
-      if (q < 16) { if (q % 2 == 0) dma_w(q / 2, kt + 2, iw); else read_next(q / 2, sl ^ 1, na, nw); }
-      else read_next(8 + (q - 16), sl ^ 1, na, nw);
+#pragma unroll
+      for (int op = q * OPS / MQ; op < (q + 1) * OPS / MQ; ++op) {
+        if (op < 16) { if (op % 2 == 0) dma_w(op / 2, kt + 2, iw); else read_next(op / 2, sl ^ 1, na, nw); }
+        else read_next(8 + (op - 16), sl ^ 1, na, nw);
+      }
       DFHIP_PIN;
     }
     ua = na; uw = nw;
@@ -397,11 +418,56 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
   // (the compiler does not know that the statements above write the accumulators late: every later use
   // of an accumulator is tied behind the wait states)
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) asm volatile("" : "+a"(acc[i][j]));
 
-  // scale, round to bf16, park the wave's 128x128 block in LDS, store whole 256-byte row pieces
+  if constexpr (SPLIT) {
+    // Every part leaves its fp32 block in `partials` and takes a ticket; the part that comes last adds the blocks in
+    // part order (its own too: the same bits whoever is last) and writes the tile.  Nobody waits.
+    constexpr int BLOCK = TM * 8 * 256;
+    f32x4* const blocks = reinterpret_cast<f32x4*>(partials) + (int64_t)tile * split_k * BLOCK;
+    f32x4* const mine = blocks + part * BLOCK + tid;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) store_f32x4_device_coherent(mine + (i * 8 + j) * 256, acc[i][j]);
+    wait_vmcnt<0>();
+    __syncthreads();
+    int* const ticket_cell = reinterpret_cast<int*>(smem);
+    if (tid == 0) *ticket_cell = atomicAdd(arrivals + tile, 1);
+    __syncthreads();
+    const int ticket = *ticket_cell;
+    if (ticket != split_k - 1) return;
+    if (tid == 0) atomicExch(arrivals + tile, 0);     // counters are left at zero
+    __syncthreads();                                  // the ticket has been read before the tile is parked over it
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(blocks, 0, split_k * BLOCK * 16, 0x00027000);
+    constexpr int SC1 = 16;                           // read from the memory side, as the stores were written
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p = 0; p < split_k; ++p) {
+      const int base = p * (BLOCK * 16);
+#pragma unroll
+      for (int i = 0; i < TM; i += 2) {             // 16 loads in flight before the first is used
+        f32x4 v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          v[j] = __builtin_bit_cast(
+              f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16, base + (i * 8 + j) * 4096, SC1));
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          f32x4& sum = acc[i + j / 8][j % 8];
+          sum += v[j];
+          asm volatile("" : "+a"(sum));             // back to its accumulation registers
+        }
+      }
+    }
+  }
+
+  // scale, round to bf16, park the wave's block in LDS, store whole 256-byte row pieces
   const float sa = a_scale[0];
   uint8_t* park = smem + wave * (128 * F8_EROW);
 #pragma unroll
@@ -410,7 +476,7 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
     n = n < N ? n : N - 4;   // columns past the edge are never stored; keep the scale load in bounds
     const f32x4 ws = *reinterpret_cast<const f32x4*>((FUSED && wave_n ? w2_scale : w_scale) + n);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < TM; ++i) {
       u32x2 v;
       v[0] = pack2_bf16(acc[i][j][0] * (sa * ws[0]), acc[i][j][1] * (sa * ws[1]));
       v[1] = pack2_bf16(acc[i][j][2] * (sa * ws[2]), acc[i][j][3] * (sa * ws[3]));
@@ -419,15 +485,15 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
   }
   DFHIP_PIN;
   if (FUSED) {
-    // gate blocks sit in the parks of waves 0, 1 (rows 0..127, 128..255), up blocks in those of waves 2, 3;
-    // wave w combines rows (w & 1) * 128 + (w >> 1) * 64 .. + 64 of the tile
+    // gate blocks sit in the parks of waves 0, 1 (the two halves of the rows), up blocks in those of waves 2, 3;
+    // wave w combines half (w >> 1) of the rows of park w & 1
     __syncthreads();
     const uint8_t* gpark = smem + (wave & 1) * (128 * F8_EROW);
     const uint8_t* upark = smem + ((wave & 1) + 2) * (128 * F8_EROW);
-    const int row0 = (wave >> 1) * 64;
+    const int row0 = (wave >> 1) * (8 * TM);
     float vmax = 0.0f;
 #pragma unroll 4
-    for (int p = 0; p < 16; ++p) {
+    for (int p = 0; p < 2 * TM; ++p) {
       const int id = p * 64 + lane;
       const int row = row0 + (id >> 4), c = id & 15;
       const u32x4 gv = *reinterpret_cast<const u32x4*>(gpark + row * F8_EROW + c * 16);
@@ -439,7 +505,7 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
         const float hi = silu_f32(__uint_as_float(gv[w] & 0xffff0000u)) * __uint_as_float(uv[w] & 0xffff0000u);
         o[w] = pack2_bf16(lo, hi);
       }
-      const int m = m0 + (wave & 1) * 128 + row, n = n0 + c * 8;
+      const int m = m0 + (wave & 1) * (16 * TM) + row, n = n0 + c * 8;
       if (m < M && n < N) {
         *reinterpret_cast<u32x4*>(C + (int64_t)m * ldc + n) = o;
 #pragma unroll
@@ -453,9 +519,9 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
     if (lane == 0) atomic_max_nonneg(amax, vmax);
     return;
   }
-  const int m_base = m0 + wave_m * 128, n_base = n0 + wave_n * 128;
+  const int m_base = m0 + wave_m * (16 * TM), n_base = n0 + wave_n * 128;
 #pragma unroll 4
-  for (int p = 0; p < 32; ++p) {
+  for (int p = 0; p < 4 * TM; ++p) {
     const int id = p * 64 + lane;
     const int row = id >> 4, c = id & 15;
     const u32x4 v = *reinterpret_cast<const u32x4*>(park + row * F8_EROW + c * 16);
@@ -464,28 +530,35 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
   }
 }
 
+template <int TM, bool SPLIT>
 int launch_fp8_ring(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
-                    const float* a_scale, const float* w_scale, int M, int N, int K, hipStream_t stream) {
+                    const float* a_scale, const float* w_scale, int M, int N, int K, int split_k, void* workspace,
+                    hipStream_t stream) {
+  auto kernel = gemm_fp8_ring_kernel<false, TM, SPLIT>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
-  if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(gemm_fp8_ring_kernel<false>), F8_RING_LDS, lds_opted_in)) return rc;
-  const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
-  hipLaunchKernelGGL(gemm_fp8_ring_kernel<false>, dim3(tiles_m * tiles_n), dim3(256), F8_RING_LDS, stream,
+  if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), F8_RING_LDS, lds_opted_in)) return rc;
+  const int tiles_m = (M + 32 * TM - 1) / (32 * TM), tiles_n = (N + 255) / 256;
+  float* partials = nullptr;
+  if (SPLIT) partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area((size_t)tiles_m * tiles_n));
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(256), F8_RING_LDS, stream,
                      static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), nullptr,
                      static_cast<uint16_t*>(C), a_scale, w_scale, nullptr, nullptr, M, N, K, lda, ldw, ldc, tiles_m,
-                     tiles_n);
+                     tiles_n, split_k, partials, static_cast<int*>(workspace));
   return dfhip_check_launch();
 }
 
+template <int TM>
 int launch_fp8_ring_fused(const void* A, int64_t lda, const void* Wg, const void* Wu, int64_t ldw, void* act,
                           int64_t ld_act, const float* a_scale, const float* wg_scale, const float* wu_scale,
                           float* amax, int M, int I, int K, hipStream_t stream) {
+  auto kernel = gemm_fp8_ring_kernel<true, TM, false>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
-  if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(gemm_fp8_ring_kernel<true>), F8_RING_LDS, lds_opted_in)) return rc;
-  const int tiles_m = (M + 255) / 256, tiles_n = (I + 127) / 128;
-  hipLaunchKernelGGL(gemm_fp8_ring_kernel<true>, dim3(tiles_m * tiles_n), dim3(256), F8_RING_LDS, stream,
+  if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), F8_RING_LDS, lds_opted_in)) return rc;
+  const int tiles_m = (M + 32 * TM - 1) / (32 * TM), tiles_n = (I + 127) / 128;
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(256), F8_RING_LDS, stream,
                      static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(Wg), static_cast<const uint8_t*>(Wu),
                      static_cast<uint16_t*>(act), a_scale, wg_scale, wu_scale, amax, M, I, K, lda, ldw, ld_act,
-                     tiles_m, tiles_n);
+                     tiles_m, tiles_n, 1, nullptr, nullptr);
   return dfhip_check_launch();
 }
 
@@ -674,13 +747,6 @@ int launch_fp8_ring224(const void* A, int64_t lda, const void* W, int64_t ldw, v
   return dfhip_check_launch();
 }
 
-// Fraction of the CU-rounds that do work when [M, N] is cut into 256 x tile_n tiles dealt to 256 CUs in rounds.
-double fp8_round_fill(int M, int N, int tile_n) {
-  const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + tile_n - 1) / tile_n);
-  const int64_t rounds = (tiles + 255) / 256;
-  return (double)M * N / ((double)rounds * 256 * 256 * tile_n);
-}
-
 template <int BM, int BN>
 int launch_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
                const float* w_scale, int M, int N, int K, hipStream_t stream) {
@@ -698,6 +764,55 @@ int launch_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, 
 // Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip); with 16 rows and more from K = 4096
 // on, as for bf16 rows of the same bytes.
 bool stream_planned(int M, int N, int K) { return dfhip_stream_fits(M, N, K, 1) && (M < 16 || K >= 4096); }
+
+constexpr int F8_MAX_SPLIT = 16;
+
+// 16-row blocks per wave of a ring tile (256 columns), 0 for the other kernels
+int ring_blocks(int variant) { return variant == 0 ? 8 : variant == 3 ? 6 : variant == 4 ? 4 : 0; }
+
+struct TilePlan { int variant, split_k; double cost; };
+
+// What one launch (or `share` of one shape side by side) costs in us: rounds of 256 workgroups, each the slabs of a
+// part at the kernel's time per slab and a fixed start and end, plus the hand-over of the fp32 blocks of a split, whose
+// reader takes split_k blocks one after the other.  A shorter tile is hardly faster per slab (the loads bound it), so
+// it pays where it saves a round or leaves tiles to split; the 224-column kernel enters with a rate of its own.  The
+// register-staged 128 x 128 kernel is never faster than the 128-row ring (17 .. 300 rows, 256 .. 8192 columns and K: 6
+// against 6 us at the smallest, 51 against 40 at K = 8192).  Against about 200 measured launches (65 .. 2048 rows, 8192 x 28672, 4096 x 14336,
+// 28672 x 8192 and 14336 x 4096) the choice is the fastest or within 8 % of it.
+double tile_cost(int64_t tiles, int split_k, int share, int K, double per_slab, int tm) {
+  const double rounds = (double)((tiles * split_k * share + 255) / 256);
+  return rounds * ((double)(K / FBK) / split_k * per_slab + 6.0) + (split_k > 1 ? 0.9 * tm * split_k + 4.0 : 0.0);
+}
+struct RingTile { int variant, tm; double per_slab; };
+constexpr RingTile F8_RINGS[3] = {{0, 8, 1.07}, {3, 6, 0.97}, {4, 4, 0.85}};
+
+// The tile shape and the parts of K.  K is only cut where K > N, the projection back to the model width, which has few
+// tiles and a long K (8192 x 28672, us at 128 / 350 / 1024 rows: 244 / 230 / 244 before, 64 / 96 / 182 now); the
+// projections in front of it keep one order of their sums, that of the fused launch.  At least eight slabs a part.
+TilePlan plan_tile(int M, int N, int K, int share, bool may_split) {
+  TilePlan best{2, 1, tile_cost((int64_t)((M + 255) / 256) * ((N + F8_TBN - 1) / F8_TBN), 1, share, K, 1.0, 0)};
+  for (const RingTile& ring : F8_RINGS) {
+    const int64_t tiles = (int64_t)((M + 32 * ring.tm - 1) / (32 * ring.tm)) * ((N + 255) / 256);
+    for (int s = 1; s <= F8_MAX_SPLIT; ++s) {
+      if (s > 1 && (!may_split || K <= N || K / FBK < 8 * s || tiles * s * share > 256)) break;
+      const TilePlan plan{ring.variant, s, tile_cost(tiles, s, share, K, ring.per_slab, ring.tm)};
+      if (plan.cost < best.cost) best = plan;
+    }
+  }
+  return best;
+}
+
+int check_gemm(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
+               const float* w_scale, int M, int N, int K) {
+  if (!A || !W || !C || !a_scale || !w_scale) return DFHIP_ERR_NULL_POINTER;
+  if (M < 1 || N < 1 || K < 1 || K % FBK != 0 || N % 8 != 0) return DFHIP_ERR_BAD_SHAPE;
+  if (lda < K || ldw < K || ldc < N) return DFHIP_ERR_BAD_STRIDE;
+  if (lda >= (1 << 23) || ldw >= (1 << 23)) return DFHIP_ERR_BAD_STRIDE;   // 256 rows of a tile within 32-bit byte offsets
+  if (lda % 16 || ldw % 16 || ldc % 8 || !dfhip_aligned16(A) || !dfhip_aligned16(W) || !dfhip_aligned16(C) ||
+      !dfhip_aligned16(w_scale))
+    return DFHIP_ERR_BAD_ALIGNMENT;
+  return DFHIP_OK;
+}
 
 int check_q(const void* x, int64_t ld, int M, int D) {
   if (!x) return DFHIP_ERR_NULL_POINTER;
@@ -756,27 +871,55 @@ extern "C" int dfhip_silu_mul_absmax_bf16(const void* gate, int64_t ld_gate, con
 extern "C" int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
                                          int64_t ldc, const float* a_scale, const float* w_scale, int M, int N,
                                          int K, int variant, dfhip_stream_t stream) {
-  if (!A || !W || !C || !a_scale || !w_scale) return DFHIP_ERR_NULL_POINTER;
-  if (M < 1 || N < 1 || K < 1 || K % FBK != 0 || N % 8 != 0) return DFHIP_ERR_BAD_SHAPE;
-  if (lda < K || ldw < K || ldc < N) return DFHIP_ERR_BAD_STRIDE;
-  if (lda >= (1 << 23) || ldw >= (1 << 23)) return DFHIP_ERR_BAD_STRIDE;   // 256 rows of a tile within 32-bit byte offsets
-  if (lda % 16 || ldw % 16 || ldc % 8 || !dfhip_aligned16(A) || !dfhip_aligned16(W) || !dfhip_aligned16(C) ||
-      !dfhip_aligned16(w_scale))
-    return DFHIP_ERR_BAD_ALIGNMENT;
+  if (int rc = check_gemm(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (variant < 0 && stream_planned(M, N, K))
     return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
-  if (variant < 0) {   // the planned kernel
-    const int64_t big_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-    variant = 1;
-    if (M > 128 && N > 128 && big_tiles >= 32)
-      variant = fp8_round_fill(M, N, F8_TBN) > fp8_round_fill(M, N, 256) + 0.05 ? 2 : 0;
-  }
+  if (variant < 0) variant = plan_tile(M, N, K, 1, false).variant;
   switch (variant) {
-    case 0: return launch_fp8_ring(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
+    case 0: return launch_fp8_ring<8, false>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, nullptr, s);
     case 1: return launch_fp8<128, 128>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
     case 2: return launch_fp8_ring224(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
+    case 3: return launch_fp8_ring<6, false>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, nullptr, s);
+    case 4: return launch_fp8_ring<4, false>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, nullptr, s);
     default: return DFHIP_ERR_BAD_ARGUMENT;
+  }
+}
+
+extern "C" int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k) {
+  if (!variant || !split_k) return DFHIP_ERR_NULL_POINTER;
+  if (M < 1 || N < 1 || K < 1) return DFHIP_ERR_BAD_SHAPE;
+  if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
+  *variant = -1;
+  *split_k = 1;
+  if (stream_planned(M, N, K)) return DFHIP_OK;
+  const TilePlan plan = plan_tile(M, N, K, share, true);
+  *variant = plan.variant;
+  *split_k = plan.split_k;
+  return DFHIP_OK;
+}
+
+extern "C" size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k) {
+  const int tm = ring_blocks(variant);
+  if (M < 1 || N < 1 || split_k < 2 || split_k > F8_MAX_SPLIT || !tm) return 0;
+  const size_t tiles = (size_t)((M + 32 * tm - 1) / (32 * tm)) * ((N + 255) / 256);
+  return dfhip_counter_area(tiles) + tiles * split_k * (size_t)(32 * tm) * 256 * sizeof(float);
+}
+
+extern "C" int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
+                                        const float* a_scale, const float* w_scale, int M, int N, int K, int variant,
+                                        int split_k, void* workspace, size_t workspace_bytes, dfhip_stream_t stream) {
+  if (int rc = check_gemm(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K)) return rc;
+  const int tm = ring_blocks(variant);
+  if (!tm || split_k < 2 || split_k > F8_MAX_SPLIT || K / FBK < 2 * split_k) return DFHIP_ERR_BAD_ARGUMENT;
+  if (!workspace) return DFHIP_ERR_NULL_POINTER;
+  if (!dfhip_aligned16(workspace)) return DFHIP_ERR_BAD_ALIGNMENT;
+  if (workspace_bytes < dfhip_gemm_fp8_splitk_workspace_bytes(M, N, variant, split_k)) return DFHIP_ERR_BAD_ARGUMENT;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (tm) {
+    case 8: return launch_fp8_ring<8, true>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, split_k, workspace, s);
+    case 6: return launch_fp8_ring<6, true>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, split_k, workspace, s);
+    default: return launch_fp8_ring<4, true>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, split_k, workspace, s);
   }
 }
 
@@ -796,8 +939,23 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, co
   if (stream_planned(M, I, K))
     return dfhip_stream_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I,
                                     K, static_cast<hipStream_t>(stream));
-  return launch_fp8_ring_fused(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I,
-                               K, static_cast<hipStream_t>(stream));
+  // the height of the tile that costs least in rounds (see tile_cost); every height adds in the same order
+  const RingTile* ring = &F8_RINGS[0];
+  double least = 0.0;
+  for (const RingTile& r : F8_RINGS) {
+    const int64_t tiles = (int64_t)((M + 32 * r.tm - 1) / (32 * r.tm)) * ((I + 127) / 128);
+    const double cost = tile_cost(tiles, 1, 1, K, r.per_slab, r.tm);
+    if (&r == &F8_RINGS[0] || cost < least) { ring = &r; least = cost; }
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (ring->tm) {
+    case 8: return launch_fp8_ring_fused<8>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax,
+                                            M, I, K, s);
+    case 6: return launch_fp8_ring_fused<6>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax,
+                                            M, I, K, s);
+    default: return launch_fp8_ring_fused<4>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale,
+                                             amax, M, I, K, s);
+  }
 }
 
 extern "C" int dfhip_gemm_fp8_nt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,

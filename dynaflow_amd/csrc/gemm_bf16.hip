@@ -223,14 +223,6 @@ constexpr int EROW = 272;    // padded row of the epilogue staging area (bytes)
 // Split-K: the bound of the last part's wait for the others (sleeps of about a microsecond: a second).
 constexpr int SPLITK_SPIN_LIMIT = 1 << 20;
 
-// Split-K workspaces start with the arrival counters.  Both split-K kernels use the same size of
-// counter area for a workspace (at least 4 KiB), so that the fp32 blocks one of them leaves behind
-// never lie where the other expects counters that are zero.
-size_t counter_area(size_t tiles) {
-  const size_t need = ((tiles * sizeof(int)) + 255) & ~(size_t)255;
-  return need > 4096 ? need : 4096;
-}
-
 // Which output the W row at position `pos` of a run of paired MFMA blocks belongs to.  MFMA block j = pos / 16
 // hands lane quad q = (pos % 16) / 4 the four outputs r = pos % 4; blocks are paired (0,1), (2,3), ... over 32
 // outputs each, and quad q owns outputs 8q .. 8q+3 of a pair through the even block and 8q+4 .. 8q+7 through the
@@ -588,7 +580,7 @@ int launch_ring(const void* A, int64_t lda, const void* W, const void* W2, int64
   float* partials = nullptr;
   int lead_slabs = K / BK;
   if (split_k > 1) {
-    partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + counter_area((size_t)tiles_m * tiles_n));
+    partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area((size_t)tiles_m * tiles_n));
     lead_slabs = (K / BK) / split_k;   // an even split measured best (a smaller share for the parts that only leave a block did not pay)
   }
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(RTHREADS), RING_LDS, stream,
@@ -1521,7 +1513,7 @@ gemm_bf16_skinny_wide_kernel(const uint16_t* __restrict__ A, const uint16_t* __r
 }
 
 size_t skinny_tiles(int M, int N) { return (size_t)((M + SK_BM - 1) / SK_BM) * ((N + SK_BN - 1) / SK_BN); }
-size_t skinny_counter_bytes(int M, int N) { return counter_area(skinny_tiles(M, N)); }
+size_t skinny_counter_bytes(int M, int N) { return dfhip_counter_area(skinny_tiles(M, N)); }
 
 template <bool FUSED>
 int launch_skinny(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc, int M,
@@ -1701,7 +1693,7 @@ extern "C" int dfhip_gemm_bf16_nt(const void* A, int64_t lda, const void* W, int
 extern "C" size_t dfhip_gemm_bf16_splitk_workspace_bytes(int M, int N, int split_k) {
   if (M < 1 || N < 1 || split_k < 2) return 0;
   const size_t tiles = (size_t)((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN);
-  const size_t ring = counter_area(tiles) + tiles * split_k * (size_t)RBM * RBN * sizeof(float);
+  const size_t ring = dfhip_counter_area(tiles) + tiles * split_k * (size_t)RBM * RBN * sizeof(float);
   if (M > SK_MAX_M) return ring;
   // the weight-streaming kernel (M <= 1024) has its own layout; a caller sizes for whichever is used
   const size_t skinny = skinny_counter_bytes(M, N) + skinny_tiles(M, N) * split_k * (size_t)SK_BM * SK_BN * sizeof(float);
@@ -1858,7 +1850,7 @@ extern "C" int dfhip_gemm_bf16_nt_splitk_static(const void* A, int64_t lda, cons
     // poison the next one.  The two split-K kernels size their counter areas differently; the larger one is
     // cleared (what lies behind the counters are partial blocks, written before they are read).
     const size_t tiles_ring = (size_t)((M + RBM - 1) / RBM) * ((N + RBN - 1) / RBN);
-    size_t counters = counter_area(tiles_ring);
+    size_t counters = dfhip_counter_area(tiles_ring);
     if (M <= SK_MAX_M && skinny_counter_bytes(M, N) > counters) counters = skinny_counter_bytes(M, N);
     if (int rc = dfhip_fill_u32(ws, 0u, (int64_t)(counters / 4), stream)) return rc;
   }

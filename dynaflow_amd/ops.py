@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import math
 import contextlib
+import ctypes
 import os
 import weakref
 import threading
@@ -169,8 +170,6 @@ def _splitk_workspace(device: torch.device, stream: int, nbytes: int) -> torch.T
 
 def _plan_bf16(lib, M: int, N: int, K: int) -> tuple[int, int]:
     """(kernel variant, split of K) for a bf16 GEMM, for as many launches side by side as the forward declared."""
-    import ctypes
-
     variant, split_k = ctypes.c_int(0), ctypes.c_int(1)
     _cabi.check("dfhip_gemm_bf16_plan_shared", lib.dfhip_gemm_bf16_plan_shared(
         M, N, K, _side_by_side(), ctypes.byref(variant), ctypes.byref(split_k)))
@@ -791,11 +790,27 @@ def _linear_fp8_impl(x_q, w_q, x_scale, w_scale, variant: int = -1, to_output: b
         raise RuntimeError("linear_fp8: shape mismatch")
     out = _new_output(M, N, torch.bfloat16, x_q.device, to_output)
     if M > 0:
-        rc = lib.dfhip_gemm_fp8_nt_variant(
-            a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N,
-            x_scale.data_ptr(), w_scale.contiguous().data_ptr(), M, N, K, variant, _stream(),
-        )
-        _cabi.check("dfhip_gemm_fp8_nt_variant", rc)
+        stream, split_k = _stream(), 1
+        if variant < 0:
+            planned, parts = ctypes.c_int(-1), ctypes.c_int(1)
+            _cabi.check("dfhip_gemm_fp8_plan_shared", lib.dfhip_gemm_fp8_plan_shared(
+                M, N, K, _side_by_side(), ctypes.byref(planned), ctypes.byref(parts)))
+            if SPLIT_K_ENABLED or parts.value == 1:
+                variant, split_k = planned.value, parts.value
+        scale = w_scale.contiguous()
+        if split_k > 1:
+            ws = _splitk_workspace(x_q.device, stream, lib.dfhip_gemm_fp8_splitk_workspace_bytes(M, N, variant, split_k))
+            rc = lib.dfhip_gemm_fp8_nt_splitk(
+                a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, x_scale.data_ptr(), scale.data_ptr(), M, N, K,
+                variant, split_k, ws.data_ptr(), ws.numel(), stream,
+            )
+            _cabi.check("dfhip_gemm_fp8_nt_splitk", rc)
+        else:
+            rc = lib.dfhip_gemm_fp8_nt_variant(
+                a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, x_scale.data_ptr(), scale.data_ptr(), M, N, K,
+                variant, stream,
+            )
+            _cabi.check("dfhip_gemm_fp8_nt_variant", rc)
     return out.view(*x_q.shape[:-1], N)
 
 

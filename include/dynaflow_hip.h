@@ -215,12 +215,24 @@ int dfhip_gemm_fp8_nt(const void* A, int64_t lda, const void* W, int64_t ldw, vo
                       int64_t ldc, const float* a_scale, const float* w_scale, int M, int N,
                       int K, dfhip_stream_t stream);
 /* The same with an explicit kernel, for tuning and tests (the choice has no counterpart in the
- * reference): 0 = 256x256 LDS-DMA ring,
+ * reference): 0, 3, 4 = LDS-DMA ring with tiles of 256, 192 and 128 rows by 256 columns,
  * 1 = register-staged 128x128, 2 = 256x224 LDS-DMA ring (N = 7 * 2^k), negative =
  * the choice dfhip_gemm_fp8_nt makes. */
 int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
                               const float* a_scale, const float* w_scale, int M, int N, int K, int variant,
                               dfhip_stream_t stream);
+/* The same with K cut into split_k parts (2 .. 16, at least two slabs of 128 each), for outputs of too few tiles to
+ * fill the GPU; variant 0, 3 or 4.  workspace: dfhip_gemm_fp8_splitk_workspace_bytes bytes, 16-byte aligned, whose
+ * arrival counters (4 bytes a tile at its start) are zero; they are left zero.  Launches that may overlap need one
+ * each.  The parts are added in part order: the same bits in every run.
+ * dfhip_gemm_fp8_plan_shared: the variant and split for `share` launches of this shape side by side (variant < 0: the
+ * launch without a split decides).  K is only cut where K > N (the projection back to the model width): the projections
+ * in front of it keep one order of their sums, that of dfhip_gemm_fp8_gate_up_silu_absmax. */
+int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
+size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k);
+int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
+                             const float* a_scale, const float* w_scale, int M, int N, int K, int variant, int split_k,
+                             void* workspace, size_t workspace_bytes, dfhip_stream_t stream);
 /* Gate and up projection of the fp8 MLP block with the SiLU*mul as the epilogue of ONE launch:
  *   g = bf16(a_scale * wg_scale[i] * A W_gate^T), u likewise with W_up,
  *   act[m,i] = bf16( silu(g) * u ),   amax[0] = max(amax[0], max |act|)

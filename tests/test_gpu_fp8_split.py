@@ -1,0 +1,112 @@
+"""The fp8 ring tiles of 256, 192 and 128 rows, and K cut into parts that meet in a workspace."""
+import ctypes
+
+import pytest
+import torch
+
+from dynaflow_amd import _cabi
+
+F8 = torch.float8_e4m3fn
+
+
+def randn(shape, seed, std=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(shape, generator=g, device="cuda") * std).bfloat16()
+
+
+def operands(M, N, K):
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
+
+    xq, xs = ops.quant_fp8(randn((M, K), 1))
+    return (xq, *quantize_weight_per_channel(randn((N, K), 2, 0.05)), xs)
+
+
+def test_planned_fp8_splits_are_launchable():
+    """Every plan names a kernel and a split that the entry points take, and only projections with K > N are cut."""
+    lib, v, s = _cabi.load(), ctypes.c_int(), ctypes.c_int()
+    cut = 0
+    for M in (1, 16, 64, 65, 128, 129, 192, 193, 350, 700, 1024, 2048, 5000):
+        for N, K in ((8192, 28672), (28672, 8192), (4096, 14336), (14336, 4096), (8, 128), (264, 1152), (2048, 4096)):
+            for share in (1, 2, 4, 16):
+                assert lib.dfhip_gemm_fp8_plan_shared(M, N, K, share, ctypes.byref(v), ctypes.byref(s)) == 0
+                assert v.value in (-1, 0, 1, 2, 3, 4) and 1 <= s.value <= 16
+                if s.value > 1:
+                    cut += 1
+                    assert K > N and K // 128 >= 8 * s.value
+                    assert lib.dfhip_gemm_fp8_splitk_workspace_bytes(M, N, v.value, s.value) > 0
+    assert cut > 20
+    assert lib.dfhip_gemm_fp8_splitk_workspace_bytes(100, 256, 1, 2) == 0       # a kernel that does not split
+    args = (16, 1024, 16, 1024, 16, 8, 16, 16, 1, 8, 1024)
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 4, 2, None, 0, None) == -1       # no workspace
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 4, 2, 16, 100, None) == -7       # too small
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 1, 2, 16, 1 << 30, None) == -7   # not a ring tile
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 4, 5, 16, 1 << 30, None) == -7   # less than two slabs a part
+
+
+# rows at the edges of 128, 192 and 256-row tiles, ragged columns, 1 slab of K, an odd number, an even one
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128), (65, 264, 384), (128, 256, 256), (129, 520, 640), (192, 1032, 1152),
+                                   (193, 264, 384), (385, 1544, 1024)])
+@pytest.mark.parametrize("variant", [0, 3, 4])
+def test_fp8_tile_heights_add_in_one_order(M, N, K, variant):
+    from dynaflow_amd import ops
+
+    xq, wq, ws, xs = operands(M, N, K)
+    got = ops.linear_fp8_variant(xq, wq, xs, ws, variant)
+    want = (xq.float() * xs) @ (wq.float() * ws[:, None]).t()
+    assert (got.float() - want).abs().max().item() <= 2.0 ** -7 * want.abs().max().item()
+    assert torch.equal(got, ops.linear_fp8_variant(xq, wq, xs, ws, 1))
+
+
+# parts of two slabs (the shortest), of uneven lengths (9 slabs in 2 and 4 parts, 37 in 16), ragged tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", [0, 3, 4])
+@pytest.mark.parametrize("M,N,K,split", [(1, 8, 512, 2), (200, 264, 1152, 2), (130, 520, 1152, 4), (390, 1032, 4736, 16),
+                                         (512, 2048, 4096, 3)])
+def test_fp8_split_launch(M, N, K, split, variant):
+    """Against the fp32 product: bf16 rounding of the result (2^-8 of it) and the fp32 sums; the same bits in every run,
+    with counters left at zero in between."""
+    lib = _cabi.load()
+    xq, wq, ws, xs = operands(M, N, K)
+    nbytes = lib.dfhip_gemm_fp8_splitk_workspace_bytes(M, N, variant, split)
+    workspace = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+    want = (xq.float() * xs) @ (wq.float() * ws[:, None]).t()
+    runs = []
+    for _ in range(3):
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert lib.dfhip_gemm_fp8_nt_splitk(
+            xq.data_ptr(), K, wq.data_ptr(), K, out.data_ptr(), N, xs.data_ptr(), ws.data_ptr(), M, N, K, variant, split,
+            workspace.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream) == 0
+        runs.append(out)
+    assert (runs[0].float() - want).abs().max().item() <= 2.0 ** -7 * want.abs().max().item()
+    assert torch.equal(runs[0], runs[1]) and torch.equal(runs[0], runs[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,I,K", [(65, 1024, 2048), (128, 3592, 512), (180, 2048, 1024), (350, 7168, 384), (600, 264, 640)])
+def test_fused_fp8_tile_heights(M, I, K):
+    """The fused launch with tiles of 128, 192 and 256 rows: codes and scale of the separate operators."""
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
+
+    xq, wq, ws, xs = operands(M, I, K)
+    uq, us = quantize_weight_per_channel(randn((I, K), 3, 0.05))
+    q, scale = ops.gate_up_silu_quant_fp8(xq, wq, uq, xs, ws, us)
+    want_q, want_scale = ops.silu_mul_quant_fp8(ops.linear_fp8_variant(xq, wq, xs, ws, 1),
+                                                ops.linear_fp8_variant(xq, uq, xs, us, 1))
+    assert torch.equal(scale, want_scale) and torch.equal(q.view(torch.uint8), want_q.view(torch.uint8))
+
+
+@pytest.mark.gpu
+def test_split_launches_of_both_types_share_a_workspace():
+    """What an fp8 launch leaves in the workspace of a stream is nothing a bf16 launch takes for a counter."""
+    from dynaflow_amd import ops
+
+    xq, wq, ws, xs = operands(130, 1032, 4096)
+    x, w = randn((17, 4096), 4), randn((4096, 4096), 5, 0.05)      # 2 parts, up to 256 counters
+    want8, want16 = (xq.float() * xs) @ (wq.float() * ws[:, None]).t(), x.float() @ w.float().t()
+    for _ in range(2):
+        got8, got16 = ops.linear_fp8(xq, wq, xs, ws), ops.linear(x, w)
+        assert (got8.float() - want8).abs().max().item() <= 2.0 ** -7 * want8.abs().max().item()
+        assert (got16.float() - want16).abs().max().item() <= 2.0 ** -7 * want16.abs().max().item()
