@@ -23,6 +23,13 @@
 // by far; a workgroup in which a row's sum of exponentials ends beyond SAFE_SUM runs the safe pass behind the
 // fast one (running maximum, rescaling whenever the maximum moves by more than 2^RESCALE_THRESHOLD) and
 // stores its rows again.
+//
+// Sequences whose length is no multiple of 64 (RAGGED) end in a block that is partly there: its missing key rows
+// re-read the sequence's last one (only rows past the sequence see them: the causal mask covers the others), its
+// missing values are zeros that pack_v_kernel wrote, and rows past the sequence are not stored.  A form of its own,
+// so that whole sequences do not select between two sets of key offsets.  Operator with pack_v, 32 heads on 8, us (PyTorch's
+// fused attention, which took these lengths before): 1 x 333 21 (32), 1 x 777 30 (57), 4 x 333 25 (58), 4 x 1500 105 (382),
+// 4 x 2047 165 (543); level with it below about 100 tokens.  4 x 2048 through either form 154 - 158.
 #include <type_traits>
 
 #include "dfhip_common.h"
@@ -117,7 +124,7 @@ DFHIP_DEVICE void map_workgroup(int B, int S, int q_heads, int kv_heads, int& b,
 // pinned - the P V MFMAs of tile t, the score MFMAs of tile t+2, and the softmax (VALU) of tile t+1.  Score
 // tiles and probability fragments alternate between two register sets (A: even tiles, B: odd tiles).  K/V
 // blocks live in a ring of 4 stages: block j (V in use), j+1 (K in use), j+2 and j+3 landing.
-template <int HPW>
+template <int HPW, bool RAGGED>
 __global__ void __launch_bounds__(256)
 causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint16_t* __restrict__ k, int64_t ld_k,
                         const uint16_t* __restrict__ v_blk, uint16_t* __restrict__ out, int64_t ld_o, int B, int S,
@@ -140,10 +147,12 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
   // ---- DMA sources: uniform bases that advance by one block, per-lane offsets fixed for the whole kernel
   // (per block: 4 K instructions + 4 V instructions per wave, 1 KiB each)
   const uint8_t* kseq = reinterpret_cast<const uint8_t*>(k + (int64_t)b * S * ld_k + (int64_t)kvh * AD);
-  const uint8_t* vseq = reinterpret_cast<const uint8_t*>(v_blk) + ((int64_t)(b * kv_heads + kvh) * S) * (AD * 2) +
+  const int s_blocks = RAGGED ? (S + KVB - 1) / KVB * KVB : S;   // positions of a sequence in v_blk
+  const uint8_t* vseq = reinterpret_cast<const uint8_t*>(v_blk) + ((int64_t)(b * kv_heads + kvh) * s_blocks) * (AD * 2) +
                         wave * 4096;
   const int64_t k_block_bytes = (int64_t)KVB * ld_k * 2;
-  uint32_t k_off[4], v_off[4];
+  uint32_t k_off[4], k_off_tail[4], v_off[4];
+  const int tail_block = S / KVB, tail_last = S - 1 - tail_block * KVB;   // RAGGED: the partial block, its last position
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int row = (wave * 4 + t) * 4 + (lane >> 4);          // LDS row 0..63 (MFMA row order)
@@ -151,13 +160,18 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
     const int pos = (row & 32) | pi(row & 31);                 // position inside the block
     const int chunk = (slot & 8) | ((slot & 7) ^ (row & 7));   // logical 16-byte chunk held by this slot
     k_off[t] = (uint32_t)(pos * ld_k * 2 + chunk * 16);
+    if (RAGGED) k_off_tail[t] = (uint32_t)((pos < tail_last ? pos : tail_last) * ld_k * 2 + chunk * 16);
     v_off[t] = (uint32_t)(t * 1024 + lane * 16);
   }
+  auto dma_k = [&](int stage, int j, int t) {
+    const uint32_t off = RAGGED && j == tail_block ? k_off_tail[t] : k_off[t];
+    dma16_base(stage * STAGE_BYTES + (wave * 4 + t) * 1024, kseq + j * k_block_bytes, off);
+  };
   // piece t of block j: 4 K instructions (t = 0..3), then 4 V instructions; nothing past the last block
   auto issue_piece = [&](int j, int t) {
     if (j > last_block_wg) return;
     const int stage = j % STAGES;
-    if (t < 4) dma16_base(stage * STAGE_BYTES + (wave * 4 + t) * 1024, kseq + j * k_block_bytes, k_off[t]);
+    if (t < 4) dma_k(stage, j, t);
     else dma16_base(stage * STAGE_BYTES + K_BYTES + (wave * 4 + t - 4) * 1024, vseq + (int64_t)j * (KVB * AD * 2),
                     v_off[t - 4]);
   };
@@ -172,7 +186,7 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
   auto issue_piece_or_dummy = [&](int j, int t) {
     const int src = j < last_block_wg ? j : last_block_wg;
     const int stage = j % STAGES;
-    if (t < 4) dma16_base(stage * STAGE_BYTES + (wave * 4 + t) * 1024, kseq + src * k_block_bytes, k_off[t]);
+    if (t < 4) dma_k(stage, src, t);
     else dma16_base(stage * STAGE_BYTES + K_BYTES + (wave * 4 + t - 4) * 1024, vseq + (int64_t)src * (KVB * AD * 2),
                     v_off[t - 4]);
   };
@@ -510,42 +524,45 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
   store_rows(safe_sum);
 }
 
-// v[T, ld_v] (head h at column h*128) -> v_blk[B][kv_heads][S/8][128][8]
+// v[T, ld_v] (head h at column h*128) -> v_blk[B][kv_heads][pbs][128][8], pbs = S / 8 or, ragged, the eighths of
+// whole blocks of 64 positions; positions past the sequence are zeros
 __global__ void __launch_bounds__(128)
-pack_v_kernel(const uint16_t* __restrict__ v, int64_t ld_v, uint16_t* __restrict__ v_blk, int S, int kv_heads) {
-  const int pbs = S / 8;
+pack_v_kernel(const uint16_t* __restrict__ v, int64_t ld_v, uint16_t* __restrict__ v_blk, int S, int pbs,
+              int kv_heads) {
   const int pb = blockIdx.x % pbs;
   const int h = (blockIdx.x / pbs) % kv_heads;
   const int b = blockIdx.x / (pbs * kv_heads);
   const int d = threadIdx.x;
-  const uint16_t* src = v + ((int64_t)b * S + pb * 8) * ld_v + (int64_t)h * AD + d;
+  const uint16_t* src = v + (int64_t)b * S * ld_v + (int64_t)h * AD + d;
+  auto value = [&](int pos) { return pos < S ? (uint32_t)src[pos * ld_v] : 0u; };
   uint32_t w[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = (uint32_t)src[(2 * i) * ld_v] | ((uint32_t)src[(2 * i + 1) * ld_v] << 16);
+  for (int i = 0; i < 4; ++i) w[i] = value(pb * 8 + 2 * i) | (value(pb * 8 + 2 * i + 1) << 16);
   u32x4 o = {w[0], w[1], w[2], w[3]};
   *reinterpret_cast<u32x4*>(v_blk + ((((int64_t)b * kv_heads + h) * pbs + pb) * AD + d) * 8) = o;
 }
 
-}  // namespace
-
-extern "C" int dfhip_pack_v_bf16(const void* v, int64_t ld_v, void* v_blk, int B, int S, int kv_heads, int head_dim,
-                                 dfhip_stream_t stream) {
+int pack_v(const void* v, int64_t ld_v, void* v_blk, int B, int S, int kv_heads, int head_dim, bool ragged,
+           hipStream_t stream) {
   if (!v || !v_blk) return DFHIP_ERR_NULL_POINTER;
-  if (B < 1 || S < 8 || S % 8 != 0 || kv_heads < 1 || head_dim != AD ||
-      (int64_t)B * kv_heads * (S / 8) >= (int64_t)1 << 31)
+  if (B < 1 || S < (ragged ? 1 : 8) || (!ragged && S % 8 != 0) || S > INT32_MAX - KVB || kv_heads < 1 || head_dim != AD)
     return DFHIP_ERR_BAD_SHAPE;
+  const int pbs = ragged ? (S + KVB - 1) / KVB * (KVB / 8) : S / 8;
+  if ((int64_t)B * kv_heads * pbs >= (int64_t)1 << 31) return DFHIP_ERR_BAD_SHAPE;
   if (ld_v < (int64_t)kv_heads * AD) return DFHIP_ERR_BAD_STRIDE;
   if (!dfhip_aligned16(v_blk)) return DFHIP_ERR_BAD_ALIGNMENT;
-  hipLaunchKernelGGL(pack_v_kernel, dim3(B * kv_heads * (S / 8)), dim3(128), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(v), ld_v, static_cast<uint16_t*>(v_blk), S, kv_heads);
+  hipLaunchKernelGGL(pack_v_kernel, dim3(B * kv_heads * pbs), dim3(128), 0, stream, static_cast<const uint16_t*>(v), ld_v,
+                     static_cast<uint16_t*>(v_blk), S, pbs, kv_heads);
   return dfhip_check_launch();
 }
 
-extern "C" int dfhip_causal_attention_bf16(const void* q, int64_t ld_q, const void* k, int64_t ld_k,
-                                           const void* v_blk, void* out, int64_t ld_o, int B, int S, int q_heads,
-                                           int kv_heads, int head_dim, float scale, dfhip_stream_t stream) {
+template <bool RAGGED>
+int causal_attention(const void* q, int64_t ld_q, const void* k, int64_t ld_k, const void* v_blk, void* out,
+                     int64_t ld_o, int B, int S, int q_heads, int kv_heads, int head_dim, float scale,
+                     hipStream_t stream) {
   if (!q || !k || !v_blk || !out) return DFHIP_ERR_NULL_POINTER;
-  if (B < 1 || S < KVB || S % KVB != 0 || q_heads < 1 || kv_heads < 1 || q_heads % kv_heads != 0 || head_dim != AD)
+  if (B < 1 || S < (RAGGED ? 1 : KVB) || (!RAGGED && S % KVB != 0) || S > INT32_MAX - 4 * WAVE_ROWS || q_heads < 1 ||
+      kv_heads < 1 || q_heads % kv_heads != 0 || head_dim != AD)
     return DFHIP_ERR_BAD_SHAPE;
   const int group = q_heads / kv_heads;
   const int hpw = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;      // query heads per workgroup
@@ -560,11 +577,10 @@ extern "C" int dfhip_causal_attention_bf16(const void* q, int64_t ld_q, const vo
     return DFHIP_ERR_BAD_ALIGNMENT;
   auto launch = [&](auto heads_per_workgroup) {
     constexpr int HPW = decltype(heads_per_workgroup)::value;
+    auto kernel = causal_attention_kernel<HPW, RAGGED>;
     static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
-    if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(causal_attention_kernel<HPW>), ATT_LDS, lds_opted_in))
-      return rc;
-    hipLaunchKernelGGL(causal_attention_kernel<HPW>, dim3((unsigned)groups), dim3(256), ATT_LDS,
-                       static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(q), ld_q,
+    if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), ATT_LDS, lds_opted_in)) return rc;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(256), ATT_LDS, stream, static_cast<const uint16_t*>(q), ld_q,
                        static_cast<const uint16_t*>(k), ld_k, static_cast<const uint16_t*>(v_blk),
                        static_cast<uint16_t*>(out), ld_o, B, S, q_heads, kv_heads, scale * 1.4426950408889634f);
     return dfhip_check_launch();
@@ -572,4 +588,30 @@ extern "C" int dfhip_causal_attention_bf16(const void* q, int64_t ld_q, const vo
   if (hpw == 4) return launch(std::integral_constant<int, 4>{});
   if (hpw == 2) return launch(std::integral_constant<int, 2>{});
   return launch(std::integral_constant<int, 1>{});
+}
+
+}  // namespace
+
+extern "C" int dfhip_pack_v_bf16(const void* v, int64_t ld_v, void* v_blk, int B, int S, int kv_heads, int head_dim,
+                                 dfhip_stream_t stream) {
+  return pack_v(v, ld_v, v_blk, B, S, kv_heads, head_dim, false, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int dfhip_pack_v_ragged_bf16(const void* v, int64_t ld_v, void* v_blk, int B, int S, int kv_heads,
+                                        int head_dim, dfhip_stream_t stream) {
+  return pack_v(v, ld_v, v_blk, B, S, kv_heads, head_dim, true, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int dfhip_causal_attention_bf16(const void* q, int64_t ld_q, const void* k, int64_t ld_k,
+                                           const void* v_blk, void* out, int64_t ld_o, int B, int S, int q_heads,
+                                           int kv_heads, int head_dim, float scale, dfhip_stream_t stream) {
+  return causal_attention<false>(q, ld_q, k, ld_k, v_blk, out, ld_o, B, S, q_heads, kv_heads, head_dim, scale,
+                                 static_cast<hipStream_t>(stream));
+}
+
+extern "C" int dfhip_causal_attention_ragged_bf16(const void* q, int64_t ld_q, const void* k, int64_t ld_k,
+                                                  const void* v_blk, void* out, int64_t ld_o, int B, int S, int q_heads,
+                                                  int kv_heads, int head_dim, float scale, dfhip_stream_t stream) {
+  return causal_attention<true>(q, ld_q, k, ld_k, v_blk, out, ld_o, B, S, q_heads, kv_heads, head_dim, scale,
+                                static_cast<hipStream_t>(stream));
 }

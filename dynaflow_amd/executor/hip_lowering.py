@@ -9,7 +9,8 @@ it deep-copies the sub-``GraphModule`` and replaces
 * ``rms_norm(x, (H,), w, eps)`` (bf16, last dim)      -> ``dynaflow_hip.rms_norm``
 * ``apply_rope(t, cos, sin)`` (bf16, one graph node)  -> ``dynaflow_hip.rope``
 * ``attend_and_append(qkv, k_cache, v_cache, ...)``   -> ``dynaflow_hip.decode_attention``
-* ``causal_gqa_attention(q, k, v)`` (bf16, d 128, S%64) -> ``dynaflow_hip.causal_attention``
+* ``causal_gqa_attention(q, k, v)`` (bf16, d 128)    -> ``dynaflow_hip.causal_attention`` or, S % 64 != 0,
+  ``causal_attention_ragged``; sequences shorter than a block of 64 stay on the tensor operations
 
 * ``add(r, linear(x, w))`` (bf16, same shapes, the linear used once) -> ``dynaflow_hip.linear_add``
   (the residual addition as the GEMM's epilogue; same roundings, same bits)
@@ -76,6 +77,15 @@ def _traced_int(value: Any) -> int | None:
         hint = getattr(value.node, "hint", None)
         return int(hint) if hint is not None else None
     return value if isinstance(value, int) else None
+
+
+def _one_causal_batch(q: Any, k: Any, v: Any) -> bool:
+    """What the ragged attention kernel takes: bf16 q, k, v of the same sequences, whole groups of query heads."""
+    if not all(isinstance(t, torch.Tensor) and t.dtype == torch.bfloat16 and t.dim() == 4 for t in (q, k, v)):
+        return False
+    sizes = [[_traced_int(n) for n in t.shape] for t in (q, k, v)]
+    return (sizes[1] == sizes[2] and sizes[0][:2] == sizes[1][:2] and sizes[0][3] == sizes[1][3]
+            and sizes[0][2] % sizes[1][2] == 0)
 
 
 def _linear_supported(x: Any, w: Any) -> bool:
@@ -208,10 +218,13 @@ def lower_to_hip(gm: fx.GraphModule, fuse_silu_epilogue: bool = False,
         if not isinstance(et, torch.Tensor) or et.dtype != torch.bfloat16 or et.dim() != 4:
             continue
         seq, d = _traced_int(et.shape[1]), _static_int(et.shape[3])
-        if seq is None or seq % 64 or d != 128:
+        if seq is None or seq < 64 or d != 128:
+            continue
+        if seq % 64 and not _one_causal_batch(*(_example(a) for a in node.args)):
             continue
         with graph.inserting_before(node):
-            new = graph.call_function(ops.causal_attention, tuple(node.args))
+            kernel = ops.causal_attention if seq % 64 == 0 else ops.causal_attention_ragged
+            new = graph.call_function(kernel, tuple(node.args))
         new.meta = dict(node.meta)
         node.replace_all_uses_with(new)
         graph.erase_node(node)

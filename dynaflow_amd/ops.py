@@ -46,6 +46,7 @@ _lib.define("transpose_weight(Tensor w) -> Tensor")
 _lib.define("rope(Tensor t, Tensor cos, Tensor sin) -> Tensor")
 _lib.define("rope_pair(Tensor q, Tensor k, Tensor cos, Tensor sin) -> (Tensor, Tensor)")
 _lib.define("causal_attention(Tensor q, Tensor k, Tensor v) -> Tensor")
+_lib.define("causal_attention_ragged(Tensor q, Tensor k, Tensor v) -> Tensor")
 _lib.define("linear_add(Tensor x, Tensor weight, Tensor residual) -> Tensor")
 _lib.define("linear_to_output(Tensor x, Tensor weight) -> Tensor")
 _lib.define("linear_multi(Tensor x, Tensor[] weights) -> Tensor[]")
@@ -531,6 +532,13 @@ def _token_rows(t: torch.Tensor, what: str):
     return t, t.stride(1)
 
 
+def _aligned_rows(t: torch.Tensor, ld: int):
+    """Token rows that start on 16 bytes: a copy where a view's offset or row stride says otherwise."""
+    if t.data_ptr() % 16 or ld % 8:
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t, t.stride(1)
+
+
 # ------------------------------------------------------------------ rope
 def _rope_impl(t: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
     """t [B, S, heads, d] bf16 (contiguous), cos/sin [S, d/2] fp32 -> rotated tensor of the same shape."""
@@ -584,8 +592,11 @@ torch.library.register_fake("dynaflow_hip::rope", lambda t, cos, sin: torch.empt
 
 
 # ------------------------------------------------------ prefill attention
-def _causal_attention_impl(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-    """q [B, S, Hq, 128], k / v [B, S, Hkv, 128] (bf16) -> softmax(q k^T / sqrt(128), causal) v as [B, S, Hq, 128]."""
+def _causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ragged: bool) -> torch.Tensor:
+    """q [B, S, Hq, 128], k / v [B, S, Hkv, 128] (bf16) -> softmax(q k^T / sqrt(128), causal) v as [B, S, Hq, 128].
+
+    ``ragged``: any S; otherwise multiples of 64, whose kernel does without the care for a partial block.
+    """
     _require_device(q, k, v)
     lib = _cabi.load()
     if q.dtype != torch.bfloat16 or k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
@@ -594,27 +605,33 @@ def _causal_attention_impl(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) ->
         raise RuntimeError("causal_attention: q [B,S,Hq,128] and k, v [B,S,Hkv,128] expected")
     B, S, Hq, d = q.shape
     Hkv = k.shape[2]
-    if S % 64 != 0 or Hq % Hkv != 0:
+    if (S % 64 != 0 and not ragged) or Hq % Hkv != 0:
         raise RuntimeError("causal_attention: sequence length must be a multiple of 64, q heads a multiple of kv heads")
     q, ld_q = _token_rows(q, "q")
     k, ld_k = _token_rows(k, "k")
     v, ld_v = _token_rows(v, "v")
+    if ragged:
+        q, ld_q = _aligned_rows(q, ld_q)
+        k, ld_k = _aligned_rows(k, ld_k)
     out = torch.empty((B, S, Hq, d), dtype=q.dtype, device=q.device)
     if B > 0:
-        v_blk = torch.empty((B, Hkv, S // 8, d, 8), dtype=q.dtype, device=q.device)
+        suffix = "_ragged_bf16" if ragged else "_bf16"
+        v_blk = torch.empty((B, Hkv, (S + 63) // 64 * 8, d, 8), dtype=q.dtype, device=q.device)
         stream = _stream()
-        rc = lib.dfhip_pack_v_bf16(v.data_ptr(), ld_v, v_blk.data_ptr(), B, S, Hkv, d, stream)
-        _cabi.check("dfhip_pack_v_bf16", rc)
-        rc = lib.dfhip_causal_attention_bf16(
+        rc = getattr(lib, "dfhip_pack_v" + suffix)(v.data_ptr(), ld_v, v_blk.data_ptr(), B, S, Hkv, d, stream)
+        _cabi.check("dfhip_pack_v" + suffix, rc)
+        rc = getattr(lib, "dfhip_causal_attention" + suffix)(
             q.data_ptr(), ld_q, k.data_ptr(), ld_k, v_blk.data_ptr(), out.data_ptr(), Hq * d, B, S, Hq, Hkv, d,
             1.0 / math.sqrt(d), stream,
         )
-        _cabi.check("dfhip_causal_attention_bf16", rc)
+        _cabi.check("dfhip_causal_attention" + suffix, rc)
     return out
 
 
-_lib.impl("causal_attention", _causal_attention_impl, "CUDA")
-torch.library.register_fake("dynaflow_hip::causal_attention", lambda q, k, v: torch.empty_like(q), lib=_lib)
+_lib.impl("causal_attention", lambda q, k, v: _causal_attention(q, k, v, False), "CUDA")
+_lib.impl("causal_attention_ragged", lambda q, k, v: _causal_attention(q, k, v, True), "CUDA")
+for _name in ("causal_attention", "causal_attention_ragged"):
+    torch.library.register_fake(f"dynaflow_hip::{_name}", lambda q, k, v: torch.empty_like(q), lib=_lib)
 
 
 # ------------------------------------------------------- decode attention
@@ -863,6 +880,7 @@ rope = torch.ops.dynaflow_hip.rope
 rope_pair = torch.ops.dynaflow_hip.rope_pair
 decode_attention = torch.ops.dynaflow_hip.decode_attention
 causal_attention = torch.ops.dynaflow_hip.causal_attention
+causal_attention_ragged = torch.ops.dynaflow_hip.causal_attention_ragged
 linear_add = torch.ops.dynaflow_hip.linear_add
 linear_to_output = torch.ops.dynaflow_hip.linear_to_output
 linear_multi = torch.ops.dynaflow_hip.linear_multi

@@ -304,6 +304,14 @@ int dfhip_causal_attention_bf16(const void* q, int64_t ld_q, const void* k, int6
                                 void* out, int64_t ld_o, int B, int S, int q_heads, int kv_heads, int head_dim,
                                 float scale, dfhip_stream_t stream);
 
+/* The same for sequences of any length S >= 1: v_blk is [B][kv_heads][8 ceil(S/64)][128][8], whole blocks of 64
+ * positions, the ones past S zeros (which dfhip_pack_v_ragged_bf16 writes). */
+int dfhip_pack_v_ragged_bf16(const void* v, int64_t ld_v, void* v_blk, int B, int S, int kv_heads, int head_dim,
+                             dfhip_stream_t stream);
+int dfhip_causal_attention_ragged_bf16(const void* q, int64_t ld_q, const void* k, int64_t ld_k, const void* v_blk,
+                                       void* out, int64_t ld_o, int B, int S, int q_heads, int kv_heads, int head_dim,
+                                       float scale, dfhip_stream_t stream);
+
 /* Decode step against a static KV cache (bf16, head_dim 128).  Cache layout, per
  * sequence slot and kv head, `capacity` positions (capacity % 32 == 0):
  *   k_cache [num_slots][kv_heads][capacity][128]

@@ -45,6 +45,30 @@ def test_causal_attention_against_oracle(ops, B, S, Hq, Hkv):
     assert bool((err < 0.05).all()), err.argmax()
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv", [(1, 1, 4, 1), (2, 63, 1, 1), (1, 65, 2, 1), (3, 127, 8, 2), (2, 129, 4, 1),
+                                        (1, 257, 3, 3), (8, 191, 8, 1), (2, 300, 6, 3), (3, 777, 8, 2), (2, 128, 2, 1),
+                                        (1, 1025, 4, 1)])
+def test_causal_attention_ragged_against_oracle(ops, B, S, Hq, Hkv):
+    """Sequences that end inside a block of 64 (whole ones too): q and k as column ranges of a wider buffer whose
+    remaining columns and following rows are NaN, so that a row read past the sequences would show."""
+    q, k, v = inputs(B, S, Hq, Hkv, 7 * S + Hq)
+    print(f"ragged causal attention B={B} S={S} Hq={Hq} Hkv={Hkv}", flush=True)
+    wide = torch.full((B * S + 64, Hq + 2 * Hkv + 1, D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    rows = wide[:B * S].view(B, S, Hq + 2 * Hkv + 1, D)
+    views = rows[:, :, :Hq], rows[:, :, Hq:Hq + Hkv], rows[:, :, Hq + Hkv:Hq + 2 * Hkv]
+    for view, t in zip(views, (q, k, v)):
+        view.copy_(t)
+    got = ops.causal_attention_ragged(*views)
+    torch.cuda.synchronize()
+    want = ref.attention(q.double(), k.double(), v.double())
+    assert got.shape == (B, S, Hq, D) and got.dtype == torch.bfloat16
+    assert rel_err(got.float(), want) < TOL_BF16
+    err = (got.double().cpu() - want).abs().amax(dim=(0, 2, 3))
+    assert bool((err < 0.05).all()), err.argmax()
+    if S % 64 == 0:
+        assert torch.equal(got, ops.causal_attention(*views))
+
+
 def test_causal_attention_first_token_and_constant_values(ops):
     q, k, v = inputs(2, 192, 4, 2, 5)
     got = ops.causal_attention(q.cuda(), k.cuda(), v.cuda()).cpu()

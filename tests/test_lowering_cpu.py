@@ -1,4 +1,5 @@
 """The HIP lowering pass on traced graphs (graph surgery only; nothing runs)."""
+import pytest
 import torch
 
 from dynaflow_amd import matching, ops
@@ -125,6 +126,22 @@ def test_decoder_layer_attention_is_lowered_for_head_dim_128():
     torch.compile(layer, backend=backend, fullgraph=True)(ids)
     _, stats = lower_to_hip(captured["gm"])
     assert "causal_attention" not in stats
+
+
+@pytest.mark.parametrize("heads,seq_len,lowered_to", [(4, 64, "causal_attention"), (4, 65, "causal_attention_ragged"),
+                                                      (4, 127, "causal_attention_ragged"), (4, 63, None)])
+def test_attention_kernel_by_sequence_length(heads, seq_len, lowered_to):
+    from dynaflow_amd.decoder import causal_gqa_attention
+
+    graph = torch.fx.Graph()
+    nodes = [graph.placeholder(name) for name in "qkv"]
+    for node, h in zip(nodes, (heads, 2, 2)):
+        node.meta["example_value"] = torch.empty(2, seq_len, h, 128, dtype=torch.bfloat16, device="meta")
+    graph.output((graph.call_function(causal_gqa_attention, tuple(nodes)),))
+    lowered, stats = lower_to_hip(torch.fx.GraphModule(torch.nn.Module(), graph))
+    assert stats.get("causal_attention", 0) == (lowered_to is not None)
+    if lowered_to:
+        assert targets(lowered).count(getattr(ops, lowered_to)) == 1
 
 
 def test_stacked_weight_cache_keys_and_lifetime():
