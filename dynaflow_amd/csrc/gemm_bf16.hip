@@ -1157,49 +1157,75 @@ int launch_walk(const void* A, int64_t lda, const void* W, const void* W2, int64
 // non-temporal ones of the large-tile kernels: they are a few MB that the next kernel of the chain reads at once
 // (decode step 16.85 -> 16.72 ms).
 // (a ring of five units, one more slab in flight, measured no faster on any decode shape)
-constexpr int SK_BM = 128, SK_BN = 128, SK_UNITS = 4, SK_UNIT = 32768, SK_LDS = SK_UNITS * SK_UNIT;
-constexpr int SK_AHEAD = SK_UNITS - 1;          // slabs issued ahead of the one being multiplied
-constexpr int SK_FLIGHT = (SK_AHEAD - 2) * 8;   // DMA instructions of a wave that may still be in flight at a barrier
+constexpr int SK_BM = 128, SK_BN = 128;
 constexpr int SK_MAX_M = 1024;
 
+// Up to 64 rows take tiles of 64 rows (four waves side by side instead of two by two): a slab holds half as many
+// activation bytes - the rows past M of a tile are loaded like the others - and the ring more slabs, and the parts of K
+// hand over half as much.  FUSED tiles of 64 rows also come with 128 outputs (256 W rows), for launches that run side by
+// side.  [us at 64 rows, tiles of 128 rows -> 64, 8B shapes, lone / pair on two streams: q/k/v 22.8 -> 18.2 / 30.0 -> 26.0,
+// o 19.6 -> 15.9 / 25.4 -> 20.0, down 36.5 -> 30.7 / 51.5 -> 45.6, gate + up + SiLU*mul 53 -> 48 / 82 - 88 either way:
+// 470 MB for the two launches at what reaches the XCDs from memory or its cache, about 5.5 TB/s]
+template <int BM, int BW>
+struct SkinnyTile {
+  static constexpr int WAVES_M = BM / 64, WAVES_N = 4 / WAVES_M;
+  static constexpr int WROWS = BW / WAVES_N;              // W rows of a wave
+  static constexpr int JN = WROWS / 32;                   // MFMA blocks of a wave along W
+  static constexpr int A_DMA = BM / 32, W_DMA = BW / 32;  // DMA instructions (8 rows each) of a wave per slab
+  static constexpr int A_BYTES = BM * 128, UNIT_BYTES = (BM + BW) * 128;
+  static constexpr int UNITS = BM == 128 && BW == 128 ? 4 : 163840 / UNIT_BYTES;
+  static constexpr int LDS = UNITS * UNIT_BYTES;
+  static constexpr int AHEAD = UNITS - 1;                 // slabs issued ahead of the one being multiplied
+  // DMA instructions of a wave that may still be in flight at a barrier
+  static constexpr int FLIGHT = (AHEAD - 2) * (A_DMA + W_DMA);
+};
+
 // FUSED: C[M, N] = silu(A W^T) * (A W2^T) (gate and up weights, N = the intermediate size, K not split):
-// a tile is 128 rows x 64 columns, its W half holds, per wave column, 32 gate rows and the 32 matching up
-// rows, so MFMA block j = 0 is the gate and j = 1 the up projection of the same outputs.
-template <bool FUSED>
+// a tile has BW / 2 columns, its W half holds, per wave column, 32 gate rows and the 32 matching up rows, so MFMA
+// block j = 0 is the gate and j = 1 the up projection of the same outputs; where a wave has one block (JN = 1) its
+// rows are 16 gate and 16 up rows, and the accumulators g and g + 2 of a lane belong together.
+template <bool FUSED, int BM, int BW>
 __global__ void __launch_bounds__(RTHREADS)
 gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                         const uint16_t* __restrict__ W2, uint16_t* __restrict__ C,
                         int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, int tiles_m, int tiles_n,
                         int split_k, float* __restrict__ partials, int* __restrict__ arrivals) {
-  constexpr int TILE_N = FUSED ? SK_BN / 2 : SK_BN;
+  using T = SkinnyTile<BM, BW>;
+  constexpr int JN = T::JN, HALF = T::WROWS / 2;   // FUSED: gate rows of a wave
+  constexpr int TILE_N = FUSED ? BW / 2 : BW;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave_m = wave & 1, wave_n = wave >> 1;
+  const int wave_m = wave % T::WAVES_M, wave_n = wave / T::WAVES_M;
   const int tiles = tiles_m * tiles_n;
   const int work = remap_xcd(blockIdx.x, tiles * split_k);
   const int part = work / tiles;
   const int tile = work - part * tiles;        // column tile major, row tile minor
   const int tile_n = tile / tiles_m;
-  const int m0 = (tile - tile_n * tiles_m) * SK_BM;
+  const int m0 = (tile - tile_n * tiles_m) * BM;
   const int n0 = tile_n * TILE_N;
   const int slabs_total = K / BK;
   const int slab0 = (int)((int64_t)slabs_total * part / split_k);
   const int KT = (int)((int64_t)slabs_total * (part + 1) / split_k) - slab0;
 
-  // DMA: a half is 128 rows x 128 bytes = 16 instructions of 8 rows, 4 per wave
-  const uint8_t* a_src[4];
-  const uint8_t* w_src[4];
+  // DMA: instructions of 8 rows x 128 bytes, the rows of a slab dealt to the waves in runs
+  const uint8_t* a_src[T::A_DMA];
+  const uint8_t* w_src[T::W_DMA];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int row = (wave * 4 + t) * 8 + (lane >> 3);
+  for (int t = 0; t < T::A_DMA; ++t) {
+    const int row = (wave * T::A_DMA + t) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
     const int ar = m0 + row < M ? m0 + row : M - 1;
     a_src[t] = reinterpret_cast<const uint8_t*>(A + (int64_t)ar * lda + chunk * 8);
+  }
+#pragma unroll
+  for (int t = 0; t < T::W_DMA; ++t) {
+    const int row = (wave * T::W_DMA + t) * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
     if (FUSED) {
-      const int block = row >> 5;                       // 32-row block: wave column block/2, (0: gate, 1: up)
-      int wr = n0 + (block >> 1) * 32 + (row & 31); wr = wr < N ? wr : N - 1;
-      w_src[t] = reinterpret_cast<const uint8_t*>(((block & 1) ? W2 : W) + (int64_t)wr * ldw + chunk * 8);
+      const int piece = row / HALF;                     // wave column piece / 2, (0: gate, 1: up)
+      int wr = n0 + (piece >> 1) * HALF + row % HALF; wr = wr < N ? wr : N - 1;
+      w_src[t] = reinterpret_cast<const uint8_t*>(((piece & 1) ? W2 : W) + (int64_t)wr * ldw + chunk * 8);
     } else {
       int wr = n0 + row; wr = wr < N ? wr : N - 1;
       w_src[t] = reinterpret_cast<const uint8_t*>(W + (int64_t)wr * ldw + chunk * 8);
@@ -1208,42 +1234,43 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
   auto issue = [&](int slab, int unit) {
     const int64_t off = (int64_t)(slab0 + (slab < KT ? slab : KT - 1)) * (BK * 2);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) dma16(unit * SK_UNIT + (wave * 4 + t) * 1024, a_src[t] + off);
+    for (int t = 0; t < T::A_DMA; ++t) dma16(unit * T::UNIT_BYTES + (wave * T::A_DMA + t) * 1024, a_src[t] + off);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) dma16(unit * SK_UNIT + 16384 + (wave * 4 + t) * 1024, w_src[t] + off);
+    for (int t = 0; t < T::W_DMA; ++t)
+      dma16(unit * T::UNIT_BYTES + T::A_BYTES + (wave * T::W_DMA + t) * 1024, w_src[t] + off);
   };
 
   const int frow = lane & 31, fhalf = lane >> 5, fswz = (frow >> 1) & 7;
   int koff[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) koff[ks] = ((2 * ks + fhalf) ^ fswz) * 16;
-  const int a_lane = (wave_m * 64 + frow) * 128, w_lane = 16384 + (wave_n * 64 + frow) * 128;
+  const int a_lane = (wave_m * 64 + frow) * 128, w_lane = T::A_BYTES + (wave_n * T::WROWS + frow) * 128;
 
-  f32x16 acc[2][2];
+  f32x16 acc[2][JN];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < JN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
   // Fragments are double-buffered by hand: the reads of k-step s+1 (or of the next slab's first k-step)
   // are issued before the MFMAs of step s, so no LDS latency is exposed inside a slab or across slabs.
-  bf16x8 fa[2][2], fw[2][2];
+  bf16x8 fa[2][2], fw[2][JN];
   auto read_frags = [&](int slab, int ks, int slot) {
-    const uint8_t* u = smem + (slab % SK_UNITS) * SK_UNIT;
+    const uint8_t* u = smem + (slab % T::UNITS) * T::UNIT_BYTES;
 #pragma unroll
     for (int i = 0; i < 2; ++i) fa[slot][i] = *reinterpret_cast<const bf16x8*>(u + a_lane + i * 4096 + koff[ks]);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) fw[slot][j] = *reinterpret_cast<const bf16x8*>(u + w_lane + j * 4096 + koff[ks]);
+    for (int j = 0; j < JN; ++j) fw[slot][j] = *reinterpret_cast<const bf16x8*>(u + w_lane + j * 4096 + koff[ks]);
   };
 #pragma unroll
-  for (int u = 0; u < SK_AHEAD; ++u) issue(u, u);
-  wait_vmcnt<SK_FLIGHT>();   // slabs 0 and 1 have landed
+  for (int u = 0; u < T::AHEAD; ++u) issue(u, u);
+  wait_vmcnt<T::FLIGHT>();   // slabs 0 and 1 have landed
   workgroup_barrier();
   read_frags(0, 0, 0);
   for (int kt = 0; kt < KT; ++kt) {
-    issue(kt + SK_AHEAD, (kt + SK_AHEAD) % SK_UNITS);   // into the unit of slab kt-1: everybody passed the barrier after it
+    issue(kt + T::AHEAD, (kt + T::AHEAD) % T::UNITS);   // into the unit of slab kt-1: everybody passed the barrier after it
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const int slot = ks & 1;
@@ -1252,27 +1279,28 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < JN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[slot][j], fa[slot][i], acc[i][j], 0, 0, 0);
       DFHIP_PIN;
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // every read of slab kt (and the prefetch) has returned
-    wait_vmcnt<SK_FLIGHT>();   // slab kt+2 has landed; only the slabs after it may be in flight
+    wait_vmcnt<T::FLIGHT>();   // slab kt+2 has landed; only the slabs after it may be in flight
     workgroup_barrier();
   }
   wait_vmcnt<0>();
   workgroup_barrier();
 
   if (split_k > 1) {
-    f32x4* mine = reinterpret_cast<f32x4*>(partials) + ((int64_t)tile * split_k + part) * (16 * RTHREADS) + tid;
+    constexpr int PIECES = 8 * JN;               // f32x4 of a lane
+    f32x4* mine = reinterpret_cast<f32x4*>(partials) + ((int64_t)tile * split_k + part) * (PIECES * RTHREADS) + tid;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < JN; ++j)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           f32x4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-          store_f32x4_device_coherent(mine + ((i * 2 + j) * 4 + g) * RTHREADS, v);
+          store_f32x4_device_coherent(mine + ((i * JN + j) * 4 + g) * RTHREADS, v);
         }
     wait_vmcnt<0>();
     __syncthreads();
@@ -1284,46 +1312,52 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
     if (ticket != split_k - 1) return;
     if (tid == 0) atomicExch(arrivals + tile, 0);
     // the last arriver adds the parts in part order (its own is read back like the others)
-    const f32x4* all = reinterpret_cast<const f32x4*>(partials) + (int64_t)tile * split_k * (16 * RTHREADS) + tid;
+    const f32x4* all = reinterpret_cast<const f32x4*>(partials) + (int64_t)tile * split_k * (PIECES * RTHREADS) + tid;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < JN; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    for (int p = 0; p < split_k; ++p) {
+    // TOGETHER parts are on their way at a time: a load from the memory side takes a microsecond and more, and what is
+    // in flight costs nothing but registers
+    constexpr int TOGETHER = 32 / PIECES;
+    for (int p0 = 0; p0 < split_k; p0 += TOGETHER) {
+      f32x4 v[TOGETHER][PIECES];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        f32x4 v[8];
+      for (int h = 0; h < TOGETHER; ++h) {
+        const int p = p0 + h < split_k ? p0 + h : split_k - 1;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) v[c] = load_f32x4_device_coherent(all + ((int64_t)p * 16 + h * 8 + c) * RTHREADS);
+        for (int c = 0; c < PIECES; ++c) v[h][c] = load_f32x4_device_coherent(all + ((int64_t)p * PIECES + c) * RTHREADS);
+      }
 #pragma unroll
-        for (int c = 0; c < 8; ++c) wait_loaded(v[c]);
+      for (int h = 0; h < TOGETHER; ++h)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const int i = h, j = c >> 2, g = c & 3;
-          acc[i][j][4 * g] += v[c][0];
-          acc[i][j][4 * g + 1] += v[c][1];
-          acc[i][j][4 * g + 2] += v[c][2];
-          acc[i][j][4 * g + 3] += v[c][3];
-        }
+        for (int c = 0; c < PIECES; ++c) wait_loaded(v[h][c]);
+#pragma unroll
+      for (int h = 0; h < TOGETHER; ++h) {
+        if (p0 + h >= split_k) break;
+#pragma unroll
+        for (int c = 0; c < PIECES; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[c / (4 * JN)][c / 4 % JN][4 * (c % 4) + e] += v[h][c][e];
       }
     }
   }
 
   if (FUSED) {
     // the roundings of the separate kernels: bf16 projections, bf16 silu, bf16 product
-    constexpr int FROW = 80;
+    constexpr int OUTS = HALF, FROW = OUTS * 2 + 16, RUNS = OUTS / 8;   // outputs, padded bytes, 16-byte pieces of a row
     uint8_t* fpark = smem + wave * (64 * FROW);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
+      for (int g = 0; g < RUNS; ++g) {
         float p[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float gt = bf16_bits_to_f32(f32_to_bf16_bits(acc[i][0][4 * g + e]));
-          const float ut = bf16_bits_to_f32(f32_to_bf16_bits(acc[i][1][4 * g + e]));
+          const float ut = bf16_bits_to_f32(f32_to_bf16_bits(JN == 1 ? acc[i][0][4 * g + 8 + e] : acc[i][JN - 1][4 * g + e]));
           p[e] = bf16_bits_to_f32(f32_to_bf16_bits(silu_fast(gt))) * ut;
         }
         u32x2 v;
@@ -1332,11 +1366,11 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
         *reinterpret_cast<u32x2*>(fpark + (i * 32 + frow) * FROW + (g * 8 + fhalf * 4) * 2) = v;
       }
     DFHIP_PIN;
-    const int fm_base = m0 + wave_m * 64, fn_base = n0 + wave_n * 32;
+    const int fm_base = m0 + wave_m * 64, fn_base = n0 + wave_n * OUTS;
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < RUNS; ++p) {
       const int id = p * 64 + lane;
-      const int row = id >> 2, c = id & 3;
+      const int row = id / RUNS, c = id % RUNS;
       const u32x4 v = *reinterpret_cast<const u32x4*>(fpark + row * FROW + c * 16);
       const int m = fm_base + row, n = fn_base + c * 8;
       if (m < M && n < N) *reinterpret_cast<u32x4*>(C + (int64_t)m * ldc + n) = v;
@@ -1344,13 +1378,13 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
     return;
   }
 
-  // park 64 rows x 64 columns per wave (144-byte rows), then whole 128-byte row pieces
-  constexpr int PROW = 144;
+  // park 64 rows x 32 JN columns per wave (padded rows), then whole row pieces
+  constexpr int PROW = 64 * JN + 16, RUNS = 4 * JN;
   uint8_t* park = smem + wave * (64 * PROW);
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < JN; ++j)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         u32x2 v;
@@ -1359,11 +1393,11 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
         *reinterpret_cast<u32x2*>(park + (i * 32 + frow) * PROW + (j * 32 + g * 8 + fhalf * 4) * 2) = v;
       }
   DFHIP_PIN;
-  const int m_base = m0 + wave_m * 64, n_base = n0 + wave_n * 64;
+  const int m_base = m0 + wave_m * 64, n_base = n0 + wave_n * T::WROWS;
 #pragma unroll 4
-  for (int p = 0; p < 8; ++p) {
+  for (int p = 0; p < RUNS; ++p) {
     const int id = p * 64 + lane;
-    const int row = id >> 3, c = id & 7;
+    const int row = id / RUNS, c = id % RUNS;
     u32x4 v = *reinterpret_cast<const u32x4*>(park + row * PROW + c * 16);
     const int m = m_base + row, n = n_base + c * 8;
     if (m < M && n < N) {
@@ -1515,24 +1549,32 @@ gemm_bf16_skinny_wide_kernel(const uint16_t* __restrict__ A, const uint16_t* __r
 size_t skinny_tiles(int M, int N) { return (size_t)((M + SK_BM - 1) / SK_BM) * ((N + SK_BN - 1) / SK_BN); }
 size_t skinny_counter_bytes(int M, int N) { return dfhip_counter_area(skinny_tiles(M, N)); }
 
-template <bool FUSED>
-int launch_skinny(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc, int M,
-                  int N, int K, int split_k, void* workspace, hipStream_t stream) {
-  if (M > SK_MAX_M || (FUSED && split_k != 1)) return DFHIP_ERR_BAD_SHAPE;
-  auto kernel = gemm_bf16_skinny_kernel<FUSED>;
+template <bool FUSED, int BM, int BW>
+int launch_skinny_tile(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
+                       int M, int N, int K, int split_k, void* workspace, hipStream_t stream) {
+  auto kernel = gemm_bf16_skinny_kernel<FUSED, BM, BW>;
+  constexpr int LDS = SkinnyTile<BM, BW>::LDS;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
-  if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), SK_LDS, lds_opted_in)) return rc;
-  constexpr int TILE_N = FUSED ? SK_BN / 2 : SK_BN;
-  const int tiles_m = (M + SK_BM - 1) / SK_BM;
+  if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), LDS, lds_opted_in)) return rc;
+  constexpr int TILE_N = FUSED ? BW / 2 : BW;
+  const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = (N + TILE_N - 1) / TILE_N;
   int* arrivals = static_cast<int*>(workspace);
   float* partials = nullptr;
   if (split_k > 1) partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + skinny_counter_bytes(M, N));
-  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(RTHREADS), SK_LDS, stream,
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(RTHREADS), LDS, stream,
                      static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(W),
                      static_cast<const uint16_t*>(W2), static_cast<uint16_t*>(C), M, N, K, lda, ldw, ldc, tiles_m,
                      tiles_n, split_k, partials, arrivals);
   return dfhip_check_launch();
+}
+
+template <bool FUSED>
+int launch_skinny(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc, int M,
+                  int N, int K, int split_k, void* workspace, hipStream_t stream) {
+  if (M > SK_MAX_M || (FUSED && split_k != 1)) return DFHIP_ERR_BAD_SHAPE;
+  auto launch = M <= 64 ? launch_skinny_tile<FUSED, 64, SK_BN> : launch_skinny_tile<FUSED, SK_BM, SK_BN>;
+  return launch(A, lda, W, W2, ldw, C, ldc, M, N, K, split_k, workspace, stream);
 }
 
 // The few-rows kernel with K cut into parts: arrival counters and fp32 blocks of the workspace as in launch_skinny.
@@ -1545,6 +1587,8 @@ int launch_stream(const void* A, int64_t lda, const void* W, const void* R, int6
 int launch_skinny_wide(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                        int M, int N, int K, hipStream_t stream) {
   if (M > SK_MAX_M || K / BK < 2) return DFHIP_ERR_BAD_SHAPE;
+  if (M <= 64)
+    return launch_skinny_tile<true, 64, 2 * SKW_BN>(A, lda, W, W2, ldw, C, ldc, M, N, K, 1, nullptr, stream);
   auto kernel = gemm_bf16_skinny_wide_kernel;
   static std::atomic<uint64_t> lds_opted_in{0};
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), SKW_LDS, lds_opted_in)) return rc;

@@ -58,3 +58,30 @@ def test_few_row_fp8_launches(M, N, K):
     q, scale = ops.gate_up_silu_quant_fp8(xq, wq, uq, xs, ws, us)
     want_q, want_scale = ops.silu_mul_quant_fp8(y, ops.linear_fp8(xq, uq, xs, us))
     assert torch.equal(scale, want_scale) and torch.equal(q.view(torch.uint8), want_q.view(torch.uint8))
+
+
+# 64-row tiles (33 .. 64 rows; 16 .. 32 with a short K) and the first row that has the 128-row ones; ragged columns, K in
+# up to 10 parts
+@pytest.mark.parametrize("M,N,K", [(16, 1032, 1088), (33, 1024, 1024), (48, 4096, 14336), (64, 6152, 4096),
+                                   (64, 1032, 8192), (57, 14344, 1152), (65, 1032, 8192)])
+def test_tiles_of_64_rows(M, N, K):
+    """Against the fp32 product (bound as above); the fused launch in both of its forms (lone and beside another one)
+    with the bits of the separate launches whose K is whole; rows of a launch of more than 64, whose K is whole, with the
+    bits of a launch of few."""
+    from dynaflow_amd import ops
+
+    x, w, up, r = randn((M, K), 11), randn((N, K), 12, 0.05), randn((N, K), 13, 0.05), randn((M, N), 14)
+    want = x.float() @ w.float().t()
+    limit = 2.0 ** -7 * want.abs().max().item()
+    for side_by_side in (1, 2):
+        with ops.launch_options(side_by_side):
+            y = ops.linear(x, w)
+            assert (y.float() - want).abs().max().item() <= limit
+            assert torch.equal(ops.linear(x, w), y)
+            assert torch.equal(ops.linear_add(x, w, r), r + y)
+            fused = ops.gate_up_silu(x, w, up)
+        whole = [ops.linear_variant(x, t, 6) for t in (w, up)]
+        assert (whole[0].float() - want).abs().max().item() <= limit
+        assert torch.equal(fused, ops.silu_mul(*whole, True))
+    few = x[:40].contiguous()
+    assert torch.equal(ops.linear_variant(few, w, 6), whole[0][:40])
