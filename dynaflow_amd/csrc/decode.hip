@@ -284,7 +284,7 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
     for (int w = 1; w < 4; ++w) mm = fmaxf(mm, m_lds[w * group + h]);
     f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
     float den = 0.0f;
-    if (!SPLIT || mm > -INFINITY) {                         // (a part can be without a chunk, a token cannot)
+    if (!SPLIT || chunk0 < chunks) {                        // (a part can be without a chunk, a token cannot)
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
         const float f = exp2f(m_lds[w * group + h] - mm);   // 0 for a wave that had no chunk (m = -inf)
@@ -337,7 +337,8 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
           }
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            if (q0 + c * lanes >= parts || ml[c][0] == -INFINITY) continue;
+            // a part without a chunk left zeros; one whose scores are all NaN or -inf has the same maximum, and counts
+            if (q0 + c * lanes >= parts || (ml[c][0] == -INFINITY && ml[c][1] == 0.0f)) continue;
             const float m_new = fmaxf(mm, ml[c][0]);
             const float keep = exp2f(mm - m_new), add = exp2f(ml[c][0] - m_new);
 #pragma unroll

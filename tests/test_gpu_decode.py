@@ -206,6 +206,25 @@ def test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, len
         assert int(ws[:4096].view(torch.int32).abs().sum()) == 0
 
 
+def test_decode_attention_cut_over_positions_keeps_nan(ops):
+    """A part all of whose scores are NaN has no maximum, like a part without positions, and still reaches the output:
+    one kv head's keys are NaN in whole parts (2, 3) of 256 positions; the other heads and tokens stay finite."""
+    from dynaflow_amd.decoder import rope_tables
+
+    T, heads, kv_heads, capacity = 2, 32, 8, 8192
+    g = torch.Generator(device="cuda").manual_seed(5)
+    qkv = torch.randn(T, (heads + 2 * kv_heads) * D, generator=g, device="cuda").bfloat16()
+    k = torch.randn(T, kv_heads, capacity, D, generator=g, device="cuda").bfloat16()
+    v = torch.randn(T, kv_heads, capacity // 8, D, 8, generator=g, device="cuda").bfloat16()
+    k[0, 3, 512:1024] = float("nan")
+    slots, lens = (torch.tensor(t, dtype=torch.int32, device="cuda") for t in ([0, 1], [capacity, capacity]))
+    cos, sin = (t.cuda() for t in rope_tables(capacity, D, 500000.0))
+    out = ops.decode_attention(qkv, k, v, slots, lens, cos, sin, heads, kv_heads).view(T, heads, D)
+    want = torch.zeros(T, heads, D, dtype=torch.bool, device="cuda")
+    want[0, 12:16] = True
+    assert torch.equal(out.isnan(), want)
+
+
 def test_decode_attention_ignores_what_lies_past_the_length(ops):
     """Caches are usually allocated uninitialised or hold recycled slots: NaN and Inf patterns in positions
     from lengths[t] on (keys and values) must not reach the output, and the result is the one a cache with
