@@ -36,6 +36,7 @@
 // gemm_bf16_nt_kernel (generic, register staged, any tile shape of the template)
 //   16-byte global loads into registers while the previous slab multiplies, parked
 //   in two padded LDS buffers, one barrier per slab.  Used for small shapes.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -600,9 +601,13 @@ int launch_ring(const void* A, int64_t lda, const void* W, const void* W2, int64
 // j + 7 are the two projections of the same outputs: bf16(bf16(silu(g)) * u) - the roundings of the
 // two-kernel path - is computed in registers and stored from there, 8 bytes per lane.
 constexpr int TBN = 224;
-// The column count is a template parameter: 224 as described, and 128 (4 x 8 blocks per wave, not FUSED) for
+// The tile is a template parameter: 256 x 224 as described; 256 x 128 (4 x 8 blocks per wave, not FUSED) for
 // shapes whose 256 x 256 tiling has at most half as many tiles as the GPU has CUs - 256 x 128 tiles then fill
-// a round without a split along K and its fp32 partial blocks.
+// a round without a split along K and its fp32 partial blocks; and 192 x 256 (2 x 2 waves of 6 x 8 blocks, which
+// read 14 fragments for 48 MFMAs where four waves of 3 x 16 would read 19) for row counts that 256 cuts badly
+// (rows192_cheaper).  FUSED, 256 W rows are 64 gate and 64 up rows for each of the two wave columns, and a lane's blocks j
+// and j + 4 belong together.  Every tile adds in the same order of K: the same bits.  Bound: MFMA / power, and for a launch
+// of one or two rounds the share of them that does work.
 
 // Fused 224-wide tile: which of the tile's 112 outputs the W row at position `pos` (0..111 within the gate or
 // the up part of the W half) belongs to.  MFMA block j = pos / 16 hands lane quad q = (pos % 16) / 4 the four
@@ -612,38 +617,45 @@ constexpr int TBN = 224;
 // a tile went out as twice as many 32-byte requests).  The seventh block keeps the plain order.
 DFHIP_DEVICE int fused224_output_of(int pos) { return pos < 96 ? fused_pair_output_of(pos) : pos; }
 
-template <bool FUSED, int TN>
+template <bool FUSED, int TN, int TM>
 __global__ void __launch_bounds__(RTHREADS)
 gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
                          const uint16_t* __restrict__ W2, uint16_t* __restrict__ C,
                          int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, int tiles_m, int tiles_n) {
   constexpr int OUT_N = FUSED ? TN / 2 : TN;
-  constexpr int JB = TN / 16;          // 16-column MFMA blocks of a wave: 14 or 8
-  constexpr int WP = TN / 32;          // DMA instructions of a W half per wave: 7 or 4
-  constexpr int NR = 4 + JB;           // fragment reads per k-step
-  constexpr int MQ = 4 * JB;           // MFMAs per k-step
-  constexpr int TROW = TN * 2 + 16;    // padded row of the staging area (bytes)
-  static_assert(!FUSED || TN == TBN, "the fused form exists for the 224-wide tile only");
+  constexpr int WAVES_N = TN == 256 ? 2 : 1;   // waves along the columns
+  constexpr int IB = TM * WAVES_N / 64;        // 16-row MFMA blocks of a wave: 4 or 6
+  constexpr int JB = TN / WAVES_N / 16;        // 16-column MFMA blocks of a wave: 14 or 8
+  constexpr int AP = TM / 32, WP = TN / 32;    // DMA instructions of an A / W half per wave
+  constexpr int NR = IB + JB;                  // fragment reads per k-step
+  constexpr int MQ = IB * JB;                  // MFMAs per k-step
+  constexpr int TROW = JB * 32 + 16;           // padded row of the staging area (bytes)
+  static_assert(!FUSED || TN != 128, "the fused form exists for the 224 and 256 W rows of a slab");
+  static_assert(MQ >= NR + AP && MQ >= 4 * WP + NR, "reads and DMA pieces of a k-step behind its MFMAs");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
 
   const int tile = remap_xcd(blockIdx.x, tiles_m * tiles_n);
   const int per_panel = GROUP_M * tiles_n;
   const int first_m = (tile / per_panel) * GROUP_M;
   const int rows_in_panel = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
   const int in_panel = tile % per_panel;
-  const int m0 = (first_m + in_panel % rows_in_panel) * RBM;
+  const int m0 = (first_m + in_panel % rows_in_panel) * TM;
   const int n0 = (in_panel / rows_in_panel) * OUT_N;
   const int KT = K / BK;
 
-  // DMA sources.  A half: 32 instructions of 8 rows, 8 per wave.  W half: 28 instructions, 7 per wave
-  // (FUSED: 14 of gate rows, then 14 of up rows: waves 0, 1 read W, waves 2, 3 read W2).  The address is a
-  // wave-uniform tile base (scalar registers, advanced per slab) plus a 32-bit byte offset per lane.
-  uint32_t a_off[8], w_off[WP];
+  // DMA sources, instructions of 8 rows, AP of the A half and WP of the W half per wave (FUSED: the gate rows of a
+  // wave column, then its up rows - a wave reads one kind: with 224 rows waves 0, 1 read W and 2, 3 read W2, with two
+  // wave columns 0, 2 and 1, 3).  The address is a wave-uniform tile base (scalar registers, advanced per slab) plus a
+  // 32-bit byte offset per lane.
+  constexpr int HALF = OUT_N / WAVES_N;        // FUSED: gate rows of a wave column
+  const bool up_rows = FUSED && (wave * WP * 8 / HALF) % 2 == 1;
+  uint32_t a_off[AP], w_off[WP];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const int row = (wave * 8 + t) * 8 + (lane >> 3);
+  for (int t = 0; t < AP; ++t) {
+    const int row = (wave * AP + t) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
     int ar = m0 + row; ar = ar < M ? ar : M - 1;
     a_off[t] = (uint32_t)((int64_t)(ar - m0) * lda * 2 + chunk * 16);
@@ -652,15 +664,15 @@ gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restr
   for (int t = 0; t < WP; ++t) {
     const int row = (wave * WP + t) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-    int wr = n0 + (FUSED ? fused224_output_of(row >= OUT_N ? row - OUT_N : row) : row);
+    int wr = n0 + (FUSED ? row / (2 * HALF) * HALF + fused224_output_of(row % HALF) : row);
     wr = wr < N ? wr : N - 1;
     w_off[t] = (uint32_t)((int64_t)(wr - n0) * ldw * 2 + chunk * 16);
   }
   const uint8_t* const a_tile = reinterpret_cast<const uint8_t*>(A + (int64_t)m0 * lda);
-  const uint8_t* const w_tile = reinterpret_cast<const uint8_t*>(((FUSED && wave >= 2) ? W2 : W) + (int64_t)n0 * ldw);
+  const uint8_t* const w_tile = reinterpret_cast<const uint8_t*>((up_rows ? W2 : W) + (int64_t)n0 * ldw);
   auto dma_a = [&](int t, int slab, int unit) {
     const int s = slab < KT ? slab : KT - 1;
-    dma16_base(unit * UNIT + (wave * 8 + t) * 1024, a_tile + (int64_t)s * (BK * 2), a_off[t]);
+    dma16_base(unit * UNIT + (wave * AP + t) * 1024, a_tile + (int64_t)s * (BK * 2), a_off[t]);
   };
   auto dma_w = [&](int t, int slab, int unit) {
     const int s = slab < KT ? slab : KT - 1;
@@ -671,27 +683,27 @@ gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restr
   int koff[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) koff[ks] = ((4 * ks + fquad) ^ fswz) * 16;
-  const int a_lane = (wave * 64 + frow) * 128, w_lane = frow * 128;
+  const int a_lane = (wave_m * (16 * IB) + frow) * 128, w_lane = (wave_n * (16 * JB) + frow) * 128;
 
-  f32x4 acc[4][JB];
+  f32x4 acc[IB][JB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IB; ++i)
 #pragma unroll
     for (int j = 0; j < JB; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
 #pragma unroll
-  for (int t = 0; t < 8; ++t) dma_a(t, 0, 0);
+  for (int t = 0; t < AP; ++t) dma_a(t, 0, 0);
 #pragma unroll
   for (int t = 0; t < WP; ++t) dma_w(t, 0, 1);
 #pragma unroll
-  for (int t = 0; t < 8; ++t) dma_a(t, 1, 2);
+  for (int t = 0; t < AP; ++t) dma_a(t, 1, 2);
 #pragma unroll
   for (int t = 0; t < WP; ++t) dma_w(t, 1, 3);
-  wait_vmcnt<8 + WP>();   // slab 0 has landed; slab 1 may still be in flight
+  wait_vmcnt<AP + WP>();   // slab 0 has landed; slab 1 may still be in flight
   workgroup_barrier();
 
-  bf16x8 fa[2][4], fw[2][JB];
-  // fragments in the order the MFMAs need them: W block 0, A block 0, W blocks 1.., A blocks 1..3
+  bf16x8 fa[2][IB], fw[2][JB];
+  // fragments in the order the MFMAs need them: W block 0, A block 0, W blocks 1.., A blocks 1..
   auto read_frag = [&](int pos, int ks, int slot, int unit_a, int unit_w) {
     const bool is_a = pos == 1 || pos > JB;
     const int blk = pos <= 1 ? 0 : pos <= JB ? pos - 1 : pos - JB;
@@ -710,18 +722,18 @@ gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restr
 #pragma unroll
   for (int pos = 0; pos < NR; ++pos) read_frag(pos, 0, 0, ua, uw);
   for (int kt = 0; kt < KT; ++kt) {
-    // k-step 0: the fragments of k-step 1 behind the first MFMAs, the 8 pieces of A(kt+2) spread over the rest
-    constexpr int A0 = TN == TBN ? NR + 2 : NR, AS = (MQ - A0) / 8;
+    // k-step 0: the fragments of k-step 1 behind the first MFMAs, the AP pieces of A(kt+2) spread over the rest
+    constexpr int A0 = TN == TBN ? NR + 2 : NR, AS = (MQ - A0) / AP;
 #pragma unroll
     for (int q = 0; q < MQ; ++q) {
       mfma(q, 0);
       if (q < NR) read_frag(q, 1, 1, ua, uw);
-      else if (q >= A0 && (q - A0) % AS == 0 && (q - A0) / AS < 8) dma_a((q - A0) / AS, kt + 2, ia);
+      else if (q >= A0 && (q - A0) % AS == 0 && (q - A0) / AS < AP) dma_a((q - A0) / AS, kt + 2, ia);
       DFHIP_PIN;
     }
     // all LDS reads of slab kt issued; slab kt+1 must have landed, only A(kt+2) may be in flight
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wait_vmcnt<8>();
+    wait_vmcnt<AP>();
     workgroup_barrier();
     int na = ua + 2; if (na >= NUNITS) na -= NUNITS;
     int nw = uw + 2; if (nw >= NUNITS) nw -= NUNITS;
@@ -743,15 +755,15 @@ gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restr
   // (the compiler does not know that the statements above write the accumulators late: every later use
   // of an accumulator is tied behind the wait states)
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IB; ++i)
 #pragma unroll
     for (int j = 0; j < JB; ++j) asm volatile("" : "+a"(acc[i][j]));
 
   if (FUSED) {
-    // silu(gate) * up in registers (blocks j and j + 7 hold the two projections of the same outputs) and
+    // silu(gate) * up in registers (blocks j and j + JB / 2 hold the two projections of the same outputs) and
     // stores straight from the registers: a lane owns 8 consecutive outputs of one row per pair of blocks
     // (see fused224_output_of) and 4 of the seventh block
-    const int m_first = m0 + wave * 64 + frow;
+    const int m_first = m0 + wave_m * (16 * IB) + frow, n_first = n0 + wave_n * HALF;
     auto product = [&](int i, int j) {
       u32x2 packed;
 #pragma unroll
@@ -764,25 +776,27 @@ gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restr
       return packed;
     };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < IB; ++i) {
       const int m = m_first + i * 16;
 #pragma unroll
-      for (int pr = 0; pr < 3; ++pr) {
+      for (int pr = 0; pr < JB / 4; ++pr) {
         const u32x2 even = product(i, 2 * pr), odd = product(i, 2 * pr + 1);
         const u32x4 v = {even[0], even[1], odd[0], odd[1]};
-        const int n = n0 + pr * 32 + fquad * 8;   // N % 8 == 0: the run is entirely inside or outside
+        const int n = n_first + pr * 32 + fquad * 8;   // N % 8 == 0: the run is entirely inside or outside
         if (m < M && n < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(C + (int64_t)m * ldc + n));
       }
-      const u32x2 v = product(i, 6);
-      const int n = n0 + 96 + fquad * 4;
-      if (m < M && n < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(C + (int64_t)m * ldc + n));
+      if constexpr (JB / 2 % 2 == 1) {
+        const u32x2 v = product(i, JB / 2 - 1);
+        const int n = n_first + 96 + fquad * 4;
+        if (m < M && n < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x2*>(C + (int64_t)m * ldc + n));
+      }
     }
     return;
   }
-  // park 64 rows x 224 columns per wave as bf16, then store whole row pieces
-  uint8_t* park = smem + wave * (64 * TROW);
+  // park a wave's block as bf16, then store whole row pieces
+  uint8_t* park = smem + wave * (16 * IB * TROW);
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < IB; ++i)
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
       u32x2 v;
@@ -791,14 +805,14 @@ gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restr
       *reinterpret_cast<u32x2*>(park + (i * 16 + frow) * TROW + (j * 16 + fquad * 4) * 2) = v;
     }
   DFHIP_PIN;
-  const int m_base = m0 + wave * 64;
-  constexpr int CPR = TN / 8;   // 16-byte pieces of a row
+  const int m_base = m0 + wave_m * (16 * IB), n_base = n0 + wave_n * (16 * JB);
+  constexpr int CPR = JB * 2;   // 16-byte pieces of a row
 #pragma unroll 4
-  for (int p = 0; p < CPR; ++p) {
+  for (int p = 0; p < CPR * IB / 4; ++p) {
     const int id = p * 64 + lane;
     const int row = id / CPR, c = id - row * CPR;
     u32x4 v = *reinterpret_cast<const u32x4*>(park + row * TROW + c * 16);
-    const int m = m_base + row, n = n0 + c * 8;
+    const int m = m_base + row, n = n_base + c * 8;
     if (m < M && n < N) {
       if (W2) {            // not FUSED: W2 is the optional residual [M, N] (leading dimension ldc)
         const u32x4 r = *reinterpret_cast<const u32x4*>(W2 + (int64_t)m * ldc + n);
@@ -810,14 +824,14 @@ gemm_bf16_ring224_kernel(const uint16_t* __restrict__ A, const uint16_t* __restr
   }
 }
 
-template <bool FUSED, int TN = TBN>
+template <bool FUSED, int TN = TBN, int TM = RBM>
 int launch_ring224(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                    int M, int N, int K, hipStream_t stream) {
-  auto kernel = gemm_bf16_ring224_kernel<FUSED, TN>;
+  auto kernel = gemm_bf16_ring224_kernel<FUSED, TN, TM>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), RING_LDS, lds_opted_in)) return rc;
   constexpr int OUT_N = FUSED ? TN / 2 : TN;
-  const int tiles_m = (M + RBM - 1) / RBM;
+  const int tiles_m = (M + TM - 1) / TM;
   const int tiles_n = (N + OUT_N - 1) / OUT_N;
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(RTHREADS), RING_LDS, stream,
                      static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(W),
@@ -1626,6 +1640,22 @@ double round_fill(int M, int N, int tile_n, int share = 1) {
   return (double)M * N * share / ((double)rounds * 256 * RBM * tile_n);
 }
 
+// Whether tiles of 192 rows x 256 W rows (128 outputs where gate and up meet in a tile) cost clearly less than those of 256
+// rows with `wide` or `narrow` columns.  A launch costs its rounds of 256 workgroups times what a round of the tile takes:
+// 1 / 0.93 / 0.84 for 256 x 256 / 256 x 224 / 192 x 256 (74 / 69 / 62 us at K = 4096; less than the area says, because the
+// clock is higher while units idle).  Measured at M = 300 .. 6000 on four weights, the tile is 6 - 18 % faster wherever
+// this says so: 670 x 14336 x 4096 71 -> 64 us, 2331 x 4096 x 14336 236 -> 210, 2880 x 6144 x 4096 142 -> 124, gate + up +
+// SiLU*mul 2 x 14336 x 4096 at 560 / 1100 / 1554 rows 144 / 228 / 308 -> 124 / 199 / 291; where it says no, the tile is up
+// to 60 % slower (777 x 14336 x 4096: 1.09 rounds, 81 -> 122) or at best 4 % faster.
+bool rows192_cheaper(int M, int N, int wide, int narrow, int share) {
+  auto cost = [&](int tile_m, int tile_n, double per_round) {
+    const int64_t tiles = (int64_t)((M + tile_m - 1) / tile_m) * ((N + tile_n - 1) / tile_n) * share;
+    return (double)((tiles + 255) / 256) * per_round;
+  };
+  const double best = std::min(cost(RBM, wide, 1.0), cost(RBM, narrow, 0.93));
+  return cost(192, wide, 0.84) < 0.95 * best;
+}
+
 // Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip), whatever runs beside it.
 // With 16 rows and more a K below 2048 keeps the 128-row tiles.  Weights of more than 2^27 elements keep them too: there
 // a row has the same bits in a launch of few rows and of many, which is worth more than the gain (2 x 28672 x 8192 with
@@ -1664,6 +1694,7 @@ extern "C" int dfhip_gemm_bf16_nt_variant(const void* A, int64_t lda, const void
     case 3: return launch<256, 128, 2, 2>(A, lda, W, ldw, C, ldc, M, N, K, s);
     case 5: return launch_ring224<false>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, s);
     case 7: return launch_ring224<false, 128>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, s);
+    case 9: return launch_ring224<false, 256, 192>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, s);
     case 6: return launch_skinny<false>(A, lda, W, nullptr, ldw, C, ldc, M, N, K, 1, nullptr, s);
     case 8:
       if (!dfhip_stream_fits(M, N, (int64_t)K * 2, 1)) return DFHIP_ERR_BAD_SHAPE;
@@ -1676,7 +1707,8 @@ extern "C" int dfhip_gemm_bf16_plan(int M, int N, int K, int* variant, int* spli
   return dfhip_gemm_bf16_plan_shared(M, N, K, 1, variant, split_k);
 }
 
-extern "C" int dfhip_gemm_bf16_plan_shared(int M, int N, int K, int share, int* variant, int* split_k) {
+// The plan among the tiles of 256 rows (and the small ones), which is also what says whether a caller may split K.
+static int plan_rows256(int M, int N, int K, int share, int* variant, int* split_k) {
   if (!variant || !split_k) return DFHIP_ERR_NULL_POINTER;
   if (M < 1 || N < 1 || K < 1) return DFHIP_ERR_BAD_SHAPE;
   if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
@@ -1724,6 +1756,12 @@ extern "C" int dfhip_gemm_bf16_plan_shared(int M, int N, int K, int share, int* 
     // 256 x 224 tiles when they fill the rounds of 256 workgroups clearly better (N = 7 * 2^k)
     if (s <= 1 && round_fill(M, N, TBN, share) > round_fill(M, N, RBN, share) + 0.05) *variant = 5;
   }
+  return DFHIP_OK;
+}
+
+extern "C" int dfhip_gemm_bf16_plan_shared(int M, int N, int K, int share, int* variant, int* split_k) {
+  if (int rc = plan_rows256(M, N, K, share, variant, split_k)) return rc;
+  if ((*variant == 0 || *variant == 5) && *split_k == 1 && rows192_cheaper(M, N, RBN, TBN, share)) *variant = 9;
   return DFHIP_OK;
 }
 
@@ -1800,6 +1838,9 @@ extern "C" int dfhip_gemm_bf16_gate_up_silu_shared(const void* A, int64_t lda, c
     return launch_skinny<true>(A, lda, W_gate, W_up, ldw, Out, ldo, M, I, K, 1, nullptr,
                                static_cast<hipStream_t>(stream));
   }
+  // 192 x (128 + 128) where it takes clearly fewer of its shorter rounds
+  if (rows192_cheaper(M, I, 128, TBN / 2, share))
+    return launch_ring224<true, 256, 192>(A, lda, W_gate, W_up, ldw, Out, ldo, M, I, K, static_cast<hipStream_t>(stream));
   // the 256 x (112 + 112) tile when it fills the rounds of 256 workgroups clearly better than the 256 x (128 + 128)
   // one, which moves fewer bytes through LDS per flop; launches that run side by side take their rounds together
   // (two launches of the 8B shape at 2048 rows: 2 x 896 square tiles are exactly 7 rounds)
@@ -1824,7 +1865,8 @@ extern "C" int dfhip_gemm_bf16_nt_add(const void* A, int64_t lda, const void* W,
   if (int rc = check_args(A, lda, W, ldw, C, ldc, M, N, K)) return rc;
   if (!dfhip_aligned16(R)) return DFHIP_ERR_BAD_ALIGNMENT;
   int variant = 2, planned = 1;
-  if (int rc = dfhip_gemm_bf16_plan(M, N, K, &variant, &planned)) return rc;
+  const auto plan = split_k > 1 ? plan_rows256 : dfhip_gemm_bf16_plan_shared;   // (tiles of 192 rows do not split K)
+  if (int rc = plan(M, N, K, 1, &variant, &planned)) return rc;
   if (split_k < 1 || split_k > 16 || K / BK < split_k) return DFHIP_ERR_BAD_ARGUMENT;
   if (split_k > 1) {
     if (variant != 0 && variant != 6 && variant != 8) return DFHIP_ERR_BAD_ARGUMENT;   // the planned kernel does not split K
@@ -1838,6 +1880,7 @@ extern "C" int dfhip_gemm_bf16_nt_add(const void* A, int64_t lda, const void* W,
     case 0: return launch_ring<false>(A, lda, W, R, ldw, C, ldc, M, N, K, split_k, workspace, s);
     case 5: return launch_ring224<false>(A, lda, W, R, ldw, C, ldc, M, N, K, s);
     case 7: return launch_ring224<false, 128>(A, lda, W, R, ldw, C, ldc, M, N, K, s);
+    case 9: return launch_ring224<false, 256, 192>(A, lda, W, R, ldw, C, ldc, M, N, K, s);
     case 6: return launch_skinny<false>(A, lda, W, R, ldw, C, ldc, M, N, K, split_k, workspace, s);
     case 8:
       if (!dfhip_stream_fits(M, N, (int64_t)K * 2, split_k))

@@ -97,6 +97,8 @@ int dfhip_gemm_bf16_nt(const void* A, int64_t lda, const void* W, int64_t ldw, v
  *          parts that meet as with variant 6 (needs K >= 1024 and K / split_k >= 1024; the
  *          plan picks it up to 32 rows for K >= 2048, below 16 rows for every such K, and
  *          weights of at most 2^27 elements);
+ *          9 = 192x256 tile, LDS-DMA ring (chosen instead of 0 and 5 where its shorter rounds of
+ *              256 workgroups cost less, e.g. 670 rows of N = 14336; the same bits);
  *          register-staged tiles: 1 = 256x256 / 8 waves, 2 = 128x128 / 4 waves,
  *          3 = 256x128 / 4 waves, 4 = 256x256 / 4 waves. */
 int dfhip_gemm_bf16_nt_variant(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
