@@ -27,9 +27,13 @@
 // Sequences whose length is no multiple of 64 (RAGGED) end in a block that is partly there: its missing key rows
 // re-read the sequence's last one (only rows past the sequence see them: the causal mask covers the others), its
 // missing values are zeros that pack_v_kernel wrote, and rows past the sequence are not stored.  A form of its own,
-// so that whole sequences do not select between two sets of key offsets.  Operator with pack_v, 32 heads on 8, us (PyTorch's
-// fused attention, which took these lengths before): 1 x 333 21 (32), 1 x 777 30 (57), 4 x 333 25 (58), 4 x 1500 105 (382),
-// 4 x 2047 165 (543); level with it below about 100 tokens.  4 x 2048 through either form 154 - 158.
+// so that whole sequences do not select between two sets of key offsets.  These lengths went to PyTorch's fused
+// attention, whose weights are relative to the row's running maximum, so that the largest of them are exact in bf16; with
+// the fixed reference above every weight is rounded, and the result lay further from float64 (2-norm, rows from 64 on of
+// 777: 2.15e-3 against 1.94e-3).  The ragged form therefore multiplies two bf16 parts of a weight: 1.66e-3, the rounding
+// of the result alone, for 48 MFMAs a step instead of 36.  Operator with pack_v, 32 heads on 8, us (one part; PyTorch's):
+// 1 x 65 13 (13; 18), 1 x 333 23 (20; 31), 1 x 777 36 (28; 55), 4 x 333 26 (23; 56), 4 x 1500 131 (101; 375),
+// 4 x 2047 207 (157; 538).
 #include <type_traits>
 
 #include "dfhip_common.h"
@@ -133,6 +137,7 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, half = lane >> 5;
+  constexpr int PARTS = RAGGED ? 2 : 1;        // bf16 parts of a probability
   constexpr int WPH = 4 / HPW;                 // waves per head
   constexpr int QROWS = WAVE_ROWS * WPH;       // query rows per workgroup
   int b, kvh, hq, qb;
@@ -248,9 +253,15 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
   // nearly every MFMA of a step: a slice turns one score into a probability (an even register's waits for its
   // odd neighbour to be packed with it).  No maximum is taken and no sum: the row sums come out of the matrix
   // pipe (an all-ones A operand against the probabilities), and whether a row's scores outgrew its reference
-  // shows in that sum at the end.
+  // shows in that sum at the end.  RAGGED: the probabilities go into P V in two parts, bf16(e) and the bf16 of what that
+  // rounding left, and the row sums are added up here in fp32 (PARTS).
   float held = 0.0f;                          // the probability of an even register until its odd neighbour follows
-  auto softmax_slice = [&](auto diag, int i, int block, int sb, const f32x16 (&s)[2], bf16x8 (&pf)[2][2]) {
+  float l_lane[2] = {0.0f, 0.0f};             // RAGGED: the lane's share of the row sums
+  auto put_rest = [&](bf16x8 (&pf)[PARTS][2][2], int nb, int r, float e) {   // behind bf16(e), which is in part 0
+    if constexpr (RAGGED)
+      pf[1][nb][r >> 3][r & 7] = static_cast<bf16_t>(e - static_cast<float>(pf[0][nb][r >> 3][r & 7]));
+  };
+  auto softmax_slice = [&](auto diag, int i, int block, int sb, const f32x16 (&s)[2], bf16x8 (&pf)[PARTS][2][2]) {
     const int nb = i >> 4, r = i & 15;
     float x = s[nb][r];
     if (decltype(diag)::value) {
@@ -259,9 +270,12 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
       if (pos > qrow) x = -INFINITY;
     }
     const float e = __builtin_amdgcn_exp2f(fmaf(x, scale_log2, neg_ref[nb]));
+    if (RAGGED) l_lane[nb] += e;
     if (r & 1) {
-      pf[nb][r >> 3][(r & 7) - 1] = static_cast<bf16_t>(held);
-      pf[nb][r >> 3][r & 7] = static_cast<bf16_t>(e);
+      pf[0][nb][r >> 3][(r & 7) - 1] = static_cast<bf16_t>(held);
+      pf[0][nb][r >> 3][r & 7] = static_cast<bf16_t>(e);
+      put_rest(pf, nb, r - 1, held);
+      put_rest(pf, nb, r, e);
     } else {
       held = e;
     }
@@ -286,20 +300,22 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
   for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
     for (int r = 0; r < 16; ++r) l_acc[nb][r] = 0.0f;
-  auto step = [&](auto do_s, auto do_sm, auto diag, int vb, int vsb, const bf16x8 (&pf_in)[2][2], int kb, int ksb,
-                  f32x16 (&s_out)[2], int mb, int msb, const f32x16 (&s_in)[2], bf16x8 (&pf_out)[2][2], int nvb,
+  auto step = [&](auto do_s, auto do_sm, auto diag, int vb, int vsb, const bf16x8 (&pf_in)[PARTS][2][2], int kb, int ksb,
+                  f32x16 (&s_out)[2], int mb, int msb, const f32x16 (&s_in)[2], bf16x8 (&pf_out)[PARTS][2][2], int nvb,
                   int nvsb, int dma_block) {
     constexpr bool DO_S = decltype(do_s)::value, DO_SM = decltype(do_sm)::value;
     constexpr int FRAGS = DO_S ? 16 : 8;       // pairs that consume an A fragment: 8 of P V, 8 of the scores
-    constexpr int PAIRS = FRAGS + 2;           // + the row sums of the two k-steps
+    constexpr int SUMS = RAGGED ? 0 : 2;       // the row sums of the two k-steps
+    constexpr int PAIRS = FRAGS + SUMS;
+    constexpr int MFMAS = 2 * PAIRS + 16 * (PARTS - 1);
     bf16x8 fr[FRAGS + AHEAD];
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) fr[a] = vpre[a];
 #pragma unroll
     for (int pq = 0; pq < PAIRS; ++pq) {
-      // pair order: pv0..pv3, sum(t=0), pv4..pv7, sum(t=1), score k-steps 0..7
-      const bool is_sum = pq == 4 || pq == 9;
-      const int f = pq < 4 ? pq : pq < 9 ? pq - 1 : pq - 2;      // fragment index of a consuming pair
+      // pair order: pv0..pv3, sum(t=0), pv4..pv7, sum(t=1), score k-steps 0..7 (a fragment of V serves all parts)
+      const bool is_sum = SUMS > 0 && (pq == 4 || pq == 9);
+      const int f = SUMS == 0 || pq < 4 ? pq : pq < 9 ? pq - 1 : pq - 2;      // fragment index of a consuming pair
       // the 8 LDS-DMA instructions of the block that enters the ring in this iteration, spread over the step
       // (4 waves issuing them in one burst keep the address unit, and with it the waves, busy for ~500 cycles)
       if (dma_block >= 0) {
@@ -311,22 +327,24 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
         else if (n < FRAGS) fr[n] = k_frag(kb, ksb, n - 8);
         else fr[n] = v_frag(nvb, nvsb, n - FRAGS);
       }
+      const int parts = !is_sum && f < 8 ? PARTS : 1;
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
+      for (int u = 0; u < 2 * parts; ++u) {
+        const int nb = u & 1;
         if (is_sum) {
-          l_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pf_in[nb][pq == 4 ? 0 : 1], l_acc[nb], 0, 0, 0);
+          l_acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, pf_in[0][nb][pq == 4 ? 0 : 1], l_acc[nb], 0, 0, 0);
         } else if (f < 8) {
           const int t = f >> 2, db = f & 3;
-          o[db][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], pf_in[nb][t], o[db][nb], 0, 0, 0);
+          o[db][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f], pf_in[u >> 1][nb][t], o[db][nb], 0, 0, 0);
         } else if (f == 8) {
           s_out[nb] = mfma_scores_first(fr[f], qf[nb][0]);
         } else {
           mfma_scores_next(s_out[nb], fr[f], qf[nb][f - 8]);
         }
         if (DO_SM) {
-          const int m = 2 * pq + nb;           // slices [32 m / (2 PAIRS), 32 (m+1) / (2 PAIRS))
+          const int m = 2 * pq + u + (f < 8 ? 2 * f : 16) * (PARTS - 1);   // of MFMAS: slices 32 m / MFMAS and on
 #pragma unroll
-          for (int i = 32 * m / (2 * PAIRS); i < 32 * (m + 1) / (2 * PAIRS); ++i)
+          for (int i = 32 * m / MFMAS; i < 32 * (m + 1) / MFMAS; ++i)
             softmax_slice(diag, i, mb, msb, s_in, pf_out);
         }
         DFHIP_PIN;
@@ -340,7 +358,7 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
   using no = std::false_type;
 
   f32x16 sA[2], sB[2];
-  bf16x8 pfA[2][2], pfB[2][2];
+  bf16x8 pfA[PARTS][2][2], pfB[PARTS][2][2];
   wait_vmcnt<0>();                           // Q and the first blocks have landed
   workgroup_barrier();
   // from here on the Q fragments live in accumulation registers (see mfma_scores_first)
@@ -429,7 +447,10 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
       }
     }
   };
-  const float fast_sum[2] = {l_acc[0][0], l_acc[1][0]};
+  float fast_sum[2] = {l_acc[0][0], l_acc[1][0]};
+  if (RAGGED)
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) fast_sum[nb] = l_lane[nb] + __shfl_xor(l_lane[nb], 32, 64);
   store_rows(fast_sum);
   for (++j; j <= last_block_wg; ++j) {
     turn_ring(j);
@@ -479,7 +500,7 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
       }
       // register r of this lane: position p_base + 16*(r/8) + (r%8), query row my_qrow0 + 32 nb
       const int p_base = jb * KVB + sb * 32 + 8 * half;
-      bf16x8 pf[2][2];
+      bf16x8 pf[PARTS][2][2];
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb) {
         if (diagonal) {
@@ -508,15 +529,17 @@ causal_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, const uint
         for (int r = 0; r < 16; ++r) {
           const float p = __builtin_amdgcn_exp2f(fmaf(s[nb][r], scale_log2, -mc));
           lsum += p;
-          pf[nb][r >> 3][r & 7] = static_cast<bf16_t>(p);
+          pf[0][nb][r >> 3][r & 7] = static_cast<bf16_t>(p);
+          put_rest(pf, nb, r, p);
         }
         l_run[nb] += lsum;
       }
 #pragma unroll
       for (int p = 0; p < 8; ++p) {
         const bf16x8 vf = v_frag(jb, sb, p);
-        o[p & 3][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[0][p >> 2], o[p & 3][0], 0, 0, 0);
-        o[p & 3][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[1][p >> 2], o[p & 3][1], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2 * PARTS; ++u)
+          o[p & 3][u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[u >> 1][u & 1][p >> 2], o[p & 3][u & 1], 0, 0, 0);
       }
     }
   }
@@ -612,6 +635,7 @@ extern "C" int dfhip_causal_attention_bf16(const void* q, int64_t ld_q, const vo
 extern "C" int dfhip_causal_attention_ragged_bf16(const void* q, int64_t ld_q, const void* k, int64_t ld_k,
                                                   const void* v_blk, void* out, int64_t ld_o, int B, int S, int q_heads,
                                                   int kv_heads, int head_dim, float scale, dfhip_stream_t stream) {
-  return causal_attention<true>(q, ld_q, k, ld_k, v_blk, out, ld_o, B, S, q_heads, kv_heads, head_dim, scale,
-                                static_cast<hipStream_t>(stream));
+  auto form = S % KVB == 0 ? causal_attention<false> : causal_attention<true>;   // whole blocks: the same layout, no tail
+  return form(q, ld_q, k, ld_k, v_blk, out, ld_o, B, S, q_heads, kv_heads, head_dim, scale,
+              static_cast<hipStream_t>(stream));
 }

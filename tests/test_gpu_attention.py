@@ -69,6 +69,25 @@ def test_causal_attention_ragged_against_oracle(ops, B, S, Hq, Hkv):
         assert torch.equal(got, ops.causal_attention(*views))
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv,std", [(1, 65, 8, 2, 1.28), (2, 127, 4, 2, 1.28), (1, 333, 8, 2, 2.5),
+                                            (1, 777, 4, 4, 1.28), (1, 1025, 8, 1, 1.28)])
+def test_causal_attention_ragged_is_as_exact_as_weights_relative_to_the_row_maximum(ops, B, S, Hq, Hkv, std):
+    """Lengths that are no multiple of 64 go to PyTorch's fused attention otherwise, which rounds a weight to bf16 relative
+    to its row's maximum (the largest weight is exact).  The distance from float64 is no larger than that of an evaluation
+    with exactly this rounding and the one of the result.  Rows from 32 on: behind the first tile of positions the row's
+    reference is not its maximum."""
+    q, k, v = (t * std for t in inputs(B, S, Hq, Hkv, S))
+    got = ops.causal_attention_ragged(q.cuda(), k.cuda(), v.cuda()).double().cpu()[:, 32:]
+    want = ref.attention(q.double(), k.double(), v.double())[:, 32:]
+    heads = [t.double().permute(0, 2, 1, 3).repeat_interleave(Hq // t.shape[2], dim=1) for t in (q, k, v)]
+    scores = heads[0] @ heads[1].transpose(2, 3) / D ** 0.5
+    scores = scores.masked_fill(torch.ones(S, S, dtype=torch.bool).triu(1), float("-inf"))
+    weights = torch.exp(scores - scores.amax(-1, keepdim=True))
+    rounded = (weights.bfloat16().double() @ heads[2] / weights.sum(-1, keepdim=True)).transpose(1, 2)[:, 32:]
+    bound = (rounded.bfloat16().double() - want).norm()
+    assert (got - want).norm() <= bound, ((got - want).norm() / want.norm(), bound / want.norm())
+
+
 def test_causal_attention_first_token_and_constant_values(ops):
     q, k, v = inputs(2, 192, 4, 2, 5)
     got = ops.causal_attention(q.cuda(), k.cuda(), v.cuda()).cpu()
