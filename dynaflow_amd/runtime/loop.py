@@ -12,21 +12,28 @@ from collections.abc import Coroutine
 from typing import Any
 
 
-class _ThreadLoop(threading.local):
-    def __init__(self) -> None:
-        self.loop: asyncio.AbstractEventLoop | None = None
+class _KeptLoop:
+    """A loop and whoever closes it: the thread's locals hold this object and the loop does not, so it goes, and the loop
+    is closed, when they are dropped at the end of the thread.  (A loop by itself is part of reference cycles and would
+    keep its descriptors until the collector finds it.)"""
 
-    def get(self) -> asyncio.AbstractEventLoop:
-        if self.loop is None or self.loop.is_closed():
-            self.loop = asyncio.new_event_loop()
-        return self.loop
+    def __init__(self) -> None:
+        self.loop = asyncio.new_event_loop()
 
     def __del__(self) -> None:
-        if self.loop is not None and not self.loop.is_closed() and not self.loop.is_running():
-            self.loop.close()
+        loop = getattr(self, "loop", None)
+        if loop is not None and not loop.is_closed() and not loop.is_running():
+            loop.close()
 
 
-_thread = _ThreadLoop()
+_thread = threading.local()
+
+
+def _thread_loop() -> asyncio.AbstractEventLoop:
+    kept = getattr(_thread, "kept", None)
+    if kept is None or kept.loop.is_closed():
+        kept = _thread.kept = _KeptLoop()
+    return kept.loop
 
 
 def run_coroutine(coroutine: Coroutine) -> Any:
@@ -38,7 +45,7 @@ def run_coroutine(coroutine: Coroutine) -> Any:
     else:
         coroutine.close()
         raise RuntimeError("a forward cannot be called from a running event loop")
-    loop = _thread.get()
+    loop = _thread_loop()
     try:
         return loop.run_until_complete(coroutine)
     finally:
