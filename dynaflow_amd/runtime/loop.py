@@ -7,6 +7,7 @@ loop is closed with the thread.
 from __future__ import annotations
 
 import asyncio
+import os
 import threading
 from collections.abc import Coroutine
 from typing import Any
@@ -19,19 +20,28 @@ class _KeptLoop:
 
     def __init__(self) -> None:
         self.loop = asyncio.new_event_loop()
+        self.process = os.getpid()
 
     def __del__(self) -> None:
         loop = getattr(self, "loop", None)
-        if loop is not None and not loop.is_closed() and not loop.is_running():
+        if loop is None or loop.is_closed() or loop.is_running():
+            return
+        if self.process != os.getpid():
+            _inherited.append(loop)
+        else:
             loop.close()
 
+
+#: Loops of a parent process that a fork has brought here.  They share the parent's epoll object: closing one (its own
+#: ``__del__`` does that too) would take the parent's wake-up descriptor out of it, so they stay as they are.
+_inherited: list[asyncio.AbstractEventLoop] = []
 
 _thread = threading.local()
 
 
 def _thread_loop() -> asyncio.AbstractEventLoop:
     kept = getattr(_thread, "kept", None)
-    if kept is None or kept.loop.is_closed():
+    if kept is None or kept.process != os.getpid() or kept.loop.is_closed():
         kept = _thread.kept = _KeptLoop()
     return kept.loop
 

@@ -1,9 +1,12 @@
 """The event loop that a thread keeps for its forwards: what ``asyncio.run`` did for each of them is still done."""
+import asyncio
 import gc
+import multiprocessing
 import os
 import subprocess
 import sys
 import threading
+import time
 import warnings
 
 from dynaflow_amd.runtime.loop import run_coroutine
@@ -44,3 +47,29 @@ def test_a_loop_is_closed_at_the_end_of_the_process():
             "assert run_coroutine(nothing()) == 7\n")
     done = subprocess.run([sys.executable, "-X", "dev", "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
     assert done.returncode == 0 and "event loop" not in done.stderr and "loop.py" not in done.stderr, done.stderr
+
+
+def _in_a_forked_child():
+    from dynaflow_amd.runtime import loop
+
+    assert run_coroutine(nothing()) == 7
+    loop._thread.__dict__.clear()            # what the end of a thread does
+    gc.collect()
+
+
+def test_a_forked_child_leaves_its_parents_loop_alone():
+    """A child shares the parent's epoll object.  One that closes the inherited loop takes the parent's wake-up descriptor
+    out of it, and the parent's coroutines then sleep through what other threads finish for them."""
+    async def other_thread():
+        started = time.monotonic()
+        await asyncio.wait_for(asyncio.get_running_loop().run_in_executor(None, time.sleep, 0.02), 10)
+        return time.monotonic() - started
+
+    assert run_coroutine(nothing()) == 7
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", DeprecationWarning)      # a fork beside torch's threads
+        child = multiprocessing.get_context("fork").Process(target=_in_a_forked_child)
+        child.start()
+    child.join(60)
+    assert child.exitcode == 0
+    assert run_coroutine(other_thread()) < 5
