@@ -64,3 +64,7 @@ def run_coroutine(coroutine: Coroutine) -> Any:
             for task in left:
                 task.cancel()
             loop.run_until_complete(asyncio.gather(*left, return_exceptions=True))
+            for task in left:
+                if not task.cancelled() and task.exception() is not None:
+                    loop.call_exception_handler({"message": "a task that outlived its forward failed while it was cancelled",
+                                                 "exception": task.exception(), "task": task})

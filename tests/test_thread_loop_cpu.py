@@ -1,6 +1,7 @@
 """The event loop that a thread keeps for its forwards: what ``asyncio.run`` did for each of them is still done."""
 import asyncio
 import gc
+import logging
 import multiprocessing
 import os
 import subprocess
@@ -73,3 +74,19 @@ def test_a_forked_child_leaves_its_parents_loop_alone():
     child.join(60)
     assert child.exitcode == 0
     assert run_coroutine(other_thread()) < 5
+
+
+def test_a_left_over_task_that_fails_while_it_is_cancelled_is_reported(caplog):
+    async def fails_on_cancel():
+        try:
+            await asyncio.sleep(60)
+        finally:
+            raise ValueError("lost work")
+
+    async def leaves_it():
+        asyncio.get_running_loop().create_task(fails_on_cancel())
+        await asyncio.sleep(0)
+
+    with caplog.at_level(logging.ERROR, "asyncio"):
+        run_coroutine(leaves_it())
+    assert any(r.exc_info and "lost work" in str(r.exc_info[1]) for r in caplog.records)
