@@ -110,7 +110,10 @@ class OperatorHandle:
 
 class ExecutionContext:
     """What a scheduler talks to the engine through: a forward that it drives directly (``forward``, an object with
-    ``next_operator`` and ``launch``), or two queues with an engine coroutine at their other end."""
+    ``next_operator``, ``launch`` and ``give_way``), or two queues with an engine coroutine at their other end.
+
+    A scheduler may run several coroutines, say one per nano-batch: ``execute`` lets the others have their turn, so
+    operators are launched in the order in which the coroutines ask for them, one each in turn."""
 
     def __init__(
         self,
@@ -148,6 +151,7 @@ class ExecutionContext:
         """
         if self._forward is not None:
             self._forward.launch(operator, func)
+            await self._forward.give_way()
             return
         if isinstance(operator, OperatorHandle):
             operator = (operator,)

@@ -37,6 +37,7 @@ from dynaflow_amd.config import DynaFlowConfig
 from dynaflow_amd.interface import OperatorHandle, SplitConfig
 from dynaflow_amd.runtime.device import get_device
 from dynaflow_amd.runtime.env import ExecutionEnvironment, set_op_handle
+from dynaflow_amd.runtime.loop import may_have_other_tasks
 
 _DEFAULT_MAX_TOKENS = 16384
 
@@ -435,6 +436,7 @@ class ScheduledForward:
         self.split = split_config
         self.args = args
         self.device = get_device()
+        self.origin_stream = self.device.current_stream()
         lanes = split_config.num_nano_batches
         self.env = ExecutionEnvironment(lanes)
         engine.last_env = self.env
@@ -494,7 +496,15 @@ class ScheduledForward:
         """Wait for another coroutine's launch."""
         moved = asyncio.Event()
         self._waiting.append(moved)
-        await moved.wait()
+        with self.device.stream(self.origin_stream):
+            await moved.wait()
+
+    async def give_way(self) -> None:
+        """Let the scheduler's other coroutines go on, if it has any.  The current stream belongs to the thread and a
+        coroutine may wait here inside its own ``with device.stream(...)``: the others find the caller's stream."""
+        if may_have_other_tasks():
+            with self.device.stream(self.origin_stream):
+                await asyncio.sleep(0)
 
     def launch(self, operators: "OperatorHandle | tuple[OperatorHandle, ...]", func: Callable | None = None) -> None:
         """Enqueue operators on the current stream, behind the previous work of their nano-batches."""

@@ -13,6 +13,17 @@ from collections.abc import Coroutine
 from typing import Any
 
 
+class _TaskFactory:
+    """Makes a loop's tasks and counts the ones of a run."""
+
+    def __init__(self) -> None:
+        self.made = 0
+
+    def __call__(self, loop: asyncio.AbstractEventLoop, coroutine: Coroutine, **kwargs: Any) -> asyncio.Task:
+        self.made += 1
+        return asyncio.Task(coroutine, loop=loop, **kwargs)
+
+
 class _KeptLoop:
     """A loop and whoever closes it: the thread's locals hold this object and the loop does not, so it goes, and the loop
     is closed, when they are dropped at the end of the thread.  (A loop by itself is part of reference cycles and would
@@ -20,6 +31,8 @@ class _KeptLoop:
 
     def __init__(self) -> None:
         self.loop = asyncio.new_event_loop()
+        self.tasks = _TaskFactory()
+        self.loop.set_task_factory(self.tasks)
         self.process = os.getpid()
 
     def __del__(self) -> None:
@@ -39,11 +52,21 @@ _inherited: list[asyncio.AbstractEventLoop] = []
 _thread = threading.local()
 
 
-def _thread_loop() -> asyncio.AbstractEventLoop:
+def _kept_loop() -> _KeptLoop:
     kept = getattr(_thread, "kept", None)
     if kept is None or kept.process != os.getpid() or kept.loop.is_closed():
         kept = _thread.kept = _KeptLoop()
-    return kept.loop
+    return kept
+
+
+def may_have_other_tasks() -> bool:
+    """False if the coroutine of ``run_coroutine`` that runs now is the only one: it has started no task.  (Half a
+    microsecond where a turn of the loop takes three.)"""
+    kept = getattr(_thread, "kept", None)
+    loop = asyncio.get_running_loop()
+    if kept is None or kept.loop is not loop or loop.get_task_factory() is not kept.tasks:
+        return True
+    return kept.tasks.made > 1
 
 
 def run_coroutine(coroutine: Coroutine) -> Any:
@@ -55,7 +78,8 @@ def run_coroutine(coroutine: Coroutine) -> Any:
     else:
         coroutine.close()
         raise RuntimeError("a forward cannot be called from a running event loop")
-    loop = _thread_loop()
+    kept = _kept_loop()
+    loop, kept.tasks.made = kept.loop, 0
     try:
         return loop.run_until_complete(coroutine)
     finally:

@@ -509,3 +509,56 @@ def test_engine_coroutine_behind_queues_issues_what_the_manager_issues(host_devi
     for got, want in zip(y_queues if isinstance(y_queues, tuple) else (y_queues,),
                          y_direct if isinstance(y_direct, tuple) else (y_direct,)):
         assert torch.equal(got, want)
+
+
+class LaneScheduler(MLPOverlapScheduler):
+    """One coroutine per nano-batch, each on a stream of its own."""
+
+    async def schedule(self, context):
+        from dynaflow_amd.runtime.device import get_device
+
+        async def lane(b, stream):
+            while (op := await context.pop(b)) is not None:
+                with get_device().stream(stream):
+                    await context.execute((op,))
+
+        lanes = range(context.split_config.num_nano_batches)
+        await asyncio.gather(*(lane(b, self.lane_streams[b]) for b in lanes))
+
+
+class TwoLayers(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.layers = torch.nn.ModuleList(SwiGLUMLP(32, 96, dtype=torch.float32) for _ in range(2))
+
+    def forward(self, x):
+        for layer in self.layers:
+            x = layer(x)
+        return x
+
+
+@pytest.mark.parametrize("lanes", [2, 3])
+def test_a_coroutine_per_nano_batch_is_launched_in_turn(host_device, lanes):
+    """Schedulers that run one coroutine per nano-batch: every launch lets the other coroutines have their turn, as the
+    hand-over to an engine coroutine does, and a coroutine that waits inside its ``with device.stream`` neither lends its
+    stream to another one's launch nor leaves it behind."""
+    torch._dynamo.reset()
+    cfg = make_config(lanes, num_nano_batches=lanes)
+    scheduler = LaneScheduler(cfg)
+    scheduler.lane_streams = [host_device.new_stream(f"lane{b}") for b in range(lanes)]
+    torch.manual_seed(0)
+    model, manager, x = TwoLayers(), DynaFlowManager(), torch.randn(96, 32)
+    torch._dynamo.mark_dynamic(x, 0)
+    compiled = torch.compile(model, backend=make_backend(manager, cfg, scheduler), fullgraph=True)
+    manager.prepare(96, [96])
+    with torch.no_grad():
+        compiled(x)
+        assert manager.prepare(96, [96]).num_nano_batches == lanes
+        host_device.log.clear()
+        y = compiled(x)
+    torch.testing.assert_close(y, model(x), rtol=0, atol=0)
+    subgraphs = [name for name in top_level(manager) if isinstance(name, tuple)]
+    assert len(subgraphs) >= 4
+    assert manager.engine.issue_trace == [(name, b) for _, name in subgraphs for b in range(lanes)]
+    assert [e[2] for e in host_device.log if e[0] == "range"] == [f"lane{b}" for _ in subgraphs for b in range(lanes)]
+    assert host_device.current_stream().name == "default"
