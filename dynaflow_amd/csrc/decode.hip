@@ -312,6 +312,7 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
     __syncthreads();
     if (ticket != parts - 1) return;
     if (tid == 0) atomicExch(arrivals + pair, 0);
+    const auto left = coherent_blocks(blocks, parts * part_block(group) * 16);
     // Two threads share an item's parts (part q: thread q % 2) where there are threads enough; their sums meet in LDS,
     // in the room of the waves' partial results.
     const int lanes = 2 * items <= DEC_THREADS ? 2 : 1;
@@ -327,14 +328,11 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             const int q = q0 + c * lanes < parts ? q0 + c * lanes : q0;
-            v[c] = load_f32x4_device_coherent(blocks + q * part_block(group) + it);
-            ml[c] = load_f32x4_device_coherent(blocks + q * part_block(group) + items + (it >> 5));
+            const int at = (q * part_block(group) + it) * 16, head_at = (q * part_block(group) + items + (it >> 5)) * 16;
+            v[c] = load_f32x4_device_coherent(left, at, 0);
+            ml[c] = load_f32x4_device_coherent(left, head_at, 0);
           }
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            wait_loaded(v[c]);
-            wait_loaded(ml[c]);
-          }
+          DFHIP_PIN;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             // a part without a chunk left zeros; one whose scores are all NaN or -inf has the same maximum, and counts

@@ -136,19 +136,22 @@ DFHIP_DEVICE void wait_vmcnt() {
 // 16-byte store / load that is coherent across the XCDs (sc1: written through to, and read
 // from, the memory side instead of the XCD-private L2).  Used for split-K partial blocks so
 // that no L2-wide write-back or invalidate is needed to hand them from one XCD to another.
+// A load is a builtin and not inline assembly: the compiler takes an asm output as written at once, so it
+// may copy or reuse the registers of a load that is still on its way, and it places no wait for it.
 // A store of more than 8 bytes reads its data registers for a few cycles after issue and the compiler
 // cannot see that this statement is one: the wait states keep the next write to those registers away.
 DFHIP_DEVICE void store_f32x4_device_coherent(f32x4* p, f32x4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
-DFHIP_DEVICE f32x4 load_f32x4_device_coherent(const f32x4* p) {
-  f32x4 v;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
-  return v;
+// The blocks that the parts of one tile left: `base` is the same for the whole wave.
+DFHIP_DEVICE __amdgpu_buffer_rsrc_t coherent_blocks(const void* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00027000);
 }
-// The loads above are invisible to the compiler's own wait-count bookkeeping: a value may only
-// be used after this, which ties the wait to the register so that the use cannot move above it.
-DFHIP_DEVICE void wait_loaded(f32x4& v) { asm volatile("s_waitcnt vmcnt(0)" : "+v"(v)::"memory"); }
+// `at` bytes (of the lane) + `uniform` bytes (of the wave) into them
+DFHIP_DEVICE f32x4 load_f32x4_device_coherent(__amdgpu_buffer_rsrc_t blocks, int at, int uniform) {
+  constexpr int SC1 = 16;
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(blocks, at, uniform, SC1));
+}
 
 // one float, coherent across the XCDs
 DFHIP_DEVICE void store_device_coherent(float* p, float v) {

@@ -441,9 +441,7 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
     if (ticket != split_k - 1) return;
     if (tid == 0) atomicExch(arrivals + tile, 0);     // counters are left at zero
     __syncthreads();                                  // the ticket has been read before the tile is parked over it
-    const __amdgpu_buffer_rsrc_t rsrc =
-        __builtin_amdgcn_make_buffer_rsrc(blocks, 0, split_k * BLOCK * 16, 0x00027000);
-    constexpr int SC1 = 16;                           // read from the memory side, as the stores were written
+    const auto left = coherent_blocks(blocks, split_k * BLOCK * 16);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -455,8 +453,7 @@ gemm_fp8_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ 
         f32x4 v[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j)
-          v[j] = __builtin_bit_cast(
-              f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16, base + (i * 8 + j) * 4096, SC1));
+          v[j] = load_f32x4_device_coherent(left, tid * 16, base + (i * 8 + j) * 4096);
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           f32x4& sum = acc[i + j / 8][j % 8];

@@ -490,15 +490,17 @@ gemm_bf16_ring_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict
       __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // counters are left at zero
     }
     __syncthreads();
-    const f32x4* all = reinterpret_cast<const f32x4*>(partials) + (int64_t)tile * split_k * (64 * RTHREADS) + tid;
+    constexpr int BLOCK = 64 * RTHREADS * 16;   // bytes of a part
+    const auto all = coherent_blocks(reinterpret_cast<const uint8_t*>(partials) + (int64_t)tile * split_k * BLOCK,
+                                     split_k * BLOCK);
     for (int p = 0; p < split_k - 1; ++p) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         f32x4 v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = load_f32x4_device_coherent(all + ((int64_t)p * 64 + i * 8 + j) * RTHREADS);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) wait_loaded(v[j]);
+        for (int j = 0; j < 8; ++j)
+          v[j] = load_f32x4_device_coherent(all, tid * 16, p * BLOCK + (i * 8 + j) * (RTHREADS * 16));
+        DFHIP_PIN;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           acc[i][j] += v[j];
@@ -1326,7 +1328,9 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
     if (ticket != split_k - 1) return;
     if (tid == 0) atomicExch(arrivals + tile, 0);
     // the last arriver adds the parts in part order (its own is read back like the others)
-    const f32x4* all = reinterpret_cast<const f32x4*>(partials) + (int64_t)tile * split_k * (PIECES * RTHREADS) + tid;
+    constexpr int BLOCK = PIECES * RTHREADS * 16;   // bytes of a part
+    const auto all = coherent_blocks(reinterpret_cast<const uint8_t*>(partials) + (int64_t)tile * split_k * BLOCK,
+                                     split_k * BLOCK);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -1342,12 +1346,10 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
       for (int h = 0; h < TOGETHER; ++h) {
         const int p = p0 + h < split_k ? p0 + h : split_k - 1;
 #pragma unroll
-        for (int c = 0; c < PIECES; ++c) v[h][c] = load_f32x4_device_coherent(all + ((int64_t)p * PIECES + c) * RTHREADS);
+        for (int c = 0; c < PIECES; ++c)
+          v[h][c] = load_f32x4_device_coherent(all, tid * 16, p * BLOCK + c * (RTHREADS * 16));
       }
-#pragma unroll
-      for (int h = 0; h < TOGETHER; ++h)
-#pragma unroll
-        for (int c = 0; c < PIECES; ++c) wait_loaded(v[h][c]);
+      DFHIP_PIN;
 #pragma unroll
       for (int h = 0; h < TOGETHER; ++h) {
         if (p0 + h >= split_k) break;

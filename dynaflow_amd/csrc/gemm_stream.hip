@@ -169,7 +169,6 @@ gemm_stream_kernel(const StreamArgs p) {
   // The waves' sums meet in LDS, [wave][i][j][lane] with 16 bytes a lane; RI row blocks at a time, so that a workgroup
   // never asks for more than 64 KiB and a second one fits beside it (the launches of two nano-batches share the units).
   constexpr int RI = rows_per_round(MB, NB), ITEMS = RI * NB * 64;
-  const f32x4* const all = reinterpret_cast<const f32x4*>(p.partials) + (int64_t)tile * p.split_k * (MB * NB * 64);
   float vmax = 0.0f;
   const float sa = FP8 ? p.a_scale[0] : 1.0f;
   auto total = [&](int i, int j, int l) {
@@ -225,7 +224,9 @@ gemm_stream_kernel(const StreamArgs p) {
 
   if constexpr (SPLIT) {
     // the parts of a tile meet in memory: each leaves its sums, the part that arrives last adds them in part order
-    f32x4* const block = const_cast<f32x4*>(all) + (int64_t)part * (MB * NB * 64);
+    constexpr int BLOCK = MB * NB * 64 * 16;     // bytes of a part
+    f32x4* const all = reinterpret_cast<f32x4*>(p.partials) + (int64_t)tile * p.split_k * (MB * NB * 64);
+    f32x4* const block = all + (int64_t)part * (MB * NB * 64);
 #pragma unroll
     for (int i0 = 0; i0 < MB; i0 += RI) {
       gather(i0);
@@ -244,6 +245,7 @@ gemm_stream_kernel(const StreamArgs p) {
     __syncthreads();
     if (*ticket_cell != p.split_k - 1) return;
     if (tid == 0) atomicExch(p.arrivals + tile, 0);
+    const auto parts = coherent_blocks(all, p.split_k * BLOCK);
     for (int id = tid; id < MB * NB * 64; id += THREADS) {
       f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
       for (int q0 = 0; q0 < p.split_k; q0 += 4) {
@@ -251,10 +253,9 @@ gemm_stream_kernel(const StreamArgs p) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const int q = q0 + c < p.split_k ? q0 + c : p.split_k - 1;
-          more[c] = load_f32x4_device_coherent(all + (int64_t)q * (MB * NB * 64) + id);
+          more[c] = load_f32x4_device_coherent(parts, id * 16, q * BLOCK);
         }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) wait_loaded(more[c]);
+        DFHIP_PIN;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
           if (q0 + c < p.split_k) v += more[c];
