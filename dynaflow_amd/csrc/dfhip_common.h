@@ -38,11 +38,19 @@ static inline int dfhip_check_launch() {
 }
 
 // Split-K workspaces start with the arrival counters.  All split-K kernels, bf16 and fp8, use the same size of
-// counter area for a workspace (at least 4 KiB), so that the fp32 blocks one of them leaves behind
-// never lie where another expects counters that are zero.
+// counter area up to 1024 tiles (4 KiB), so that the fp32 blocks one of them leaves behind do not lie where another
+// expects counters that are zero.  A launch of more tiles has counters where smaller ones leave blocks, and clears
+// those first (a fill kernel, legal inside a captured graph).
+constexpr size_t DFHIP_COMMON_COUNTERS = 4096;
 static inline size_t dfhip_counter_area(size_t tiles) {
   const size_t need = ((tiles * sizeof(int)) + 255) & ~(size_t)255;
-  return need > 4096 ? need : 4096;
+  return need > DFHIP_COMMON_COUNTERS ? need : DFHIP_COMMON_COUNTERS;
+}
+static inline int dfhip_clear_uncommon_counters(void* workspace, size_t tiles, hipStream_t stream) {
+  const size_t area = dfhip_counter_area(tiles);
+  if (area == DFHIP_COMMON_COUNTERS) return DFHIP_OK;
+  return dfhip_fill_u32(static_cast<uint8_t*>(workspace) + DFHIP_COMMON_COUNTERS, 0u,
+                        (int64_t)((area - DFHIP_COMMON_COUNTERS) / 4), stream);
 }
 
 // bf16 <-> fp32 on raw 16-bit storage

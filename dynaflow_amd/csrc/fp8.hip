@@ -536,7 +536,11 @@ int launch_fp8_ring(const void* A, int64_t lda, const void* W, int64_t ldw, void
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), F8_RING_LDS, lds_opted_in)) return rc;
   const int tiles_m = (M + 32 * TM - 1) / (32 * TM), tiles_n = (N + 255) / 256;
   float* partials = nullptr;
-  if (SPLIT) partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area((size_t)tiles_m * tiles_n));
+  if (SPLIT) {
+    const size_t tiles = (size_t)tiles_m * tiles_n;
+    if (int rc = dfhip_clear_uncommon_counters(workspace, tiles, stream)) return rc;
+    partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area(tiles));
+  }
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(256), F8_RING_LDS, stream,
                      static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), nullptr,
                      static_cast<uint16_t*>(C), a_scale, w_scale, nullptr, nullptr, M, N, K, lda, ldw, ldc, tiles_m,

@@ -583,7 +583,9 @@ int launch_ring(const void* A, int64_t lda, const void* W, const void* W2, int64
   float* partials = nullptr;
   int lead_slabs = K / BK;
   if (split_k > 1) {
-    partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area((size_t)tiles_m * tiles_n));
+    const size_t tiles = (size_t)tiles_m * tiles_n;
+    if (int rc = dfhip_clear_uncommon_counters(workspace, tiles, stream)) return rc;
+    partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area(tiles));
     lead_slabs = (K / BK) / split_k;   // an even split measured best (a smaller share for the parts that only leave a block did not pay)
   }
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(RTHREADS), RING_LDS, stream,
@@ -1577,7 +1579,10 @@ int launch_skinny_tile(const void* A, int64_t lda, const void* W, const void* W2
   const int tiles_n = (N + TILE_N - 1) / TILE_N;
   int* arrivals = static_cast<int*>(workspace);
   float* partials = nullptr;
-  if (split_k > 1) partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + skinny_counter_bytes(M, N));
+  if (split_k > 1) {
+    if (int rc = dfhip_clear_uncommon_counters(workspace, skinny_tiles(M, N), stream)) return rc;
+    partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + skinny_counter_bytes(M, N));
+  }
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(RTHREADS), LDS, stream,
                      static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(W),
                      static_cast<const uint16_t*>(W2), static_cast<uint16_t*>(C), M, N, K, lda, ldw, ldc, tiles_m,

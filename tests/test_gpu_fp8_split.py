@@ -110,3 +110,29 @@ def test_split_launches_of_both_types_share_a_workspace():
         got8, got16 = ops.linear_fp8(xq, wq, xs, ws), ops.linear(x, w)
         assert (got8.float() - want8).abs().max().item() <= 2.0 ** -7 * want8.abs().max().item()
         assert (got16.float() - want16).abs().max().item() <= 2.0 ** -7 * want16.abs().max().item()
+
+
+@pytest.mark.gpu
+def test_split_launches_of_more_tiles_than_the_common_counters_share_a_workspace():
+    """More than 1024 tiles: their counters lie where a launch of few tiles leaves its partial sums."""
+    lib, stream = _cabi.load(), torch.cuda.current_stream().cuda_stream
+    few, many = (130, 1032, 4096, 4), (4, 256 * 1030, 512, 2)
+    x, w, g = randn((20, 1024), 4), randn((128 * 1030, 1024), 5, 0.05), torch.Generator(device="cuda").manual_seed(6)
+    nbytes = max([lib.dfhip_gemm_fp8_splitk_workspace_bytes(M, N, 4, s) for M, N, _, s in (few, many)]
+                 + [lib.dfhip_gemm_bf16_splitk_workspace_bytes(20, 128 * 1030, 2)])
+    workspace = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+    for _ in range(2):
+        for M, N, K, split in (few, many):
+            xq, wq = ((torch.randn(s, generator=g, device="cuda") * 16).to(F8) for s in ((M, K), (N, K)))
+            xs, ws = torch.full((1,), 0.01, device="cuda"), torch.full((N,), 0.01, device="cuda")
+            out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+            assert lib.dfhip_gemm_fp8_nt_splitk(
+                xq.data_ptr(), K, wq.data_ptr(), K, out.data_ptr(), N, xs.data_ptr(), ws.data_ptr(), M, N, K, 4, split,
+                workspace.data_ptr(), nbytes, stream) == 0
+            want = (xq.float() @ wq.float().t()) * 1e-4
+            assert (out.float() - want).abs().max().item() <= 2.0 ** -7 * want.abs().max().item()
+        out = torch.full((20, 128 * 1030), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert lib.dfhip_gemm_bf16_nt_splitk(x.data_ptr(), 1024, w.data_ptr(), 1024, out.data_ptr(), 128 * 1030, 20,
+                                             128 * 1030, 1024, 2, workspace.data_ptr(), nbytes, stream) == 0
+        want = x.float() @ w.float().t()
+        assert (out.float() - want).abs().max().item() <= 2.0 ** -7 * want.abs().max().item()
