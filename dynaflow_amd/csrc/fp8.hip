@@ -787,9 +787,9 @@ double tile_cost(int64_t tiles, int split_k, int share, int K, double per_slab, 
 struct RingTile { int variant, tm; double per_slab; };
 constexpr RingTile F8_RINGS[3] = {{0, 8, 1.07}, {3, 6, 0.97}, {4, 4, 0.85}};
 
-// The tile shape and the parts of K.  K is only cut where K > N, the projection back to the model width, which has few
-// tiles and a long K (8192 x 28672, us at 128 / 350 / 1024 rows: 244 / 230 / 244 before, 64 / 96 / 182 now); the
-// projections in front of it keep one order of their sums, that of the fused launch.  At least eight slabs a part.
+// The tile shape and the parts of K.  K is only cut where the caller allows it, for the projection back to the model
+// width, and where K > N: few tiles and a long K (8192 x 28672, us at 128 / 350 / 1024 rows: 245 / 236 / 242 before,
+// 78 / 90 / 183 now).  At least eight slabs a part.
 TilePlan plan_tile(int M, int N, int K, int share, bool may_split) {
   TilePlan best{2, 1, tile_cost((int64_t)((M + 255) / 256) * ((N + F8_TBN - 1) / F8_TBN), 1, share, K, 1.0, 0)};
   for (const RingTile& ring : F8_RINGS) {

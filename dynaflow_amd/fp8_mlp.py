@@ -53,11 +53,11 @@ class Fp8SwiGLU(nn.Module):
         xq, xs = ops.quant_fp8(x)
         if self.fuse_gate_up:
             aq, a_s = ops.gate_up_silu_quant_fp8(xq, self.w_gate_q, self.w_up_q, xs, self.w_gate_s, self.w_up_s)
-            return ops.linear_fp8(aq, self.w_down_q, a_s, self.w_down_s)
+            return ops.linear_fp8(aq, self.w_down_q, a_s, self.w_down_s, True)
         g = ops.linear_fp8(xq, self.w_gate_q, xs, self.w_gate_s)
         u = ops.linear_fp8(xq, self.w_up_q, xs, self.w_up_s)
         aq, a_s = ops.silu_mul_quant_fp8(g, u)
-        return ops.linear_fp8(aq, self.w_down_q, a_s, self.w_down_s)
+        return ops.linear_fp8(aq, self.w_down_q, a_s, self.w_down_s, True)
 
     def forward_schedule(self, x: torch.Tensor, split_indices: list[int]) -> torch.Tensor:
         """The split schedule issued directly, one nano-batch after the other."""

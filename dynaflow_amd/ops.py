@@ -57,9 +57,9 @@ _lib.define(
 )
 _lib.define("quant_fp8(Tensor x) -> (Tensor, Tensor)")
 _lib.define("silu_mul_quant_fp8(Tensor gate, Tensor up) -> (Tensor, Tensor)")
-_lib.define("linear_fp8(Tensor x_q, Tensor w_q, Tensor x_scale, Tensor w_scale) -> Tensor")
+_lib.define("linear_fp8(Tensor x_q, Tensor w_q, Tensor x_scale, Tensor w_scale, bool cut_k=False) -> Tensor")
 _lib.define("linear_fp8_variant(Tensor x_q, Tensor w_q, Tensor x_scale, Tensor w_scale, int variant) -> Tensor")
-_lib.define("linear_fp8_to_output(Tensor x_q, Tensor w_q, Tensor x_scale, Tensor w_scale) -> Tensor")
+_lib.define("linear_fp8_to_output(Tensor x_q, Tensor w_q, Tensor x_scale, Tensor w_scale, bool cut_k=False) -> Tensor")
 _lib.define(
     "gate_up_silu_quant_fp8(Tensor x_q, Tensor w_gate_q, Tensor w_up_q, Tensor x_scale, Tensor w_gate_scale, "
     "Tensor w_up_scale) -> (Tensor, Tensor)"
@@ -794,7 +794,9 @@ def _gate_up_silu_quant_fp8_impl(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w
     return q.view(*x_q.shape[:-1], I), scale
 
 
-def _linear_fp8_impl(x_q, w_q, x_scale, w_scale, variant: int = -1, to_output: bool = False):
+def _linear_fp8_impl(x_q, w_q, x_scale, w_scale, variant: int = -1, to_output: bool = False, cut_k: bool = False):
+    """``cut_k``: K may be cut into parts that are summed one after the other, where that is faster (the projection back
+    to the model width).  Without it the sums have the order of ``gate_up_silu_quant_fp8``, whatever the widths are."""
     _require_device(x_q, w_q, x_scale, w_scale)
     lib = _cabi.load()
     if x_q.dtype != FP8_DTYPE or w_q.dtype != FP8_DTYPE:
@@ -808,7 +810,7 @@ def _linear_fp8_impl(x_q, w_q, x_scale, w_scale, variant: int = -1, to_output: b
     out = _new_output(M, N, torch.bfloat16, x_q.device, to_output)
     if M > 0:
         stream, split_k = _stream(), 1
-        if variant < 0:
+        if variant < 0 and (cut_k or K <= N):         # (K <= N is not cut; the plan knows the launches side by side)
             planned, parts = ctypes.c_int(-1), ctypes.c_int(1)
             _cabi.check("dfhip_gemm_fp8_plan_shared", lib.dfhip_gemm_fp8_plan_shared(
                 M, N, K, _side_by_side(), ctypes.byref(planned), ctypes.byref(parts)))
@@ -840,9 +842,10 @@ torch.library.register_fake(
                                        x_q.new_empty((1,), dtype=torch.float32)),
     lib=_lib,
 )
-_lib.impl("linear_fp8", lambda x_q, w_q, xs, ws: _linear_fp8_impl(x_q, w_q, xs, ws), "CUDA")
+_lib.impl("linear_fp8", lambda x_q, w_q, xs, ws, cut_k=False: _linear_fp8_impl(x_q, w_q, xs, ws, cut_k=cut_k), "CUDA")
 _lib.impl("linear_fp8_variant", lambda x_q, w_q, xs, ws, v: _linear_fp8_impl(x_q, w_q, xs, ws, v), "CUDA")
-_lib.impl("linear_fp8_to_output", lambda x_q, w_q, xs, ws: _linear_fp8_impl(x_q, w_q, xs, ws, to_output=True), "CUDA")
+_lib.impl("linear_fp8_to_output",
+          lambda x_q, w_q, xs, ws, cut_k=False: _linear_fp8_impl(x_q, w_q, xs, ws, to_output=True, cut_k=cut_k), "CUDA")
 torch.library.register_fake(
     "dynaflow_hip::quant_fp8",
     lambda x: (x.new_empty(x.shape, dtype=FP8_DTYPE), x.new_empty((1,), dtype=torch.float32)),
@@ -855,12 +858,12 @@ torch.library.register_fake(
 )
 torch.library.register_fake(
     "dynaflow_hip::linear_fp8",
-    lambda x_q, w_q, xs, ws: x_q.new_empty((*x_q.shape[:-1], w_q.shape[0]), dtype=torch.bfloat16),
+    lambda x_q, w_q, xs, ws, cut_k=False: x_q.new_empty((*x_q.shape[:-1], w_q.shape[0]), dtype=torch.bfloat16),
     lib=_lib,
 )
 torch.library.register_fake(
     "dynaflow_hip::linear_fp8_to_output",
-    lambda x_q, w_q, xs, ws: x_q.new_empty((*x_q.shape[:-1], w_q.shape[0]), dtype=torch.bfloat16),
+    lambda x_q, w_q, xs, ws, cut_k=False: x_q.new_empty((*x_q.shape[:-1], w_q.shape[0]), dtype=torch.bfloat16),
     lib=_lib,
 )
 torch.library.register_fake(

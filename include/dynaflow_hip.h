@@ -228,8 +228,9 @@ int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void* W, int64_t
  * arrival counters (4 bytes a tile at its start) are zero; they are left zero.  Launches that may overlap need one
  * each.  The parts are added in part order: the same bits in every run.
  * dfhip_gemm_fp8_plan_shared: the variant and split for `share` launches of this shape side by side (variant < 0: the
- * launch without a split decides).  K is only cut where K > N (the projection back to the model width): the projections
- * in front of it keep one order of their sums, that of dfhip_gemm_fp8_gate_up_silu_absmax. */
+ * launch without a split decides).  For the projection back to the model width: K is only cut where K > N, and the
+ * projections in front of it, which keep the order of sums of dfhip_gemm_fp8_gate_up_silu_absmax, are launched without a
+ * split whatever their widths are. */
 int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
 size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k);
 int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,

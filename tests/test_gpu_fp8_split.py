@@ -99,6 +99,57 @@ def test_fused_fp8_tile_heights(M, I, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,I,K", [(128, 1024, 4096), (256, 4096, 8192), (350, 1536, 7168)])
+def test_fused_fp8_launch_with_an_intermediate_width_below_the_model_width(M, I, K):
+    """The planned gate and up launches, whose K > N could be cut, keep the order of sums of the fused one: the same codes
+    and scale, alone and side by side, and the same block output.  Operands over many binades, so that the order of the
+    fp32 sums shows in some of the results."""
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import Fp8SwiGLU, quantize_weight_per_channel
+
+    spread = lambda shape, seed: randn(shape, seed) * torch.exp2(randn(shape, seed + 50, 4.0))
+    xq, xs = ops.quant_fp8(spread((M, K), 1))
+    (wq, ws), (uq, us) = (quantize_weight_per_channel(spread((I, K), seed)) for seed in (2, 3))
+    whole = [ops.linear_fp8_variant(xq, w, xs, s, 0) for w, s in ((wq, ws), (uq, us))]
+    for share in (1, 2):
+        with ops.launch_options(share):
+            q, scale = ops.gate_up_silu_quant_fp8(xq, wq, uq, xs, ws, us)
+            gate, up = ops.linear_fp8(xq, wq, xs, ws), ops.linear_fp8(xq, uq, xs, us)
+        assert torch.equal(gate, whole[0]) and torch.equal(up, whole[1])
+        want_q, want_scale = ops.silu_mul_quant_fp8(gate, up)
+        assert torch.equal(scale, want_scale) and torch.equal(q.view(torch.uint8), want_q.view(torch.uint8))
+    outs = [Fp8SwiGLU.from_weights(spread((I, K), 6), spread((I, K), 7), spread((K, I), 8), fuse_gate_up=fused)(
+        spread((M, K), 9)) for fused in (False, True)]
+    assert torch.equal(*outs)
+
+
+@pytest.mark.gpu
+def test_fp8_block_cuts_the_projection_back_to_the_model_width():
+    """The block's down projection is the launch in parts (which takes the workspace), the caller's plain one is not."""
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import Fp8SwiGLU
+
+    hidden, inter, x = 1024, 4096, randn((130, 1024), 9)
+    model = Fp8SwiGLU.from_weights(randn((inter, hidden), 6, 0.05), randn((inter, hidden), 7, 0.05),
+                                   randn((hidden, inter), 8, 0.05))
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    taken = lambda: sum(key[-1] == stream.cuda_stream for key in ops._splitk_workspaces)
+    with torch.cuda.stream(stream):
+        xq, xs = ops.quant_fp8(x)
+        aq, scale = ops.gate_up_silu_quant_fp8(xq, model.w_gate_q, model.w_up_q, xs, model.w_gate_s, model.w_up_s)
+        before = taken()
+        whole = ops.linear_fp8(aq, model.w_down_q, scale, model.w_down_s)
+        assert taken() == before
+        y = model(x)
+        cut = ops.linear_fp8(aq, model.w_down_q, scale, model.w_down_s, True)
+    stream.synchronize()
+    assert before == 0 and taken() == 1
+    assert torch.equal(y, cut)
+    assert (cut.float() - whole.float()).abs().max().item() <= 2.0 ** -7 * whole.float().abs().max().item()
+
+
+@pytest.mark.gpu
 def test_split_launches_of_both_types_share_a_workspace():
     """What an fp8 launch leaves in the workspace of a stream is nothing a bf16 launch takes for a counter."""
     from dynaflow_amd import ops
@@ -107,7 +158,7 @@ def test_split_launches_of_both_types_share_a_workspace():
     x, w = randn((17, 4096), 4), randn((4096, 4096), 5, 0.05)      # 2 parts, up to 256 counters
     want8, want16 = (xq.float() * xs) @ (wq.float() * ws[:, None]).t(), x.float() @ w.float().t()
     for _ in range(2):
-        got8, got16 = ops.linear_fp8(xq, wq, xs, ws), ops.linear(x, w)
+        got8, got16 = ops.linear_fp8(xq, wq, xs, ws, True), ops.linear(x, w)
         assert (got8.float() - want8).abs().max().item() <= 2.0 ** -7 * want8.abs().max().item()
         assert (got16.float() - want16).abs().max().item() <= 2.0 ** -7 * want16.abs().max().item()
 
