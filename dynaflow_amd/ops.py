@@ -533,8 +533,9 @@ def _token_rows(t: torch.Tensor, what: str):
 
 
 def _aligned_rows(t: torch.Tensor, ld: int):
-    """Token rows that start on 16 bytes: a copy where a view's offset or row stride says otherwise."""
-    if t.data_ptr() % 16 or ld % 8:
+    """Token rows that start on 16 bytes, less than 2^24 elements apart: a copy where a view's offset or stride says
+    otherwise."""
+    if t.data_ptr() % 16 or ld % 8 or ld >= 1 << 24:
         t = t.clone(memory_format=torch.contiguous_format)
     return t, t.stride(1)
 

@@ -255,3 +255,14 @@ def test_side_by_side_option_and_the_plan_for_shared_launches():
     assert plan(128, 6144, 4096, 2) == (6, 2) and plan(128, 14336, 4096, 2) == (6, 1)
     v, k = ctypes.c_int(), ctypes.c_int()
     assert lib.dfhip_gemm_bf16_plan_shared(2048, 4096, 14336, 0, ctypes.byref(v), ctypes.byref(k)) == -7
+
+
+@pytest.mark.parametrize("stride", [1 << 24, 1 << 26])
+def test_ragged_attention_takes_rows_that_are_far_apart(stride):
+    """The kernel keeps a block's byte offsets in 32 bits and refuses wider rows; PyTorch's attention, which took the
+    lengths that are no multiple of 64 before, did not."""
+    far = torch.empty_strided((1, 65, 8, 128), (65 * stride, stride, 128, 1), dtype=torch.bfloat16, device="meta")
+    t, ld = ops._aligned_rows(*ops._token_rows(far, "k"))
+    assert ld == 8 * 128 and t.stride() == (65 * ld, ld, 128, 1)
+    near = torch.empty_strided((1, 65, 8, 128), (65 * 2048, 2048, 128, 1), dtype=torch.bfloat16, device="meta")
+    assert ops._aligned_rows(*ops._token_rows(near, "k"))[0] is near
