@@ -254,7 +254,7 @@ class HipDevice:
         return current_stream()
 
     def stream(self, stream: "torch.cuda.Stream"):
-        if stream.device_index != torch._C._cuda_getDevice():
+        if stream is None or stream.device_index != torch._C._cuda_getDevice():
             return torch.cuda.stream(stream)
         return _CurrentStream(stream)
 

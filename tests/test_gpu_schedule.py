@@ -737,3 +737,13 @@ def test_decoder_layer_whole_schedule_graph_with_padded_capture_size():
             assert y.shape == eager.shape and torch.equal(y, eager), f"replay {i}"
             torch.randn(256, 256, device="cuda").sum().item()
     assert len(manager._schedule_graphs) == 1
+
+
+def test_a_scheduler_may_name_no_stream():
+    """``device.stream(None)`` leaves the current stream as it is, like ``torch.cuda.stream(None)``."""
+    from dynaflow_amd.runtime.device import get_device
+
+    device, side = get_device(), torch.cuda.Stream()
+    with device.stream(side), device.stream(None):
+        assert torch.cuda.current_stream() == side and device.current_stream() == side
+    assert torch.cuda.current_stream() == torch.cuda.default_stream()
