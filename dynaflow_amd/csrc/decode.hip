@@ -46,6 +46,16 @@ DFHIP_DEVICE void store_row(uint16_t* out_row, int it, f32x4 num, float den) {
 // 16-byte words of a part's block in the workspace: the sums of `group` heads, then one word (maximum, sum) per head.
 __host__ __device__ constexpr int part_block(int group) { return group * (HD / 4 + 1); }
 
+// Parts of a sequence of `len` positions where the launch has `parts` workgroups for each: at least 256 positions (two
+// chunks per wave) a part, and at least three parts, since the meeting costs about 3 us.  Shorter sequences stay whole:
+// the bits of an uncut launch, and its time but for the start of the workgroups that end at once.  [us, uncut / cut by the
+// capacity alone / by the length: 2 sequences in a cache of 8192 positions, of 33 6.4 / 13.4 / 6.6, of 512 9.8 / 14.3 /
+// 9.9, of 2048 27 - 31 / 16.8 / 11.6, of 8192 111 / 21.9 / 21.0]
+DFHIP_DEVICE int sequence_parts(int len, int parts) {
+  if (len < 3 * 256) return 1;
+  return len / 256 < parts ? len / 256 : parts;
+}
+
 // One workgroup per (token, kv head).  Wave w takes the chunks w, w+4, ... of 32 positions.
 // MFMA row i of a score tile is mapped to position 8*(i/4) + i%4 (+4 for the second tile of the
 // chunk), so that after the two tiles lane (head = lane%16, g = lane/16) holds the scores of its
@@ -59,10 +69,10 @@ __host__ __device__ constexpr int part_block(int group) { return group * (HD / 4
 // barrier: the wave that wrote the LDS words is the one that reads them; the other three waves only rotate their
 // copies of the query heads).
 //
-// SPLIT: a (token, kv head) pair has `parts` workgroups, each with its share of the token's chunks, for launches with too
-// few pairs to fill the chip (attention_parts says when).  A part leaves its unnormalised sums, maximum and sum of exponentials in `partials`
-// ([pair][part][part_block(group)] words of 16 bytes), counts itself in and is done; the part that arrives last combines
-// them, in the same order whoever that is.
+// SPLIT: a (token, kv head) pair has `parts` workgroups, for launches with too few pairs to fill the chip (attention_parts
+// says when), of which the token's length takes as many as pay (sequence_parts); the others end at once.  A part leaves
+// its unnormalised sums, maximum and sum of exponentials in `partials` ([pair][part][part_block(group)] words of 16
+// bytes), counts itself in and is done; the part that arrives last combines them, in the same order whoever that is.
 template <bool APPEND, bool SPLIT>
 __global__ void __launch_bounds__(DEC_THREADS)
 decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* __restrict__ kc,
@@ -77,8 +87,11 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
   float* const o_lds = combine_lds;                       // [4][group][HD]
   float* const m_lds = combine_lds + 4 * group * HD;      // [4][group]
   float* const l_lds = m_lds + 4 * group;                 // [4][group]
-  const int pair = SPLIT ? blockIdx.x / parts : blockIdx.x;
-  const int part = SPLIT ? blockIdx.x - pair * parts : 0;
+  // Part-major: the parts that every sequence uses are dispatched first and lie on all XCDs.  (Pair-major, the only
+  // workgroups with work of 8 short sequences are every eighth one, on one XCD: 512 positions 20.2 us, so 12.5.)
+  const int pairs = SPLIT ? gridDim.x / parts : gridDim.x;
+  const int part = SPLIT ? blockIdx.x / pairs : 0;
+  const int pair = blockIdx.x - part * pairs;
   const int t = pair / kv_heads, kvh = pair - t * kv_heads;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hq = lane & 15, g = lane >> 4;
@@ -93,6 +106,8 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
   const int pos = len - 1;                     // APPEND: the new token's position (before the clamp below)
   const bool append = APPEND && pos < capacity;
   len = len < capacity ? len : capacity;
+  const int used = SPLIT ? sequence_parts(len, parts) : 1;   // workgroups that share this pair
+  if (SPLIT && part >= used) return;
   const int64_t head_base = ((int64_t)slot * kv_heads + kvh) * capacity * HD;
   uint16_t* kbase = kc + head_base;
   uint16_t* vbase = vc + head_base;
@@ -210,8 +225,8 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
 
   // two fragment sets in turn: the loads of the next chunk are in flight while one is multiplied
   const int all_chunks = (len + CHUNK - 1) / CHUNK;
-  const int chunk0 = SPLIT ? (int)((int64_t)all_chunks * part / parts) : 0;
-  const int chunks = SPLIT ? (int)((int64_t)all_chunks * (part + 1) / parts) : all_chunks;   // end of this part's
+  const int chunk0 = SPLIT ? (int)((int64_t)all_chunks * part / used) : 0;
+  const int chunks = SPLIT ? (int)((int64_t)all_chunks * (part + 1) / used) : all_chunks;   // end of this part's
   KVFrags fa, fb;
   if (chunk0 + wave < chunks) load(fa, chunk0 + wave);
   // (the first chunk's loads are on their way while the query heads are rotated)
@@ -284,17 +299,15 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
     for (int w = 1; w < 4; ++w) mm = fmaxf(mm, m_lds[w * group + h]);
     f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
     float den = 0.0f;
-    if (!SPLIT || chunk0 < chunks) {                        // (a part can be without a chunk, a token cannot)
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const float f = exp2f(m_lds[w * group + h] - mm);   // 0 for a wave that had no chunk (m = -inf)
-        const f32x4 v = reinterpret_cast<const f32x4*>(o_lds)[w * items + it];
+    for (int w = 0; w < 4; ++w) {
+      const float f = exp2f(m_lds[w * group + h] - mm);   // 0 for a wave that had no chunk (m = -inf)
+      const f32x4 v = reinterpret_cast<const f32x4*>(o_lds)[w * items + it];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) num[e] += v[e] * f;
-        den += l_lds[w * group + h] * f;
-      }
+      for (int e = 0; e < 4; ++e) num[e] += v[e] * f;
+      den += l_lds[w * group + h] * f;
     }
-    if constexpr (SPLIT) {
+    if (SPLIT && used > 1) {
       f32x4* const mine = blocks + part * part_block(group);
       store_f32x4_device_coherent(mine + it, num);
       if ((it & 31) == 0) store_f32x4_device_coherent(mine + items + h, f32x4{mm, den, 0.0f, 0.0f});
@@ -303,6 +316,7 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
     }
   }
   if constexpr (SPLIT) {
+    if (used == 1) return;
     wait_vmcnt<0>();
     __syncthreads();
     int* const ticket_cell = reinterpret_cast<int*>(combine_lds);
@@ -310,9 +324,9 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
     __syncthreads();
     const int ticket = *ticket_cell;
     __syncthreads();
-    if (ticket != parts - 1) return;
+    if (ticket != used - 1) return;
     if (tid == 0) atomicExch(arrivals + pair, 0);
-    const auto left = coherent_blocks(blocks, parts * part_block(group) * 16);
+    const auto left = coherent_blocks(blocks, used * part_block(group) * 16);
     // Two threads share an item's parts (part q: thread q % 2) where there are threads enough; their sums meet in LDS,
     // in the room of the waves' partial results.
     const int lanes = 2 * items <= DEC_THREADS ? 2 : 1;
@@ -323,11 +337,11 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
       for (int it = it0; it < items; it += lanes > 1 ? items : DEC_THREADS) {
         f32x4 num = {0.0f, 0.0f, 0.0f, 0.0f};
         float mm = -INFINITY, den = 0.0f;
-        for (int q0 = share; q0 < parts; q0 += 4 * lanes) {
+        for (int q0 = share; q0 < used; q0 += 4 * lanes) {
           f32x4 v[4], ml[4];
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            const int q = q0 + c * lanes < parts ? q0 + c * lanes : q0;
+            const int q = q0 + c * lanes < used ? q0 + c * lanes : q0;
             const int at = (q * part_block(group) + it) * 16, head_at = (q * part_block(group) + items + (it >> 5)) * 16;
             v[c] = load_f32x4_device_coherent(left, at, 0);
             ml[c] = load_f32x4_device_coherent(left, head_at, 0);
@@ -335,8 +349,7 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
           DFHIP_PIN;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            // a part without a chunk left zeros; one whose scores are all NaN or -inf has the same maximum, and counts
-            if (q0 + c * lanes >= parts || (ml[c][0] == -INFINITY && ml[c][1] == 0.0f)) continue;
+            if (q0 + c * lanes >= used) continue;
             const float m_new = fmaxf(mm, ml[c][0]);
             const float keep = exp2f(mm - m_new), add = exp2f(ml[c][0] - m_new);
 #pragma unroll
@@ -453,11 +466,11 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
 }
 
 // Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), with at least 256 positions of
-// a full cache each (two chunks per wave).  From 257 pairs on nothing is cut: the meeting of the parts costs about 10 us
-// of latency and an uncut launch fills the chip.  [us, uncut -> cut: 2 sequences of up to 8192 positions 111 -> 18
-// (their bytes at 6.7 TB/s: 8), 8 of 2048 33 -> 18 (10), 20 of up to 4096 68 -> 48 (32), 20 of 4096 74 -> 62 (50); 40 of
-// up to 1024 30 -> 30, 64 of 2048 87 -> 95, so those stay whole.]  The lengths are on the device: a short sequence in a
-// large cache is cut too finely rather than not at all, its parts without a chunk cost their start.
+// a full cache each (two chunks per wave).  The lengths are on the device: the launch is sized for full caches and each
+// sequence takes its share of it (sequence_parts).  A launch with fewer than MIN_PARTS of them, from 171 pairs on, cuts
+// nothing.  [us, uncut / cut: 2 sequences of 8192 positions 111 / 21.0 (their bytes at 6.7 TB/s: 10), 8 of 2048 33 / 16.8
+// (10), 20 of 4096 69 / 58 (50); in two parts, not taken: 32 of 512, 2048 and 4096 14.6 / 16.5, 42.9 / 46.0, 79 / 84]
+constexpr int MIN_PARTS = 3;
 static int attention_parts(int T, int kv_heads, int capacity) {
   const int64_t pairs = (int64_t)T * kv_heads;
   int64_t parts = 512 / pairs;
@@ -485,6 +498,7 @@ static int decode_attention_append(const void* qkv, int64_t ld_qkv, void* k_cach
     return DFHIP_ERR_BAD_ALIGNMENT;
   const int group = q_heads / kv_heads;
   const size_t lds_bytes = (size_t)4 * group * (HD + 2) * sizeof(float) + 2 * HD * sizeof(uint16_t);
+  if (parts < MIN_PARTS) parts = 1;
   const auto kernel = parts > 1 ? decode_attention_kernel<true, true> : decode_attention_kernel<true, false>;
   float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + ATTENTION_COUNTER_BYTES);
   hipLaunchKernelGGL(kernel, dim3(T * kv_heads * parts), dim3(DEC_THREADS), lds_bytes,

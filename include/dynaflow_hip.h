@@ -365,9 +365,9 @@ int dfhip_decode_attention_append_bf16(const void* qkv, int64_t ld_qkv, void* k_
                                        float scale, dfhip_stream_t stream);
 
 /* dfhip_decode_attention_append_bf16 for a step with few sequences: where T * kv_heads is too small to fill the chip, the
- * positions of a sequence are cut into parts (as many as T, kv_heads and capacity give) whose partial sums meet in
- * `workspace` (device memory, 16-byte aligned, at least dfhip_decode_attention_workspace_bytes; that is 0, and the
- * workspace may be null, where nothing is cut).  The workspace starts with arrival counters that must be zero before the
+ * positions of a long sequence (768 and more) are cut into parts - as many as T, kv_heads and capacity give workgroups
+ * for and its length makes worth it - whose partial sums meet in `workspace` (device memory, 16-byte aligned, at least
+ * dfhip_decode_attention_workspace_bytes; where that is 0 nothing is cut and the workspace may be null).  The workspace starts with arrival counters that must be zero before the
  * first use and are left zero; launches that may overlap in time need workspaces of their own.  The parts are combined
  * in a fixed order: the same bits in every run, but for a cut launch not those of the uncut one.  (The same node of the
  * host framework as above, examples/ae/scheduler/vllm/nanoflow.py:89-95.) */

@@ -164,11 +164,13 @@ def test_one_launch_decode_attention_has_the_bits_of_the_two_launches(heads, kv_
 
 
 @pytest.mark.parametrize("heads,kv_heads,capacity,lengths", [
-    (32, 8, 512, [1, 512, 33, 256]),                 # two parts: one position, the cut on and beside a chunk's edge
-    (4, 1, 8192, [8192, 1, 300]),                    # 32 parts, most of them without a chunk for the short ones
+    (32, 8, 512, [1, 512, 33, 256]),                 # room for two parts, which do not pay: whole
+    (4, 1, 8192, [8192, 1, 300]),                    # 32 parts for the long one, the short ones whole
     (16, 1, 4096, [4095, 2049, 7, 65]),              # 16 query heads on one kv head
     (3, 3, 1024, [1024, 31, 513] * 7),               # no grouping
-    (32, 8, 2048, [2048 - 31 * i for i in range(32)]),   # the most pairs that are still cut
+    (32, 8, 2048, [2048 - 31 * i for i in range(32)]),   # two parts again
+    (32, 8, 2048, [2048 - 64 * i for i in range(21)]),   # the most pairs that are still cut: three parts each
+    (8, 2, 4096, [767, 768, 1023, 1024, 1025, 4096]),    # around the lengths that take one, three and four parts
 ])
 def test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, lengths):
     """Few (token, kv head) pairs: several workgroups share a token's positions and the last to arrive combines them.
@@ -204,6 +206,30 @@ def test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, len
     assert rel_err(outs[0], want) < 2 ** -7
     for ws in ops._attention_workspaces.values():
         assert int(ws[:4096].view(torch.int32).abs().sum()) == 0
+
+
+@pytest.mark.parametrize("T,capacity,lengths", [(2, 8192, [1, 33, 512, 767]), (8, 1024, [64, 767]), (32, 2048, [2048, 700])])
+def test_decode_attention_stays_whole_where_parts_do_not_pay(ops, T, capacity, lengths):
+    """Sequences too short for three parts of 256 positions, and launches with room for two parts only: the bits of the
+    uncut launch."""
+    from dynaflow_amd import _cabi
+    from dynaflow_amd.decoder import rope_tables
+
+    heads, kv_heads = 32, 8
+    g = torch.Generator(device="cuda").manual_seed(T)
+    qkv = torch.randn(T, (heads + 2 * kv_heads) * D, generator=g, device="cuda").bfloat16()
+    slots = torch.arange(T, dtype=torch.int32, device="cuda")
+    lens = torch.tensor([lengths[i % len(lengths)] for i in range(T)], dtype=torch.int32, device="cuda")
+    cos, sin = (t.cuda() for t in rope_tables(capacity, D, 500000.0))
+    k = torch.randn(T, kv_heads, capacity, D, generator=g, device="cuda").bfloat16()
+    v = torch.randn(T, kv_heads, capacity // 8, D, 8, generator=g, device="cuda").bfloat16()
+    k1, v1, want = k.clone(), v.clone(), torch.empty(T, heads * D, dtype=torch.bfloat16, device="cuda")
+    _cabi.check("append", _cabi.load().dfhip_decode_attention_append_bf16(
+        qkv.data_ptr(), qkv.stride(0), k1.data_ptr(), v1.data_ptr(), slots.data_ptr(), lens.data_ptr(), cos.data_ptr(),
+        sin.data_ptr(), want.data_ptr(), heads * D, T, heads, kv_heads, D, T, capacity, capacity, D ** -0.5,
+        torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(ops.decode_attention(qkv, k, v, slots, lens, cos, sin, heads, kv_heads), want)
+    assert torch.equal(k, k1) and torch.equal(v, v1)
 
 
 def test_decode_attention_cut_over_positions_keeps_nan(ops):
