@@ -77,6 +77,7 @@ SIGNATURES: dict[str, tuple] = {
     "dfhip_gemm_bf16_gate_up_silu_shared": (c_int, [_P, c_int64, _P, _P, c_int64, _P, c_int64, c_int, c_int, c_int,
                                                     c_int, _P]),
     "dfhip_gemm_f32_nt": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P]),
+    "dfhip_gemm_f32_nt_shared": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_int, _P]),
     "dfhip_gemm_fp8_nt": (
         c_int,
         [_P, c_int64, _P, c_int64, _P, c_int64, _P, _P, c_int, c_int, c_int, _P],

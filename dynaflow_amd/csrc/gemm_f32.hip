@@ -4,9 +4,9 @@
 //   per workgroup so that a small product still has a workgroup for every compute unit; its four waves share the blocks
 //   and take the 128-byte slabs of K in turn, operands go straight from memory (L2) to registers, and the four partial
 //   sums meet in LDS.  Bound by the matrix pipes' fp32 rate and, at these sizes, by how evenly the blocks fall.
-// gemm_f32_nt_kernel (v_mfma_f32_32x32x2_f32, any K that is a multiple of 4): a 128x128 tile per workgroup, K walked in
-//   slabs of 16 through one LDS buffer.  LDS rows hold 16 floats padded to 17 so that the 32 lanes of a fragment read
-//   (one float each, rows 17 words apart) hit 32 different banks.
+// gemm_f32_nt_kernel (v_mfma_f32_32x32x2_f32, any K that is a multiple of 4; many rows with a K up to about 3000): a
+//   128x128 tile per workgroup, K walked in slabs of 16 through one LDS buffer.  LDS rows hold 16 floats padded to 17 so
+//   that the 32 lanes of a fragment read (one float each, rows 17 words apart) hit 32 different banks.
 #include "dfhip_common.h"
 
 namespace {
@@ -216,19 +216,39 @@ int launch_deep(const F32Args& p, hipStream_t stream) {
 // Smallest tile for which a wave's share of K has two slabs in flight.
 constexpr int SPLIT_MIN_K = 32 * SWAVES * 2;
 
-// The tile whose rounds of 256 workgroups take the least: a round costs its blocks and about 1.5 blocks' worth of start,
-// loads and meeting.  [us at [128 x 1024] x [2816 x 1024]^T / [128 x 2816] x [1024 x 2816]^T, with the workgroups in
-// parentheses: 2 x 3 blocks 12.4 (236) / 27.5 (88), 4 x 2 14.9 (176) / 32.7 (64), 2 x 2 17.2 (352) / 22.2 (128), 2 x 1
-// 18.4 (704) / 16.9 (256); the 128 x 128 tiles used before 105 (22) / 274 (8).  Floor at the fp32 rate: 4.9.]
-int launch_f32(const F32Args& p, hipStream_t stream) {
+int launch_tile128(const F32Args& p, hipStream_t stream) {
+  dim3 grid((p.N + FBN - 1) / FBN, (p.M + FBM - 1) / FBM);
+  hipLaunchKernelGGL(gemm_f32_nt_kernel, grid, dim3(FTHREADS), 0, stream, p.A, p.W, p.C, p.M, p.N, p.K, p.lda, p.ldw, p.ldc);
+  return dfhip_check_launch();
+}
+
+// The split tile that takes the least: one round of 256 workgroups costs its blocks and about 1.5 blocks' worth of start,
+// loads and meeting; of several rounds, whose workgroups overlap, each costs 0.6 of its blocks and of seven more for the
+// operands (per round at K = 2048: 4 x 4 blocks 37 us, 4 x 3 31, 4 x 2 25).  [us at [128 x 1024] x [2816 x 1024]^T / [128 x
+// 2816] x [1024 x 2816]^T, with the workgroups in parentheses: 2 x 3 blocks 12.4 (236) / 27.5 (88), 4 x 2 14.9 (176) /
+// 32.7 (64), 2 x 2 17.2 (352) / 22.2 (128), 2 x 1 18.4 (704) / 16.9 (256); the 128 x 128 tiles 105 (22) / 274 (8).  Floor at
+// the fp32 rate: 4.9.]
+// Many rows and a K up to about 3000 keep the 128 x 128 tiles, which read their operands half as often: both are priced
+// in us, fitted to about 190 launches (0.5 * 10^9 .. 10^12 flops, K = 288 .. 14336, alone and in pairs), the 128 x 128
+// tiles by their rounds (of all launches side by side: they fill each other's units).  [us, 128 x 128 / split: 8192 x 2816
+// x 512 250 / 319, 8192 x 5632 x 1024 801 / 978, 8192 x 5632 x 2048 1511 / 1623, 8192 x 4096 x 4096 2133 / 2123; a pair of
+// 3000 x 2816 x 1024 337 / 402, of 1500 x 2816 x 512 126 / 140]
+int launch_f32(const F32Args& p, int share, hipStream_t stream) {
   constexpr int SHAPES[8][2] = {{4, 4}, {4, 3}, {4, 2}, {2, 3}, {2, 2}, {2, 1}, {1, 2}, {1, 1}};
   int best = 0;
   double least = 0.0;
   for (int i = 0; i < 8; ++i) {
     const int64_t rounds = (split_tiles(p, SHAPES[i][0], SHAPES[i][1]) + 255) / 256;
-    const double cost = (double)rounds * (SHAPES[i][0] * SHAPES[i][1] + 1.5);
+    const int blocks = SHAPES[i][0] * SHAPES[i][1];
+    const double cost = rounds == 1 ? blocks + 1.5 : 0.6 * (double)rounds * (blocks + 7);
     if (i == 0 || cost < least) { best = i; least = cost; }
   }
+  const double k = p.K / 1024.0;
+  const int64_t tiles128 = (int64_t)((p.M + FBM - 1) / FBM) * ((p.N + FBN - 1) / FBN);
+  const double rounds128 = (double)((tiles128 * share + 255) / 256);
+  const bool fits = (p.M + FBM - 1) / FBM <= 65535;          // (the rows are the grid's second dimension)
+  if (fits && k * (45.0 + 58.0 * rounds128) + 8.0 * rounds128 < 1.06 * share * least * (0.52 + 1.06 * k))
+    return launch_tile128(p, stream);
   switch (best) {
     case 0: return launch_deep<4, 4>(p, stream);
     case 1: return launch_deep<4, 3>(p, stream);
@@ -243,20 +263,21 @@ int launch_f32(const F32Args& p, hipStream_t stream) {
 
 }  // namespace
 
-extern "C" int dfhip_gemm_f32_nt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
-                                 int M, int N, int K, dfhip_stream_t stream) {
+extern "C" int dfhip_gemm_f32_nt_shared(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
+                                        int M, int N, int K, int share, dfhip_stream_t stream) {
   if (!A || !W || !C) return DFHIP_ERR_NULL_POINTER;
   if (M < 1 || N < 1 || K < 1 || K % 4 != 0) return DFHIP_ERR_BAD_SHAPE;
   if (lda < K || ldw < K || ldc < N) return DFHIP_ERR_BAD_STRIDE;
   if (lda % 4 || ldw % 4 || !dfhip_aligned16(A) || !dfhip_aligned16(W) ||
       (reinterpret_cast<uintptr_t>(C) & 3u))
     return DFHIP_ERR_BAD_ALIGNMENT;
-  if (K % 32 == 0 && K >= SPLIT_MIN_K)
-    return launch_f32({static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N, K, lda,
-                       ldw, ldc}, static_cast<hipStream_t>(stream));
-  dim3 grid((N + FBN - 1) / FBN, (M + FBM - 1) / FBM);
-  hipLaunchKernelGGL(gemm_f32_nt_kernel, grid, dim3(FTHREADS), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N,
-                     K, lda, ldw, ldc);
-  return dfhip_check_launch();
+  if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
+  const F32Args p{static_cast<const float*>(A), static_cast<const float*>(W), static_cast<float*>(C), M, N, K, lda, ldw, ldc};
+  if (K % 32 == 0 && K >= SPLIT_MIN_K) return launch_f32(p, share, static_cast<hipStream_t>(stream));
+  return launch_tile128(p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int dfhip_gemm_f32_nt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
+                                 int M, int N, int K, dfhip_stream_t stream) {
+  return dfhip_gemm_f32_nt_shared(A, lda, W, ldw, C, ldc, M, N, K, 1, stream);
 }

@@ -245,10 +245,10 @@ def _linear_impl(x: torch.Tensor, weight: torch.Tensor, variant: int = -1, split
                     )
                     _cabi.check("dfhip_gemm_bf16_nt", rc)
         elif x.dtype == torch.float32:
-            rc = lib.dfhip_gemm_f32_nt(
-                a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, M, N, K, _stream()
+            rc = lib.dfhip_gemm_f32_nt_shared(
+                a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, M, N, K, _side_by_side(), _stream()
             )
-            _cabi.check("dfhip_gemm_f32_nt", rc)
+            _cabi.check("dfhip_gemm_f32_nt_shared", rc)
         else:
             raise RuntimeError(f"linear: unsupported dtype {x.dtype}")
     return out.view(*x.shape[:-1], N)

@@ -205,6 +205,11 @@ int dfhip_gemm_bf16_gate_up_silu_shared(const void* A, int64_t lda, const void* 
  * Requires K % 4 == 0, 16-byte aligned pointers, lda/ldw % 4 == 0. */
 int dfhip_gemm_f32_nt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
                       int64_t ldc, int M, int N, int K, dfhip_stream_t stream);
+/* The same for a launch that runs side by side with `share` - 1 others of its shape (1 <= share <= 16, as for
+ * dfhip_gemm_bf16_plan_shared): the kernel is the one whose launches take the least time together.  The kernels add
+ * in different orders. */
+int dfhip_gemm_f32_nt_shared(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
+                             int64_t ldc, int M, int N, int K, int share, dfhip_stream_t stream);
 
 /* fp8 e4m3fn inputs, fp32 accumulate, bf16 output (the `linear` node, dynaflow/runtime/engine.py:381,
  * of a host model whose weights are quantised per output channel and whose activations are

@@ -23,3 +23,24 @@ def test_gemm_f32_tiles(M, N, K):
     bound = K * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
     assert bool(((got.double() - a.double() @ w.double().t()).abs() <= bound).all())
     assert torch.equal(ops.linear(a, w), got)
+
+
+# (rows, columns, K, launches side by side, whether the 128 x 128 tiles take it): both sides of the line between them
+@pytest.mark.parametrize("M,N,K,share,tile128", [(8192, 2816, 512, 1, True), (3000, 2816, 512, 1, True),
+                                                 (3000, 5632, 1024, 1, True), (2816, 2816, 1024, 2, True),
+                                                 (1024, 5632, 1024, 2, True), (3000, 2816, 1024, 1, False),
+                                                 (512, 5632, 2048, 2, False), (256, 2816, 1024, 2, False)])
+def test_gemm_f32_of_many_rows(M, N, K, share, tile128):
+    """Against float64 as above.  The 128 x 128 kernel is known by its bits: it also takes a K that is no multiple of 32,
+    and four columns of zeros at the end of K change none of its sums."""
+    from dynaflow_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a = torch.randn(M, K, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda")
+    with ops.launch_options(share):
+        got = ops.linear(a, w)
+    bound = K * 2.0 ** -24 * (a[::97].double().abs() @ w.double().abs().t())
+    assert bool(((got[::97].double() - a[::97].double() @ w.double().t()).abs() <= bound).all())
+    padded = ops.linear(*(torch.nn.functional.pad(t, (0, 4)) for t in (a, w)))
+    assert torch.equal(got, padded) == tile128
