@@ -763,8 +763,17 @@ int launch_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, 
 }
 
 // Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip); with 16 rows and more from K = 4096
-// on, as for bf16 rows of the same bytes.
-bool stream_planned(int M, int N, int K) { return dfhip_stream_fits(M, N, K, 1) && (M < 16 || K >= 4096); }
+// on, as for bf16 rows of the same bytes.  From 33 rows on every workgroup re-reads the activations four times as wide as
+// up to 16, and two such launches side by side are bound by that; the ring tiles share what they read.  A pair of more
+// than 2^27 weights takes those, and one cut along K from 2^25 on.  [us a pair at 33 / 64 rows, streamed / ring: 28672 x
+// 8192 97 / 82 and 112 / 83, with gate + up + SiLU*mul 185 / 170 and 200 / 169; 8192 x 28672 118 / 91 and 155 / 91, 4096
+// x 14336 48 / 46 and 66 / 46; but 14336 x 4096 30 / 38 and 35 / 39, 1536 x 7168 24 / 28 and 28 / 29.  Alone 28672 x 8192
+// 53 / 71 and 64 / 72, 8192 x 28672 62 / 77 and 80 / 77]
+bool stream_planned(int M, int N, int K, int share, bool may_split) {
+  if (!dfhip_stream_fits(M, N, K, 1) || (M >= 16 && K < 4096)) return false;
+  const int64_t most = may_split && K > N ? 1 << 25 : 1 << 27;
+  return M <= 32 || share == 1 || (int64_t)N * K <= most;
+}
 
 constexpr int F8_MAX_SPLIT = 16;
 
@@ -874,9 +883,7 @@ extern "C" int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void*
                                          int K, int variant, dfhip_stream_t stream) {
   if (int rc = check_gemm(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (variant < 0 && stream_planned(M, N, K))
-    return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
-  if (variant < 0) variant = plan_tile(M, N, K, 1, false).variant;
+  if (variant < 0) return dfhip_gemm_fp8_nt_shared(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, stream);
   switch (variant) {
     case 0: return launch_fp8_ring<8, false>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, nullptr, s);
     case 1: return launch_fp8<128, 128>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
@@ -887,13 +894,24 @@ extern "C" int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void*
   }
 }
 
+extern "C" int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
+                                        const float* a_scale, const float* w_scale, int M, int N, int K, int share,
+                                        dfhip_stream_t stream) {
+  if (int rc = check_gemm(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K)) return rc;
+  if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
+  if (stream_planned(M, N, K, share, false))
+    return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, static_cast<hipStream_t>(stream));
+  return dfhip_gemm_fp8_nt_variant(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K,
+                                   plan_tile(M, N, K, share, false).variant, stream);
+}
+
 extern "C" int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k) {
   if (!variant || !split_k) return DFHIP_ERR_NULL_POINTER;
   if (M < 1 || N < 1 || K < 1) return DFHIP_ERR_BAD_SHAPE;
   if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
   *variant = -1;
   *split_k = 1;
-  if (stream_planned(M, N, K)) return DFHIP_OK;
+  if (stream_planned(M, N, K, share, true)) return DFHIP_OK;
   const TilePlan plan = plan_tile(M, N, K, share, true);
   *variant = plan.variant;
   *split_k = plan.split_k;
@@ -924,10 +942,11 @@ extern "C" int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* 
   }
 }
 
-extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, const void* W_gate, const void* W_up,
-                                                  int64_t ldw, void* act, int64_t ld_act, const float* a_scale,
-                                                  const float* w_gate_scale, const float* w_up_scale, float* amax,
-                                                  int M, int I, int K, dfhip_stream_t stream) {
+extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t lda, const void* W_gate,
+                                                         const void* W_up, int64_t ldw, void* act, int64_t ld_act,
+                                                         const float* a_scale, const float* w_gate_scale,
+                                                         const float* w_up_scale, float* amax, int M, int I, int K,
+                                                         int share, dfhip_stream_t stream) {
   if (!A || !W_gate || !W_up || !act || !a_scale || !w_gate_scale || !w_up_scale || !amax)
     return DFHIP_ERR_NULL_POINTER;
   if (M < 1 || I < 8 || K < 1 || K % FBK != 0 || I % 8 != 0) return DFHIP_ERR_BAD_SHAPE;
@@ -937,15 +956,19 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, co
       !dfhip_aligned16(W_up) || !dfhip_aligned16(act) || !dfhip_aligned16(w_gate_scale) ||
       !dfhip_aligned16(w_up_scale))
     return DFHIP_ERR_BAD_ALIGNMENT;
-  if (stream_planned(M, I, K))
+  if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
+  if (stream_planned(M, I, K, share, false))
     return dfhip_stream_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I,
                                     K, static_cast<hipStream_t>(stream));
-  // the height of the tile that costs least in rounds (see tile_cost); every height adds in the same order
+  // the height of the tile that costs least in rounds (see tile_cost); every height adds in the same order.  A pair of
+  // 2 x 14336 x 4096 at 192 / 256 rows: one round of 192 and 256-row tiles 53 / 59 us, two of 128-row ones 66 / 68.  (Of a
+  // pair the last round runs beside the other launch, and can cost less than it is priced at: 2 x 12288 x 6144 at 700
+  // rows takes 192-row tiles and 181 us where 256-row ones take 167.)
   const RingTile* ring = &F8_RINGS[0];
   double least = 0.0;
   for (const RingTile& r : F8_RINGS) {
     const int64_t tiles = (int64_t)((M + 32 * r.tm - 1) / (32 * r.tm)) * ((I + 127) / 128);
-    const double cost = tile_cost(tiles, 1, 1, K, r.per_slab, r.tm);
+    const double cost = tile_cost(tiles, 1, share, K, r.per_slab, r.tm);
     if (&r == &F8_RINGS[0] || cost < least) { ring = &r; least = cost; }
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -957,6 +980,14 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, co
     default: return launch_fp8_ring_fused<4>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale,
                                              amax, M, I, K, s);
   }
+}
+
+extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, const void* W_gate, const void* W_up,
+                                                  int64_t ldw, void* act, int64_t ld_act, const float* a_scale,
+                                                  const float* w_gate_scale, const float* w_up_scale, float* amax,
+                                                  int M, int I, int K, dfhip_stream_t stream) {
+  return dfhip_gemm_fp8_gate_up_silu_absmax_shared(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale,
+                                                   w_up_scale, amax, M, I, K, 1, stream);
 }
 
 extern "C" int dfhip_gemm_fp8_nt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,

@@ -762,7 +762,8 @@ def _silu_mul_quant_fp8_impl(gate: torch.Tensor, up: torch.Tensor):
 
 def _gate_up_silu_quant_fp8_impl(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w_up_scale):
     """The fp8 gate and up projections with SiLU*mul as the GEMM's epilogue, then the re-quantisation:
-    returns what ``silu_mul_quant_fp8(linear_fp8(x, w_gate), linear_fp8(x, w_up))`` returns, bit for bit."""
+    returns what ``silu_mul_quant_fp8(linear_fp8(x, w_gate), linear_fp8(x, w_up))`` returns beside as many launches, bit
+    for bit."""
     _require_device(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w_up_scale)
     lib = _cabi.load()
     if x_q.dtype != FP8_DTYPE or w_gate_q.dtype != FP8_DTYPE or w_up_q.dtype != FP8_DTYPE:
@@ -783,12 +784,12 @@ def _gate_up_silu_quant_fp8_impl(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w
     q = torch.empty((M, I), dtype=FP8_DTYPE, device=x_q.device)
     if M > 0:
         _fill_zero(amax)
-        rc = lib.dfhip_gemm_fp8_gate_up_silu_absmax(
+        rc = lib.dfhip_gemm_fp8_gate_up_silu_absmax_shared(
             a.data_ptr(), lda, wg.data_ptr(), wu.data_ptr(), ldg, act.data_ptr(), I, x_scale.data_ptr(),
             w_gate_scale.contiguous().data_ptr(), w_up_scale.contiguous().data_ptr(), amax.data_ptr(), M, I, K,
-            _stream(),
+            _side_by_side(), _stream(),
         )
-        _cabi.check("dfhip_gemm_fp8_gate_up_silu_absmax", rc)
+        _cabi.check("dfhip_gemm_fp8_gate_up_silu_absmax_shared", rc)
         rc = lib.dfhip_quant_fp8_bf16(act.data_ptr(), I, q.data_ptr(), I, M, I, amax.data_ptr(), scale.data_ptr(),
                                       _stream())
         _cabi.check("dfhip_quant_fp8_bf16", rc)
@@ -811,26 +812,21 @@ def _linear_fp8_impl(x_q, w_q, x_scale, w_scale, variant: int = -1, to_output: b
     out = _new_output(M, N, torch.bfloat16, x_q.device, to_output)
     if M > 0:
         stream, split_k = _stream(), 1
-        if variant < 0 and (cut_k or K <= N):         # (K <= N is not cut; the plan knows the launches side by side)
+        if cut_k and SPLIT_K_ENABLED:
             planned, parts = ctypes.c_int(-1), ctypes.c_int(1)
             _cabi.check("dfhip_gemm_fp8_plan_shared", lib.dfhip_gemm_fp8_plan_shared(
                 M, N, K, _side_by_side(), ctypes.byref(planned), ctypes.byref(parts)))
-            if SPLIT_K_ENABLED or parts.value == 1:
-                variant, split_k = planned.value, parts.value
+            variant, split_k = planned.value, parts.value
         scale = w_scale.contiguous()
+        gemm = (a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, x_scale.data_ptr(), scale.data_ptr(), M, N, K)
         if split_k > 1:
             ws = _splitk_workspace(x_q.device, stream, lib.dfhip_gemm_fp8_splitk_workspace_bytes(M, N, variant, split_k))
-            rc = lib.dfhip_gemm_fp8_nt_splitk(
-                a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, x_scale.data_ptr(), scale.data_ptr(), M, N, K,
-                variant, split_k, ws.data_ptr(), ws.numel(), stream,
-            )
+            rc = lib.dfhip_gemm_fp8_nt_splitk(*gemm, variant, split_k, ws.data_ptr(), ws.numel(), stream)
             _cabi.check("dfhip_gemm_fp8_nt_splitk", rc)
+        elif variant >= 0:
+            _cabi.check("dfhip_gemm_fp8_nt_variant", lib.dfhip_gemm_fp8_nt_variant(*gemm, variant, stream))
         else:
-            rc = lib.dfhip_gemm_fp8_nt_variant(
-                a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, x_scale.data_ptr(), scale.data_ptr(), M, N, K,
-                variant, stream,
-            )
-            _cabi.check("dfhip_gemm_fp8_nt_variant", rc)
+            _cabi.check("dfhip_gemm_fp8_nt_shared", lib.dfhip_gemm_fp8_nt_shared(*gemm, _side_by_side(), stream))
     return out.view(*x_q.shape[:-1], N)
 
 

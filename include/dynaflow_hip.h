@@ -228,12 +228,18 @@ int dfhip_gemm_fp8_nt(const void* A, int64_t lda, const void* W, int64_t ldw, vo
 int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
                               const float* a_scale, const float* w_scale, int M, int N, int K, int variant,
                               dfhip_stream_t stream);
+/* The choice of dfhip_gemm_fp8_nt for a launch that runs side by side with `share` - 1 others of its shape (1 <= share <=
+ * 16, as for dfhip_gemm_bf16_plan_shared).  From 33 to 64 rows the kernel, and with it the order of the sums, can depend
+ * on `share`; dfhip_gemm_fp8_gate_up_silu_absmax_shared makes the same choice. */
+int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
+                             const float* a_scale, const float* w_scale, int M, int N, int K, int share,
+                             dfhip_stream_t stream);
 /* The same with K cut into split_k parts (2 .. 16, at least two slabs of 128 each), for outputs of too few tiles to
  * fill the GPU; variant 0, 3 or 4.  workspace: dfhip_gemm_fp8_splitk_workspace_bytes bytes, 16-byte aligned, whose
  * arrival counters (4 bytes a tile at its start) are zero; they are left zero.  Launches that may overlap need one
  * each.  The parts are added in part order: the same bits in every run.
- * dfhip_gemm_fp8_plan_shared: the variant and split for `share` launches of this shape side by side (variant < 0: the
- * launch without a split decides).  For the projection back to the model width: K is only cut where K > N, and the
+ * dfhip_gemm_fp8_plan_shared: the variant and split for `share` launches of this shape side by side (variant < 0:
+ * dfhip_gemm_fp8_nt_shared).  For the projection back to the model width: K is only cut where K > N, and the
  * projections in front of it, which keep the order of sums of dfhip_gemm_fp8_gate_up_silu_absmax, are launched without a
  * split whatever their widths are. */
 int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
@@ -253,6 +259,11 @@ int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, const void* W
                                        int64_t ldw, void* act, int64_t ld_act, const float* a_scale,
                                        const float* w_gate_scale, const float* w_up_scale, float* amax, int M,
                                        int I, int K, dfhip_stream_t stream);
+/* The same for a launch beside `share` - 1 others of its shape: the bits of two dfhip_gemm_fp8_nt_shared launches. */
+int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t lda, const void* W_gate, const void* W_up,
+                                              int64_t ldw, void* act, int64_t ld_act, const float* a_scale,
+                                              const float* w_gate_scale, const float* w_up_scale, float* amax, int M,
+                                              int I, int K, int share, dfhip_stream_t stream);
 
 /* ------------------------------------------------------------ elementwise
  *

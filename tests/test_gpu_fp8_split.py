@@ -123,6 +123,41 @@ def test_fused_fp8_launch_with_an_intermediate_width_below_the_model_width(M, I,
     assert torch.equal(*outs)
 
 
+def test_fp8_launches_side_by_side_are_planned_as_such():
+    """From 33 rows on a pair of large launches takes the ring tiles, a lone one the streaming kernel; a pair of narrower
+    ones and up to 32 rows stay with it, and a projection that is not cut along K never is."""
+    lib, v, s = _cabi.load(), ctypes.c_int(), ctypes.c_int()
+    for M, N, K, share, streamed in ((48, 28672, 8192, 1, True), (48, 28672, 8192, 2, False), (64, 8192, 28672, 2, False),
+                                     (33, 4096, 14336, 2, False), (32, 28672, 8192, 2, True), (64, 14336, 4096, 2, True),
+                                     (64, 1536, 7168, 2, True), (65, 14336, 4096, 1, False)):
+        assert lib.dfhip_gemm_fp8_plan_shared(M, N, K, share, ctypes.byref(v), ctypes.byref(s)) == 0
+        assert (v.value < 0) == streamed, (M, N, K, share)
+    args = (16, 1024, 16, 1024, 16, 8, 16, 16, 1, 8, 1024)
+    assert lib.dfhip_gemm_fp8_nt_shared(*args, 0, None) == -7 and lib.dfhip_gemm_fp8_nt_shared(*args, 17, None) == -7
+
+
+# streamed, at its edge and beyond; one round of tall tiles instead of two of short ones; an intermediate width below the
+# model width on both sides of 2^27 weights
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,I,K", [(32, 17408, 8192), (33, 17408, 8192), (64, 17408, 8192), (192, 14336, 4096),
+                                   (256, 14336, 4096), (40, 8192, 17408), (40, 4096, 8192)])
+@pytest.mark.parametrize("share", [1, 2, 16])
+def test_fused_fp8_launch_beside_others(M, I, K, share):
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
+
+    spread = lambda shape, seed: randn(shape, seed) * torch.exp2(randn(shape, seed + 50, 4.0))
+    xq, xs = ops.quant_fp8(spread((M, K), 1))
+    (wq, ws), (uq, us) = (quantize_weight_per_channel(spread((I, K), seed)) for seed in (2, 3))
+    with ops.launch_options(share):
+        q, scale = ops.gate_up_silu_quant_fp8(xq, wq, uq, xs, ws, us)
+        gate, up = ops.linear_fp8(xq, wq, xs, ws), ops.linear_fp8(xq, uq, xs, us)
+    want_q, want_scale = ops.silu_mul_quant_fp8(gate, up)
+    assert torch.equal(scale, want_scale) and torch.equal(q.view(torch.uint8), want_q.view(torch.uint8))
+    want = (xq.float() * xs) @ (wq.float() * ws[:, None]).t()
+    assert (gate.float() - want).abs().max().item() <= 2.0 ** -6 * want.abs().max().item()
+
+
 @pytest.mark.gpu
 def test_fp8_block_cuts_the_projection_back_to_the_model_width():
     """The block's down projection is the launch in parts (which takes the workspace), the caller's plain one is not."""
