@@ -160,13 +160,5 @@ DFHIP_DEVICE f32x4 load_f32x4_device_coherent(__amdgpu_buffer_rsrc_t blocks, int
   constexpr int SC1 = 16;
   return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(blocks, at, uniform, SC1));
 }
-
-// one float, coherent across the XCDs
-DFHIP_DEVICE void store_device_coherent(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-DFHIP_DEVICE float load_device_coherent(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 DFHIP_DEVICE void workgroup_barrier() { asm volatile("s_barrier" ::: "memory"); }
 #define DFHIP_PIN __builtin_amdgcn_sched_barrier(0)

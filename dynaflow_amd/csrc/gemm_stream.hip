@@ -310,7 +310,7 @@ template <bool FP8, bool FUSED, bool SPLIT>
 int launch_rows(const StreamArgs& p, int width, hipStream_t stream) {
   if (p.M <= 16) return launch_width<FP8, 1, FUSED, SPLIT>(p, width, stream);
   if (p.M <= 32) return launch_width<FP8, 2, FUSED, SPLIT>(p, width, stream);
-  if constexpr (FUSED && !FP8) return DFHIP_ERR_BAD_SHAPE;   // the bf16 entry points stop at 32 rows
+  if constexpr (!FP8 && (FUSED || SPLIT)) return DFHIP_ERR_BAD_SHAPE;   // bf16: whole K alone, by variant
   else return launch_width<FP8, 4, FUSED, SPLIT>(p, width, stream);
 }
 
