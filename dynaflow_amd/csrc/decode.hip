@@ -48,9 +48,9 @@ __host__ __device__ constexpr int part_block(int group) { return group * (HD / 4
 
 // Parts of a sequence of `len` positions where the launch has `parts` workgroups for each: at least 256 positions (two
 // chunks per wave) a part, and at least three parts, since the meeting costs about 3 us.  Shorter sequences stay whole:
-// the bits of an uncut launch, and its time but for the start of the workgroups that end at once.  [us, uncut / cut by the
-// capacity alone / by the length: 2 sequences in a cache of 8192 positions, of 33 6.4 / 13.4 / 6.6, of 512 9.8 / 14.3 /
-// 9.9, of 2048 27 - 31 / 16.8 / 11.6, of 8192 111 / 21.9 / 21.0]
+// the bits and the time of an uncut launch.  [us, uncut / cut by the
+// capacity alone / by the length: 2 sequences in a cache of 8192 positions, of 33 6.4 / 13.4 / 6.5, of 512 9.8 / 14.3 /
+// 9.9, of 2048 27 - 31 / 16.8 / 11.6, of 8192 111 / 21.9 / 20.8]
 DFHIP_DEVICE int sequence_parts(int len, int parts) {
   if (len < 3 * 256) return 1;
   return len / 256 < parts ? len / 256 : parts;
@@ -88,10 +88,9 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
   float* const m_lds = combine_lds + 4 * group * HD;      // [4][group]
   float* const l_lds = m_lds + 4 * group;                 // [4][group]
   // Part-major: the parts that every sequence uses are dispatched first and lie on all XCDs.  (Pair-major, the only
-  // workgroups with work of 8 short sequences are every eighth one, on one XCD: 512 positions 20.2 us, so 12.5.)
-  const int pairs = SPLIT ? gridDim.x / parts : gridDim.x;
-  const int part = SPLIT ? blockIdx.x / pairs : 0;
-  const int pair = blockIdx.x - part * pairs;
+  // workgroups with work of 8 short sequences are every eighth one, on one XCD: 512 positions 20.2 us, so 12.2.)
+  const int part = SPLIT ? blockIdx.y : 0;
+  const int pair = blockIdx.x;
   const int t = pair / kv_heads, kvh = pair - t * kv_heads;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hq = lane & 15, g = lane >> 4;
@@ -468,7 +467,7 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
 // Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), with at least 256 positions of
 // a full cache each (two chunks per wave).  The lengths are on the device: the launch is sized for full caches and each
 // sequence takes its share of it (sequence_parts).  A launch with fewer than MIN_PARTS of them, from 171 pairs on, cuts
-// nothing.  [us, uncut / cut: 2 sequences of 8192 positions 111 / 21.0 (their bytes at 6.7 TB/s: 10), 8 of 2048 33 / 16.8
+// nothing.  [us, uncut / cut: 2 sequences of 8192 positions 111 / 20.8 (their bytes at 6.7 TB/s: 10), 8 of 2048 33 / 16.8
 // (10), 20 of 4096 69 / 58 (50); in two parts, not taken: 32 of 512, 2048 and 4096 14.6 / 16.5, 42.9 / 46.0, 79 / 84]
 constexpr int MIN_PARTS = 3;
 static int attention_parts(int T, int kv_heads, int capacity) {
@@ -501,7 +500,7 @@ static int decode_attention_append(const void* qkv, int64_t ld_qkv, void* k_cach
   if (parts < MIN_PARTS) parts = 1;
   const auto kernel = parts > 1 ? decode_attention_kernel<true, true> : decode_attention_kernel<true, false>;
   float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + ATTENTION_COUNTER_BYTES);
-  hipLaunchKernelGGL(kernel, dim3(T * kv_heads * parts), dim3(DEC_THREADS), lds_bytes,
+  hipLaunchKernelGGL(kernel, dim3(T * kv_heads, parts), dim3(DEC_THREADS), lds_bytes,
                      static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(qkv), ld_qkv,
                      static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), slots, lengths,
                      static_cast<uint16_t*>(out), ld_out, kv_heads, group, num_slots, capacity,
