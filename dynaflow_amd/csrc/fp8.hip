@@ -787,8 +787,8 @@ struct TilePlan { int variant, split_k; double cost; };
 // reader takes split_k blocks one after the other.  A shorter tile is hardly faster per slab (the loads bound it), so
 // it pays where it saves a round or leaves tiles to split; the 224-column kernel enters with a rate of its own.  The
 // register-staged 128 x 128 kernel is never faster than the 128-row ring (17 .. 300 rows, 256 .. 8192 columns and K: 6
-// against 6 us at the smallest, 51 against 40 at K = 8192).  Against about 200 measured launches (65 .. 2048 rows, 8192 x 28672, 4096 x 14336,
-// 28672 x 8192 and 14336 x 4096) the choice is the fastest or within 8 % of it.
+// against 6 us at the smallest, 51 against 40 at K = 8192).  The prices are good to about 15 %: 8192 x 28672 takes seven
+// parts up to 128 rows, 77 us, where eight take 64.
 double tile_cost(int64_t tiles, int split_k, int share, int K, double per_slab, int tm) {
   const double rounds = (double)((tiles * split_k * share + 255) / 256);
   return rounds * ((double)(K / FBK) / split_k * per_slab + 6.0) + (split_k > 1 ? 0.9 * tm * split_k + 4.0 : 0.0);

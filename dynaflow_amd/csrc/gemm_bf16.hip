@@ -1664,12 +1664,15 @@ bool rows192_cheaper(int M, int N, int wide, int narrow, int share) {
 }
 
 // Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip), whatever runs beside it.
-// With 16 rows and more a K below 2048 keeps the 128-row tiles.  Weights of more than 2^27 elements keep them too: there
-// a row has the same bits in a launch of few rows and of many, which is worth more than the gain (2 x 28672 x 8192 with
-// SiLU*mul, us: 154 against 186 at 1 .. 16 rows, but 193 against 182 at 64, where the re-read activations weigh more).
+// With 16 rows and more a K below 2048 keeps the 128-row tiles.
+// Weights of more than 2^27 elements keep them at every count of rows.  That is a promise and not a matter of speed: the
+// rows of a gate + up + SiLU*mul launch of 2 x 28672 x 8192 have the same bits when they are launched in pieces, down to
+// one row (a test holds them to it), while smaller weights have other bits up to 32 rows than above.  It costs 176 us
+// against 142 at 1 .. 12 rows, and as much in the plain launches of such weights, which share the rule so that fused and
+// separate launches agree.
 // From 33 rows on two such launches side by side cost what they cost one after the other - the re-read activation rows
-// bound them - where the 128-row tiles of a pair share what they read (8B layer, 2 x 48 rows: 167 against 136 us; 2 x 20
-// rows in a decode step: 161 against 190 us a layer).
+// bound them - where the 128-row tiles of a pair overlap (8B layer, 2 x 48 rows: 167 against 136 us; 2 x 20 rows in a
+// decode step: 161 against 190 us a layer).  At 32 rows a pair is about level, 5 % slower at worst.
 bool stream_planned(int M, int N, int K) {
   return M <= 32 && dfhip_stream_fits(M, N, (int64_t)K * 2, 1) && (M < 16 || K >= 2048) &&
          (int64_t)N * K <= (int64_t)1 << 27;

@@ -13,12 +13,14 @@
 //     4 KiB apart and so on one L2 channel, hence the workgroups start at different slabs;
 //   * at the end the four partial sums meet in LDS and are added in wave order.  Where K is cut into parts (a
 //     caller's workspace), the part that arrives last adds them in part order: the same bits in every run.
-// The order of K depends on K and on the cut alone, so the fused launch has the bits of the separate, uncut ones.
+// The order in which a column's K is summed depends on K, on the cut and on the column's tile, whose number says at which
+// slab its waves start: a row of W can sum in another order in a matrix of another N, or at another place in it.  The
+// fused launch has the bits of the separate, uncut ones because N, and with it the tiles, are the same.
 // Measured (weights from HBM, us; M = 2 / 16 / 32 rows, against the 128-row tiles used before): gate + up + SiLU*mul
-// 2 x 14336 x 4096 (235 MB) 40 / 38 / 41, before 55; down 4096 x 14336 22 / 22 / 26, before 207 / 38 / 39; q/k/v
-// 6144 x 4096 11 / 13 / 16, before 61 / 23 / 23; o 4096 x 4096 8 / 10 / 12, before 61 / 21 / 21.  At 2 / 16 / 32 / 64
-// rows fp8 down 8192 x 28672 (235 MB) 37 / 42 / 54 / 78, before 240; fp8 gate + up 2 x 28672 x 8192 (470 MB)
-// 84 / 87 / 95 / 113, before 117 - 121.
+// 2 x 14336 x 4096 (235 MB) 39 / 39 / 43, before 51; down 4096 x 14336 23 / 24 / 27, before 207 / 36 / 36; q/k/v
+// 6144 x 4096 12 / 15 / 18, before 62 / 22 / 22; o 4096 x 4096 8 / 10 / 13, before 61 / 21 / 21.  At 8 / 16 / 32 / 64
+// rows fp8 down 8192 x 28672 (235 MB) 37 / 42 / 54 / 79, before 240; fp8 gate + up 2 x 28672 x 8192 (470 MB)
+// 80 / 82 / 92 / 112, before 113 - 117.
 #include "dfhip_stream.h"
 
 namespace {
