@@ -7,6 +7,7 @@ loop is closed with the thread.
 from __future__ import annotations
 
 import asyncio
+import ctypes
 import os
 import threading
 from collections.abc import Coroutine
@@ -24,6 +25,12 @@ class _TaskFactory:
         return asyncio.Task(coroutine, loop=loop, **kwargs)
 
 
+#: A loop of a parent process that a fork has brought here shares the parent's epoll object: closing it (its own ``__del__``
+#: does that too, at the end of the process at the latest) would take the parent's wake-up descriptor out of it.  One
+#: reference that nobody gives back leaves it as it is.
+_keep_forever = ctypes.PYFUNCTYPE(None, ctypes.py_object)(("Py_IncRef", ctypes.pythonapi))
+
+
 class _KeptLoop:
     """A loop and whoever closes it: the thread's locals hold this object and the loop does not, so it goes, and the loop
     is closed, when they are dropped at the end of the thread.  (A loop by itself is part of reference cycles and would
@@ -35,19 +42,15 @@ class _KeptLoop:
         self.loop.set_task_factory(self.tasks)
         self.process = os.getpid()
 
-    def __del__(self) -> None:
+    def __del__(self, _process: Any = os.getpid, _keep_forever: Any = _keep_forever) -> None:   # (also at the very end)
         loop = getattr(self, "loop", None)
         if loop is None or loop.is_closed() or loop.is_running():
             return
-        if self.process != os.getpid():
-            _inherited.append(loop)
+        if self.process != _process():
+            _keep_forever(loop)
         else:
             loop.close()
 
-
-#: Loops of a parent process that a fork has brought here.  They share the parent's epoll object: closing one (its own
-#: ``__del__`` does that too) would take the parent's wake-up descriptor out of it, so they stay as they are.
-_inherited: list[asyncio.AbstractEventLoop] = []
 
 _thread = threading.local()
 

@@ -10,6 +10,8 @@ import threading
 import time
 import warnings
 
+import pytest
+
 from dynaflow_amd.runtime.loop import run_coroutine
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -74,6 +76,28 @@ def test_a_forked_child_leaves_its_parents_loop_alone():
     child.join(60)
     assert child.exitcode == 0
     assert run_coroutine(other_thread()) < 5
+
+
+@pytest.mark.parametrize("forward", [False, True])
+def test_a_forked_child_that_ends_like_any_process_leaves_its_parents_loop_alone(forward):
+    """Through the interpreter's end, where modules are already taken apart, with and without a forward of its own."""
+    code = (f"import asyncio, os, sys, time\n"
+            f"from dynaflow_amd.runtime import loop\n"
+            f"run_coroutine = loop.run_coroutine\n"
+            f"async def nothing(): return 7\n"
+            f"async def other_thread():\n"
+            f"    started = time.monotonic()\n"
+            f"    await asyncio.wait_for(asyncio.get_running_loop().run_in_executor(None, time.sleep, 0.02), 10)\n"
+            f"    return time.monotonic() - started\n"
+            f"assert run_coroutine(nothing()) == 7\n"
+            f"child = os.fork()\n"
+            f"if child == 0:\n"
+            f"    if {forward}: assert run_coroutine(nothing()) == 7\n"
+            f"    sys.exit(0)\n"
+            f"assert os.waitpid(child, 0)[1] == 0\n"
+            f"assert run_coroutine(other_thread()) < 5\n")
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0 and not done.stderr, done.stderr
 
 
 def test_a_left_over_task_that_fails_while_it_is_cancelled_is_reported(caplog):
