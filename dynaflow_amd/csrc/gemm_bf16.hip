@@ -1653,7 +1653,9 @@ double round_fill(int M, int N, int tile_n, int share = 1) {
 // clock is higher while units idle).  Measured at M = 300 .. 6000 on four weights, the tile is 6 - 18 % faster wherever
 // this says so: 670 x 14336 x 4096 71 -> 64 us, 2331 x 4096 x 14336 236 -> 210, 2880 x 6144 x 4096 142 -> 124, gate + up +
 // SiLU*mul 2 x 14336 x 4096 at 560 / 1100 / 1554 rows 144 / 228 / 308 -> 124 / 199 / 291; where it says no, the tile is up
-// to 60 % slower (777 x 14336 x 4096: 1.09 rounds, 81 -> 122) or at best 4 % faster.
+// to 60 % slower (777 x 14336 x 4096: 1.09 rounds, 81 -> 122) or at best 4 % faster.  Two launches side by side (`share`), 300
+// .. 2880 rows: from level (670 x 14336 x 4096 141 / 144, 1554 x 14336 x 4096 306 / 304) to 30 % faster (300 x 28672 x 8192
+// 363 -> 280).
 bool rows192_cheaper(int M, int N, int wide, int narrow, int share) {
   auto cost = [&](int tile_m, int tile_n, double per_round) {
     const int64_t tiles = (int64_t)((M + tile_m - 1) / tile_m) * ((N + tile_n - 1) / tile_n) * share;
