@@ -41,6 +41,7 @@ class _KeptLoop:
         self.tasks = _TaskFactory()
         self.loop.set_task_factory(self.tasks)
         self.process = os.getpid()
+        self.forks = _forks
 
     def __del__(self, _process: Any = os.getpid, _keep_forever: Any = _keep_forever) -> None:   # (also at the very end)
         loop = getattr(self, "loop", None)
@@ -54,10 +55,22 @@ class _KeptLoop:
 
 _thread = threading.local()
 
+#: Forks of this process so far.  A loop from before one shares its epoll object with the child, whatever that does with
+#: its copy: the next forward takes a new loop.
+_forks = 0
+
+
+def _count_fork() -> None:
+    global _forks
+    _forks += 1
+
+
+os.register_at_fork(after_in_parent=_count_fork)
+
 
 def _kept_loop() -> _KeptLoop:
     kept = getattr(_thread, "kept", None)
-    if kept is None or kept.process != os.getpid() or kept.loop.is_closed():
+    if kept is None or kept.process != os.getpid() or kept.forks != _forks or kept.loop.is_closed():
         kept = _thread.kept = _KeptLoop()
     return kept
 

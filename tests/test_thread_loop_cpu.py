@@ -60,7 +60,14 @@ def _in_a_forked_child():
     gc.collect()
 
 
-def test_a_forked_child_leaves_its_parents_loop_alone():
+def _closes_what_it_inherits():
+    from dynaflow_amd.runtime import loop
+
+    loop._thread.kept.loop.close()
+
+
+@pytest.mark.parametrize("child", [_in_a_forked_child, _closes_what_it_inherits])
+def test_a_forked_child_leaves_its_parents_loop_alone(child):
     """A child shares the parent's epoll object.  One that closes the inherited loop takes the parent's wake-up descriptor
     out of it, and the parent's coroutines then sleep through what other threads finish for them."""
     async def other_thread():
@@ -71,7 +78,7 @@ def test_a_forked_child_leaves_its_parents_loop_alone():
     assert run_coroutine(nothing()) == 7
     with warnings.catch_warnings():
         warnings.simplefilter("ignore", DeprecationWarning)      # a fork beside torch's threads
-        child = multiprocessing.get_context("fork").Process(target=_in_a_forked_child)
+        child = multiprocessing.get_context("fork").Process(target=child)
         child.start()
     child.join(60)
     assert child.exitcode == 0
