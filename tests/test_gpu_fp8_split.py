@@ -59,6 +59,20 @@ def test_fp8_tile_heights_add_in_one_order(M, N, K, variant):
     assert torch.equal(got, ops.linear_fp8_variant(xq, wq, xs, ws, 1))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(65, 264, 384), (193, 520, 640), (385, 1544, 1024), (300, 4032, 4096)])
+def test_fp8_ring_tiles_have_one_order_of_sums(M, N, K):
+    """Operands over many binades: fp32 sums of narrow e4m3 data are nearly exact in any order and would not tell."""
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
+
+    xq, xs = ops.quant_fp8(randn((M, K), 1) * torch.exp2(randn((M, K), 2, 4.0)))
+    wq, ws = quantize_weight_per_channel(randn((N, K), 3) * torch.exp2(randn((N, K), 4, 4.0)))
+    tall = ops.linear_fp8_variant(xq, wq, xs, ws, 0)
+    for variant in (2, 3, 4):
+        assert torch.equal(ops.linear_fp8_variant(xq, wq, xs, ws, variant), tall), variant
+
+
 # parts of two slabs (the shortest), of uneven lengths (9 slabs in 2 and 4 parts, 37 in 16), ragged tiles
 @pytest.mark.gpu
 @pytest.mark.parametrize("variant", [0, 3, 4])
