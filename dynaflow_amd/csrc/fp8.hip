@@ -16,6 +16,7 @@
 //                       with K cut into parts for few tiles: [350 x 28672] x [8192 x 28672]^T ran on 64 workgroups
 //                       (230 us, 0.71 PFLOP/s), with 192 rows and four parts it takes 96.
 // gemm_fp8_nt_kernel    register-staged double buffer, 128 x 128: an independent second kernel, by variant only.
+#include "dfhip_ring3.h"
 #include "dfhip_stream.h"
 
 namespace {
@@ -812,6 +813,55 @@ TilePlan plan_tile(int M, int N, int K, int share, bool may_split) {
   return best;
 }
 
+// Prices of the ring kernels as those of the three-slab tiles (dfhip_ring3.h), by variant.
+constexpr DfhipPrice F8_RING_PRICE[3] = {{0.774, 0.642, 7.45, 17.5, 2.35, 5.6}, {0.100, 1.010, 8.73, 5.24, 2.14, 5.6},
+                                         {0.566, 0.620, 2.00, 1.00, 1.96, 6.01}};   // of F8_RINGS
+constexpr DfhipPrice F8_RING224_PRICE = {0.861, 0.401, 8.58, 0.0, 0.0, 6.0};
+
+// Whether a three-slab tile takes the place of the planned kernel, and which: where it is 4 % cheaper, 7 % above 256 rows and
+// for gate + up, whose pairs above 128 rows need 15 % (192 rows of 2 x 28672 x 8192 in pairs, priced 8 % lower, took 228 us
+// on 224 x 192 tiles where the 192-row ones take 195).  Over 190 timed shapes
+// (those of dfhip_price) this takes 9.4 % off the mean, 9.8 % being what the best choice for each would; the worst loss is
+// 6 % (350 x 4096 x 16384 alone: 42 -> 45 us), the best gains 63 % (96 x 4096 x 14336 alone: 41 -> 25) and 44 % (96 x 8192 x 28672
+// alone: 78 -> 55).
+DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share, int variant, int split_k, bool may_split) {
+  const int tm = ring_blocks(variant);
+  const int rows = tm ? 32 * tm : 256, cols = !tm ? F8_TBN : gate_up ? 128 : 256;
+  const DfhipPrice& price = tm == 8 ? F8_RING_PRICE[0] : tm == 6 ? F8_RING_PRICE[1] : tm == 4 ? F8_RING_PRICE[2]
+                                                                                            : F8_RING224_PRICE;
+  const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+  const double now = dfhip_price(price, tiles, share, K / FBK, split_k, (double)N * K * (gate_up ? 2e-6 : 1e-6));
+  const DfhipRing3Plan best = dfhip_ring3_plan(true, gate_up, M, N, K, share, may_split);
+  const double clearly = gate_up && share > 1 && M > 128 ? 0.85 : M > 256 || gate_up ? 0.93 : 0.96;
+  const double cube = clearly * clearly * clearly;
+  return best.cost < cube * cube * now ? best : DfhipRing3Plan{-1, 1, 0.0};
+}
+
+// Up to 64 rows, what the streaming kernel of the 128-row tiles' plan (stream_planned) leaves to the 128 x 128 tile: launches
+// of 33 rows and more, unless they are alone and their weights few.  [us at 33 / 64 rows, streamed or on 128-row tiles against
+// 128 x 128: alone 28672 x 8192 53 / 63 against 55 / 56, with gate + up + SiLU*mul 103 / 110 against 91 / 94, 14336 x 4096
+// 17 / 19 against 23 / 22, with gate + up 35 / 37 against 33 / 33; in pairs 28672 x 8192 81 / 84 against 76 / 78, 14336 x 4096
+// 30 / 35 against 25 / 26.]  A product that may be cut along K goes there alone from 33 rows on, in pairs from 17, or 9 where its
+// weights are many.  [8192 x 28672 at 17 / 24 / 33 / 64 rows: in pairs 91 / 97 / 92 / 92 against 77 / 78 / 79 / 82, alone
+// 44 / 48 / 59 / 79 against 50 / 49 / 50 / 52; 4096 x 14336 in pairs 34 / 38 / 45 / 45 against 31 / 32 / 31 / 32, alone
+// 19 / 21 / 25 / 34 against 24; at 12 rows in pairs 8192 x 28672 82 against 79, 4096 x 14336 30 against 32.  Fewer than 2^25 weights
+// stay: 1536 x 7168 alone at 40 rows 15 against 18, in pairs at 12 rows 17 against 23.]
+bool few_rows_streamed(int M, int N, int K, int share, bool may_split) {
+  if (!dfhip_stream_fits(M, N, K, 1) || (M >= 16 && K < 4096)) return false;
+  const int64_t weights = (int64_t)N * K;
+  if (!may_split || K <= N) return M <= 32 || (share == 1 && weights < (int64_t)1 << 27);
+  if (weights < (int64_t)1 << 25) return M <= 32 || share == 1;
+  return M <= (share == 1 ? 32 : weights < (int64_t)1 << 27 ? 16 : 8);
+}
+
+// The plan of a launch: -1 for the streaming kernel, else a tile and the parts of K.
+TilePlan plan_launch(int M, int N, int K, int share, bool may_split) {
+  if (few_rows_streamed(M, N, K, share, may_split)) return {-1, 1, 0.0};
+  const TilePlan plan = plan_tile(M, N, K, share, may_split);
+  const DfhipRing3Plan tiles = three_slabs_cheaper(false, M, N, K, share, plan.variant, plan.split_k, may_split && K > N);
+  return tiles.tile < 0 ? plan : TilePlan{DFHIP_RING3_VARIANT + tiles.tile, tiles.split_k, tiles.cost};
+}
+
 int check_gemm(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
                const float* w_scale, int M, int N, int K) {
   if (!A || !W || !C || !a_scale || !w_scale) return DFHIP_ERR_NULL_POINTER;
@@ -890,7 +940,9 @@ extern "C" int dfhip_gemm_fp8_nt_variant(const void* A, int64_t lda, const void*
     case 2: return launch_fp8_ring224(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, s);
     case 3: return launch_fp8_ring<6, false>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, nullptr, s);
     case 4: return launch_fp8_ring<4, false>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, nullptr, s);
-    default: return DFHIP_ERR_BAD_ARGUMENT;
+    default:
+      if (!dfhip_ring3_variant(variant, true)) return DFHIP_ERR_BAD_ARGUMENT;
+      return dfhip_ring3_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, variant - DFHIP_RING3_VARIANT, 1, nullptr, s);
   }
 }
 
@@ -899,10 +951,10 @@ extern "C" int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* 
                                         dfhip_stream_t stream) {
   if (int rc = check_gemm(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K)) return rc;
   if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
-  if (stream_planned(M, N, K, share, false))
+  const TilePlan plan = plan_launch(M, N, K, share, false);
+  if (plan.variant < 0)
     return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, static_cast<hipStream_t>(stream));
-  return dfhip_gemm_fp8_nt_variant(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K,
-                                   plan_tile(M, N, K, share, false).variant, stream);
+  return dfhip_gemm_fp8_nt_variant(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, plan.variant, stream);
 }
 
 extern "C" int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k) {
@@ -918,8 +970,20 @@ extern "C" int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* v
   return DFHIP_OK;
 }
 
+extern "C" int dfhip_gemm_fp8_plan_tiles(int M, int N, int K, int share, int may_split, int* variant, int* split_k) {
+  if (!variant || !split_k) return DFHIP_ERR_NULL_POINTER;
+  if (M < 1 || N < 1 || K < 1) return DFHIP_ERR_BAD_SHAPE;
+  if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
+  const TilePlan plan = plan_launch(M, N, K, share, may_split);
+  *variant = plan.variant;
+  *split_k = plan.split_k;
+  return DFHIP_OK;
+}
+
 extern "C" size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k) {
   const int tm = ring_blocks(variant);
+  if (M >= 1 && N >= 1 && split_k >= 2 && split_k <= DFHIP_RING3_MAX_SPLIT && dfhip_ring3_variant(variant, true))
+    return dfhip_ring3_workspace_bytes(M, N, variant - DFHIP_RING3_VARIANT, split_k);
   if (M < 1 || N < 1 || split_k < 2 || split_k > F8_MAX_SPLIT || !tm) return 0;
   const size_t tiles = (size_t)((M + 32 * tm - 1) / (32 * tm)) * ((N + 255) / 256);
   return dfhip_counter_area(tiles) + tiles * split_k * (size_t)(32 * tm) * 256 * sizeof(float);
@@ -930,11 +994,15 @@ extern "C" int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* 
                                         int split_k, void* workspace, size_t workspace_bytes, dfhip_stream_t stream) {
   if (int rc = check_gemm(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K)) return rc;
   const int tm = ring_blocks(variant);
-  if (!tm || split_k < 2 || split_k > F8_MAX_SPLIT || K / FBK < 2 * split_k) return DFHIP_ERR_BAD_ARGUMENT;
+  const bool three_slabs = dfhip_ring3_variant(variant, true);
+  if ((!tm && !three_slabs) || split_k < 2 || split_k > F8_MAX_SPLIT || K / FBK < 2 * split_k) return DFHIP_ERR_BAD_ARGUMENT;
   if (!workspace) return DFHIP_ERR_NULL_POINTER;
   if (!dfhip_aligned16(workspace)) return DFHIP_ERR_BAD_ALIGNMENT;
   if (workspace_bytes < dfhip_gemm_fp8_splitk_workspace_bytes(M, N, variant, split_k)) return DFHIP_ERR_BAD_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (three_slabs)
+    return dfhip_ring3_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, variant - DFHIP_RING3_VARIANT, split_k,
+                           workspace, s);
   switch (tm) {
     case 8: return launch_fp8_ring<8, true>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, split_k, workspace, s);
     case 6: return launch_fp8_ring<6, true>(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, split_k, workspace, s);
@@ -957,7 +1025,7 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t 
       !dfhip_aligned16(w_up_scale))
     return DFHIP_ERR_BAD_ALIGNMENT;
   if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
-  if (stream_planned(M, I, K, share, false))
+  if (few_rows_streamed(M, I, K, share, false))
     return dfhip_stream_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I,
                                     K, static_cast<hipStream_t>(stream));
   // the height of the tile that costs least in rounds (see tile_cost); every height adds in the same order.  A pair of
@@ -972,6 +1040,10 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t 
     if (&r == &F8_RINGS[0] || cost < least) { ring = &r; least = cost; }
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const DfhipRing3Plan three = three_slabs_cheaper(true, M, I, K, share, ring->variant, 1, false);
+  if (three.tile >= 0)
+    return dfhip_ring3_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I, K,
+                                   three.tile, s);
   switch (ring->tm) {
     case 8: return launch_fp8_ring_fused<8>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax,
                                             M, I, K, s);

@@ -40,6 +40,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "dfhip_ring3.h"
 #include "dfhip_stream.h"
 
 // Split-K scratch of dfhip_gemm_bf16_nt_splitk_static: arrival counters followed by fp32 partial blocks,
@@ -1680,6 +1681,37 @@ bool stream_planned(int M, int N, int K) {
          (int64_t)N * K <= (int64_t)1 << 27;
 }
 
+// Prices of the kernels above, as those of the three-slab tiles (dfhip_ring3.h), by variant.
+constexpr DfhipPrice RING_PRICE = {0.764, 0.703, 4.67, 1.82, 4.25, 5.0}, RING224_PRICE = {0.540, 0.755, 8.15, 0, 0, 6.22},
+                     RING128_PRICE = {0.445, 0.388, 3.56, 0, 0, 5.0}, ROWS192_PRICE = {0.628, 0.502, 5.40, 0, 0, 5.2},
+                     SKINNY_PRICE = {0.259, 0.329, 2.79, 4.43, 0.52, 5.54};
+
+// Whether a three-slab tile takes the place of the planned kernel (`variant`, K in `split_k` parts), and which.  It has to be
+// clearly cheaper: 4 %, and more where the prices are the least sure: 13 % against weight-streaming tiles that split K (20 % up
+// to 256 rows), in pairs 8 % for gate + up and 15 % against 192-row tiles.  Over 279 timed shapes (those of dfhip_price above 128 rows) this takes 5 % off the mean, 7 % being what
+// the best choice for each would; the worst loss is 7 % (200 x 28672 x 4096 alone: 71 -> 76 us), the best gains 48 % (1100 x
+// 2048 x 5632 alone: 58 -> 39) and 44 % (300 x 4096 x 14336 in pairs: 119 -> 83).
+DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share, int variant, int split_k, bool may_split) {
+  struct Kernel { int rows, cols; DfhipPrice price; } k;
+  switch (variant) {
+    case 0: k = {RBM, RBN, RING_PRICE}; break;
+    case 5: k = {RBM, TBN, RING224_PRICE}; break;
+    case 6: k = {SK_BM, SK_BN, SKINNY_PRICE}; break;
+    case 7: k = {RBM, 128, RING128_PRICE}; break;
+    case 9: k = {192, 256, ROWS192_PRICE}; break;
+    default: return {-1, 1, 0.0};
+  }
+  if (M <= SK_BM) return {-1, 1, 0.0};
+  const int cols = gate_up ? k.cols / 2 : k.cols;
+  const int64_t tiles = (int64_t)((M + k.rows - 1) / k.rows) * ((N + cols - 1) / cols);
+  const double now = dfhip_price(k.price, tiles, share, K / BK, split_k, (double)N * K * (gate_up ? 4e-6 : 2e-6));
+  const DfhipRing3Plan best = dfhip_ring3_plan(false, gate_up, M, N, K, share, may_split);
+  const double clearly = variant == 6 && split_k > 1 ? (M <= 256 ? 0.8 : 0.87)
+                                                     : share == 1 ? 0.96 : variant == 9 ? 0.85 : gate_up ? 0.92 : 0.96;
+  const double cube = clearly * clearly * clearly;
+  return best.cost < cube * cube * now ? best : DfhipRing3Plan{-1, 1, 0.0};
+}
+
 int check_args(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
                int K) {
   if (!A || !W || !C) return DFHIP_ERR_NULL_POINTER;
@@ -1711,7 +1743,9 @@ extern "C" int dfhip_gemm_bf16_nt_variant(const void* A, int64_t lda, const void
     case 8:
       if (!dfhip_stream_fits(M, N, (int64_t)K * 2, 1)) return DFHIP_ERR_BAD_SHAPE;
       return dfhip_stream_bf16(A, lda, W, ldw, nullptr, C, ldc, M, N, K, 1, nullptr, nullptr, s);
-    default: return DFHIP_ERR_BAD_ARGUMENT;
+    default:
+      if (!dfhip_ring3_variant(variant, false)) return DFHIP_ERR_BAD_ARGUMENT;
+      return dfhip_ring3_bf16(A, lda, W, ldw, nullptr, C, ldc, M, N, K, variant - DFHIP_RING3_VARIANT, 1, nullptr, s);
   }
 }
 
@@ -1777,10 +1811,42 @@ extern "C" int dfhip_gemm_bf16_plan_shared(int M, int N, int K, int share, int* 
   return DFHIP_OK;
 }
 
+extern "C" int dfhip_gemm_bf16_plan_tiles(int M, int N, int K, int share, int may_split, int* variant, int* split_k) {
+  if (int rc = dfhip_gemm_bf16_plan_shared(M, N, K, share, variant, split_k)) return rc;
+  if (!may_split) *split_k = 1;
+  const DfhipRing3Plan tiles = three_slabs_cheaper(false, M, N, K, share, *variant, *split_k, may_split);
+  if (tiles.tile >= 0) {
+    *variant = DFHIP_RING3_VARIANT + tiles.tile;
+    *split_k = tiles.split_k;
+  }
+  return DFHIP_OK;
+}
+
+extern "C" size_t dfhip_gemm_bf16_tiles_workspace_bytes(int M, int N, int variant, int split_k) {
+  if (M < 1 || N < 1 || split_k < 2 || split_k > DFHIP_RING3_MAX_SPLIT || !dfhip_ring3_variant(variant, false)) return 0;
+  return dfhip_ring3_workspace_bytes(M, N, variant - DFHIP_RING3_VARIANT, split_k);
+}
+
+extern "C" int dfhip_gemm_bf16_nt_tiles(const void* A, int64_t lda, const void* W, int64_t ldw, const void* R, void* C,
+                                        int64_t ldc, int M, int N, int K, int variant, int split_k, void* workspace,
+                                        size_t workspace_bytes, dfhip_stream_t stream) {
+  if (int rc = check_args(A, lda, W, ldw, C, ldc, M, N, K)) return rc;
+  if (R && !dfhip_aligned16(R)) return DFHIP_ERR_BAD_ALIGNMENT;
+  if (!dfhip_ring3_variant(variant, false) || split_k < 1 || split_k > DFHIP_RING3_MAX_SPLIT || K / BK < split_k)
+    return DFHIP_ERR_BAD_ARGUMENT;
+  if (split_k > 1) {
+    if (!workspace) return DFHIP_ERR_NULL_POINTER;
+    if (!dfhip_aligned16(workspace)) return DFHIP_ERR_BAD_ALIGNMENT;
+    if (workspace_bytes < dfhip_gemm_bf16_tiles_workspace_bytes(M, N, variant, split_k)) return DFHIP_ERR_BAD_ARGUMENT;
+  }
+  return dfhip_ring3_bf16(A, lda, W, ldw, R, C, ldc, M, N, K, variant - DFHIP_RING3_VARIANT, split_k, workspace,
+                          static_cast<hipStream_t>(stream));
+}
+
 extern "C" int dfhip_gemm_bf16_nt(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
                                   int64_t ldc, int M, int N, int K, dfhip_stream_t stream) {
   int variant = 2, split_k = 1;
-  if (int rc = dfhip_gemm_bf16_plan(M, N, K, &variant, &split_k)) return rc;
+  if (int rc = dfhip_gemm_bf16_plan_tiles(M, N, K, 1, 0, &variant, &split_k)) return rc;
   return dfhip_gemm_bf16_nt_variant(A, lda, W, ldw, C, ldc, M, N, K, variant, stream);
 }
 
@@ -1850,13 +1916,18 @@ extern "C" int dfhip_gemm_bf16_gate_up_silu_shared(const void* A, int64_t lda, c
     return launch_skinny<true>(A, lda, W_gate, W_up, ldw, Out, ldo, M, I, K, 1, nullptr,
                                static_cast<hipStream_t>(stream));
   }
+  const bool rows192 = rows192_cheaper(M, I, 128, TBN / 2, share);
+  const bool narrow = round_fill(M, I, TBN / 2, share) > round_fill(M, I, 128, share) + 0.05;
+  const DfhipRing3Plan tiles = three_slabs_cheaper(true, M, I, K, share, rows192 ? 9 : narrow ? 5 : 0, 1, false);
+  if (tiles.tile >= 0)
+    return dfhip_ring3_bf16_gate_up(A, lda, W_gate, W_up, ldw, Out, ldo, M, I, K, tiles.tile, static_cast<hipStream_t>(stream));
   // 192 x (128 + 128) where it takes clearly fewer of its shorter rounds
-  if (rows192_cheaper(M, I, 128, TBN / 2, share))
+  if (rows192)
     return launch_ring224<true, 256, 192>(A, lda, W_gate, W_up, ldw, Out, ldo, M, I, K, static_cast<hipStream_t>(stream));
   // the 256 x (112 + 112) tile when it fills the rounds of 256 workgroups clearly better than the 256 x (128 + 128)
   // one, which moves fewer bytes through LDS per flop; launches that run side by side take their rounds together
   // (two launches of the 8B shape at 2048 rows: 2 x 896 square tiles are exactly 7 rounds)
-  if (round_fill(M, I, TBN / 2, share) > round_fill(M, I, 128, share) + 0.05) {
+  if (narrow) {
     // a launch that has the GPU to itself and more than one round of tiles: workgroups that walk their tiles hide
     // a tile's stores behind the next one (they hold their compute units to the end, so nothing runs beside them)
     if (share == 1 && walk_kernel_fits(M, I, K) && ldo < (1 << 22) && (int64_t)(M / RBM) * (I / (TBN / 2)) > 256)

@@ -23,6 +23,7 @@ from __future__ import annotations
 import math
 import contextlib
 import ctypes
+import functools
 import os
 import weakref
 import threading
@@ -169,12 +170,30 @@ def _splitk_workspace(device: torch.device, stream: int, nbytes: int) -> torch.T
     return _zeroed_workspace(_splitk_workspaces, device, stream, nbytes)
 
 
-def _plan_bf16(lib, M: int, N: int, K: int) -> tuple[int, int]:
-    """(kernel variant, split of K) for a bf16 GEMM, for as many launches side by side as the forward declared."""
+#: kernel variants from here on are launched by dfhip_gemm_bf16_nt_tiles
+_FIRST_TILE_VARIANT = 10
+
+
+@functools.lru_cache(maxsize=4096)
+def _plan_tiles(entry: str, M: int, N: int, K: int, share: int, may_split: bool) -> tuple[int, int]:
     variant, split_k = ctypes.c_int(0), ctypes.c_int(1)
-    _cabi.check("dfhip_gemm_bf16_plan_shared", lib.dfhip_gemm_bf16_plan_shared(
-        M, N, K, _side_by_side(), ctypes.byref(variant), ctypes.byref(split_k)))
+    _cabi.check(entry, getattr(_cabi.load(), entry)(M, N, K, share, may_split, ctypes.byref(variant), ctypes.byref(split_k)))
     return variant.value, split_k.value
+
+
+def _plan_bf16(M: int, N: int, K: int, may_split: bool = True) -> tuple[int, int]:
+    """(kernel variant, split of K) for a bf16 GEMM, for as many launches side by side as the forward declared."""
+    return _plan_tiles("dfhip_gemm_bf16_plan_tiles", M, N, K, _side_by_side(), may_split)
+
+
+def _launch_tiles(lib, a, lda: int, w, ldw: int, residual, out, M: int, N: int, K: int, variant: int, split_k: int) -> None:
+    stream, ws_ptr, ws_bytes = _stream(), 0, 0
+    if split_k > 1:
+        ws = _splitk_workspace(a.device, stream, lib.dfhip_gemm_bf16_tiles_workspace_bytes(M, N, variant, split_k))
+        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+    _cabi.check("dfhip_gemm_bf16_nt_tiles", lib.dfhip_gemm_bf16_nt_tiles(
+        a.data_ptr(), lda, w.data_ptr(), ldw, residual.data_ptr() if residual is not None else 0, out.data_ptr(), N, M, N, K,
+        variant, split_k, ws_ptr, ws_bytes, stream))
 
 
 _output_offer = threading.local()
@@ -223,8 +242,10 @@ def _linear_impl(x: torch.Tensor, weight: torch.Tensor, variant: int = -1, split
                 )
                 _cabi.check("dfhip_gemm_bf16_nt_variant", rc)
             else:
-                planned, split_k = _plan_bf16(lib, M, N, K)
-                if split_k > 1 and split_k_allowed and SPLIT_K_ENABLED:
+                planned, split_k = _plan_bf16(M, N, K, split_k_allowed and SPLIT_K_ENABLED)
+                if planned >= _FIRST_TILE_VARIANT:
+                    _launch_tiles(lib, a, lda, w, ldw, None, out, M, N, K, planned, split_k)
+                elif split_k > 1:
                     stream = _stream()
                     nbytes = lib.dfhip_gemm_bf16_splitk_workspace_bytes(M, N, split_k)
                     ws = _splitk_workspace(x.device, stream, nbytes)
@@ -396,15 +417,15 @@ def _linear_add_impl(x: torch.Tensor, weight: torch.Tensor, residual: torch.Tens
         r = r.contiguous()
     out = _new_output(M, N, x.dtype, x.device, to_output)
     if M > 0:
-        stream = _stream()
-        _, split_k = _plan_bf16(lib, M, N, K)
-        ws_ptr, ws_bytes = 0, 0
-        if split_k > 1 and SPLIT_K_ENABLED:
+        planned, split_k = _plan_bf16(M, N, K, SPLIT_K_ENABLED)
+        if planned >= _FIRST_TILE_VARIANT:
+            _launch_tiles(lib, a, lda, w, ldw, r, out, M, N, K, planned, split_k)
+            return out.view(*x.shape[:-1], N)
+        stream, ws_ptr, ws_bytes = _stream(), 0, 0
+        if split_k > 1:
             nbytes = lib.dfhip_gemm_bf16_splitk_workspace_bytes(M, N, split_k)
             ws = _splitk_workspace(x.device, stream, nbytes)
             ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
-        else:
-            split_k = 1
         rc = lib.dfhip_gemm_bf16_nt_add(
             a.data_ptr(), lda, w.data_ptr(), ldw, r.data_ptr(), out.data_ptr(), N, M, N, K, split_k, ws_ptr,
             ws_bytes, stream,
@@ -813,10 +834,7 @@ def _linear_fp8_impl(x_q, w_q, x_scale, w_scale, variant: int = -1, to_output: b
     if M > 0:
         stream, split_k = _stream(), 1
         if cut_k and SPLIT_K_ENABLED:
-            planned, parts = ctypes.c_int(-1), ctypes.c_int(1)
-            _cabi.check("dfhip_gemm_fp8_plan_shared", lib.dfhip_gemm_fp8_plan_shared(
-                M, N, K, _side_by_side(), ctypes.byref(planned), ctypes.byref(parts)))
-            variant, split_k = planned.value, parts.value
+            variant, split_k = _plan_tiles("dfhip_gemm_fp8_plan_tiles", M, N, K, _side_by_side(), True)
         scale = w_scale.contiguous()
         gemm = (a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, x_scale.data_ptr(), scale.data_ptr(), M, N, K)
         if split_k > 1:

@@ -99,6 +99,8 @@ int dfhip_gemm_bf16_nt(const void* A, int64_t lda, const void* W, int64_t ldw, v
  *          weights of at most 2^27 elements);
  *          9 = 192x256 tile, LDS-DMA ring (chosen instead of 0 and 5 where its shorter rounds of
  *              256 workgroups cost less, e.g. 670 rows of N = 14336; the same bits);
+ *          10 .. 15 = 224x192, 160x256, 128x256, 192x192, 128x192, 128x128 tiles of which LDS holds
+ *              three slabs and more (dfhip_gemm_bf16_plan_tiles; the same bits);
  *          register-staged tiles: 1 = 256x256 / 8 waves, 2 = 128x128 / 4 waves,
  *          3 = 256x128 / 4 waves, 4 = 256x256 / 4 waves. */
 int dfhip_gemm_bf16_nt_variant(const void* A, int64_t lda, const void* W, int64_t ldw, void* C,
@@ -116,6 +118,18 @@ int dfhip_gemm_bf16_plan(int M, int N, int K, int* variant, int* split_k);
  * together, so K is split less or not at all and the tile shape is chosen for the rounds they take
  * together.  1 <= share <= 16; share = 1 is dfhip_gemm_bf16_plan. */
 int dfhip_gemm_bf16_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
+
+/* The same among all tiles: variants 10 .. 15 where they cost clearly less than that choice (200 x 14336 x 4096
+ * in a pair 79 -> 64 us, 1100 x 2048 x 5632 alone 58 -> 39), which stands elsewhere.  may_split = 0: K stays whole.
+ * dfhip_gemm_bf16_nt_tiles launches variants 10 .. 15, with K in split_k parts (1 .. 16) that meet in a
+ * workspace of dfhip_gemm_bf16_tiles_workspace_bytes bytes, 16-byte aligned, whose arrival counters (4 bytes a tile at
+ * its start) are zero and left zero; the part that comes last adds all in part order, nobody waits.  R: residual
+ * [M, N] of leading dimension ldc added to the rounded product as by dfhip_gemm_bf16_nt_add, or null. */
+int dfhip_gemm_bf16_plan_tiles(int M, int N, int K, int share, int may_split, int* variant, int* split_k);
+size_t dfhip_gemm_bf16_tiles_workspace_bytes(int M, int N, int variant, int split_k);
+int dfhip_gemm_bf16_nt_tiles(const void* A, int64_t lda, const void* W, int64_t ldw, const void* R, void* C,
+                             int64_t ldc, int M, int N, int K, int variant, int split_k, void* workspace,
+                             size_t workspace_bytes, dfhip_stream_t stream);
 
 /* Split-K flavour of the fast path for shapes with few output tiles (the same `linear` node,
  * dynaflow/runtime/engine.py:381; the down projection of the host model's MLP, whose gate and up
@@ -235,14 +249,16 @@ int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* W, int64_t 
                              const float* a_scale, const float* w_scale, int M, int N, int K, int share,
                              dfhip_stream_t stream);
 /* The same with K cut into split_k parts (2 .. 16, at least two slabs of 128 each), for outputs of too few tiles to
- * fill the GPU; variant 0, 3 or 4.  workspace: dfhip_gemm_fp8_splitk_workspace_bytes bytes, 16-byte aligned, whose
+ * fill the GPU; variant 0, 3, 4, 11, 12 or 15.  workspace: dfhip_gemm_fp8_splitk_workspace_bytes bytes, 16-byte aligned, whose
  * arrival counters (4 bytes a tile at its start) are zero; they are left zero.  Launches that may overlap need one
  * each.  The parts are added in part order: the same bits in every run.
  * dfhip_gemm_fp8_plan_shared: the variant and split for `share` launches of this shape side by side (variant < 0:
  * dfhip_gemm_fp8_nt_shared).  For the projection back to the model width: K is only cut where K > N, and the
  * projections in front of it, which keep the order of sums of dfhip_gemm_fp8_gate_up_silu_absmax, are launched without a
- * split whatever their widths are. */
+ * split whatever their widths are.
+ * dfhip_gemm_fp8_plan_tiles: the same among all tiles, 11, 12 and 15 (those of dfhip_gemm_bf16_nt_variant) included. */
 int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
+int dfhip_gemm_fp8_plan_tiles(int M, int N, int K, int share, int may_split, int* variant, int* split_k);
 size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k);
 int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
                              const float* a_scale, const float* w_scale, int M, int N, int K, int variant, int split_k,
