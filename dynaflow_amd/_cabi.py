@@ -130,6 +130,10 @@ SIGNATURES: dict[str, tuple] = {
     "dfhip_transpose_bf16": (c_int, [_P, c_int64, _P, c_int64, c_int, c_int, _P]),
     "dfhip_absmax_bf16": (c_int, [_P, c_int64, c_int, c_int, _P, _P]),
     "dfhip_quant_fp8_bf16": (c_int, [_P, c_int64, _P, c_int64, c_int, c_int, _P, _P, _P]),
+    "dfhip_quant_fp8_dynamic_bf16": (c_int, [_P, c_int64, _P, c_int64, c_int, c_int, _P, _P, _P]),
+    "dfhip_silu_mul_quant_fp8_bf16": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, _P, _P,
+                                              _P]),
+    "dfhip_requant_fp8_bf16": (c_int, [_P, c_int64, _P, c_int64, c_int, c_int, _P, _P, _P]),
     "dfhip_silu_mul_absmax_bf16": (
         c_int,
         [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, _P, _P],

@@ -117,6 +117,124 @@ silu_mul_absmax_kernel(const uint16_t* __restrict__ gate, int64_t ld_gate, const
   block_max_to(amax, m);
 }
 
+// ---- quantisation without a cell that has to be cleared first: the blocks leave their maxima in `parts`, and every block
+// of the launch that quantises takes the maximum of those
+constexpr int QPARTS = DFHIP_FP8_PARTS;          // blocks at most
+
+// (address of group gi; without a gap between rows no division)
+template <bool FLAT>
+DFHIP_DEVICE int64_t group_at(uint32_t gi, uint32_t per_row, int64_t ld) {
+  if (FLAT) return (int64_t)gi * 8;
+  const uint32_t row = gi / per_row;
+  return (int64_t)row * ld + (gi - row * per_row) * 8;
+}
+DFHIP_DEVICE float absmax8(u32x4 v) {
+  float m = 0.0f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) m = fmaxf(m, fmaxf(fabsf(bf16_lo_to_f32(v[w])), fabsf(bf16_hi_to_f32(v[w]))));
+  return m;
+}
+DFHIP_DEVICE u32x2 quant8(u32x4 v, float scale) {
+  return u32x2{quant4(bf16_lo_to_f32(v[0]), bf16_hi_to_f32(v[0]), bf16_lo_to_f32(v[1]), bf16_hi_to_f32(v[1]), scale),
+               quant4(bf16_lo_to_f32(v[2]), bf16_hi_to_f32(v[2]), bf16_lo_to_f32(v[3]), bf16_hi_to_f32(v[3]), scale)};
+}
+// the block's maximum, in every thread
+template <int THREADS>
+DFHIP_DEVICE float block_max(float v) {
+  __shared__ float partial[THREADS / 64];
+  v = wave_max(v);
+  if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = partial[0];
+#pragma unroll
+  for (int w = 1; w < THREADS / 64; ++w) v = fmaxf(v, partial[w]);
+  return v;
+}
+
+// parts[block] = max |x| of the groups of the block; with `up`, x is first replaced by bf16(silu(x) * up), which is stored.
+// Bound: HBM, or up to some MB the launch.  QUNROLL groups of a thread are loaded before the first is used, and no atomics
+// queue up at one address (12 ns each): with the quantisation behind it and no launch to clear a cell, x of 12 / 350 / 2048 x
+// 8192 7.6 / 12.8 / 41.6 -> 5.6 / 8.2 / 19.5 us, SiLU*mul of 350 / 2048 x 28672 32 / 106 -> 23 / 91.
+template <bool FLAT, bool SILU>
+__global__ void __launch_bounds__(QT)
+absmax_parts_kernel(const uint16_t* __restrict__ x, int64_t ld, const uint16_t* __restrict__ up, int64_t ld_up,
+                    uint16_t* __restrict__ out, int64_t ld_out, uint32_t groups, uint32_t per_row,
+                    float* __restrict__ parts) {
+  float m = 0.0f;
+  for (uint32_t g0 = blockIdx.x * (QT * QUNROLL) + threadIdx.x; g0 < groups; g0 += gridDim.x * (QT * QUNROLL)) {
+    u32x4 v[QUNROLL], u[QUNROLL];
+#pragma unroll
+    for (int k = 0; k < QUNROLL; ++k) {
+      const uint32_t gi = g0 + k * QT < groups ? g0 + k * QT : g0;
+      v[k] = *reinterpret_cast<const u32x4*>(x + group_at<FLAT>(gi, per_row, ld));
+      if (SILU) u[k] = *reinterpret_cast<const u32x4*>(up + group_at<FLAT>(gi, per_row, ld_up));
+    }
+    DFHIP_PIN;
+#pragma unroll
+    for (int k = 0; k < QUNROLL; ++k) {
+      if (SILU) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          v[k][w] = pack2_bf16(silu_f32(bf16_lo_to_f32(v[k][w])) * bf16_lo_to_f32(u[k][w]),
+                               silu_f32(bf16_hi_to_f32(v[k][w])) * bf16_hi_to_f32(u[k][w]));
+        if (g0 + k * QT < groups)
+          *reinterpret_cast<u32x4*>(out + group_at<FLAT>(g0 + k * QT, per_row, ld_out)) = v[k];
+      }
+      m = fmaxf(m, absmax8(v[k]));               // (a group past the end repeats the first one)
+    }
+  }
+  m = block_max<QT>(m);
+  if (threadIdx.x == 0) parts[blockIdx.x] = m;
+}
+
+// q = e4m3fn(x / scale), scale = max(amax, 1e-12) / 448.  PARTS: amax is the maximum of n_parts values; else `amax` is one
+// value, which the last block to have read it clears, with the count of those that have: the cells are zero again for the
+// launch that folds the next maximum into them.
+template <bool FLAT, bool PARTS>
+__global__ void __launch_bounds__(QT)
+quant_fp8_after_kernel(const uint16_t* __restrict__ x, int64_t ld, uint8_t* __restrict__ q, int64_t ld_q, uint32_t groups,
+                       uint32_t per_row, float* __restrict__ amax, int n_parts, int* __restrict__ readers,
+                       float* __restrict__ scale_out) {
+  const uint32_t step = gridDim.x * (QT * QUNROLL);
+  uint32_t g0 = blockIdx.x * (QT * QUNROLL) + threadIdx.x;
+  u32x4 v[QUNROLL];
+  auto load = [&]() {
+#pragma unroll
+    for (int k = 0; k < QUNROLL; ++k) {
+      const uint32_t gi = g0 + k * QT < groups ? g0 + k * QT : groups - 1;
+      v[k] = *reinterpret_cast<const u32x4*>(x + group_at<FLAT>(gi, per_row, ld));
+    }
+    DFHIP_PIN;
+  };
+  load();
+  float m = 0.0f;
+  if (PARTS) {
+#pragma unroll
+    for (int p = 0; p < QPARTS / QT; ++p)
+      if (p * QT + (int)threadIdx.x < n_parts) m = fmaxf(m, amax[p * QT + threadIdx.x]);
+    m = block_max<QT>(m);
+  } else {
+    __shared__ float cell;
+    if (threadIdx.x == 0) cell = __hip_atomic_load(amax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    m = cell;
+    if (threadIdx.x == 0 && atomicAdd(readers, 1) == (int)gridDim.x - 1) {
+      __hip_atomic_store(amax, 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(readers, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  const float scale = fmaxf(m, 1e-12f) / FP8_MAX;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && scale_out != nullptr) scale_out[0] = scale;
+  while (g0 < groups) {
+#pragma unroll
+    for (int k = 0; k < QUNROLL; ++k)
+      if (g0 + k * QT < groups)
+        *reinterpret_cast<u32x2*>(q + group_at<FLAT>(g0 + k * QT, per_row, ld_q)) = quant8(v[k], scale);
+    g0 += step;
+    if (g0 < groups) load();
+  }
+}
+
 // ------------------------------------------------------------------ fp8 GEMM
 constexpr int FBK = 128;            // fp8 values (= bytes) per slab row
 constexpr int FROW = FBK + 16;      // padded LDS row in bytes
@@ -909,6 +1027,73 @@ extern "C" int dfhip_quant_fp8_bf16(const void* x, int64_t ld, void* q, int64_t 
                      static_cast<const uint16_t*>(x), ld, static_cast<uint8_t*>(q), ld_q, groups, per_row, amax,
                      scale_out);
   return dfhip_check_launch();
+}
+
+namespace {
+unsigned parts_for(uint32_t groups) {
+  const uint32_t blocks = (groups + QT * QUNROLL - 1) / (QT * QUNROLL);
+  return blocks > QPARTS ? QPARTS : blocks;
+}
+int check_q_out(const void* q, int64_t ld_q, int D) {
+  if (!q) return DFHIP_ERR_NULL_POINTER;
+  if (ld_q < D) return DFHIP_ERR_BAD_STRIDE;
+  return ld_q % 8 || (reinterpret_cast<uintptr_t>(q) & 7u) ? DFHIP_ERR_BAD_ALIGNMENT : DFHIP_OK;
+}
+template <bool PARTS>
+int launch_quant_after(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, float* amax, int n_parts, int* readers,
+                       float* scale_out, hipStream_t stream) {
+  const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
+  const auto kernel = ld == D && ld_q == D ? quant_fp8_after_kernel<true, PARTS> : quant_fp8_after_kernel<false, PARTS>;
+  hipLaunchKernelGGL(kernel, dim3(parts_for(groups)), dim3(QT), 0, stream, static_cast<const uint16_t*>(x), ld,
+                     static_cast<uint8_t*>(q), ld_q, groups, per_row, amax, n_parts, readers, scale_out);
+  return dfhip_check_launch();
+}
+}  // namespace
+
+extern "C" int dfhip_quant_fp8_dynamic_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, float* parts,
+                                            float* scale_out, dfhip_stream_t stream) {
+  if (int rc = check_q(x, ld, M, D)) return rc;
+  if (int rc = check_q_out(q, ld_q, D)) return rc;
+  if (!parts) return DFHIP_ERR_NULL_POINTER;
+  const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const auto kernel = ld == D ? absmax_parts_kernel<true, false> : absmax_parts_kernel<false, false>;
+  hipLaunchKernelGGL(kernel, dim3(parts_for(groups)), dim3(QT), 0, s, static_cast<const uint16_t*>(x), ld, nullptr, 0, nullptr,
+                     0, groups, per_row, parts);
+  if (int rc = dfhip_check_launch()) return rc;
+  return launch_quant_after<true>(x, ld, q, ld_q, M, D, parts, (int)parts_for(groups), nullptr, scale_out, s);
+}
+
+extern "C" int dfhip_silu_mul_quant_fp8_bf16(const void* gate, int64_t ld_gate, const void* up, int64_t ld_up, void* act,
+                                             int64_t ld_act, void* q, int64_t ld_q, int M, int D, float* parts,
+                                             float* scale_out, dfhip_stream_t stream) {
+  if (int rc = check_q(gate, ld_gate, M, D)) return rc;
+  if (int rc = check_q(up, ld_up, M, D)) return rc;
+  if (int rc = check_q(act, ld_act, M, D)) return rc;
+  if (int rc = check_q_out(q, ld_q, D)) return rc;
+  if (!parts) return DFHIP_ERR_NULL_POINTER;
+  const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool flat = ld_gate == D && ld_up == D && ld_act == D;
+  const auto kernel = flat ? absmax_parts_kernel<true, true> : absmax_parts_kernel<false, true>;
+  hipLaunchKernelGGL(kernel, dim3(parts_for(groups)), dim3(QT), 0, s, static_cast<const uint16_t*>(gate), ld_gate,
+                     static_cast<const uint16_t*>(up), ld_up, static_cast<uint16_t*>(act), ld_act, groups, per_row, parts);
+  if (int rc = dfhip_check_launch()) return rc;
+  return launch_quant_after<true>(act, ld_act, q, ld_q, M, D, parts, (int)parts_for(groups), nullptr, scale_out, s);
+}
+
+extern "C" int dfhip_requant_fp8_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, void* cells,
+                                      float* scale_out, dfhip_stream_t stream) {
+  if (int rc = check_q(x, ld, M, D)) return rc;
+  if (int rc = check_q_out(q, ld_q, D)) return rc;
+  if (!cells) return DFHIP_ERR_NULL_POINTER;
+  // counting readers costs 12 ns a block (350 x 28672: 21 us with 1024 of them, 11 with the launch that clears): up to 128
+  if (parts_for((uint32_t)M * (D / 8)) > 128) {
+    if (int rc = dfhip_quant_fp8_bf16(x, ld, q, ld_q, M, D, static_cast<float*>(cells), scale_out, stream)) return rc;
+    return dfhip_fill_u32(cells, 0u, 1, stream);
+  }
+  return launch_quant_after<false>(x, ld, q, ld_q, M, D, static_cast<float*>(cells), 0, static_cast<int*>(cells) + 1,
+                                   scale_out, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int dfhip_silu_mul_absmax_bf16(const void* gate, int64_t ld_gate, const void* up, int64_t ld_up,

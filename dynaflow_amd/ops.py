@@ -732,9 +732,13 @@ torch.library.register_fake(
 
 
 # --------------------------------------------------------------------- fp8
-def _fill_zero(t: torch.Tensor) -> None:
-    rc = _cabi.load().dfhip_fill_u32(t.data_ptr(), 0, t.numel(), _stream())
-    _cabi.check("dfhip_fill_u32", rc)
+#: DFHIP_FP8_PARTS: floats in which the blocks of a quantisation leave their maxima
+_FP8_PARTS = 1024
+#: cells that a fused launch folds max |act| into, and the count of blocks that have read it: zero between launches.
+#: Keyed like the split-K workspaces.
+_amax_cells: dict[tuple, torch.Tensor] = {}
+#: held from the launch that folds into a cell to the one that clears it again: threads that share a stream
+_amax_pair = threading.Lock()
 
 
 def _quant_fp8_impl(x: torch.Tensor):
@@ -744,16 +748,13 @@ def _quant_fp8_impl(x: torch.Tensor):
     if x.dtype != torch.bfloat16:
         raise RuntimeError("quant_fp8: bf16 input only")
     xr, M, D, ld = _rows(x)
-    amax = torch.empty(1, dtype=torch.float32, device=x.device)
-    scale = torch.empty(1, dtype=torch.float32, device=x.device)
+    scale = torch.empty(1 + _FP8_PARTS, dtype=torch.float32, device=x.device)
     q = torch.empty((M, D), dtype=FP8_DTYPE, device=x.device)
-    _fill_zero(amax)
-    rc = lib.dfhip_absmax_bf16(xr.data_ptr(), ld, M, D, amax.data_ptr(), _stream())
-    _cabi.check("dfhip_absmax_bf16", rc)
-    rc = lib.dfhip_quant_fp8_bf16(
-        xr.data_ptr(), ld, q.data_ptr(), D, M, D, amax.data_ptr(), scale.data_ptr(), _stream()
+    rc = lib.dfhip_quant_fp8_dynamic_bf16(
+        xr.data_ptr(), ld, q.data_ptr(), D, M, D, scale.data_ptr() + 4, scale.data_ptr(), _stream()
     )
-    _cabi.check("dfhip_quant_fp8_bf16", rc)
+    _cabi.check("dfhip_quant_fp8_dynamic_bf16", rc)
+    scale = scale[:1]
     return q.view(x.shape), scale
 
 
@@ -766,18 +767,14 @@ def _silu_mul_quant_fp8_impl(gate: torch.Tensor, up: torch.Tensor):
     g, M, D, ldg = _rows(gate)
     u, _, _, ldu = _rows(up)
     act = torch.empty((M, D), dtype=torch.bfloat16, device=gate.device)
-    amax = torch.empty(1, dtype=torch.float32, device=gate.device)
-    scale = torch.empty(1, dtype=torch.float32, device=gate.device)
+    scale = torch.empty(1 + _FP8_PARTS, dtype=torch.float32, device=gate.device)
     q = torch.empty((M, D), dtype=FP8_DTYPE, device=gate.device)
-    _fill_zero(amax)
-    rc = lib.dfhip_silu_mul_absmax_bf16(
-        g.data_ptr(), ldg, u.data_ptr(), ldu, act.data_ptr(), D, M, D, amax.data_ptr(), _stream()
+    rc = lib.dfhip_silu_mul_quant_fp8_bf16(
+        g.data_ptr(), ldg, u.data_ptr(), ldu, act.data_ptr(), D, q.data_ptr(), D, M, D, scale.data_ptr() + 4,
+        scale.data_ptr(), _stream()
     )
-    _cabi.check("dfhip_silu_mul_absmax_bf16", rc)
-    rc = lib.dfhip_quant_fp8_bf16(
-        act.data_ptr(), D, q.data_ptr(), D, M, D, amax.data_ptr(), scale.data_ptr(), _stream()
-    )
-    _cabi.check("dfhip_quant_fp8_bf16", rc)
+    _cabi.check("dfhip_silu_mul_quant_fp8_bf16", rc)
+    scale = scale[:1]
     return q.view(gate.shape), scale
 
 
@@ -800,20 +797,22 @@ def _gate_up_silu_quant_fp8_impl(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w
         wg, wu = wg.contiguous(), wu.contiguous()
         ldg = K
     act = torch.empty((M, I), dtype=torch.bfloat16, device=x_q.device)
-    amax = torch.empty(1, dtype=torch.float32, device=x_q.device)
     scale = torch.empty(1, dtype=torch.float32, device=x_q.device)
     q = torch.empty((M, I), dtype=FP8_DTYPE, device=x_q.device)
     if M > 0:
-        _fill_zero(amax)
-        rc = lib.dfhip_gemm_fp8_gate_up_silu_absmax_shared(
-            a.data_ptr(), lda, wg.data_ptr(), wu.data_ptr(), ldg, act.data_ptr(), I, x_scale.data_ptr(),
-            w_gate_scale.contiguous().data_ptr(), w_up_scale.contiguous().data_ptr(), amax.data_ptr(), M, I, K,
-            _side_by_side(), _stream(),
-        )
-        _cabi.check("dfhip_gemm_fp8_gate_up_silu_absmax_shared", rc)
-        rc = lib.dfhip_quant_fp8_bf16(act.data_ptr(), I, q.data_ptr(), I, M, I, amax.data_ptr(), scale.data_ptr(),
-                                      _stream())
-        _cabi.check("dfhip_quant_fp8_bf16", rc)
+        gate_scale, up_scale, stream = w_gate_scale.contiguous(), w_up_scale.contiguous(), _stream()
+        with _amax_pair:
+            cells = _zeroed_workspace(_amax_cells, x_q.device, stream, 256, 256)
+            rc = lib.dfhip_gemm_fp8_gate_up_silu_absmax_shared(
+                a.data_ptr(), lda, wg.data_ptr(), wu.data_ptr(), ldg, act.data_ptr(), I, x_scale.data_ptr(),
+                gate_scale.data_ptr(), up_scale.data_ptr(), cells.data_ptr(), M, I, K, _side_by_side(), stream,
+            )
+            _cabi.check("dfhip_gemm_fp8_gate_up_silu_absmax_shared", rc)
+            rc = lib.dfhip_requant_fp8_bf16(act.data_ptr(), I, q.data_ptr(), I, M, I, cells.data_ptr(), scale.data_ptr(),
+                                            stream)
+            if rc != 0:
+                lib.dfhip_fill_u32(cells.data_ptr(), 0, 2, stream)
+            _cabi.check("dfhip_requant_fp8_bf16", rc)
     return q.view(*x_q.shape[:-1], I), scale
 
 

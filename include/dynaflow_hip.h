@@ -438,6 +438,21 @@ int dfhip_silu_mul_absmax_bf16(const void* gate, int64_t ld_gate, const void* up
                                void* out, int64_t ld_out, int M, int D, float* amax,
                                dfhip_stream_t stream);
 
+/* Both without a cell to clear: the maximum and the quantisation behind it, the blocks' maxima meeting in `parts`
+ * (DFHIP_FP8_PARTS floats, contents of no matter before and after).
+ * The same codes and scale as the pairs of calls above.
+ * dfhip_silu_mul_quant_fp8_bf16: act = bf16(silu(gate) * up) [M, D] is written on the way.
+ * dfhip_requant_fp8_bf16: the launch behind dfhip_gemm_fp8_gate_up_silu_absmax; cells = the amax that one folded
+ * its maximum into, followed by a 32-bit count; both zero before, and zero again when this launch is done. */
+#define DFHIP_FP8_PARTS 1024
+int dfhip_quant_fp8_dynamic_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, float* parts,
+                                 float* scale_out, dfhip_stream_t stream);
+int dfhip_silu_mul_quant_fp8_bf16(const void* gate, int64_t ld_gate, const void* up, int64_t ld_up, void* act,
+                                  int64_t ld_act, void* q, int64_t ld_q, int M, int D, float* parts,
+                                  float* scale_out, dfhip_stream_t stream);
+int dfhip_requant_fp8_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, void* cells,
+                           float* scale_out, dfhip_stream_t stream);
+
 /* Fill `count` 32-bit words with `value` (a capture-safe replacement for
  * memset nodes, used to clear amax cells).  No counterpart in the reference (there a cudaMemset inside a
  * captured graph is fine, dynaflow/executor/cudagraph.py:84-122 captures whatever the callable issues). */

@@ -1,0 +1,97 @@
+"""Quantisation without a cell to clear: the codes and scales of the maximum and the quantisation launched one by one, at the
+sizes where the kernels change."""
+import pytest
+import torch
+
+from dynaflow_amd import _cabi
+
+pytestmark = pytest.mark.gpu
+
+
+def rows(M, D, gap, seed, special=False):
+    """[M, D] bf16 whose rows lie `gap` elements apart from another; optionally with infinities, NaN and the largest values."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    t = (torch.randn((M, D + gap), generator=g, device="cuda") * torch.exp2(torch.randn((M, 1), generator=g, device="cuda") * 4))
+    t = t.bfloat16()
+    if special:
+        t.view(-1)[:: max(1, t.numel() // 3)] = float("nan")
+    return t[:, :D]
+
+
+def one_by_one(x):
+    lib, s, (M, D) = _cabi.load(), torch.cuda.current_stream().cuda_stream, x.shape
+    amax, scale = torch.zeros(1, device="cuda"), torch.zeros(1, device="cuda")
+    q = torch.zeros((M, D), dtype=torch.uint8, device="cuda")
+    assert lib.dfhip_absmax_bf16(x.data_ptr(), x.stride(0), M, D, amax.data_ptr(), s) == 0
+    assert lib.dfhip_quant_fp8_bf16(x.data_ptr(), x.stride(0), q.data_ptr(), D, M, D, amax.data_ptr(), scale.data_ptr(), s) == 0
+    return q, scale, amax
+
+
+# one group; an odd count; a whole block and one group more; as many blocks as count their readers and one more; more than parts
+SIZES = [(1, 8), (3, 40), (1, 8192), (1, 8200), (128, 8192), (129, 8192), (4097, 2056)]
+
+
+@pytest.mark.parametrize("M,D", SIZES)
+@pytest.mark.parametrize("gap", [0, 8])
+@pytest.mark.parametrize("special", [False, True])
+def test_quant_dynamic(M, D, gap, special):
+    lib, s = _cabi.load(), torch.cuda.current_stream().cuda_stream
+    x = rows(M, D, gap, 1, special)
+    want_q, want_scale, _ = one_by_one(x)
+    parts = torch.full((1024,), float("inf"), device="cuda")
+    scale, q = torch.zeros(1, device="cuda"), torch.zeros((M, D + gap), dtype=torch.uint8, device="cuda")
+    assert lib.dfhip_quant_fp8_dynamic_bf16(x.data_ptr(), D + gap, q.data_ptr(), D + gap, M, D, parts.data_ptr(),
+                                            scale.data_ptr(), s) == 0
+    assert torch.equal(scale, want_scale) and torch.equal(q[:, :D], want_q) and not q[:, D:].any()
+    # the same behind a cell, which is zero again afterwards
+    cells = torch.zeros(2, device="cuda")
+    assert lib.dfhip_absmax_bf16(x.data_ptr(), D + gap, M, D, cells.data_ptr(), s) == 0
+    q.zero_()
+    assert lib.dfhip_requant_fp8_bf16(x.data_ptr(), D + gap, q.data_ptr(), D + gap, M, D, cells.data_ptr(), scale.data_ptr(),
+                                      s) == 0
+    assert torch.equal(scale, want_scale) and torch.equal(q[:, :D], want_q) and not cells.view(torch.int32).any()
+
+
+@pytest.mark.parametrize("M,D", SIZES)
+@pytest.mark.parametrize("gap", [0, 16])
+def test_silu_mul_quant(M, D, gap):
+    lib, s = _cabi.load(), torch.cuda.current_stream().cuda_stream
+    g, u = rows(M, D, gap, 2), rows(M, D, gap, 3)
+    act, amax = torch.zeros((M, D), dtype=torch.bfloat16, device="cuda"), torch.zeros(1, device="cuda")
+    assert lib.dfhip_silu_mul_absmax_bf16(g.data_ptr(), D + gap, u.data_ptr(), D + gap, act.data_ptr(), D, M, D,
+                                          amax.data_ptr(), s) == 0
+    want_q, want_scale, _ = one_by_one(act)
+    got, q = torch.zeros((M, D + gap), dtype=torch.bfloat16, device="cuda"), torch.zeros((M, D), dtype=torch.uint8, device="cuda")
+    scale, parts = torch.zeros(1, device="cuda"), torch.full((1024,), float("inf"), device="cuda")
+    assert lib.dfhip_silu_mul_quant_fp8_bf16(g.data_ptr(), D + gap, u.data_ptr(), D + gap, got.data_ptr(), D + gap, q.data_ptr(),
+                                             D, M, D, parts.data_ptr(), scale.data_ptr(), s) == 0
+    assert torch.equal(got[:, :D], act) and not got[:, D:].any()
+    assert torch.equal(scale, want_scale) and torch.equal(q, want_q)
+
+
+def test_fused_launches_of_two_threads_on_one_stream():
+    """The maximum of one thread's launch is not another's: the cell is theirs from the fold to the quantisation."""
+    import threading
+
+    from dynaflow_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    wq = [(torch.randn((1024, 2048), generator=g, device="cuda") * 50).to(torch.float8_e4m3fn) for _ in range(2)]
+    ws, xs = torch.full((1024,), 0.01, device="cuda"), torch.full((1,), 0.01, device="cuda")
+    xq = [(torch.randn((M, 2048), generator=g, device="cuda") * 10.0 ** i).to(torch.float8_e4m3fn) for i, M in enumerate((9, 40))]
+    want = [ops.gate_up_silu_quant_fp8(x, *wq, xs, ws, ws) for x in xq]
+    got = [[], []]
+
+    def work(i):
+        got[i] = [ops.gate_up_silu_quant_fp8(xq[i], *wq, xs, ws, ws) for _ in range(40)]
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert len(got[i]) == 40
+        for q, scale in got[i]:
+            assert torch.equal(scale, want[i][1]) and torch.equal(q.view(torch.uint8), want[i][0].view(torch.uint8))
