@@ -9,7 +9,7 @@
 // global memory (no LDS staging, no transposes):
 //   scores^T = K Q^T : A = K rows (lane: one position, 8 consecutive dims)
 //   out      = P V   : B = V     (lane: one dim, 8 consecutive positions)
-#include "dfhip_common.h"
+#include "dfhip_pairs.h"
 
 namespace {
 
@@ -500,6 +500,8 @@ static int decode_attention_append(const void* qkv, int64_t ld_qkv, void* k_cach
   if (parts < MIN_PARTS) parts = 1;
   const auto kernel = parts > 1 ? decode_attention_kernel<true, true> : decode_attention_kernel<true, false>;
   float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + ATTENTION_COUNTER_BYTES);
+  static const bool known = (dfhip_in_line(reinterpret_cast<const void*>(decode_attention_kernel<true, false>), 256), true);
+  (void)known;
   hipLaunchKernelGGL(kernel, dim3(T * kv_heads, parts), dim3(DEC_THREADS), lds_bytes,
                      static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(qkv), ld_qkv,
                      static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), slots, lengths,

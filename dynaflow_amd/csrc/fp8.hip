@@ -16,6 +16,7 @@
 //                       with K cut into parts for few tiles: [350 x 28672] x [8192 x 28672]^T ran on 64 workgroups
 //                       (230 us, 0.71 PFLOP/s), with 192 rows and four parts it takes 96.
 // gemm_fp8_nt_kernel    register-staged double buffer, 128 x 128: an independent second kernel, by variant only.
+#include "dfhip_pairs.h"
 #include "dfhip_ring3.h"
 #include "dfhip_stream.h"
 
@@ -950,7 +951,9 @@ DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share,
   const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
   const double now = dfhip_price(price, tiles, share, K / FBK, split_k, (double)N * K * (gate_up ? 2e-6 : 1e-6));
   const DfhipRing3Plan best = dfhip_ring3_plan(true, gate_up, M, N, K, share, may_split);
-  const double clearly = gate_up && share > 1 && M > 128 ? 0.85 : M > 256 || gate_up ? 0.93 : 0.96;
+  // (side by side and up to 128 rows also where it costs 5 % more: two of these launches can become one, dfhip_pairs.h)
+  const double clearly = share > 1 && M <= DFHIP_PAIR_MAX_M ? 1.05
+                         : gate_up && share > 1 ? 0.85 : M > 256 || gate_up ? 0.93 : 0.96;
   const double cube = clearly * clearly * clearly;
   return best.cost < cube * cube * now ? best : DfhipRing3Plan{-1, 1, 0.0};
 }

@@ -40,6 +40,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "dfhip_pairs.h"
 #include "dfhip_ring3.h"
 #include "dfhip_stream.h"
 
@@ -1199,16 +1200,44 @@ struct SkinnyTile {
   static constexpr int FLIGHT = (AHEAD - 2) * (A_DMA + W_DMA);
 };
 
+// Arguments of the weight-streaming kernels (strides in elements; parts of K and R, the residual, not FUSED).
+struct SkinnyArgs {
+  const uint16_t* W;
+  const uint16_t* W2;          // up weight (FUSED)
+  int N, K;
+  int tiles_m, tiles_n, split_k;
+  int64_t ldw;
+  DfhipSide side[2];
+};
+
+bool sides_skinny(const void* a, const void* b, void* both) {
+  const SkinnyArgs &x = *static_cast<const SkinnyArgs*>(a), &y = *static_cast<const SkinnyArgs*>(b);
+  if (!dfhip_sides_apart(x.side[0], y.side[0]) || x.W != y.W || x.W2 != y.W2 || x.N != y.N || x.K != y.K ||
+      x.tiles_m != y.tiles_m || x.tiles_n != y.tiles_n || x.split_k != y.split_k || x.ldw != y.ldw || x.side[0].M > DFHIP_PAIR_MAX_M ||
+      y.side[0].M > DFHIP_PAIR_MAX_M)
+    return false;
+  SkinnyArgs& out = *static_cast<SkinnyArgs*>(both);
+  out = x;
+  out.side[1] = y.side[0];
+  return true;
+}
+
 // FUSED: C[M, N] = silu(A W^T) * (A W2^T) (gate and up weights, N = the intermediate size, K not split):
 // a tile has BW / 2 columns, its W half holds, per wave column, 32 gate rows and the 32 matching up rows, so MFMA
 // block j = 0 is the gate and j = 1 the up projection of the same outputs; where a wave has one block (JN = 1) its
 // rows are 16 gate and 16 up rows, and the accumulators g and g + 2 of a lane belong together.
-template <bool FUSED, int BM, int BW>
+// MERGED: rows 0 .. 63 of a tile of 128 are side 0, 64 .. 127 side 1.
+template <bool FUSED, int BM, int BW, DfhipPaired PAIRED>
 __global__ void __launch_bounds__(RTHREADS)
-gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
-                        const uint16_t* __restrict__ W2, uint16_t* __restrict__ C,
-                        int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, int tiles_m, int tiles_n,
-                        int split_k, float* __restrict__ partials, int* __restrict__ arrivals) {
+gemm_bf16_skinny_kernel(const SkinnyArgs p) {
+  int at_side = 0;
+  const int block = PAIRED == DFHIP_BESIDE ? pair_block(blockIdx.x, gridDim.x, at_side) : blockIdx.x;
+  const uint16_t *const W = p.W, *const W2 = p.W2;
+  const int N = p.N, K = p.K, tiles_m = p.tiles_m, tiles_n = p.tiles_n;
+  const int64_t ldw = p.ldw;
+  const int split_k = p.split_k;
+  float* const partials = p.side[at_side].partials;
+  int* const arrivals = p.side[at_side].arrivals;
   using T = SkinnyTile<BM, BW>;
   constexpr int JN = T::JN, HALF = T::WROWS / 2;   // FUSED: gate rows of a wave
   constexpr int TILE_N = FUSED ? BW / 2 : BW;
@@ -1217,7 +1246,7 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave_m = wave % T::WAVES_M, wave_n = wave / T::WAVES_M;
   const int tiles = tiles_m * tiles_n;
-  const int work = remap_xcd(blockIdx.x, tiles * split_k);
+  const int work = remap_xcd(block, tiles * split_k);
   const int part = work / tiles;
   const int tile = work - part * tiles;        // column tile major, row tile minor
   const int tile_n = tile / tiles_m;
@@ -1230,12 +1259,16 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
   // DMA: instructions of 8 rows x 128 bytes, the rows of a slab dealt to the waves in runs
   const uint8_t* a_src[T::A_DMA];
   const uint8_t* w_src[T::W_DMA];
+  constexpr bool merged = PAIRED == DFHIP_MERGED;
+  static_assert(!merged || BM == 128);
+  const DfhipSide& from = p.side[merged ? wave >> 1 : at_side];   // of the A rows that this wave fetches
+  const int from0 = merged ? -64 * (wave >> 1) : m0;
 #pragma unroll
   for (int t = 0; t < T::A_DMA; ++t) {
     const int row = (wave * T::A_DMA + t) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-    const int ar = m0 + row < M ? m0 + row : M - 1;
-    a_src[t] = reinterpret_cast<const uint8_t*>(A + (int64_t)ar * lda + chunk * 8);
+    const int ar = from0 + row < from.M ? from0 + row : from.M - 1;
+    a_src[t] = reinterpret_cast<const uint8_t*>(static_cast<const uint16_t*>(from.A) + (int64_t)ar * from.lda + chunk * 8);
   }
 #pragma unroll
   for (int t = 0; t < T::W_DMA; ++t) {
@@ -1364,6 +1397,10 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
     }
   }
 
+  const DfhipSide& my = p.side[merged ? wave_m : at_side];        // of the rows that this wave has the sums of
+  uint16_t* const C = static_cast<uint16_t*>(my.C);
+  const int M = my.M, m_wave = merged ? 0 : m0 + wave_m * 64;
+  const int64_t ldc = my.ldc;
   if (FUSED) {
     // the roundings of the separate kernels: bf16 projections, bf16 silu, bf16 product
     constexpr int OUTS = HALF, FROW = OUTS * 2 + 16, RUNS = OUTS / 8;   // outputs, padded bytes, 16-byte pieces of a row
@@ -1385,7 +1422,7 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
         *reinterpret_cast<u32x2*>(fpark + (i * 32 + frow) * FROW + (g * 8 + fhalf * 4) * 2) = v;
       }
     DFHIP_PIN;
-    const int fm_base = m0 + wave_m * 64, fn_base = n0 + wave_n * OUTS;
+    const int fm_base = m_wave, fn_base = n0 + wave_n * OUTS;
 #pragma unroll
     for (int p = 0; p < RUNS; ++p) {
       const int id = p * 64 + lane;
@@ -1412,7 +1449,7 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
         *reinterpret_cast<u32x2*>(park + (i * 32 + frow) * PROW + (j * 32 + g * 8 + fhalf * 4) * 2) = v;
       }
   DFHIP_PIN;
-  const int m_base = m0 + wave_m * 64, n_base = n0 + wave_n * T::WROWS;
+  const int m_base = m_wave, n_base = n0 + wave_n * T::WROWS;
 #pragma unroll 4
   for (int p = 0; p < RUNS; ++p) {
     const int id = p * 64 + lane;
@@ -1420,8 +1457,8 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
     u32x4 v = *reinterpret_cast<const u32x4*>(park + row * PROW + c * 16);
     const int m = m_base + row, n = n_base + c * 8;
     if (m < M && n < N) {
-      if (W2) {            // not FUSED: W2 is the optional residual [M, N] (leading dimension ldc)
-        const u32x4 r = *reinterpret_cast<const u32x4*>(W2 + (int64_t)m * ldc + n);
+      if (my.R) {          // the residual [M, N] (leading dimension ldc)
+        const u32x4 r = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(my.R) + (int64_t)m * ldc + n);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = add2_bf16(v[e], r[e]);
       }
@@ -1439,15 +1476,19 @@ gemm_bf16_skinny_kernel(const uint16_t* __restrict__ A, const uint16_t* __restri
 // Same instruction and same order of K as gemm_bf16_skinny_kernel<true>: the same bits.
 constexpr int SKW_BN = 128, SKW_UNIT = 49152, SKW_UNITS = 3, SKW_LDS = SKW_UNITS * SKW_UNIT;
 
+template <bool BESIDE>
 __global__ void __launch_bounds__(RTHREADS)
-gemm_bf16_skinny_wide_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ W,
-                             const uint16_t* __restrict__ W2, uint16_t* __restrict__ C, int M, int N, int K,
-                             int64_t lda, int64_t ldw, int64_t ldc, int tiles_m, int tiles_n) {
+gemm_bf16_skinny_wide_kernel(const SkinnyArgs p) {
+  int at_side = 0;
+  const int block = BESIDE ? pair_block(blockIdx.x, gridDim.x, at_side) : blockIdx.x;
+  const uint16_t *const W = p.W, *const W2 = p.W2;
+  const int N = p.N, K = p.K, tiles_m = p.tiles_m, tiles_n = p.tiles_n;
+  const int64_t ldw = p.ldw;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave_m = wave & 1, wave_n = wave >> 1;
-  const int tile = remap_xcd(blockIdx.x, tiles_m * tiles_n);   // column tile major, row tile minor
+  const int tile = remap_xcd(block, tiles_m * tiles_n);   // column tile major, row tile minor
   const int tile_n = tile / tiles_m;
   const int m0 = (tile - tile_n * tiles_m) * SK_BM;
   const int n0 = tile_n * SKW_BN;
@@ -1457,12 +1498,13 @@ gemm_bf16_skinny_wide_kernel(const uint16_t* __restrict__ A, const uint16_t* __r
   // instructions (8 per wave); W row r of the unit: wave column r / 128, (gate, up) = (r / 64) % 2, output r % 64
   const uint8_t* a_src[4];
   const uint8_t* w_src[8];
+  const DfhipSide& my = p.side[at_side];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int row = (wave * 4 + t) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-    const int ar = m0 + row < M ? m0 + row : M - 1;
-    a_src[t] = reinterpret_cast<const uint8_t*>(A + (int64_t)ar * lda + chunk * 8);
+    const int ar = m0 + row < my.M ? m0 + row : my.M - 1;
+    a_src[t] = reinterpret_cast<const uint8_t*>(static_cast<const uint16_t*>(my.A) + (int64_t)ar * my.lda + chunk * 8);
   }
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
@@ -1554,7 +1596,9 @@ gemm_bf16_skinny_wide_kernel(const uint16_t* __restrict__ A, const uint16_t* __r
         *reinterpret_cast<u32x2*>(park + (i * 32 + frow) * PROW + (jj * 32 + g * 8 + fhalf * 4) * 2) = v;
       }
   DFHIP_PIN;
-  const int m_base = m0 + wave_m * 64, n_base = n0 + wave_n * 64;
+  uint16_t* const C = static_cast<uint16_t*>(my.C);
+  const int M = my.M, m_base = m0 + wave_m * 64, n_base = n0 + wave_n * 64;
+  const int64_t ldc = my.ldc;
 #pragma unroll 4
   for (int p = 0; p < 8; ++p) {
     const int id = p * 64 + lane;
@@ -1568,10 +1612,35 @@ gemm_bf16_skinny_wide_kernel(const uint16_t* __restrict__ A, const uint16_t* __r
 size_t skinny_tiles(int M, int N) { return (size_t)((M + SK_BM - 1) / SK_BM) * ((N + SK_BN - 1) / SK_BN); }
 size_t skinny_counter_bytes(int M, int N) { return dfhip_counter_area(skinny_tiles(M, N)); }
 
+// Two launches of up to 64 rows each against gate and up weights are one of 128-row tiles with 64 outputs (K is whole, so the
+// tile's width does not show in the sums); others sit side by side, so that K has the parts it had.  [us, a pair at 2 x 48 rows,
+// 8B shapes, on two streams / side by side in one launch / in one tile: gate + up + SiLU*mul 72 / 64 / 48, down 45 / 39 /
+// 47, whose 128 workgroups are too few]
+template <bool FUSED, int BM, int BW>
+bool join_skinny(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+  static std::atomic<uint64_t> lds_opted_in{0};
+  constexpr bool MERGED = FUSED && BM == 64;
+  using T = SkinnyTile<MERGED ? 128 : BM, MERGED ? 128 : BW>;
+  if (!sides_skinny(a, b, both)) return false;
+  if constexpr (MERGED) {
+    SkinnyArgs& out = *static_cast<SkinnyArgs*>(both);
+    out.tiles_n = (out.N + 63) / 64;
+    *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_kernel<true, 128, 128, DFHIP_MERGED>), T::LDS, (unsigned)out.tiles_n};
+  } else {
+    *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_kernel<FUSED, BM, BW, DFHIP_BESIDE>), T::LDS, 2 * grid};
+  }
+  return dfhip_opt_in_lds(joined->kernel, T::LDS, lds_opted_in) == DFHIP_OK;
+}
+bool join_skinny_wide(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+  static std::atomic<uint64_t> lds_opted_in{0};
+  *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_wide_kernel<true>), SKW_LDS, 2 * grid};
+  return sides_skinny(a, b, both) && dfhip_opt_in_lds(joined->kernel, SKW_LDS, lds_opted_in) == DFHIP_OK;
+}
+
 template <bool FUSED, int BM, int BW>
 int launch_skinny_tile(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                        int M, int N, int K, int split_k, void* workspace, hipStream_t stream) {
-  auto kernel = gemm_bf16_skinny_kernel<FUSED, BM, BW>;
+  auto kernel = gemm_bf16_skinny_kernel<FUSED, BM, BW, DFHIP_ALONE>;
   constexpr int LDS = SkinnyTile<BM, BW>::LDS;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), LDS, lds_opted_in)) return rc;
@@ -1584,10 +1653,12 @@ int launch_skinny_tile(const void* A, int64_t lda, const void* W, const void* W2
     if (int rc = dfhip_clear_uncommon_counters(workspace, skinny_tiles(M, N), stream)) return rc;
     partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + skinny_counter_bytes(M, N));
   }
-  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(RTHREADS), LDS, stream,
-                     static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(W),
-                     static_cast<const uint16_t*>(W2), static_cast<uint16_t*>(C), M, N, K, lda, ldw, ldc, tiles_m,
-                     tiles_n, split_k, partials, arrivals);
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof(SkinnyArgs), join_skinny<FUSED, BM, BW>), true);
+  (void)known;
+  const uint16_t* const w2 = static_cast<const uint16_t*>(W2);   // not FUSED: the residual
+  const SkinnyArgs args{static_cast<const uint16_t*>(W), FUSED ? w2 : nullptr, N, K, tiles_m, tiles_n, split_k, ldw,
+                        {{A, FUSED ? nullptr : w2, C, nullptr, nullptr, partials, arrivals, lda, ldc, M}, {}}};
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * split_k), dim3(RTHREADS), LDS, stream, args);
   return dfhip_check_launch();
 }
 
@@ -1611,15 +1682,16 @@ int launch_skinny_wide(const void* A, int64_t lda, const void* W, const void* W2
   if (M > SK_MAX_M || K / BK < 2) return DFHIP_ERR_BAD_SHAPE;
   if (M <= 64)
     return launch_skinny_tile<true, 64, 2 * SKW_BN>(A, lda, W, W2, ldw, C, ldc, M, N, K, 1, nullptr, stream);
-  auto kernel = gemm_bf16_skinny_wide_kernel;
+  auto kernel = gemm_bf16_skinny_wide_kernel<false>;
   static std::atomic<uint64_t> lds_opted_in{0};
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), SKW_LDS, lds_opted_in)) return rc;
   const int tiles_m = (M + SK_BM - 1) / SK_BM;
   const int tiles_n = (N + SKW_BN - 1) / SKW_BN;
-  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(RTHREADS), SKW_LDS, stream,
-                     static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(W),
-                     static_cast<const uint16_t*>(W2), static_cast<uint16_t*>(C), M, N, K, lda, ldw, ldc, tiles_m,
-                     tiles_n);
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof(SkinnyArgs), join_skinny_wide), true);
+  (void)known;
+  const SkinnyArgs args{static_cast<const uint16_t*>(W), static_cast<const uint16_t*>(W2), N, K, tiles_m, tiles_n, 1, ldw,
+                        {{A, nullptr, C, nullptr, nullptr, nullptr, nullptr, lda, ldc, M}, {}}};
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(RTHREADS), SKW_LDS, stream, args);
   return dfhip_check_launch();
 }
 

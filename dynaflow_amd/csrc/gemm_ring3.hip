@@ -18,6 +18,7 @@
 // 777 x 4096 x 14336 104 -> 93, 300 x 4096 x 14336 in pairs 126 -> 83, 1554 x 2048 x 5632 59 -> 41.
 // Tried and taken back: touching the W lines of later slabs (one 4-byte DMA per line, so that they wait in L2) - 5 to 10 us
 // slower everywhere; 192 x 224, 256 x 160 and 64-row tiles - never the best of those that remain by more than 2 %.
+#include "dfhip_pairs.h"
 #include "dfhip_ring3.h"
 
 namespace {
@@ -25,21 +26,27 @@ namespace {
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
 struct Ring3Args {
-  const uint8_t* A;
   const uint8_t* W;
   const uint8_t* W2;          // up weight (FUSED)
-  const uint16_t* R;          // residual [M, N] with the row stride of C, or null (bf16, not FUSED)
-  uint16_t* C;
-  const float* a_scale;       // fp8: one float; per output channel for the weights
-  const float* w_scale;
+  const float* w_scale;       // fp8: per output channel
   const float* w2_scale;
-  float* amax;                // fp8 FUSED
-  int M, N, slabs;            // slabs of 128 bytes per row
-  int64_t lda, ldw, ldc;      // bytes, bytes, elements
+  int N, slabs;               // slabs of 128 bytes per row
   int tiles_m, tiles_n, split_k;
-  float* partials;
-  int* arrivals;
+  int64_t ldw;                // bytes (the strides of A too; that of C in elements)
+  DfhipSide side[2];          // R (residual [M, N] with the row stride of C, or null): bf16, not FUSED
 };
+
+bool sides_ring3(const void* a, const void* b, void* both) {
+  const Ring3Args &x = *static_cast<const Ring3Args*>(a), &y = *static_cast<const Ring3Args*>(b);
+  if (!dfhip_sides_apart(x.side[0], y.side[0]) || x.W != y.W || x.W2 != y.W2 || x.w_scale != y.w_scale ||
+      x.w2_scale != y.w2_scale || x.N != y.N || x.slabs != y.slabs || x.split_k != y.split_k || x.ldw != y.ldw || x.tiles_m != y.tiles_m || x.tiles_n != y.tiles_n ||
+      x.side[0].M > DFHIP_PAIR_MAX_M || y.side[0].M > DFHIP_PAIR_MAX_M)
+    return false;
+  Ring3Args& out = *static_cast<Ring3Args*>(both);
+  out = x;
+  out.side[1] = y.side[0];
+  return true;
+}
 
 constexpr int GROUP_M = 4;    // tiles of one XCD are walked in panels of GROUP_M tile rows
 constexpr int SLAB = 128;     // bytes of K
@@ -52,7 +59,7 @@ constexpr int units(int tm, int tn) { const int u = 160 * 1024 / ((tm + tn) * SL
 template <bool FP8>
 DFHIP_DEVICE int chunk_of(int s) { return FP8 ? 2 * (s & 3) + (s >> 2) : s; }
 
-template <bool FP8, bool FUSED, int TM, int TN, bool SPLIT>
+template <bool FP8, bool FUSED, int TM, int TN, bool SPLIT, bool BESIDE>
 __global__ void __launch_bounds__(256)
 gemm_ring3_kernel(const Ring3Args p) {
   static_assert(!(FUSED && SPLIT), "the fused form keeps K whole");
@@ -66,9 +73,13 @@ gemm_ring3_kernel(const Ring3Args p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave_m = wave & 1, wave_n = wave >> 1;
 
+  int at_side = 0;
+  const int block = BESIDE ? pair_block(blockIdx.x, gridDim.x, at_side) : blockIdx.x;
+  const DfhipSide& my = p.side[at_side];
+  const int M = my.M;
   int tile, part = 0;
-  if (SPLIT) splitk_work_of(blockIdx.x, p.tiles_m * p.tiles_n, tile, part);
-  else tile = remap_xcd(blockIdx.x, p.tiles_m * p.tiles_n);
+  if (SPLIT) splitk_work_of(block, p.tiles_m * p.tiles_n, tile, part);
+  else tile = remap_xcd(block, p.tiles_m * p.tiles_n);
   const int per_panel = GROUP_M * p.tiles_n;
   const int first_m = (tile / per_panel) * GROUP_M;
   const int rows_in_panel = (p.tiles_m - first_m) < GROUP_M ? (p.tiles_m - first_m) : GROUP_M;
@@ -84,8 +95,8 @@ gemm_ring3_kernel(const Ring3Args p) {
 #pragma unroll
   for (int t = 0; t < IB; ++t) {
     const int row = (wave * IB + t) * 8 + (lane >> 3);
-    int ar = m0 + row; ar = ar < p.M ? ar : p.M - 1;
-    a_off[t] = (uint32_t)((int64_t)(ar - m0) * p.lda + chunk_of<FP8>((lane & 7) ^ ((row >> 1) & 7)) * 16);
+    int ar = m0 + row; ar = ar < M ? ar : M - 1;
+    a_off[t] = (uint32_t)((int64_t)(ar - m0) * my.lda + chunk_of<FP8>((lane & 7) ^ ((row >> 1) & 7)) * 16);
   }
 #pragma unroll
   for (int t = 0; t < JB; ++t) {
@@ -93,7 +104,7 @@ gemm_ring3_kernel(const Ring3Args p) {
     int wr = n0 + (FUSED ? row % OUT_N : row); wr = wr < p.N ? wr : p.N - 1;
     w_off[t] = (uint32_t)((int64_t)(wr - n0) * p.ldw + chunk_of<FP8>((lane & 7) ^ ((row >> 1) & 7)) * 16);
   }
-  const uint8_t* const a_tile = p.A + (int64_t)m0 * p.lda + (int64_t)slab0 * SLAB;
+  const uint8_t* const a_tile = static_cast<const uint8_t*>(my.A) + (int64_t)m0 * my.lda + (int64_t)slab0 * SLAB;
   const uint8_t* const w_tile = ((FUSED && wave >= 2) ? p.W2 : p.W) + (int64_t)n0 * p.ldw + (int64_t)slab0 * SLAB;
   auto dma = [&](int t, int slab, int unit) {  // instruction t of a slab: A first, then W
     const int64_t s = (int64_t)(slab < KT ? slab : KT - 1) * SLAB;
@@ -193,7 +204,7 @@ gemm_ring3_kernel(const Ring3Args p) {
     // Every part leaves its fp32 block and takes a ticket; the part that comes last adds the blocks in part order (its own
     // too: the same bits whoever is last) and writes the tile.  Nobody waits.
     constexpr int BLOCK = MQ * 256;            // f32x4 of a part
-    f32x4* const blocks = reinterpret_cast<f32x4*>(p.partials) + (int64_t)tile * p.split_k * BLOCK;
+    f32x4* const blocks = reinterpret_cast<f32x4*>(my.partials) + (int64_t)tile * p.split_k * BLOCK;
     f32x4* const mine = blocks + part * BLOCK + tid;
 #pragma unroll
     for (int i = 0; i < IB; ++i)
@@ -202,11 +213,11 @@ gemm_ring3_kernel(const Ring3Args p) {
     wait_vmcnt<0>();
     __syncthreads();
     int* const ticket_cell = reinterpret_cast<int*>(smem);
-    if (tid == 0) *ticket_cell = atomicAdd(p.arrivals + tile, 1);
+    if (tid == 0) *ticket_cell = atomicAdd(my.arrivals + tile, 1);
     __syncthreads();
     const int ticket = *ticket_cell;
     if (ticket != p.split_k - 1) return;
-    if (tid == 0) atomicExch(p.arrivals + tile, 0);      // counters are left at zero
+    if (tid == 0) atomicExch(my.arrivals + tile, 0);      // counters are left at zero
     __syncthreads();                                     // the ticket has been read before the tile is parked over it
     const auto left = coherent_blocks(blocks, p.split_k * BLOCK * 16);
     // 4 JB loads in flight (a load from the memory side takes microseconds when every tile is at it)
@@ -240,7 +251,7 @@ gemm_ring3_kernel(const Ring3Args p) {
 
   // round to bf16 (fp8: scale first), park the wave's block in LDS, store whole row pieces of 16 bytes
   constexpr int PROW = JB * 32 + 16, CPR = JB * 2;       // padded row of a park (bytes), pieces of a row
-  const float sa = FP8 ? p.a_scale[0] : 1.0f;
+  const float sa = FP8 ? my.a_scale[0] : 1.0f;
   uint8_t* const park = smem + wave * (16 * IB * PROW);
 #pragma unroll
   for (int j = 0; j < JB; ++j) {
@@ -275,7 +286,7 @@ gemm_ring3_kernel(const Ring3Args p) {
       const int id = q * 64 + lane;
       const int row = row0 + id / CPR, c = id % CPR;
       const int m = m0 + (wave & 1) * (16 * IB) + row, n = n0 + c * 8;
-      if (id >= 8 * IB * CPR || m >= p.M || n >= p.N) continue;   // N % 8 == 0: a piece is inside or outside
+      if (id >= 8 * IB * CPR || m >= M || n >= p.N) continue;   // N % 8 == 0: a piece is inside or outside
       const u32x4 gv = *reinterpret_cast<const u32x4*>(gpark + row * PROW + c * 16);
       const u32x4 uv = *reinterpret_cast<const u32x4*>(upark + row * PROW + c * 16);
       u32x4 o;
@@ -290,13 +301,13 @@ gemm_ring3_kernel(const Ring3Args p) {
         o[w] = pack2_bf16(lo * bf16_lo_to_f32(uv[w]), hi * bf16_hi_to_f32(uv[w]));
         if (FP8) vmax = fmaxf(vmax, fmaxf(fabsf(bf16_lo_to_f32(o[w])), fabsf(bf16_hi_to_f32(o[w]))));
       }
-      u32x4* const at = reinterpret_cast<u32x4*>(p.C + (int64_t)m * p.ldc + n);
+      u32x4* const at = reinterpret_cast<u32x4*>(static_cast<uint16_t*>(my.C) + (int64_t)m * my.ldc + n);
       if (FP8) *at = o; else __builtin_nontemporal_store(o, at);
     }
     if constexpr (FP8) {
       vmax = wave_max(vmax);
       // non-negative floats order like their bit patterns
-      if (lane == 0 && vmax > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(p.amax), __float_as_uint(vmax));
+      if (lane == 0 && vmax > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(my.amax), __float_as_uint(vmax));
     }
   } else {
     const int m_base = m0 + wave_m * (16 * IB), n_base = n0 + wave_n * (16 * JB);
@@ -305,12 +316,12 @@ gemm_ring3_kernel(const Ring3Args p) {
       const int id = q * 64 + lane;
       const int row = id / CPR, c = id % CPR;
       const int m = m_base + row, n = n_base + c * 8;
-      if (id >= 16 * IB * CPR || m >= p.M || n >= p.N) continue;
+      if (id >= 16 * IB * CPR || m >= M || n >= p.N) continue;
       u32x4 v = *reinterpret_cast<const u32x4*>(park + row * PROW + c * 16);
-      u32x4* const at = reinterpret_cast<u32x4*>(p.C + (int64_t)m * p.ldc + n);
+      u32x4* const at = reinterpret_cast<u32x4*>(static_cast<uint16_t*>(my.C) + (int64_t)m * my.ldc + n);
       if (FP8) { *at = v; continue; }
-      if (p.R) {
-        const u32x4 r = *reinterpret_cast<const u32x4*>(p.R + (int64_t)m * p.ldc + n);
+      if (my.R) {
+        const u32x4 r = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(my.R) + (int64_t)m * my.ldc + n);
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = add2_bf16(v[e], r[e]);
       }
@@ -320,20 +331,31 @@ gemm_ring3_kernel(const Ring3Args p) {
 }
 
 template <bool FP8, bool FUSED, bool SPLIT, int T>
+bool join_ring3(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+  constexpr int TM = DFHIP_RING3[T].rows, TN = DFHIP_RING3[T].cols;
+  constexpr int LDS = units(TM, TN) * (TM + TN) * SLAB;
+  static std::atomic<uint64_t> lds_opted_in{0};
+  *joined = {reinterpret_cast<const void*>(gemm_ring3_kernel<FP8, FUSED, TM, TN, SPLIT, true>), LDS, 2 * grid};
+  return sides_ring3(a, b, both) && dfhip_opt_in_lds(joined->kernel, LDS, lds_opted_in) == DFHIP_OK;
+}
+
+template <bool FP8, bool FUSED, bool SPLIT, int T>
 int launch(Ring3Args p, void* workspace, hipStream_t stream) {
   constexpr int TM = DFHIP_RING3[T].rows, TN = DFHIP_RING3[T].cols, OUT_N = FUSED ? TN / 2 : TN;
   constexpr int LDS = units(TM, TN) * (TM + TN) * SLAB;
-  auto kernel = gemm_ring3_kernel<FP8, FUSED, TM, TN, SPLIT>;
+  auto kernel = gemm_ring3_kernel<FP8, FUSED, TM, TN, SPLIT, false>;
   static std::atomic<uint64_t> lds_opted_in{0};
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), LDS, lds_opted_in)) return rc;
-  p.tiles_m = (p.M + TM - 1) / TM;
+  p.tiles_m = (p.side[0].M + TM - 1) / TM;
   p.tiles_n = (p.N + OUT_N - 1) / OUT_N;
   if (SPLIT) {
     const size_t tiles = (size_t)p.tiles_m * p.tiles_n;
     if (int rc = dfhip_clear_uncommon_counters(workspace, tiles, stream)) return rc;
-    p.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area(tiles));
-    p.arrivals = static_cast<int*>(workspace);
+    p.side[0].partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area(tiles));
+    p.side[0].arrivals = static_cast<int*>(workspace);
   }
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof p, join_ring3<FP8, FUSED, SPLIT, T>), true);
+  (void)known;
   hipLaunchKernelGGL(kernel, dim3(p.tiles_m * p.tiles_n * p.split_k), dim3(256), LDS, stream, p);
   return dfhip_check_launch();
 }
@@ -375,32 +397,28 @@ size_t dfhip_ring3_workspace_bytes(int M, int N, int tile, int split_k) {
 
 int dfhip_ring3_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const void* R, void* C, int64_t ldc, int M,
                      int N, int K, int tile, int split_k, void* workspace, hipStream_t stream) {
-  const Ring3Args p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), nullptr, static_cast<const uint16_t*>(R),
-                    static_cast<uint16_t*>(C), nullptr, nullptr, nullptr, nullptr, M, N, K / 64, lda * 2, ldw * 2, ldc, 0, 0,
-                    split_k, nullptr, nullptr};
+  const Ring3Args p{static_cast<const uint8_t*>(W), nullptr, nullptr, nullptr, N, K / 64, 0, 0, split_k, ldw * 2,
+                    {{A, R, C, nullptr, nullptr, nullptr, nullptr, lda * 2, ldc, M}, {}}};
   return split_k > 1 ? launch_tile<false, false, true>(p, tile, workspace, stream)
                      : launch_tile<false, false, false>(p, tile, nullptr, stream);
 }
 int dfhip_ring3_bf16_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                              int M, int N, int K, int tile, hipStream_t stream) {
-  const Ring3Args p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), nullptr,
-                    static_cast<uint16_t*>(C), nullptr, nullptr, nullptr, nullptr, M, N, K / 64, lda * 2, ldw * 2, ldc, 0, 0,
-                    1, nullptr, nullptr};
+  const Ring3Args p{static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), nullptr, nullptr, N, K / 64, 0, 0, 1,
+                    ldw * 2, {{A, nullptr, C, nullptr, nullptr, nullptr, nullptr, lda * 2, ldc, M}, {}}};
   return launch_tile<false, true, false>(p, tile, nullptr, stream);
 }
 int dfhip_ring3_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
                     const float* w_scale, int M, int N, int K, int tile, int split_k, void* workspace, hipStream_t stream) {
-  const Ring3Args p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), nullptr, nullptr,
-                    static_cast<uint16_t*>(C), a_scale, w_scale, nullptr, nullptr, M, N, K / 128, lda, ldw, ldc, 0, 0,
-                    split_k, nullptr, nullptr};
+  const Ring3Args p{static_cast<const uint8_t*>(W), nullptr, w_scale, nullptr, N, K / 128, 0, 0, split_k, ldw,
+                    {{A, nullptr, C, a_scale, nullptr, nullptr, nullptr, lda, ldc, M}, {}}};
   return split_k > 1 ? launch_tile<true, false, true>(p, tile, workspace, stream)
                      : launch_tile<true, false, false>(p, tile, nullptr, stream);
 }
 int dfhip_ring3_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                             const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, int M, int N,
                             int K, int tile, hipStream_t stream) {
-  const Ring3Args p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), nullptr,
-                    static_cast<uint16_t*>(C), a_scale, w_scale, w2_scale, amax, M, N, K / 128, lda, ldw, ldc, 0, 0, 1,
-                    nullptr, nullptr};
+  const Ring3Args p{static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), w_scale, w2_scale, N, K / 128, 0, 0, 1,
+                    ldw, {{A, nullptr, C, a_scale, amax, nullptr, nullptr, lda, ldc, M}, {}}};
   return launch_tile<true, true, false>(p, tile, nullptr, stream);
 }

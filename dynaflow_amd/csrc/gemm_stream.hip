@@ -21,6 +21,7 @@
 // 6144 x 4096 12 / 15 / 18, before 62 / 22 / 22; o 4096 x 4096 8 / 10 / 13, before 61 / 21 / 21.  At 8 / 16 / 32 / 64
 // rows fp8 down 8192 x 28672 (235 MB) 37 / 42 / 54 / 79, before 240; fp8 gate + up 2 x 28672 x 8192 (470 MB)
 // 80 / 82 / 92 / 112, before 113 - 117.
+#include "dfhip_pairs.h"
 #include "dfhip_stream.h"
 
 namespace {
@@ -28,21 +29,26 @@ namespace {
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 
 struct StreamArgs {
-  const uint8_t* A;
   const uint8_t* W;
   const uint8_t* W2;          // up weight (FUSED)
-  const uint16_t* R;          // residual [M, N] with the row stride of C, or null (bf16, not FUSED)
-  uint16_t* C;
-  const float* a_scale;       // fp8: one float; per output channel for the weights
-  const float* w_scale;
+  const float* w_scale;       // fp8: per output channel
   const float* w2_scale;
-  float* amax;                // fp8 FUSED
-  int M, N, slabs;            // slabs of 128 bytes per row
+  int N, slabs;               // slabs of 128 bytes per row
   int split_k;                // workgroups per tile along K (not FUSED)
-  float* partials;
-  int* arrivals;
-  int64_t lda, ldw, ldc;      // bytes, bytes, elements
+  int64_t ldw;                // bytes (the strides of A too; that of C in elements)
+  DfhipSide side[2];          // R (residual [M, N] with the row stride of C, or null): bf16, not FUSED
 };
+
+bool sides_stream(const void* a, const void* b, void* both) {
+  const StreamArgs &x = *static_cast<const StreamArgs*>(a), &y = *static_cast<const StreamArgs*>(b);
+  if (!dfhip_sides_apart(x.side[0], y.side[0]) || x.W != y.W || x.W2 != y.W2 || x.w_scale != y.w_scale ||
+      x.w2_scale != y.w2_scale || x.N != y.N || x.slabs != y.slabs || x.split_k != y.split_k || x.ldw != y.ldw)
+    return false;
+  StreamArgs& out = *static_cast<StreamArgs*>(both);
+  out = x;
+  out.side[1] = y.side[0];
+  return true;
+}
 
 constexpr int WAVES = 4;
 
@@ -53,7 +59,8 @@ constexpr int rows_per_round(int mb, int nb) {
   return r;
 }
 
-template <bool FP8, int MB, int NB, int DEPTH, bool FUSED, bool SPLIT>
+// MERGED: the first half of the row blocks is side 0, the second side 1; else all are side 0.
+template <bool FP8, int MB, int NB, int DEPTH, bool FUSED, bool SPLIT, bool MERGED>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_stream_kernel(const StreamArgs p) {
   constexpr int THREADS = WAVES * 64;
@@ -63,6 +70,10 @@ gemm_stream_kernel(const StreamArgs p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tile = SPLIT ? blockIdx.x / p.split_k : blockIdx.x;
   const int part = SPLIT ? blockIdx.x - tile * p.split_k : 0;
+  // the side of row block i, and the first row of it there
+  constexpr int second = MERGED ? MB / 2 : MB;
+  auto side_of = [&](int i) -> const DfhipSide& { return p.side[i >= second]; };
+  auto row_of = [&](int i) { return 16 * (i >= second ? i - second : i); };
   const int n0 = tile * (16 * OB);
   const int slab0 = SPLIT ? (int)((int64_t)p.slabs * part / p.split_k) : 0;
   const int slabs = SPLIT ? (int)((int64_t)p.slabs * (part + 1) / p.split_k) - slab0 : p.slabs;
@@ -80,13 +91,15 @@ gemm_stream_kernel(const StreamArgs p) {
       w_ptr[j][h] = (FUSED && j >= OB ? p.W2 : p.W) + (int64_t)n * p.ldw + (slab0 + wave) * 128 + lchunk * 16;
     }
 #pragma unroll
-  for (int i = 0; i < MB; ++i)
+  for (int i = 0; i < MB; ++i) {
+    const DfhipSide& my = side_of(i);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      int m = 16 * i + 8 * h + lrow;
-      m = m < p.M ? m : p.M - 1;
-      a_ptr[i][h] = p.A + (int64_t)m * p.lda + (slab0 + wave) * 128 + lchunk * 16;
+      int m = row_of(i) + 8 * h + lrow;
+      m = m < my.M ? m : my.M - 1;
+      a_ptr[i][h] = static_cast<const uint8_t*>(my.A) + (int64_t)m * my.lda + (slab0 + wave) * 128 + lchunk * 16;
     }
+  }
   const int n_slabs = (slabs - wave + WAVES - 1) / WAVES;   // >= DEPTH: a part has at least MIN_SLABS slabs
 
   f32x4 acc[MB][NB];
@@ -171,8 +184,7 @@ gemm_stream_kernel(const StreamArgs p) {
   // The waves' sums meet in LDS, [wave][i][j][lane] with 16 bytes a lane; RI row blocks at a time, so that a workgroup
   // never asks for more than 64 KiB and a second one fits beside it (the launches of two nano-batches share the units).
   constexpr int RI = rows_per_round(MB, NB), ITEMS = RI * NB * 64;
-  float vmax = 0.0f;
-  const float sa = FP8 ? p.a_scale[0] : 1.0f;
+  float vmax[2] = {0.0f, 0.0f};
   auto total = [&](int i, int j, int l) {
     const f32x4* at = reinterpret_cast<const f32x4*>(smem) + (i * NB + j) * 64 + l;
     f32x4 v = at[0];
@@ -188,10 +200,12 @@ gemm_stream_kernel(const StreamArgs p) {
       for (int j = 0; j < NB; ++j) mine[(i * NB + j) * 64] = acc[i0 + i][j];
     __syncthreads();
   };
-  // W was the first operand: item (i, j, l) is row 16 i + l % 16, columns 16 j + 4 (l / 16) .. + 3
+  // W was the first operand: item (i, j, l) is row l % 16 of block i, columns 16 j + 4 (l / 16) .. + 3
   auto finish = [&](int i, int j, int l, f32x4 v, f32x4 u) {
-    const int m = 16 * i + (l & 15), n = n0 + 16 * j + 4 * (l >> 4);
-    if (m >= p.M || n >= p.N) return;            // N % 8 == 0: a run of four is inside or outside
+    const DfhipSide& my = side_of(i);
+    const int m = row_of(i) + (l & 15), n = n0 + 16 * j + 4 * (l >> 4);
+    if (m >= my.M || n >= p.N) return;           // N % 8 == 0: a run of four is inside or outside
+    const float sa = FP8 ? my.a_scale[0] : 1.0f;
     if (FP8) {
       const f32x4 ws = *reinterpret_cast<const f32x4*>(p.w_scale + n);
 #pragma unroll
@@ -214,20 +228,23 @@ gemm_stream_kernel(const StreamArgs p) {
           hi = bf16_hi_to_f32(s2);
         }
         o[h] = pack2_bf16(lo * bf16_lo_to_f32(up[h]), hi * bf16_hi_to_f32(up[h]));
-        if (FP8) vmax = fmaxf(vmax, fmaxf(fabsf(bf16_lo_to_f32(o[h])), fabsf(bf16_hi_to_f32(o[h]))));
+        if (FP8) {
+          const float top = fmaxf(fabsf(bf16_lo_to_f32(o[h])), fabsf(bf16_hi_to_f32(o[h])));
+          if (i >= second) vmax[1] = fmaxf(vmax[1], top); else vmax[0] = fmaxf(vmax[0], top);
+        }
       }
-    } else if (!FP8 && p.R) {
-      const u32x2 r = *reinterpret_cast<const u32x2*>(p.R + (int64_t)m * p.ldc + n);
+    } else if (!FP8 && my.R) {
+      const u32x2 r = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(my.R) + (int64_t)m * my.ldc + n);
       o[0] = add2_bf16(o[0], r[0]);
       o[1] = add2_bf16(o[1], r[1]);
     }
-    *reinterpret_cast<u32x2*>(p.C + (int64_t)m * p.ldc + n) = o;
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(my.C) + (int64_t)m * my.ldc + n) = o;
   };
 
   if constexpr (SPLIT) {
     // the parts of a tile meet in memory: each leaves its sums, the part that arrives last adds them in part order
     constexpr int BLOCK = MB * NB * 64 * 16;     // bytes of a part
-    f32x4* const all = reinterpret_cast<f32x4*>(p.partials) + (int64_t)tile * p.split_k * (MB * NB * 64);
+    f32x4* const all = reinterpret_cast<f32x4*>(p.side[0].partials) + (int64_t)tile * p.split_k * (MB * NB * 64);
     f32x4* const block = all + (int64_t)part * (MB * NB * 64);
 #pragma unroll
     for (int i0 = 0; i0 < MB; i0 += RI) {
@@ -243,10 +260,10 @@ gemm_stream_kernel(const StreamArgs p) {
     wait_vmcnt<0>();
     __syncthreads();
     int* const ticket_cell = reinterpret_cast<int*>(smem);
-    if (tid == 0) *ticket_cell = atomicAdd(p.arrivals + tile, 1);
+    if (tid == 0) *ticket_cell = atomicAdd(p.side[0].arrivals + tile, 1);
     __syncthreads();
     if (*ticket_cell != p.split_k - 1) return;
-    if (tid == 0) atomicExch(p.arrivals + tile, 0);
+    if (tid == 0) atomicExch(p.side[0].arrivals + tile, 0);
     const auto parts = coherent_blocks(all, p.split_k * BLOCK);
     for (int id = tid; id < MB * NB * 64; id += THREADS) {
       f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -277,20 +294,51 @@ gemm_stream_kernel(const StreamArgs p) {
     if (i0 + RI < MB) __syncthreads();
   }
   if constexpr (FP8 && FUSED) {
-    vmax = wave_max(vmax);
     // non-negative floats order like their bit patterns
-    if (lane == 0 && vmax > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(p.amax), __float_as_uint(vmax));
+#pragma unroll
+    for (int c = 0; c <= MERGED; ++c) {
+      const float top = wave_max(vmax[c]);
+      if (lane == 0 && top > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(p.side[c].amax), __float_as_uint(top));
+    }
   }
 }
 
-template <bool FP8, int MB, int NB, int DEPTH, bool FUSED, bool SPLIT>
-int launch(const StreamArgs& p, hipStream_t stream) {
-  auto kernel = gemm_stream_kernel<FP8, MB, NB, DEPTH, FUSED, SPLIT>;
-  constexpr int LDS = WAVES * rows_per_round(MB, NB) * NB * 1024;
+constexpr int stream_lds(int mb, int nb) { return WAVES * rows_per_round(mb, nb) * nb * 1024; }
+// Slabs in flight per wave: as many as 256 registers hold.  `width`: 16-column blocks of the output per workgroup.
+constexpr int stream_depth(int mb, int width) { return width == 1 ? (mb == 4 ? 2 : 4) : width == 2 && mb == 1 ? 4 : 2; }
+
+template <bool FP8, int MB, int WIDTH, bool FUSED, bool SPLIT, bool MERGED>
+constexpr auto stream_kernel =
+    gemm_stream_kernel<FP8, MB, (FUSED ? 2 : 1) * WIDTH, stream_depth(MB, WIDTH), FUSED, SPLIT, MERGED>;
+
+template <bool FP8, int MB, int WIDTH, bool FUSED, bool SPLIT, bool MERGED>
+int opt_in_stream() {
+  constexpr int LDS = stream_lds(MB, (FUSED ? 2 : 1) * WIDTH);
   static std::atomic<uint64_t> lds_opted_in{0};
-  if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), LDS, lds_opted_in)) return rc;
-  constexpr int COLS = 16 * (FUSED ? NB / 2 : NB);
-  hipLaunchKernelGGL(kernel, dim3((p.N + COLS - 1) / COLS * p.split_k), dim3(WAVES * 64), LDS, stream, p);
+  return dfhip_opt_in_lds(reinterpret_cast<const void*>(stream_kernel<FP8, MB, WIDTH, FUSED, SPLIT, MERGED>), LDS, lds_opted_in);
+}
+
+// Two launches of up to 16 MB rows are one of the kernel with twice the row blocks, on the tiles (and with them the order of
+// the sums) of the one.
+template <bool FP8, int MB, int WIDTH, bool FUSED, bool SPLIT>
+bool join_stream(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+  *joined = {reinterpret_cast<const void*>(stream_kernel<FP8, 2 * MB, WIDTH, FUSED, SPLIT, true>),
+             (unsigned)stream_lds(2 * MB, (FUSED ? 2 : 1) * WIDTH), grid};
+  return sides_stream(a, b, both) && opt_in_stream<FP8, 2 * MB, WIDTH, FUSED, SPLIT, true>() == DFHIP_OK;
+}
+
+template <bool FP8, int MB, int WIDTH, bool FUSED, bool SPLIT>
+int launch(const StreamArgs& p, hipStream_t stream) {
+  const auto kernel = stream_kernel<FP8, MB, WIDTH, FUSED, SPLIT, false>;
+  if (int rc = opt_in_stream<FP8, MB, WIDTH, FUSED, SPLIT, false>()) return rc;
+  if constexpr (MB <= 2) {
+    static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof p,
+                                              join_stream<FP8, MB, WIDTH, FUSED, SPLIT>), true);
+    (void)known;
+  }
+  constexpr int COLS = 16 * WIDTH;
+  hipLaunchKernelGGL(kernel, dim3((p.N + COLS - 1) / COLS * p.split_k), dim3(WAVES * 64),
+                     stream_lds(MB, (FUSED ? 2 : 1) * WIDTH), stream, p);
   return dfhip_check_launch();
 }
 
@@ -299,19 +347,17 @@ constexpr int MIN_SLABS = 4 * WAVES;
 
 template <bool FP8, int MB, bool FUSED, bool SPLIT>
 int launch_width(const StreamArgs& p, int width, hipStream_t stream) {
-  constexpr int F = FUSED ? 2 : 1;
-  constexpr int D1 = MB == 4 ? 2 : 4;            // as many slabs in flight as 256 registers hold
   switch (width) {
-    case 1: return launch<FP8, MB, F, D1, FUSED, SPLIT>(p, stream);
-    case 2: return launch<FP8, MB, 2 * F, MB == 1 ? 4 : 2, FUSED, SPLIT>(p, stream);
-    default: return launch<FP8, MB, 4 * F, 2, FUSED, SPLIT>(p, stream);
+    case 1: return launch<FP8, MB, 1, FUSED, SPLIT>(p, stream);
+    case 2: return launch<FP8, MB, 2, FUSED, SPLIT>(p, stream);
+    default: return launch<FP8, MB, 4, FUSED, SPLIT>(p, stream);
   }
 }
 
 template <bool FP8, bool FUSED, bool SPLIT>
 int launch_rows(const StreamArgs& p, int width, hipStream_t stream) {
-  if (p.M <= 16) return launch_width<FP8, 1, FUSED, SPLIT>(p, width, stream);
-  if (p.M <= 32) return launch_width<FP8, 2, FUSED, SPLIT>(p, width, stream);
+  if (p.side[0].M <= 16) return launch_width<FP8, 1, FUSED, SPLIT>(p, width, stream);
+  if (p.side[0].M <= 32) return launch_width<FP8, 2, FUSED, SPLIT>(p, width, stream);
   if constexpr (!FP8 && (FUSED || SPLIT)) return DFHIP_ERR_BAD_SHAPE;   // bf16: whole K alone, by variant
   else return launch_width<FP8, 4, FUSED, SPLIT>(p, width, stream);
 }
@@ -366,30 +412,26 @@ int dfhip_stream_split(int M, int N, int64_t k_bytes) {
 
 int dfhip_stream_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const void* R, void* C, int64_t ldc, int M,
                       int N, int K, int split_k, void* partials, int* arrivals, hipStream_t stream) {
-  const StreamArgs p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), nullptr,
-                     static_cast<const uint16_t*>(R), static_cast<uint16_t*>(C), nullptr, nullptr, nullptr, nullptr, M, N,
-                     K / 64, split_k, static_cast<float*>(partials), arrivals, lda * 2, ldw * 2, ldc};
+  const StreamArgs p{static_cast<const uint8_t*>(W), nullptr, nullptr, nullptr, N, K / 64, split_k, ldw * 2,
+                     {{A, R, C, nullptr, nullptr, static_cast<float*>(partials), arrivals, lda * 2, ldc, M}, {}}};
   return dispatch<false, false>(p, stream);
 }
 int dfhip_stream_bf16_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                               int M, int N, int K, hipStream_t stream) {
-  const StreamArgs p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2),
-                     nullptr, static_cast<uint16_t*>(C), nullptr, nullptr, nullptr, nullptr, M, N, K / 64, 1, nullptr,
-                     nullptr, lda * 2, ldw * 2, ldc};
+  const StreamArgs p{static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), nullptr, nullptr, N, K / 64, 1, ldw * 2,
+                     {{A, nullptr, C, nullptr, nullptr, nullptr, nullptr, lda * 2, ldc, M}, {}}};
   return dispatch<false, true>(p, stream);
 }
 int dfhip_stream_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
                      const float* w_scale, int M, int N, int K, hipStream_t stream) {
-  const StreamArgs p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), nullptr, nullptr,
-                     static_cast<uint16_t*>(C), a_scale, w_scale, nullptr, nullptr, M, N, K / 128, 1, nullptr, nullptr, lda,
-                     ldw, ldc};
+  const StreamArgs p{static_cast<const uint8_t*>(W), nullptr, w_scale, nullptr, N, K / 128, 1, ldw,
+                     {{A, nullptr, C, a_scale, nullptr, nullptr, nullptr, lda, ldc, M}, {}}};
   return dispatch<true, false>(p, stream);
 }
 int dfhip_stream_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                              const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, int M, int N,
                              int K, hipStream_t stream) {
-  const StreamArgs p{static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2),
-                     nullptr, static_cast<uint16_t*>(C), a_scale, w_scale, w2_scale, amax, M, N, K / 128, 1, nullptr,
-                     nullptr, lda, ldw, ldc};
+  const StreamArgs p{static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), w_scale, w2_scale, N, K / 128, 1, ldw,
+                     {{A, nullptr, C, a_scale, amax, nullptr, nullptr, lda, ldc, M}, {}}};
   return dispatch<true, true>(p, stream);
 }

@@ -1,0 +1,184 @@
+// Pairs the launches of two nano-batches in a captured schedule (host code).
+//
+// A schedule that gives every nano-batch a stream of its own launches each projection once per nano-batch, side by side.
+// With few rows a launch is the time its weights take to arrive, and both launches fetch all of them: what reaches the XCDs
+// from memory and the memory-side cache stays at 6 - 7 TB/s however many ask, while what two workgroups of one XCD read
+// together comes at 10 - 12 TB/s.  But the two launches start some 10 us apart, the second one on other XCDs (a queue deals its
+// workgroups on from where it stopped), and whoever is behind never catches up.  So they become one launch, whose workgroups
+// multiply a weight with the rows of both (up to 32 rows each that stream their weights, up to 64 on tiles), or in which the
+// two workgroups that read the same weights sit on the same XCD and start together (pair_block).
+// [us, in a graph: 128 MB read by two launches 39 - 43, by one launch twice 24; layer of 2 x 48 tokens 126 / 90, of 2 x 12 in
+// fp8 254 / 187]
+//
+// Where every launch of a graph is one of a pair or short, nothing is left that gains from running side by side: the graph
+// becomes a chain, which saves the meetings of two queues (6 - 10 us each).  Any other graph stays as it is.  Attention
+// over a cache leaves the chip to others when its workgroups run out unevenly, and the chain has no others: it counts as
+// short up to a workgroup per compute unit.  [us of a step of 4 layers, sequences of 1/4 .. 1 of 4096 positions, two streams /
+// chain: 16 sequences 814 / 620, 40 1034 / 916, 64 1228 / 1124; 72, 288 workgroups each, 1281 / 1407, 128 1652 / 1719]
+#include <algorithm>
+#include <mutex>
+#include <unordered_map>
+#include <vector>
+
+#include "dfhip_pairs.h"
+
+namespace {
+
+constexpr unsigned SHORT_BLOCKS = 512;   // workgroups of a launch that may as well run in line, if its kernel gives no number
+
+struct Known {
+  size_t bytes = 0;
+  DfhipJoin join = nullptr;
+  unsigned in_line = SHORT_BLOCKS;
+};
+std::mutex known_mutex;
+std::unordered_map<const void*, Known>& known_kernels() {
+  static std::unordered_map<const void*, Known> kernels;
+  return kernels;
+}
+Known find_known(const void* kernel) {
+  std::lock_guard<std::mutex> guard(known_mutex);
+  const auto it = known_kernels().find(kernel);
+  return it == known_kernels().end() ? Known{} : it->second;
+}
+
+struct Node {
+  hipGraphNode_t handle;
+  bool kernel;
+  hipKernelNodeParams params;
+  Known known;
+  int pair = -1;                         // the other node of its pair
+};
+
+bool same(const dim3& a, const dim3& b) { return a.x == b.x && a.y == b.y && a.z == b.z; }
+
+// A topological order of the graph whose paired nodes are one (named by the smaller index), smallest index first; empty if
+// there is none.
+std::vector<int> order_of(const std::vector<Node>& nodes, const std::vector<std::pair<int, int>>& edges) {
+  const int n = (int)nodes.size();
+  auto name = [&](int i) { return nodes[i].pair >= 0 && nodes[i].pair < i ? nodes[i].pair : i; };
+  std::vector<std::vector<int>> next(n);
+  std::vector<int> waits(n, 0), order;
+  for (const auto& e : edges) {
+    const int a = name(e.first), b = name(e.second);
+    if (a == b) return {};
+    next[a].push_back(b);
+    ++waits[b];
+  }
+  std::vector<bool> done(n, false);
+  for (;;) {
+    int at = -1;
+    for (int i = 0; i < n && at < 0; ++i)
+      if (name(i) == i && !done[i] && waits[i] == 0) at = i;
+    if (at < 0) break;
+    done[at] = true;
+    order.push_back(at);
+    for (int b : next[at]) --waits[b];
+  }
+  for (int i = 0; i < n; ++i)
+    if (name(i) == i && !done[i]) return {};
+  return order;
+}
+
+}  // namespace
+
+void dfhip_pairable(const void* kernel, size_t bytes, DfhipJoin join) {
+  std::lock_guard<std::mutex> guard(known_mutex);
+  known_kernels()[kernel] = {bytes, bytes <= DFHIP_PAIR_MAX_ARGS ? join : nullptr, SHORT_BLOCKS};
+}
+
+void dfhip_in_line(const void* kernel, unsigned blocks) {
+  std::lock_guard<std::mutex> guard(known_mutex);
+  known_kernels()[kernel].in_line = blocks;
+}
+
+extern "C" int dfhip_graph_pair_launches(void* graph, int* pairs) {
+  if (!graph || !pairs) return DFHIP_ERR_NULL_POINTER;
+  *pairs = 0;
+  hipGraph_t g = static_cast<hipGraph_t>(graph);
+  size_t count = 0, edge_count = 0;
+  if (hipGraphGetNodes(g, nullptr, &count) != hipSuccess || hipGraphGetEdges(g, nullptr, nullptr, &edge_count) != hipSuccess)
+    return DFHIP_ERR_LAUNCH;
+  if (count < 2 || count > 2048) return DFHIP_OK;
+  std::vector<hipGraphNode_t> handles(count), from(edge_count), to(edge_count);
+  if (hipGraphGetNodes(g, handles.data(), &count) != hipSuccess) return DFHIP_ERR_LAUNCH;
+  if (edge_count && hipGraphGetEdges(g, from.data(), to.data(), &edge_count) != hipSuccess) return DFHIP_ERR_LAUNCH;
+
+  std::unordered_map<hipGraphNode_t, int> index;
+  std::vector<Node> nodes(count);
+  for (size_t i = 0; i < count; ++i) {
+    Node& node = nodes[i];
+    node.handle = handles[i];
+    index[handles[i]] = (int)i;
+    hipGraphNodeType type;
+    if (hipGraphNodeGetType(handles[i], &type) != hipSuccess) return DFHIP_ERR_LAUNCH;
+    node.kernel = type == hipGraphNodeTypeKernel;
+    if (type == hipGraphNodeTypeEmpty) continue;
+    if (!node.kernel) return DFHIP_OK;
+    if (hipGraphKernelNodeGetParams(handles[i], &node.params) != hipSuccess) return DFHIP_ERR_LAUNCH;
+    const dim3& grid = node.params.gridDim;
+    node.known = find_known(node.params.func);
+    if (node.known.join ? !node.params.kernelParams : (size_t)grid.x * grid.y * grid.z > node.known.in_line) return DFHIP_OK;
+  }
+  std::vector<std::pair<int, int>> edges(edge_count);
+  const size_t words = (count + 63) / 64;
+  std::vector<uint64_t> paths(count * words, 0);                     // bit j of row i: a path from node i to node j
+  auto reaches = [&](size_t i, size_t j) { return (paths[i * words + j / 64] >> (j % 64)) & 1; };
+  for (size_t e = 0; e < edge_count; ++e) {
+    edges[e] = {index[from[e]], index[to[e]]};
+    paths[edges[e].first * words + edges[e].second / 64] |= (uint64_t)1 << (edges[e].second % 64);
+  }
+  for (size_t k = 0; k < count; ++k)
+    for (size_t i = 0; i < count; ++i)
+      if (reaches(i, k))
+        for (size_t w = 0; w < words; ++w) paths[i * words + w] |= paths[k * words + w];
+
+  alignas(16) unsigned char both[DFHIP_PAIR_MAX_ARGS];
+  DfhipJoined joined;
+  int found = 0;
+  for (size_t i = 0; i < count; ++i) {
+    Node& a = nodes[i];
+    if (!a.kernel || !a.known.join || a.pair >= 0) continue;
+    for (size_t j = i + 1; j < count && a.pair < 0; ++j) {
+      Node& b = nodes[j];
+      if (!b.kernel || b.pair >= 0 || b.params.func != a.params.func || reaches(i, j) || reaches(j, i)) continue;
+      if (!same(a.params.gridDim, b.params.gridDim) || !same(a.params.blockDim, b.params.blockDim)) continue;
+      if (a.params.sharedMemBytes != b.params.sharedMemBytes) continue;
+      if (!a.known.join(a.params.kernelParams[0], b.params.kernelParams[0], a.params.gridDim.x, both, &joined)) continue;
+      a.pair = (int)j;
+      b.pair = (int)i;
+      ++found;
+    }
+    if (a.pair < 0) return DFHIP_OK;                                  // a launch that would lose its company
+  }
+  if (!found) return DFHIP_OK;
+  const std::vector<int> order = order_of(nodes, edges);
+  if (order.empty()) return DFHIP_OK;                                 // two pairs that wait for each other crosswise
+
+  // from here on the graph changes; a failure leaves it useless, and the caller with an error
+  if (edge_count && hipGraphRemoveDependencies(g, from.data(), to.data(), edge_count) != hipSuccess) return DFHIP_ERR_LAUNCH;
+  hipGraphNode_t last = nullptr;
+  for (int i : order) {
+    Node& node = nodes[i];
+    if (!node.kernel) {
+      if (hipGraphDestroyNode(node.handle) != hipSuccess) return DFHIP_ERR_LAUNCH;
+      continue;
+    }
+    if (node.pair >= 0) {
+      Node& other = nodes[node.pair];
+      if (!node.known.join(node.params.kernelParams[0], other.params.kernelParams[0], node.params.gridDim.x, both, &joined)) return DFHIP_ERR_LAUNCH;
+      hipKernelNodeParams params = node.params;
+      void* args[1] = {both};
+      params.kernelParams = args;
+      params.func = const_cast<void*>(joined.kernel);
+      params.gridDim.x = joined.grid;
+      params.sharedMemBytes = joined.lds;
+      if (hipGraphKernelNodeSetParams(node.handle, &params) != hipSuccess) return DFHIP_ERR_LAUNCH;
+      if (hipGraphDestroyNode(other.handle) != hipSuccess) return DFHIP_ERR_LAUNCH;
+    }
+    if (last && hipGraphAddDependencies(g, &last, &node.handle, 1) != hipSuccess) return DFHIP_ERR_LAUNCH;
+    last = node.handle;
+  }
+  *pairs = found;
+  return DFHIP_OK;
+}

@@ -21,6 +21,7 @@ scheduler and all launches.
 """
 from __future__ import annotations
 
+import ctypes
 import logging
 import os
 import tempfile
@@ -30,6 +31,7 @@ from typing import Any
 
 import torch
 
+from dynaflow_amd._cabi import KernelError, check, load
 from dynaflow_amd.config import DynaFlowConfig
 from dynaflow_amd.executor.compiler import SubgraphCompiler
 from dynaflow_amd.interface import ExecutionContext, InputInfo, OpSchedulerBase, SplitConfig
@@ -104,6 +106,14 @@ def join_results(results: dict[int, Any], num_nano_batches: int, shared_buffer: 
     return first
 
 
+def _pair_launches(graph: torch.cuda.CUDAGraph) -> int:
+    """Launches of two nano-batches against the same weights become one, where the whole schedule consists of such
+    (dfhip_graph_pair_launches); how many did."""
+    pairs = ctypes.c_int(0)
+    check("dfhip_graph_pair_launches", load().dfhip_graph_pair_launches(graph.raw_cuda_graph(), ctypes.byref(pairs)))
+    return pairs.value
+
+
 class _ScheduleGraph:
     """One captured forward: the graph, the tensors it reads and its output."""
 
@@ -128,6 +138,8 @@ class DynaFlowManager:
         self._schedule_graphs: dict[tuple, _ScheduleGraph] = {}
         #: per captured schedule: "caller" (captured from the caller's side) or "schedule" (from one of its streams)
         self.capture_origins: dict[tuple, str] = {}
+        #: per captured schedule: how many pairs of launches against the same weights became one launch
+        self.paired_launches: dict[tuple, int] = {}
 
     # ------------------------------------------------------------ set-up
     def initialize(
@@ -333,12 +345,22 @@ class DynaFlowManager:
                     "per-sub-graph graphs (CUDAGraphConfig(enabled=True)) or the eager schedule"
                 )
             torch.cuda.current_stream().synchronize()
-            graph = torch.cuda.CUDAGraph()
             # captured from the caller's side (torch's own capture stream) when that is safe, else from the
             # stream of the schedule that the others meet at
             capture_on = {} if origin == caller else {"stream": device.streams_seen[origin]}
-            with torch.cuda.graph(graph, **capture_on):
-                output = run_coroutine(self._forward_async(args, kwargs, eager_split))
+            for pairing in (bool(self.config.knob("pair_launches", True)), False):
+                graph = torch.cuda.CUDAGraph(keep_graph=True)
+                with torch.cuda.graph(graph, **capture_on):
+                    output = run_coroutine(self._forward_async(args, kwargs, eager_split))
+                self.paired_launches[key] = 0
+                if not pairing:
+                    break
+                try:
+                    self.paired_launches[key] = _pair_launches(graph)
+                    break
+                except KernelError as error:     # the graph may be half changed: the schedule once more, as it is
+                    log.warning("captured launches were not paired: %s", error)
+            graph.instantiate()
             self.capture_origins[key] = "caller" if origin == caller else "schedule"
             entry = _ScheduleGraph(graph, list(args), self._token_shaped_flags(args), output)
             self._schedule_graphs[key] = entry

@@ -458,6 +458,14 @@ int dfhip_requant_fp8_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int
  * captured graph is fine, dynaflow/executor/cudagraph.py:84-122 captures whatever the callable issues). */
 int dfhip_fill_u32(void* dst, uint32_t value, int64_t count, dfhip_stream_t stream);
 
+/* ---- captured schedules --------------------------------------------------------------------------
+ * `graph`: a hipGraph_t that has not been instantiated.  Where every kernel in it is one of two launches of up to 128
+ * rows against the same weights that do not depend on each other (a projection of two nano-batches), or a short
+ * quantisation, each two become one launch whose workgroups read a weight together, and the graph a chain of
+ * what is left, in an order that its edges allow.  Any other graph stays as it is.  *pairs: the launches that
+ * were joined.  Same results.  A negative status: the graph is of no use any more. */
+int dfhip_graph_pair_launches(void* graph, int* pairs);
+
 #ifdef __cplusplus
 }
 #endif

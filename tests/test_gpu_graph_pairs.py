@@ -1,0 +1,103 @@
+"""Launches of two nano-batches against the same weights as one, in a schedule captured as one graph: every replay has the bits
+of the eager schedule, and a schedule that is not all of such launches is left as it is."""
+import ctypes
+
+import pytest
+import torch
+
+from dynaflow_amd import _cabi
+from dynaflow_amd.backend import make_backend
+from dynaflow_amd.config import CUDAGraphConfig, DynaFlowConfig, InductorConfig
+from dynaflow_amd.fp8_mlp import Fp8SwiGLU
+from dynaflow_amd.manager import DynaFlowManager
+from dynaflow_amd.mlp import SwiGLUMLP
+
+
+def test_arguments():
+    pairs = ctypes.c_int(5)
+    assert _cabi.load().dfhip_graph_pair_launches(None, ctypes.byref(pairs)) == -1
+    assert _cabi.load().dfhip_graph_pair_launches(16, None) == -1
+
+
+def randn(shape, seed, std=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randn(shape, generator=g, device="cuda") * std).bfloat16()
+
+
+def program(model, tokens, **knobs):
+    manager = DynaFlowManager()
+    cfg = DynaFlowConfig("dynaflow_amd.schedulers:MLPOverlapScheduler", 4, InductorConfig(enabled=True),
+                         CUDAGraphConfig(enabled=False, capture_sizes=[tokens]),
+                         {"min_nano_split_tokens": 1, "num_nano_batches": 2, "dump_graph": False, "whole_graph": True,
+                          "streams": "by_nano_batch", "fuse_silu_epilogue": True, **knobs})
+    x = randn((tokens, model.hidden), 1)
+    torch._dynamo.mark_dynamic(x, 0)
+    torch._dynamo.reset()
+    compiled = torch.compile(model, backend=make_backend(manager, cfg), fullgraph=True)
+    with torch.no_grad():
+        manager.prepare(tokens, [tokens])
+        compiled(x)
+    return manager, compiled
+
+
+def forward(manager, compiled, x, graph):
+    with torch.no_grad():
+        manager.prepare(len(x), [1] * len(x), use_cudagraph=graph)
+        return compiled(x)
+
+
+def mlp(kind, hidden, inter):
+    weights = randn((inter, hidden), 2, 0.03), randn((inter, hidden), 3, 0.03), randn((hidden, inter), 4, 0.03)
+    if kind == "fp8":
+        model = Fp8SwiGLU.from_weights(*weights, fuse_gate_up=True)
+    else:
+        model = SwiGLUMLP(hidden, inter, dtype=torch.bfloat16, device="cuda")
+        with torch.no_grad():
+            for layer, w in zip((model.gate_proj, model.up_proj, model.down_proj), weights):
+                layer.weight.copy_(w)
+    model.hidden = hidden
+    return model
+
+
+# separate gate and up projections pair like the fused one: their product is a short launch
+@pytest.mark.gpu
+def test_short_launches_between_pairs():
+    manager, compiled = program(mlp("bf16", 2048, 5632), 64, fuse_silu_epilogue=False)
+    x = randn((64, 2048), 5)
+    want = forward(manager, compiled, x, False).clone()
+    for _ in range(3):
+        assert torch.equal(forward(manager, compiled, x, True), want)
+    assert list(manager.paired_launches.values()) == [2]
+
+
+# streamed weights; rows of the two nano-batches that differ; tiles of 64 and 128 rows; a grid that is no multiple of eight
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,tokens,hidden,inter", [
+    ("bf16", 2, 2048, 5632), ("bf16", 25, 2048, 5696), ("bf16", 64, 4096, 14336), ("bf16", 96, 2048, 5696),
+    ("bf16", 255, 4096, 14336), ("fp8", 24, 4096, 14336), ("fp8", 29, 2048, 5760), ("fp8", 80, 8192, 8192),
+    ("fp8", 190, 4096, 14336)])
+def test_paired_replays_have_the_bits_of_the_eager_schedule(kind, tokens, hidden, inter):
+    manager, compiled = program(mlp(kind, hidden, inter), tokens)
+    x = randn((tokens, hidden), 5)
+    forward(manager, compiled, x, True)
+    assert list(manager.paired_launches.values()) == [2], manager.paired_launches
+    for seed in (6, 7, 8):
+        x = randn((tokens, hidden), seed, 2.0 ** (seed - 6))
+        want = forward(manager, compiled, x, False).clone()
+        torch.cuda.synchronize()
+        for _ in range(2):
+            got = forward(manager, compiled, x, True)
+            assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,knobs", [(64, {"streams": "by_kind"}), (64, {"pair_launches": False}), (1024, {}),
+                                          (96, {"num_nano_batches": 3})])
+def test_other_schedules_stay_as_they_are(tokens, knobs):
+    """One stream per kind (a launch waits for the other), switched off, many rows, a launch without a partner."""
+    manager, compiled = program(mlp("bf16", 2048, 5632), tokens, **knobs)
+    x = randn((tokens, 2048), 5)
+    want = forward(manager, compiled, x, False).clone()
+    for _ in range(3):
+        assert torch.equal(forward(manager, compiled, x, True), want)
+    assert list(manager.paired_launches.values()) == [0]
