@@ -106,6 +106,10 @@ def join_results(results: dict[int, Any], num_nano_batches: int, shared_buffer: 
     return first
 
 
+#: Rows of a nano-batch up to which two of its launches may become one (DFHIP_PAIR_MAX_M).
+PAIR_MAX_ROWS = 128
+
+
 def _pair_launches(graph: torch.cuda.CUDAGraph) -> int:
     """Launches of two nano-batches against the same weights become one, where the whole schedule consists of such
     (dfhip_graph_pair_launches); how many did."""
@@ -138,6 +142,7 @@ class DynaFlowManager:
         self._schedule_graphs: dict[tuple, _ScheduleGraph] = {}
         #: per captured schedule: "caller" (captured from the caller's side) or "schedule" (from one of its streams)
         self.capture_origins: dict[tuple, str] = {}
+        self._side_by_side: int | None = None     # instead of launches_side_by_side while a schedule is captured in pairs
         #: per captured schedule: how many pairs of launches against the same weights became one launch
         self.paired_launches: dict[tuple, int] = {}
 
@@ -245,7 +250,7 @@ class DynaFlowManager:
         assert split is not None
         from dynaflow_amd import ops
 
-        with ops.launch_options(side_by_side=self.launches_side_by_side(split)):
+        with ops.launch_options(side_by_side=self._side_by_side or self.launches_side_by_side(split)):
             if split.is_dryrun:
                 results, events = self.engine.dryrun(args, kwargs, split)
             else:
@@ -292,6 +297,58 @@ class DynaFlowManager:
         return asked
 
     # ------------------------------------------------- whole-schedule graphs
+    def _logged_pass(self, args: tuple, kwargs: dict, split: SplitConfig) -> list:
+        """An eager pass before a capture: lazy one-time set-up (kernel attributes, allocator growth) must not happen
+        under capture, and the event log says from which stream the schedule can be captured."""
+        device = get_device()
+        device.trace = []
+        try:
+            run_coroutine(self._forward_async(args, kwargs, split))
+        finally:
+            event_log, device.trace = device.trace, None
+        return event_log
+
+    def _capture(self, args: tuple, kwargs: dict, split: SplitConfig, capture_on: dict) -> tuple:
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, **capture_on):
+            output = run_coroutine(self._forward_async(args, kwargs, split))
+        return graph, output
+
+    def _capture_paired(self, args: tuple, kwargs: dict, split: SplitConfig, caller, origin, capture_on: dict) -> tuple:
+        """The schedule with the launches of two nano-batches against the same weights as one: (graph, output, pairs);
+        the graph is None where nothing is to be gained by pairs or it failed half-way.
+
+        Streams by kind order the launches of a kind, and only a stream per nano-batch tells which of them need not wait
+        for each other.  What becomes a chain of paired launches has no use for either policy, so it is captured with the
+        latter, and with the kernels that the schedule's own policy plans.  [us, a decode step of 4 layers
+        by kind / in pairs: 8 sequences of 512 positions 711 / 496, 40 of 4096 1177 / 918, 64 of 4096 1410 / 1122; fp8 layer
+        of 2 x 50 tokens 373 / 254]"""
+        assert self.config is not None and self.scheduler is not None
+        policy = getattr(self.scheduler, "stream_policy", None)
+        one_stream = getattr(self.scheduler, "comp_stream", None) is getattr(self.scheduler, "comm_stream", None)
+        if not self.config.knob("pair_launches", True) or self.config.knob("cu_split", None) or one_stream:
+            return None, None, 0
+        if policy == "by_nano_batch":
+            graph, output = self._capture(args, kwargs, split, capture_on)
+        elif policy == "by_kind" and split.num_nano_batches == 2 and max(split.num_tokens) <= PAIR_MAX_ROWS:
+            self._side_by_side = self.launches_side_by_side(split)
+            self.scheduler.stream_policy = "by_nano_batch"
+            try:
+                if capture_plan.join_cycle(self._logged_pass(args, kwargs, split), caller, origin) is not None:
+                    return None, None, 0
+                torch.cuda.current_stream().synchronize()
+                graph, output = self._capture(args, kwargs, split, capture_on)
+            finally:
+                self.scheduler.stream_policy, self._side_by_side = policy, None
+        else:
+            return None, None, 0
+        try:
+            pairs = _pair_launches(graph)
+        except KernelError as error:     # the graph may be half changed
+            log.warning("captured launches were not paired: %s", error)
+            return None, None, 0
+        return (graph, output, pairs) if pairs or policy == "by_nano_batch" else (None, None, 0)
+
     def _wants_whole_graph(self, split: SplitConfig) -> bool:
         assert self.config is not None
         return (
@@ -328,14 +385,7 @@ class DynaFlowManager:
         )
         entry = self._schedule_graphs.get(key)
         if entry is None:
-            # one eager pass first: lazy one-time set-up (kernel attributes, allocator growth) must not
-            # happen under capture; its event log says from which stream the schedule can be captured
-            device = get_device()
-            device.trace = []
-            try:
-                run_coroutine(self._forward_async(args, kwargs, eager_split))
-            finally:
-                event_log, device.trace = device.trace, None
+            event_log = self._logged_pass(args, kwargs, eager_split)
             caller = stream_key(torch.cuda.current_stream())
             origin = capture_plan.choose_origin(event_log, caller)
             if origin is None:
@@ -347,20 +397,12 @@ class DynaFlowManager:
             torch.cuda.current_stream().synchronize()
             # captured from the caller's side (torch's own capture stream) when that is safe, else from the
             # stream of the schedule that the others meet at
-            capture_on = {} if origin == caller else {"stream": device.streams_seen[origin]}
-            for pairing in (bool(self.config.knob("pair_launches", True)), False):
-                graph = torch.cuda.CUDAGraph(keep_graph=True)
-                with torch.cuda.graph(graph, **capture_on):
-                    output = run_coroutine(self._forward_async(args, kwargs, eager_split))
-                self.paired_launches[key] = 0
-                if not pairing:
-                    break
-                try:
-                    self.paired_launches[key] = _pair_launches(graph)
-                    break
-                except KernelError as error:     # the graph may be half changed: the schedule once more, as it is
-                    log.warning("captured launches were not paired: %s", error)
+            capture_on = {} if origin == caller else {"stream": get_device().streams_seen[origin]}
+            graph, output, pairs = self._capture_paired(args, kwargs, eager_split, caller, origin, capture_on)
+            if graph is None:
+                graph, output = self._capture(args, kwargs, eager_split, capture_on)
             graph.instantiate()
+            self.paired_launches[key] = pairs
             self.capture_origins[key] = "caller" if origin == caller else "schedule"
             entry = _ScheduleGraph(graph, list(args), self._token_shaped_flags(args), output)
             self._schedule_graphs[key] = entry

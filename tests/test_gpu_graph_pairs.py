@@ -59,10 +59,13 @@ def mlp(kind, hidden, inter):
     return model
 
 
-# separate gate and up projections pair like the fused one: their product is a short launch
+# separate gate and up projections pair like the fused one: their product is a short launch; and streams by kind, whose
+# order of the launches of a kind is nobody's need
 @pytest.mark.gpu
-def test_short_launches_between_pairs():
-    manager, compiled = program(mlp("bf16", 2048, 5632), 64, fuse_silu_epilogue=False)
+@pytest.mark.parametrize("knobs", [{"fuse_silu_epilogue": False}, {"streams": "by_kind"},
+                                   {"streams": "by_kind", "fuse_silu_epilogue": False}])
+def test_short_launches_between_pairs_and_streams_by_kind(knobs):
+    manager, compiled = program(mlp("bf16", 2048, 5632), 64, **knobs)
     x = randn((64, 2048), 5)
     want = forward(manager, compiled, x, False).clone()
     for _ in range(3):
@@ -91,10 +94,11 @@ def test_paired_replays_have_the_bits_of_the_eager_schedule(kind, tokens, hidden
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tokens,knobs", [(64, {"streams": "by_kind"}), (64, {"pair_launches": False}), (1024, {}),
-                                          (96, {"num_nano_batches": 3})])
+@pytest.mark.parametrize("tokens,knobs", [(64, {"pair_launches": False}), (64, {"streams": "by_kind", "pair_launches": False}),
+                                          (64, {"streams": "by_kind", "serialize": True}), (1024, {}),
+                                          (1024, {"streams": "by_kind"}), (96, {"num_nano_batches": 3})])
 def test_other_schedules_stay_as_they_are(tokens, knobs):
-    """One stream per kind (a launch waits for the other), switched off, many rows, a launch without a partner."""
+    """Switched off, one stream, many rows, a launch without a partner."""
     manager, compiled = program(mlp("bf16", 2048, 5632), tokens, **knobs)
     x = randn((tokens, 2048), 5)
     want = forward(manager, compiled, x, False).clone()
