@@ -138,7 +138,7 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, _P, _P],
     ),
-    "dfhip_graph_pair_launches": (c_int, [_P, ctypes.POINTER(c_int)]),
+    "dfhip_graph_pair_launches": (c_int, [_P, c_int, ctypes.POINTER(c_int)]),
     "dfhip_fill_u32": (c_int, [_P, c_uint32, c_int64, _P]),
 }
 

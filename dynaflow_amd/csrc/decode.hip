@@ -74,13 +74,12 @@ DFHIP_DEVICE int sequence_parts(int len, int parts) {
 // its unnormalised sums, maximum and sum of exponentials in `partials` ([pair][part][part_block(group)] words of 16
 // bytes), counts itself in and is done; the part that arrives last combines them, in the same order whoever that is.
 template <bool APPEND, bool SPLIT>
-__global__ void __launch_bounds__(DEC_THREADS)
-decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* __restrict__ kc,
-                        uint16_t* __restrict__ vc, const int32_t* __restrict__ slots,
-                        const int32_t* __restrict__ lengths, uint16_t* __restrict__ out, int64_t ld_out,
-                        int kv_heads, int group, int num_slots, int capacity, float scale_log2,
-                        const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table_rows, int parts,
-                        float* __restrict__ partials, int* __restrict__ arrivals) {
+DFHIP_DEVICE void decode_attention(int pair, const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* __restrict__ kc,
+                                   uint16_t* __restrict__ vc, const int32_t* __restrict__ slots,
+                                   const int32_t* __restrict__ lengths, uint16_t* __restrict__ out, int64_t ld_out,
+                                   int kv_heads, int group, int num_slots, int capacity, float scale_log2,
+                                   const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table_rows,
+                                   int parts, float* __restrict__ partials, int* __restrict__ arrivals) {
   // partial results of the four waves, sized by the launch for the real group (a workgroup that asks for
   // little LDS leaves room for a GEMM workgroup of the other nano-batch on the same CU)
   extern __shared__ __attribute__((aligned(16))) float combine_lds[];
@@ -90,7 +89,6 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
   // Part-major: the parts that every sequence uses are dispatched first and lie on all XCDs.  (Pair-major, the only
   // workgroups with work of 8 short sequences are every eighth one, on one XCD: 512 positions 20.2 us, so 12.2.)
   const int part = SPLIT ? blockIdx.y : 0;
-  const int pair = blockIdx.x;
   const int t = pair / kv_heads, kvh = pair - t * kv_heads;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hq = lane & 15, g = lane >> 4;
@@ -383,6 +381,43 @@ decode_attention_kernel(const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* 
   }
 }
 
+struct DecodeAttention {
+  const uint16_t* q;
+  uint16_t *kc, *vc;
+  const int32_t *slots, *lengths;
+  uint16_t* out;
+  const float *cos_t, *sin_t;
+  float* partials;
+  int* arrivals;
+  int64_t ld_q, ld_out;
+  int kv_heads, group, num_slots, capacity, table_rows, parts;
+  float scale_log2;
+};
+template <bool APPEND, bool SPLIT>
+struct DecodeAttentionOf : DecodeAttention {
+  static constexpr int THREADS = DEC_THREADS;
+  DFHIP_DEVICE void run(unsigned block, unsigned) const {
+    decode_attention<APPEND, SPLIT>(block, q, ld_q, kc, vc, slots, lengths, out, ld_out, kv_heads, group, num_slots, capacity,
+                                    scale_log2, cos_t, sin_t, table_rows, parts, partials, arrivals);
+  }
+  bool beside(const DecodeAttentionOf& other) const {
+    return kc == other.kc && vc == other.vc && out != other.out && (!SPLIT || arrivals != other.arrivals);
+  }
+};
+template <bool APPEND, bool SPLIT>
+__global__ void __launch_bounds__(DEC_THREADS) decode_attention_kernel(const DecodeAttentionOf<APPEND, SPLIT> p) {
+  p.run(blockIdx.x, gridDim.x);
+}
+template <bool APPEND, bool SPLIT>
+int launch_attention(const DecodeAttention& args, int pairs, size_t lds_bytes, hipStream_t stream) {
+  using K = DecodeAttentionOf<APPEND, SPLIT>;
+  const auto kernel = decode_attention_kernel<APPEND, SPLIT>;
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), dfhip_join_beside<K>, DFHIP_SHORT_BLOCKS), true);
+  (void)known;
+  hipLaunchKernelGGL(kernel, dim3(pairs, args.parts), dim3(DEC_THREADS), lds_bytes, stream, K{args});
+  return dfhip_check_launch();
+}
+
 // One workgroup per token: rotate q and k of the new token (position lengths[t] - 1), store q,
 // append k and v to the caches of slot slots[t].
 __global__ void __launch_bounds__(256)
@@ -456,12 +491,11 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
   const float scale_log2 = scale * 1.4426950408889634f;
   const int group = q_heads / kv_heads;
   const size_t combine_bytes = (size_t)4 * group * (HD + 2) * sizeof(float);
-  hipLaunchKernelGGL((decode_attention_kernel<false, false>), dim3(T * kv_heads), dim3(DEC_THREADS), combine_bytes,
-                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(q), ld_q,
-                     static_cast<uint16_t*>(const_cast<void*>(k_cache)), static_cast<uint16_t*>(const_cast<void*>(v_cache)),
-                     slots, lengths, static_cast<uint16_t*>(out), ld_out, kv_heads, group, num_slots, capacity,
-                     scale_log2, nullptr, nullptr, 1, 1, nullptr, nullptr);
-  return dfhip_check_launch();
+  const DecodeAttention args{static_cast<const uint16_t*>(q), static_cast<uint16_t*>(const_cast<void*>(k_cache)),
+                             static_cast<uint16_t*>(const_cast<void*>(v_cache)), slots, lengths, static_cast<uint16_t*>(out),
+                             nullptr, nullptr, nullptr, nullptr, ld_q, ld_out, kv_heads, group, num_slots, capacity, 1, 1,
+                             scale_log2};
+  return launch_attention<false, false>(args, T * kv_heads, combine_bytes, static_cast<hipStream_t>(stream));
 }
 
 // Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), with at least 256 positions of
@@ -498,17 +532,13 @@ static int decode_attention_append(const void* qkv, int64_t ld_qkv, void* k_cach
   const int group = q_heads / kv_heads;
   const size_t lds_bytes = (size_t)4 * group * (HD + 2) * sizeof(float) + 2 * HD * sizeof(uint16_t);
   if (parts < MIN_PARTS) parts = 1;
-  const auto kernel = parts > 1 ? decode_attention_kernel<true, true> : decode_attention_kernel<true, false>;
   float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + ATTENTION_COUNTER_BYTES);
-  static const bool known = (dfhip_in_line(reinterpret_cast<const void*>(decode_attention_kernel<true, false>), 256), true);
-  (void)known;
-  hipLaunchKernelGGL(kernel, dim3(T * kv_heads, parts), dim3(DEC_THREADS), lds_bytes,
-                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(qkv), ld_qkv,
-                     static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache), slots, lengths,
-                     static_cast<uint16_t*>(out), ld_out, kv_heads, group, num_slots, capacity,
-                     scale * 1.4426950408889634f, cos_table, sin_table, table_rows, parts,
-                     parts > 1 ? partials : nullptr, static_cast<int*>(workspace));
-  return dfhip_check_launch();
+  const DecodeAttention args{static_cast<const uint16_t*>(qkv), static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache),
+                             slots, lengths, static_cast<uint16_t*>(out), cos_table, sin_table, parts > 1 ? partials : nullptr,
+                             static_cast<int*>(workspace), ld_qkv, ld_out, kv_heads, group, num_slots, capacity, table_rows,
+                             parts, scale * 1.4426950408889634f};
+  const auto launch = parts > 1 ? launch_attention<true, true> : launch_attention<true, false>;
+  return launch(args, T * kv_heads, lds_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int dfhip_decode_attention_append_bf16(const void* qkv, int64_t ld_qkv, void* k_cache, void* v_cache,

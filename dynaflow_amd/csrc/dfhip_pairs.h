@@ -44,12 +44,30 @@ constexpr int DFHIP_PAIR_MAX_M = 128;
 enum DfhipPaired { DFHIP_ALONE = 0, DFHIP_BESIDE = 1, DFHIP_MERGED = 2 };
 
 // The launch that two become.
-struct DfhipJoined { const void* kernel; unsigned lds; unsigned grid; };
+struct DfhipJoined { const void* kernel; unsigned lds; dim3 grid; };
 
-// Makes `kernel` known to dfhip_graph_pair_launches: its arguments are one struct of `bytes` bytes, and `join` makes those
-// of a paired launch of two of `grid` workgroups each (false: not the same weights).
-typedef bool (*DfhipJoin)(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined);
+// Makes `kernel` known to dfhip_graph_pair_launches: its arguments are one struct, and `join` makes those of the launch that
+// two of grids ga and gb become (false: they are not the same work on different rows).  `in_line`: how many workgroups a
+// launch without a partner may have that runs in line with paired ones; none at all for those that read weights.
+typedef bool (*DfhipJoin)(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined);
 constexpr size_t DFHIP_PAIR_MAX_ARGS = 512;
-void dfhip_pairable(const void* kernel, size_t bytes, DfhipJoin join);
-// How many workgroups a launch of `kernel` may have that runs in line with paired ones (the default: SHORT_BLOCKS).
-void dfhip_in_line(const void* kernel, unsigned blocks);
+constexpr unsigned DFHIP_SHORT_BLOCKS = 512;     // also that of a kernel that is not known
+void dfhip_pairable(const void* kernel, DfhipJoin join, unsigned in_line = 0);
+inline bool dfhip_same(dim3 a, dim3 b) { return a.x == b.x && a.y == b.y && a.z == b.z; }
+
+// A launch without weights is K::run(workgroup) of K::THREADS threads; two of them sit one behind the other.
+template <class K>
+struct DfhipBoth { K side[2]; unsigned blocks; };
+template <class K>
+__global__ void __launch_bounds__(K::THREADS) dfhip_beside_kernel(const DfhipBoth<K> p) {
+  const unsigned second = blockIdx.x >= p.blocks;
+  p.side[second].run(blockIdx.x - (second ? p.blocks : 0), second ? gridDim.x - p.blocks : p.blocks);
+}
+template <class K>
+bool dfhip_join_beside(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
+  static_assert(sizeof(DfhipBoth<K>) <= DFHIP_PAIR_MAX_ARGS);
+  const K &x = *static_cast<const K*>(a), &y = *static_cast<const K*>(b);
+  *joined = {reinterpret_cast<const void*>(dfhip_beside_kernel<K>), joined->lds, dim3(ga.x + gb.x, ga.y > gb.y ? ga.y : gb.y)};
+  *static_cast<DfhipBoth<K>*>(both) = {{x, y}, ga.x};
+  return x.beside(y);
+}

@@ -3,7 +3,7 @@
 // All of them move 16 bytes per lane per access (global_load/store_dwordx4) from
 // many small workgroups and do their arithmetic in fp32 with a single rounding at
 // the store.
-#include "dfhip_common.h"
+#include "dfhip_pairs.h"
 
 namespace {
 
@@ -85,12 +85,11 @@ silu_mul_f32_kernel(const float* __restrict__ gate, int64_t ld_gate, const float
 constexpr int NORM_THREADS = 256;
 constexpr int NORM_MAX_CHUNKS = 8;  // 8 chunks * 8 elements * 256 lanes = 16384 columns
 
-__global__ void __launch_bounds__(NORM_THREADS)
-rmsnorm_bf16_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual,
-                    const uint16_t* __restrict__ weight, uint16_t* __restrict__ out,
-                    uint16_t* __restrict__ residual_out, int H, float eps) {
+DFHIP_DEVICE void rmsnorm_row(unsigned at, const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual,
+                              const uint16_t* __restrict__ weight, uint16_t* __restrict__ out,
+                              uint16_t* __restrict__ residual_out, int H, float eps) {
   __shared__ float partial[NORM_THREADS / 64];
-  const int64_t row_off = (int64_t)blockIdx.x * H;
+  const int64_t row_off = (int64_t)at * H;
   const int chunks = H / 8;
   u32x4 h[NORM_MAX_CHUNKS];
   float sumsq = 0.0f;
@@ -153,6 +152,18 @@ rmsnorm_bf16_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__
     }
   }
 }
+struct RmsNorm {
+  static constexpr int THREADS = NORM_THREADS;
+  const uint16_t *x, *residual, *weight;
+  uint16_t *out, *residual_out;
+  int H;
+  float eps;
+  DFHIP_DEVICE void run(unsigned block, unsigned) const { rmsnorm_row(block, x, residual, weight, out, residual_out, H, eps); }
+  bool beside(const RmsNorm& other) const {
+    return out != other.out && (!residual_out || residual_out != other.residual_out) && weight == other.weight && H == other.H;
+  }
+};
+__global__ void __launch_bounds__(NORM_THREADS) rmsnorm_bf16_kernel(const RmsNorm p) { p.run(blockIdx.x, gridDim.x); }
 
 // out[n, k] = in[k, n]; 64x64 tiles through LDS (padded against bank conflicts).
 constexpr int TR_TILE = 64;
@@ -268,10 +279,13 @@ extern "C" int dfhip_rmsnorm_bf16(const void* x, const void* residual, const voi
   if (!dfhip_aligned16(x) || !dfhip_aligned16(weight) || !dfhip_aligned16(out) ||
       (residual && !dfhip_aligned16(residual)) || (residual_out && !dfhip_aligned16(residual_out)))
     return DFHIP_ERR_BAD_ALIGNMENT;
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(rmsnorm_bf16_kernel), dfhip_join_beside<RmsNorm>,
+                                            DFHIP_SHORT_BLOCKS), true);
+  (void)known;
   hipLaunchKernelGGL(rmsnorm_bf16_kernel, dim3(M), dim3(NORM_THREADS), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(residual),
-                     static_cast<const uint16_t*>(weight), static_cast<uint16_t*>(out),
-                     static_cast<uint16_t*>(residual_out), H, eps);
+                     RmsNorm{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(residual),
+                             static_cast<const uint16_t*>(weight), static_cast<uint16_t*>(out),
+                             static_cast<uint16_t*>(residual_out), H, eps});
   return dfhip_check_launch();
 }
 

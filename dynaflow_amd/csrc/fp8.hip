@@ -157,12 +157,11 @@ DFHIP_DEVICE float block_max(float v) {
 // queue up at one address (12 ns each): with the quantisation behind it and no launch to clear a cell, x of 12 / 350 / 2048 x
 // 8192 7.6 / 12.8 / 41.6 -> 5.6 / 8.2 / 19.5 us, SiLU*mul of 350 / 2048 x 28672 32 / 106 -> 23 / 91.
 template <bool FLAT, bool SILU>
-__global__ void __launch_bounds__(QT)
-absmax_parts_kernel(const uint16_t* __restrict__ x, int64_t ld, const uint16_t* __restrict__ up, int64_t ld_up,
-                    uint16_t* __restrict__ out, int64_t ld_out, uint32_t groups, uint32_t per_row,
-                    float* __restrict__ parts) {
+DFHIP_DEVICE void absmax_part(unsigned block, unsigned blocks, const uint16_t* __restrict__ x, int64_t ld,
+                              const uint16_t* __restrict__ up, int64_t ld_up, uint16_t* __restrict__ out, int64_t ld_out,
+                              uint32_t groups, uint32_t per_row, float* __restrict__ parts) {
   float m = 0.0f;
-  for (uint32_t g0 = blockIdx.x * (QT * QUNROLL) + threadIdx.x; g0 < groups; g0 += gridDim.x * (QT * QUNROLL)) {
+  for (uint32_t g0 = block * (QT * QUNROLL) + threadIdx.x; g0 < groups; g0 += blocks * (QT * QUNROLL)) {
     u32x4 v[QUNROLL], u[QUNROLL];
 #pragma unroll
     for (int k = 0; k < QUNROLL; ++k) {
@@ -185,19 +184,35 @@ absmax_parts_kernel(const uint16_t* __restrict__ x, int64_t ld, const uint16_t* 
     }
   }
   m = block_max<QT>(m);
-  if (threadIdx.x == 0) parts[blockIdx.x] = m;
+  if (threadIdx.x == 0) parts[block] = m;
 }
+template <bool FLAT, bool SILU>
+struct AbsmaxParts {
+  static constexpr int THREADS = QT;
+  const uint16_t* x;
+  const uint16_t* up;
+  uint16_t* out;
+  float* parts;
+  int64_t ld, ld_up, ld_out;
+  uint32_t groups, per_row;
+  DFHIP_DEVICE void run(unsigned block, unsigned blocks) const {
+    absmax_part<FLAT, SILU>(block, blocks, x, ld, up, ld_up, out, ld_out, groups, per_row, parts);
+  }
+  bool beside(const AbsmaxParts& other) const { return parts != other.parts && (!SILU || out != other.out); }
+};
+template <bool FLAT, bool SILU>
+__global__ void __launch_bounds__(QT) absmax_parts_kernel(const AbsmaxParts<FLAT, SILU> p) { p.run(blockIdx.x, gridDim.x); }
 
 // q = e4m3fn(x / scale), scale = max(amax, 1e-12) / 448.  PARTS: amax is the maximum of n_parts values; else `amax` is one
 // value, which the last block to have read it clears, with the count of those that have: the cells are zero again for the
 // launch that folds the next maximum into them.
 template <bool FLAT, bool PARTS>
-__global__ void __launch_bounds__(QT)
-quant_fp8_after_kernel(const uint16_t* __restrict__ x, int64_t ld, uint8_t* __restrict__ q, int64_t ld_q, uint32_t groups,
-                       uint32_t per_row, float* __restrict__ amax, int n_parts, int* __restrict__ readers,
-                       float* __restrict__ scale_out) {
-  const uint32_t step = gridDim.x * (QT * QUNROLL);
-  uint32_t g0 = blockIdx.x * (QT * QUNROLL) + threadIdx.x;
+DFHIP_DEVICE void quant_after(unsigned block, unsigned blocks, const uint16_t* __restrict__ x, int64_t ld,
+                              uint8_t* __restrict__ q, int64_t ld_q, uint32_t groups, uint32_t per_row,
+                              float* __restrict__ amax, int n_parts, int* __restrict__ readers,
+                              float* __restrict__ scale_out) {
+  const uint32_t step = blocks * (QT * QUNROLL);
+  uint32_t g0 = block * (QT * QUNROLL) + threadIdx.x;
   u32x4 v[QUNROLL];
   auto load = [&]() {
 #pragma unroll
@@ -219,13 +234,13 @@ quant_fp8_after_kernel(const uint16_t* __restrict__ x, int64_t ld, uint8_t* __re
     if (threadIdx.x == 0) cell = __hip_atomic_load(amax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     m = cell;
-    if (threadIdx.x == 0 && atomicAdd(readers, 1) == (int)gridDim.x - 1) {
+    if (threadIdx.x == 0 && atomicAdd(readers, 1) == (int)blocks - 1) {
       __hip_atomic_store(amax, 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(readers, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   const float scale = fmaxf(m, 1e-12f) / FP8_MAX;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && scale_out != nullptr) scale_out[0] = scale;
+  if (block == 0 && threadIdx.x == 0 && scale_out != nullptr) scale_out[0] = scale;
   while (g0 < groups) {
 #pragma unroll
     for (int k = 0; k < QUNROLL; ++k)
@@ -234,6 +249,45 @@ quant_fp8_after_kernel(const uint16_t* __restrict__ x, int64_t ld, uint8_t* __re
     g0 += step;
     if (g0 < groups) load();
   }
+}
+template <bool FLAT, bool PARTS>
+struct QuantAfter {
+  static constexpr int THREADS = QT;
+  const uint16_t* x;
+  uint8_t* q;
+  float* amax;
+  int* readers;
+  float* scale_out;
+  int64_t ld, ld_q;
+  uint32_t groups, per_row;
+  int n_parts;
+  DFHIP_DEVICE void run(unsigned block, unsigned blocks) const {
+    quant_after<FLAT, PARTS>(block, blocks, x, ld, q, ld_q, groups, per_row, amax, n_parts, readers, scale_out);
+  }
+  bool beside(const QuantAfter& other) const {
+    return q != other.q && amax != other.amax && (!scale_out || scale_out != other.scale_out);
+  }
+};
+template <bool FLAT, bool PARTS>
+__global__ void __launch_bounds__(QT) quant_fp8_after_kernel(const QuantAfter<FLAT, PARTS> p) { p.run(blockIdx.x, gridDim.x); }
+
+template <bool FLAT, bool SILU>
+int launch_absmax_parts(const AbsmaxParts<FLAT, SILU>& args, unsigned blocks, hipStream_t stream) {
+  const auto kernel = absmax_parts_kernel<FLAT, SILU>;
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), dfhip_join_beside<AbsmaxParts<FLAT, SILU>>,
+                                            DFHIP_SHORT_BLOCKS), true);
+  (void)known;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(QT), 0, stream, args);
+  return dfhip_check_launch();
+}
+template <bool FLAT, bool PARTS>
+int launch_quant_after(const QuantAfter<FLAT, PARTS>& args, unsigned blocks, hipStream_t stream) {
+  const auto kernel = quant_fp8_after_kernel<FLAT, PARTS>;
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), dfhip_join_beside<QuantAfter<FLAT, PARTS>>,
+                                            DFHIP_SHORT_BLOCKS), true);
+  (void)known;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(QT), 0, stream, args);
+  return dfhip_check_launch();
 }
 
 // ------------------------------------------------------------------ fp8 GEMM
@@ -1046,10 +1100,21 @@ template <bool PARTS>
 int launch_quant_after(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, float* amax, int n_parts, int* readers,
                        float* scale_out, hipStream_t stream) {
   const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
-  const auto kernel = ld == D && ld_q == D ? quant_fp8_after_kernel<true, PARTS> : quant_fp8_after_kernel<false, PARTS>;
-  hipLaunchKernelGGL(kernel, dim3(parts_for(groups)), dim3(QT), 0, stream, static_cast<const uint16_t*>(x), ld,
-                     static_cast<uint8_t*>(q), ld_q, groups, per_row, amax, n_parts, readers, scale_out);
-  return dfhip_check_launch();
+  const QuantAfter<false, PARTS> args{static_cast<const uint16_t*>(x), static_cast<uint8_t*>(q), amax, readers, scale_out, ld,
+                                      ld_q, groups, per_row, n_parts};
+  if (ld != D || ld_q != D) return launch_quant_after(args, parts_for(groups), stream);
+  return launch_quant_after(QuantAfter<true, PARTS>{args.x, args.q, amax, readers, scale_out, ld, ld_q, groups, per_row, n_parts},
+                            parts_for(groups), stream);
+}
+template <bool SILU>
+int launch_absmax_parts(const void* x, int64_t ld, const void* up, int64_t ld_up, void* out, int64_t ld_out, int M, int D,
+                        bool flat, float* parts, hipStream_t stream) {
+  const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
+  const AbsmaxParts<false, SILU> args{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(up),
+                                      static_cast<uint16_t*>(out), parts, ld, ld_up, ld_out, groups, per_row};
+  if (!flat) return launch_absmax_parts(args, parts_for(groups), stream);
+  return launch_absmax_parts(AbsmaxParts<true, SILU>{args.x, args.up, args.out, parts, ld, ld_up, ld_out, groups, per_row},
+                             parts_for(groups), stream);
 }
 }  // namespace
 
@@ -1058,13 +1123,9 @@ extern "C" int dfhip_quant_fp8_dynamic_bf16(const void* x, int64_t ld, void* q, 
   if (int rc = check_q(x, ld, M, D)) return rc;
   if (int rc = check_q_out(q, ld_q, D)) return rc;
   if (!parts) return DFHIP_ERR_NULL_POINTER;
-  const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const auto kernel = ld == D ? absmax_parts_kernel<true, false> : absmax_parts_kernel<false, false>;
-  hipLaunchKernelGGL(kernel, dim3(parts_for(groups)), dim3(QT), 0, s, static_cast<const uint16_t*>(x), ld, nullptr, 0, nullptr,
-                     0, groups, per_row, parts);
-  if (int rc = dfhip_check_launch()) return rc;
-  return launch_quant_after<true>(x, ld, q, ld_q, M, D, parts, (int)parts_for(groups), nullptr, scale_out, s);
+  if (int rc = launch_absmax_parts<false>(x, ld, nullptr, 0, nullptr, 0, M, D, ld == D, parts, s)) return rc;
+  return launch_quant_after<true>(x, ld, q, ld_q, M, D, parts, (int)parts_for((uint32_t)M * (D / 8)), nullptr, scale_out, s);
 }
 
 extern "C" int dfhip_silu_mul_quant_fp8_bf16(const void* gate, int64_t ld_gate, const void* up, int64_t ld_up, void* act,
@@ -1075,14 +1136,11 @@ extern "C" int dfhip_silu_mul_quant_fp8_bf16(const void* gate, int64_t ld_gate, 
   if (int rc = check_q(act, ld_act, M, D)) return rc;
   if (int rc = check_q_out(q, ld_q, D)) return rc;
   if (!parts) return DFHIP_ERR_NULL_POINTER;
-  const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const bool flat = ld_gate == D && ld_up == D && ld_act == D;
-  const auto kernel = flat ? absmax_parts_kernel<true, true> : absmax_parts_kernel<false, true>;
-  hipLaunchKernelGGL(kernel, dim3(parts_for(groups)), dim3(QT), 0, s, static_cast<const uint16_t*>(gate), ld_gate,
-                     static_cast<const uint16_t*>(up), ld_up, static_cast<uint16_t*>(act), ld_act, groups, per_row, parts);
-  if (int rc = dfhip_check_launch()) return rc;
-  return launch_quant_after<true>(act, ld_act, q, ld_q, M, D, parts, (int)parts_for(groups), nullptr, scale_out, s);
+  if (int rc = launch_absmax_parts<true>(gate, ld_gate, up, ld_up, act, ld_act, M, D, flat, parts, s)) return rc;
+  return launch_quant_after<true>(act, ld_act, q, ld_q, M, D, parts, (int)parts_for((uint32_t)M * (D / 8)), nullptr, scale_out,
+                                  s);
 }
 
 extern "C" int dfhip_requant_fp8_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, void* cells,

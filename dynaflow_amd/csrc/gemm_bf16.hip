@@ -1209,6 +1209,7 @@ struct SkinnyArgs {
   int64_t ldw;
   DfhipSide side[2];
 };
+static_assert(sizeof(SkinnyArgs) <= DFHIP_PAIR_MAX_ARGS);
 
 bool sides_skinny(const void* a, const void* b, void* both) {
   const SkinnyArgs &x = *static_cast<const SkinnyArgs*>(a), &y = *static_cast<const SkinnyArgs*>(b);
@@ -1617,24 +1618,24 @@ size_t skinny_counter_bytes(int M, int N) { return dfhip_counter_area(skinny_til
 // 8B shapes, on two streams / side by side in one launch / in one tile: gate + up + SiLU*mul 72 / 64 / 48, down 45 / 39 /
 // 47, whose 128 workgroups are too few]
 template <bool FUSED, int BM, int BW>
-bool join_skinny(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+bool join_skinny(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
   static std::atomic<uint64_t> lds_opted_in{0};
   constexpr bool MERGED = FUSED && BM == 64;
   using T = SkinnyTile<MERGED ? 128 : BM, MERGED ? 128 : BW>;
-  if (!sides_skinny(a, b, both)) return false;
+  if (!dfhip_same(ga, gb) || !sides_skinny(a, b, both)) return false;
   if constexpr (MERGED) {
     SkinnyArgs& out = *static_cast<SkinnyArgs*>(both);
     out.tiles_n = (out.N + 63) / 64;
-    *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_kernel<true, 128, 128, DFHIP_MERGED>), T::LDS, (unsigned)out.tiles_n};
+    *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_kernel<true, 128, 128, DFHIP_MERGED>), T::LDS, dim3(out.tiles_n)};
   } else {
-    *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_kernel<FUSED, BM, BW, DFHIP_BESIDE>), T::LDS, 2 * grid};
+    *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_kernel<FUSED, BM, BW, DFHIP_BESIDE>), T::LDS, dim3(2 * ga.x)};
   }
   return dfhip_opt_in_lds(joined->kernel, T::LDS, lds_opted_in) == DFHIP_OK;
 }
-bool join_skinny_wide(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+bool join_skinny_wide(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
   static std::atomic<uint64_t> lds_opted_in{0};
-  *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_wide_kernel<true>), SKW_LDS, 2 * grid};
-  return sides_skinny(a, b, both) && dfhip_opt_in_lds(joined->kernel, SKW_LDS, lds_opted_in) == DFHIP_OK;
+  *joined = {reinterpret_cast<const void*>(gemm_bf16_skinny_wide_kernel<true>), SKW_LDS, dim3(2 * ga.x)};
+  return dfhip_same(ga, gb) && sides_skinny(a, b, both) && dfhip_opt_in_lds(joined->kernel, SKW_LDS, lds_opted_in) == DFHIP_OK;
 }
 
 template <bool FUSED, int BM, int BW>
@@ -1653,7 +1654,7 @@ int launch_skinny_tile(const void* A, int64_t lda, const void* W, const void* W2
     if (int rc = dfhip_clear_uncommon_counters(workspace, skinny_tiles(M, N), stream)) return rc;
     partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + skinny_counter_bytes(M, N));
   }
-  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof(SkinnyArgs), join_skinny<FUSED, BM, BW>), true);
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), join_skinny<FUSED, BM, BW>), true);
   (void)known;
   const uint16_t* const w2 = static_cast<const uint16_t*>(W2);   // not FUSED: the residual
   const SkinnyArgs args{static_cast<const uint16_t*>(W), FUSED ? w2 : nullptr, N, K, tiles_m, tiles_n, split_k, ldw,
@@ -1687,7 +1688,7 @@ int launch_skinny_wide(const void* A, int64_t lda, const void* W, const void* W2
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), SKW_LDS, lds_opted_in)) return rc;
   const int tiles_m = (M + SK_BM - 1) / SK_BM;
   const int tiles_n = (N + SKW_BN - 1) / SKW_BN;
-  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof(SkinnyArgs), join_skinny_wide), true);
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), join_skinny_wide), true);
   (void)known;
   const SkinnyArgs args{static_cast<const uint16_t*>(W), static_cast<const uint16_t*>(W2), N, K, tiles_m, tiles_n, 1, ldw,
                         {{A, nullptr, C, nullptr, nullptr, nullptr, nullptr, lda, ldc, M}, {}}};

@@ -35,6 +35,7 @@ struct Ring3Args {
   int64_t ldw;                // bytes (the strides of A too; that of C in elements)
   DfhipSide side[2];          // R (residual [M, N] with the row stride of C, or null): bf16, not FUSED
 };
+static_assert(sizeof(Ring3Args) <= DFHIP_PAIR_MAX_ARGS);
 
 bool sides_ring3(const void* a, const void* b, void* both) {
   const Ring3Args &x = *static_cast<const Ring3Args*>(a), &y = *static_cast<const Ring3Args*>(b);
@@ -331,12 +332,12 @@ gemm_ring3_kernel(const Ring3Args p) {
 }
 
 template <bool FP8, bool FUSED, bool SPLIT, int T>
-bool join_ring3(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+bool join_ring3(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
   constexpr int TM = DFHIP_RING3[T].rows, TN = DFHIP_RING3[T].cols;
   constexpr int LDS = units(TM, TN) * (TM + TN) * SLAB;
   static std::atomic<uint64_t> lds_opted_in{0};
-  *joined = {reinterpret_cast<const void*>(gemm_ring3_kernel<FP8, FUSED, TM, TN, SPLIT, true>), LDS, 2 * grid};
-  return sides_ring3(a, b, both) && dfhip_opt_in_lds(joined->kernel, LDS, lds_opted_in) == DFHIP_OK;
+  *joined = {reinterpret_cast<const void*>(gemm_ring3_kernel<FP8, FUSED, TM, TN, SPLIT, true>), LDS, dim3(2 * ga.x)};
+  return dfhip_same(ga, gb) && sides_ring3(a, b, both) && dfhip_opt_in_lds(joined->kernel, LDS, lds_opted_in) == DFHIP_OK;
 }
 
 template <bool FP8, bool FUSED, bool SPLIT, int T>
@@ -354,7 +355,7 @@ int launch(Ring3Args p, void* workspace, hipStream_t stream) {
     p.side[0].partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + dfhip_counter_area(tiles));
     p.side[0].arrivals = static_cast<int*>(workspace);
   }
-  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof p, join_ring3<FP8, FUSED, SPLIT, T>), true);
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), join_ring3<FP8, FUSED, SPLIT, T>), true);
   (void)known;
   hipLaunchKernelGGL(kernel, dim3(p.tiles_m * p.tiles_n * p.split_k), dim3(256), LDS, stream, p);
   return dfhip_check_launch();

@@ -38,6 +38,7 @@ struct StreamArgs {
   int64_t ldw;                // bytes (the strides of A too; that of C in elements)
   DfhipSide side[2];          // R (residual [M, N] with the row stride of C, or null): bf16, not FUSED
 };
+static_assert(sizeof(StreamArgs) <= DFHIP_PAIR_MAX_ARGS);
 
 bool sides_stream(const void* a, const void* b, void* both) {
   const StreamArgs &x = *static_cast<const StreamArgs*>(a), &y = *static_cast<const StreamArgs*>(b);
@@ -321,10 +322,10 @@ int opt_in_stream() {
 // Two launches of up to 16 MB rows are one of the kernel with twice the row blocks, on the tiles (and with them the order of
 // the sums) of the one.
 template <bool FP8, int MB, int WIDTH, bool FUSED, bool SPLIT>
-bool join_stream(const void* a, const void* b, unsigned grid, void* both, DfhipJoined* joined) {
+bool join_stream(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
   *joined = {reinterpret_cast<const void*>(stream_kernel<FP8, 2 * MB, WIDTH, FUSED, SPLIT, true>),
-             (unsigned)stream_lds(2 * MB, (FUSED ? 2 : 1) * WIDTH), grid};
-  return sides_stream(a, b, both) && opt_in_stream<FP8, 2 * MB, WIDTH, FUSED, SPLIT, true>() == DFHIP_OK;
+             (unsigned)stream_lds(2 * MB, (FUSED ? 2 : 1) * WIDTH), ga};
+  return dfhip_same(ga, gb) && sides_stream(a, b, both) && opt_in_stream<FP8, 2 * MB, WIDTH, FUSED, SPLIT, true>() == DFHIP_OK;
 }
 
 template <bool FP8, int MB, int WIDTH, bool FUSED, bool SPLIT>
@@ -332,8 +333,7 @@ int launch(const StreamArgs& p, hipStream_t stream) {
   const auto kernel = stream_kernel<FP8, MB, WIDTH, FUSED, SPLIT, false>;
   if (int rc = opt_in_stream<FP8, MB, WIDTH, FUSED, SPLIT, false>()) return rc;
   if constexpr (MB <= 2) {
-    static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), sizeof p,
-                                              join_stream<FP8, MB, WIDTH, FUSED, SPLIT>), true);
+    static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), join_stream<FP8, MB, WIDTH, FUSED, SPLIT>), true);
     (void)known;
   }
   constexpr int COLS = 16 * WIDTH;

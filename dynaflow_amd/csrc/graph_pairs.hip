@@ -11,10 +11,12 @@
 // fp8 254 / 187]
 //
 // Where every launch of a graph is one of a pair or short, nothing is left that gains from running side by side: the graph
-// becomes a chain, which saves the meetings of two queues (6 - 10 us each).  Any other graph stays as it is.  Attention
-// over a cache leaves the chip to others when its workgroups run out unevenly, and the chain has no others: it counts as
-// short up to a workgroup per compute unit.  [us of a step of 4 layers, sequences of 1/4 .. 1 of 4096 positions, two streams /
-// chain: 16 sequences 814 / 620, 40 1034 / 916, 64 1228 / 1124; 72, 288 workgroups each, 1281 / 1407, 128 1652 / 1719]
+// becomes a chain, which saves the meetings of two queues (6 - 10 us each).  Any other graph stays as it is.  Short launches and
+// attention over a cache pair as well (their workgroups side by side: one launch's gap less, and of attention one tail).
+// A schedule with a stream per nano-batch (`side_by_side`) runs long attention of one beside the projections of the other, which
+// is worth as much from 512 workgroups on: it stays.  [us of a decode step of 4 layers, sequences of 1/4 .. 1 of 4096 positions,
+// streams by nano-batch / by kind / chain: 16 sequences 835 / 883 / -, 40 1037 / 1179 / 859, 64 1230 / 1410 / 1060, 128 1644 / 2030 /
+// 1622 (by kind's plans 1688); 256 of 2048 positions each 2117 / 2533 / 2145 (2333)]
 #include <algorithm>
 #include <mutex>
 #include <unordered_map>
@@ -24,12 +26,9 @@
 
 namespace {
 
-constexpr unsigned SHORT_BLOCKS = 512;   // workgroups of a launch that may as well run in line, if its kernel gives no number
-
 struct Known {
-  size_t bytes = 0;
   DfhipJoin join = nullptr;
-  unsigned in_line = SHORT_BLOCKS;
+  unsigned in_line = DFHIP_SHORT_BLOCKS;
 };
 std::mutex known_mutex;
 std::unordered_map<const void*, Known>& known_kernels() {
@@ -50,7 +49,10 @@ struct Node {
   int pair = -1;                         // the other node of its pair
 };
 
-bool same(const dim3& a, const dim3& b) { return a.x == b.x && a.y == b.y && a.z == b.z; }
+size_t blocks_of(const Node& node) {
+  const dim3& grid = node.params.gridDim;
+  return (size_t)grid.x * grid.y * grid.z;
+}
 
 // A topological order of the graph whose paired nodes are one (named by the smaller index), smallest index first; empty if
 // there is none.
@@ -82,17 +84,12 @@ std::vector<int> order_of(const std::vector<Node>& nodes, const std::vector<std:
 
 }  // namespace
 
-void dfhip_pairable(const void* kernel, size_t bytes, DfhipJoin join) {
+void dfhip_pairable(const void* kernel, DfhipJoin join, unsigned in_line) {
   std::lock_guard<std::mutex> guard(known_mutex);
-  known_kernels()[kernel] = {bytes, bytes <= DFHIP_PAIR_MAX_ARGS ? join : nullptr, SHORT_BLOCKS};
+  known_kernels()[kernel] = {join, in_line};
 }
 
-void dfhip_in_line(const void* kernel, unsigned blocks) {
-  std::lock_guard<std::mutex> guard(known_mutex);
-  known_kernels()[kernel].in_line = blocks;
-}
-
-extern "C" int dfhip_graph_pair_launches(void* graph, int* pairs) {
+extern "C" int dfhip_graph_pair_launches(void* graph, int side_by_side, int* pairs) {
   if (!graph || !pairs) return DFHIP_ERR_NULL_POINTER;
   *pairs = 0;
   hipGraph_t g = static_cast<hipGraph_t>(graph);
@@ -116,9 +113,9 @@ extern "C" int dfhip_graph_pair_launches(void* graph, int* pairs) {
     if (type == hipGraphNodeTypeEmpty) continue;
     if (!node.kernel) return DFHIP_OK;
     if (hipGraphKernelNodeGetParams(handles[i], &node.params) != hipSuccess) return DFHIP_ERR_LAUNCH;
-    const dim3& grid = node.params.gridDim;
     node.known = find_known(node.params.func);
-    if (node.known.join ? !node.params.kernelParams : (size_t)grid.x * grid.y * grid.z > node.known.in_line) return DFHIP_OK;
+    if (node.known.join && !node.params.kernelParams) node.known.join = nullptr;
+    if (!node.known.join && blocks_of(node) > node.known.in_line) return DFHIP_OK;
   }
   std::vector<std::pair<int, int>> edges(edge_count);
   const size_t words = (count + 63) / 64;
@@ -135,6 +132,10 @@ extern "C" int dfhip_graph_pair_launches(void* graph, int* pairs) {
 
   alignas(16) unsigned char both[DFHIP_PAIR_MAX_ARGS];
   DfhipJoined joined;
+  auto join_of = [&](const Node& a, const Node& b) {
+    joined.lds = a.params.sharedMemBytes;
+    return a.known.join(a.params.kernelParams[0], b.params.kernelParams[0], a.params.gridDim, b.params.gridDim, both, &joined);
+  };
   int found = 0;
   for (size_t i = 0; i < count; ++i) {
     Node& a = nodes[i];
@@ -142,14 +143,14 @@ extern "C" int dfhip_graph_pair_launches(void* graph, int* pairs) {
     for (size_t j = i + 1; j < count && a.pair < 0; ++j) {
       Node& b = nodes[j];
       if (!b.kernel || b.pair >= 0 || b.params.func != a.params.func || reaches(i, j) || reaches(j, i)) continue;
-      if (!same(a.params.gridDim, b.params.gridDim) || !same(a.params.blockDim, b.params.blockDim)) continue;
-      if (a.params.sharedMemBytes != b.params.sharedMemBytes) continue;
-      if (!a.known.join(a.params.kernelParams[0], b.params.kernelParams[0], a.params.gridDim.x, both, &joined)) continue;
+      if (!dfhip_same(a.params.blockDim, b.params.blockDim) || a.params.sharedMemBytes != b.params.sharedMemBytes) continue;
+      if (!join_of(a, b)) continue;
       a.pair = (int)j;
       b.pair = (int)i;
-      ++found;
+      found += a.known.in_line == 0;
     }
-    if (a.pair < 0) return DFHIP_OK;                                  // a launch that would lose its company
+    // a launch that would lose its company
+    if (blocks_of(a) > a.known.in_line && (a.pair < 0 || (side_by_side && a.known.in_line > 0))) return DFHIP_OK;
   }
   if (!found) return DFHIP_OK;
   const std::vector<int> order = order_of(nodes, edges);
@@ -166,12 +167,12 @@ extern "C" int dfhip_graph_pair_launches(void* graph, int* pairs) {
     }
     if (node.pair >= 0) {
       Node& other = nodes[node.pair];
-      if (!node.known.join(node.params.kernelParams[0], other.params.kernelParams[0], node.params.gridDim.x, both, &joined)) return DFHIP_ERR_LAUNCH;
+      if (!join_of(node, other)) return DFHIP_ERR_LAUNCH;
       hipKernelNodeParams params = node.params;
       void* args[1] = {both};
       params.kernelParams = args;
       params.func = const_cast<void*>(joined.kernel);
-      params.gridDim.x = joined.grid;
+      params.gridDim = joined.grid;
       params.sharedMemBytes = joined.lds;
       if (hipGraphKernelNodeSetParams(node.handle, &params) != hipSuccess) return DFHIP_ERR_LAUNCH;
       if (hipGraphDestroyNode(other.handle) != hipSuccess) return DFHIP_ERR_LAUNCH;

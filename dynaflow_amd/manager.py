@@ -110,11 +110,12 @@ def join_results(results: dict[int, Any], num_nano_batches: int, shared_buffer: 
 PAIR_MAX_ROWS = 128
 
 
-def _pair_launches(graph: torch.cuda.CUDAGraph) -> int:
+def _pair_launches(graph: torch.cuda.CUDAGraph, side_by_side: bool) -> int:
     """Launches of two nano-batches against the same weights become one, where the whole schedule consists of such
     (dfhip_graph_pair_launches); how many did."""
     pairs = ctypes.c_int(0)
-    check("dfhip_graph_pair_launches", load().dfhip_graph_pair_launches(graph.raw_cuda_graph(), ctypes.byref(pairs)))
+    check("dfhip_graph_pair_launches",
+          load().dfhip_graph_pair_launches(graph.raw_cuda_graph(), side_by_side, ctypes.byref(pairs)))
     return pairs.value
 
 
@@ -343,7 +344,7 @@ class DynaFlowManager:
         else:
             return None, None, 0
         try:
-            pairs = _pair_launches(graph)
+            pairs = _pair_launches(graph, policy == "by_nano_batch")
         except KernelError as error:     # the graph may be half changed
             log.warning("captured launches were not paired: %s", error)
             return None, None, 0

@@ -15,8 +15,8 @@ from dynaflow_amd.mlp import SwiGLUMLP
 
 def test_arguments():
     pairs = ctypes.c_int(5)
-    assert _cabi.load().dfhip_graph_pair_launches(None, ctypes.byref(pairs)) == -1
-    assert _cabi.load().dfhip_graph_pair_launches(16, None) == -1
+    assert _cabi.load().dfhip_graph_pair_launches(None, 0, ctypes.byref(pairs)) == -1
+    assert _cabi.load().dfhip_graph_pair_launches(16, 0, None) == -1
 
 
 def randn(shape, seed, std=1.0):
