@@ -73,11 +73,12 @@ def test_short_launches_between_pairs_and_streams_by_kind(knobs):
     assert list(manager.paired_launches.values()) == [2]
 
 
-# streamed weights; rows of the two nano-batches that differ; tiles of 64 and 128 rows; a grid that is no multiple of eight
+# streamed weights, the rows of both in one to four blocks of 16; rows of the two nano-batches that differ; tiles of 64 and 128 rows; a grid that is no multiple of eight
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind,tokens,hidden,inter", [
-    ("bf16", 2, 2048, 5632), ("bf16", 25, 2048, 5696), ("bf16", 64, 4096, 14336), ("bf16", 96, 2048, 5696),
-    ("bf16", 255, 4096, 14336), ("fp8", 24, 4096, 14336), ("fp8", 29, 2048, 5760), ("fp8", 80, 8192, 8192),
+    ("bf16", 2, 2048, 5632), ("bf16", 16, 2048, 5632), ("bf16", 25, 2048, 5696), ("bf16", 35, 2048, 5632),
+    ("bf16", 48, 4096, 14336), ("bf16", 64, 4096, 14336), ("bf16", 96, 2048, 5696),
+    ("bf16", 255, 4096, 14336), ("fp8", 9, 4096, 14336), ("fp8", 24, 4096, 14336), ("fp8", 29, 2048, 5760), ("fp8", 80, 8192, 8192),
     ("fp8", 190, 4096, 14336)])
 def test_paired_replays_have_the_bits_of_the_eager_schedule(kind, tokens, hidden, inter):
     manager, compiled = program(mlp(kind, hidden, inter), tokens)
