@@ -85,3 +85,25 @@ def test_tiles_of_64_rows(M, N, K):
         assert torch.equal(fused, ops.silu_mul(*whole, True))
     few = x[:40].contiguous()
     assert torch.equal(ops.linear_variant(few, w, 6), whole[0][:40])
+
+
+# 256 and 161 tiles of three blocks, the last one ragged, whole and in two parts
+@pytest.mark.parametrize("M,N,K", [(1, 12280, 1024), (16, 12288, 1088), (32, 12264, 2048), (17, 6136, 4096), (24, 7720, 2112)])
+def test_tiles_of_three_blocks(M, N, K):
+    """Within the bound of the other few-row launches of the fp32 product, bf16 and fp8."""
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
+
+    x, w, r = randn((M, K), 1), randn((N, K), 2, 0.05), randn((M, N), 3)
+    want = x.float() @ w.float().t()
+    limit = 2.0 ** -7 * want.abs().max().item()
+    y = ops.linear(x, w)
+    assert (y.float() - want).abs().max().item() <= limit
+    assert (ops.linear_variant(x, w, 8).float() - want).abs().max().item() <= limit
+    assert torch.equal(ops.linear_add(x, w, r), r + y)
+    if K % 128 == 0:
+        xq, xs = ops.quant_fp8(x)
+        wq, ws = quantize_weight_per_channel(w)
+        y = ops.linear_fp8(xq, wq, xs, ws)
+        want = (xq.float() * xs) @ (wq.float() * ws[:, None]).t()
+        assert (y.float() - want).abs().max().item() <= 2.0 ** -6 * want.abs().max().item()
