@@ -503,15 +503,21 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
 // sequence takes its share of it (sequence_parts).  A launch with fewer than MIN_PARTS of them, from 171 pairs on, cuts
 // nothing.  [us, uncut / cut: 2 sequences of 8192 positions 111 / 20.8 (their bytes at 6.7 TB/s: 10), 8 of 2048 33 / 16.8
 // (10), 20 of 4096 69 / 58 (50); in two parts, not taken: 32 of 512, 2048 and 4096 14.6 / 16.5, 42.9 / 46.0, 79 / 84]
+// A compute unit takes in no more than 29 GB/s, so a few pairs more than units take twice the time: 257 .. 384 of them are cut
+// in four where the cache has room for 2048 positions, and so are 171 .. 192, which leave a quarter of the units idle, where it
+// has room for 4096.  [us, uncut / four parts, all full / of 1/4 .. 1 of the capacity, 8 kv heads: 34 sequences of 2048 70 / 58,
+// 42 / 47; 36 of 4096 139 / 109, 94 / 83; 40 of 8192 275 / 213, 223 / 167; 48 of 2048 80 / 76, 62 / 60; 24 of 4096 75 / 71, 68 / 65, of
+// 8192 142 / 130, 129 / 109; not taken: 36 of 1024 38.5 / 38, 26 of 4096 78 / 85, 69 / 66, 54 of 2048 80 / 85, 68 / 68]
 constexpr int MIN_PARTS = 3;
 static int attention_parts(int T, int kv_heads, int capacity) {
   const int64_t pairs = (int64_t)T * kv_heads;
+  if ((pairs > 256 && pairs <= 384 && capacity >= 2048) || (pairs > 170 && pairs <= 192 && capacity >= 4096)) return 4;
   int64_t parts = 512 / pairs;
   if (parts > capacity / 256) parts = capacity / 256;
   if (parts > 32) parts = 32;
   return parts < 1 ? 1 : (int)parts;
 }
-// The arrival counters at the start of the workspace: a launch that splits has at most 256 pairs, and the area is the same
+// The arrival counters at the start of the workspace: a launch that splits has at most 384 pairs, and the area is the same
 // for every shape, so that no launch's partial sums lie where another's counters are expected to be zero.
 constexpr size_t ATTENTION_COUNTER_BYTES = 4096;
 

@@ -49,9 +49,10 @@ struct Node {
   int pair = -1;                         // the other node of its pair
 };
 
+// (the parts of a sequence that attention cuts, grid.y, count as one)
 size_t blocks_of(const Node& node) {
   const dim3& grid = node.params.gridDim;
-  return (size_t)grid.x * grid.y * grid.z;
+  return node.known.join ? grid.x : (size_t)grid.x * grid.y * grid.z;
 }
 
 // A topological order of the graph whose paired nodes are one (named by the smaller index), smallest index first; empty if

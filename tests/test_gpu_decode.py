@@ -208,6 +208,22 @@ def test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, len
         assert int(ws[:4096].view(torch.int32).abs().sum()) == 0
 
 
+@pytest.mark.parametrize("heads,kv_heads,capacity,lengths", [
+    (32, 8, 2048, [2048 - 61 * i for i in range(33)]),   # the fewest and the most pairs of a little more than one per unit
+    (32, 8, 2048, [767 + 31 * i for i in range(41)] + [1, 768, 4096, 2048, 1023, 33, 2017]),
+    (43, 43, 4096, [4096, 1, 2500, 1024]),               # the fewest and the most pairs below one per unit
+    (32, 8, 4096, [4096 - 171 * i for i in range(24)]),
+])
+def test_decode_attention_cut_in_four(ops, heads, kv_heads, capacity, lengths):
+    """Pairs that would leave the compute units unevenly loaded."""
+    from dynaflow_amd import _cabi
+
+    T = len(lengths)
+    counters, block = 4096, heads // kv_heads * (D // 4 + 1) * 16
+    assert _cabi.load().dfhip_decode_attention_workspace_bytes(T, heads, kv_heads, capacity) == counters + T * kv_heads * 4 * block
+    test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, lengths)
+
+
 @pytest.mark.parametrize("T,capacity,lengths", [(2, 8192, [1, 33, 512, 767]), (8, 1024, [64, 767]), (32, 2048, [2048, 700])])
 def test_decode_attention_stays_whole_where_parts_do_not_pay(ops, T, capacity, lengths):
     """Sequences too short for three parts of 256 positions, and launches with room for two parts only: the bits of the
