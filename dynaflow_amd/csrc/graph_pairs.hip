@@ -8,14 +8,14 @@
 // multiply a weight with the rows of both (up to 32 rows each that stream their weights, up to 64 on tiles), or in which the
 // two workgroups that read the same weights sit on the same XCD and start together (pair_block).
 // [us, in a graph: 128 MB read by two launches 39 - 43, by one launch twice 24; layer of 2 x 48 tokens 126 / 90, of 2 x 12 in
-// fp8 254 / 187]
+// fp8 254 / 170]
 //
 // Where every launch of a graph is one of a pair or short, nothing is left that gains from running side by side: the graph
 // becomes a chain, which saves the meetings of two queues (6 - 10 us each).  Any other graph stays as it is.  Short launches and
 // attention over a cache pair as well (their workgroups side by side: one launch's gap less, and of attention one tail).
 // A schedule with a stream per nano-batch (`side_by_side`) runs long attention of one beside the projections of the other, which
 // is worth as much from 512 workgroups on: it stays.  [us of a decode step of 4 layers, sequences of 1/4 .. 1 of 4096 positions,
-// streams by nano-batch / by kind / chain: 16 sequences 835 / 883 / -, 40 1037 / 1179 / 859, 64 1230 / 1410 / 1060, 128 1644 / 2030 /
+// streams by nano-batch / by kind / chain: 40 sequences 1036 / 1179 / 824, 64 1230 / 1410 / 1058, 128 1644 / 2030 /
 // 1622 (by kind's plans 1688); 256 of 2048 positions each 2117 / 2533 / 2145 (2333)]
 #include <algorithm>
 #include <mutex>
