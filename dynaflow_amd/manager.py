@@ -327,7 +327,10 @@ class DynaFlowManager:
         assert self.config is not None and self.scheduler is not None
         policy = getattr(self.scheduler, "stream_policy", None)
         one_stream = getattr(self.scheduler, "comp_stream", None) is getattr(self.scheduler, "comm_stream", None)
-        if not self.config.knob("pair_launches", True) or self.config.knob("cu_split", None) or one_stream:
+        # (a collective looks like a short launch and waits for other ranks: what ran beside it stays beside it)
+        several_ranks = torch.distributed.is_available() and torch.distributed.is_initialized() and \
+            torch.distributed.get_world_size() > 1
+        if not self.config.knob("pair_launches", True) or self.config.knob("cu_split", None) or one_stream or several_ranks:
             return None, None, 0
         if policy == "by_nano_batch":
             graph, output = self._capture(args, kwargs, split, capture_on)

@@ -95,6 +95,18 @@ def test_paired_replays_have_the_bits_of_the_eager_schedule(kind, tokens, hidden
 
 
 @pytest.mark.gpu
+def test_ranks_keep_their_schedule(monkeypatch):
+    """Collectives are kernels of few workgroups: with several ranks nothing is put in line."""
+    monkeypatch.setattr(torch.distributed, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.distributed, "get_world_size", lambda: 2)
+    manager, compiled = program(mlp("bf16", 2048, 5632), 64)
+    x = randn((64, 2048), 5)
+    want = forward(manager, compiled, x, False).clone()
+    assert torch.equal(forward(manager, compiled, x, True), want)
+    assert list(manager.paired_launches.values()) == [0]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tokens,knobs", [(64, {"pair_launches": False}), (64, {"streams": "by_kind", "pair_launches": False}),
                                           (64, {"streams": "by_kind", "serialize": True}), (1024, {}),
                                           (1024, {"streams": "by_kind"}), (96, {"num_nano_batches": 3})])
