@@ -354,7 +354,7 @@ gemm_stream_kernel(const StreamArgs p) {
 
 constexpr int stream_lds(int mb, int nb) { return WAVES * rows_per_round(mb, nb) * nb * 1024; }
 // Slabs in flight per wave: as many as 256 registers hold.  `width`: 16-column blocks of the output per workgroup.
-constexpr int stream_depth(int mb, int width) { return width == 1 ? (mb == 4 ? 2 : 4) : (width == 2 || width == 3) && mb == 1 ? 4 : 2; }
+constexpr int stream_depth(int mb, int width) { return width == 1 ? (mb == 4 ? 2 : 4) : width == 2 && mb == 1 ? 4 : 2; }
 
 template <bool FP8, int MB, int WIDTH, bool FUSED, bool SPLIT, bool MERGED>
 constexpr auto stream_kernel =
@@ -406,7 +406,6 @@ int launch_width(const StreamArgs& p, int width, hipStream_t stream) {
   switch (width) {
     case 1: return launch<FP8, MB, 1, FUSED, SPLIT>(p, stream);
     case 2: return launch<FP8, MB, 2, FUSED, SPLIT>(p, stream);
-    case 3: return launch<FP8, MB, 3, FUSED, SPLIT>(p, stream);
     default: return launch<FP8, MB, 4, FUSED, SPLIT>(p, stream);
   }
 }
@@ -424,28 +423,15 @@ int launch_rows(const StreamArgs& p, int width, hipStream_t stream) {
 // does not: the widest tile that leaves 160.  [us, 8B shapes, weights from HBM: o 4096 x 4096 at 16 rows 9.7 with 256
 // workgroups of 16 columns, 12.9 with 128 of 32; q/k/v 6144 x 4096 16.7 with 384 of 16, 13.3 with 192 of 32; gate +
 // up + SiLU*mul 2 x 14336 x 4096 at 64 rows 88 / 64 / 49 with 16 / 32 / 64 outputs a workgroup]
-// A compute unit takes in no more than 29 GB/s, so the launch is as long as the unit that takes in the most, rows of the
-// weights and of the activations (whole blocks) counted alike: a narrower tile with which that is 10 % less, lone and side by side together.
-// [us, the widest of 1, 2 and 4 blocks -> this, lone / side by side: q/k/v 6144 x 4096 in two parts at 24 rows 17.8 -> 15.2 / 29.1 ->
-// 26.4, 12288 x 4096 at 16 rows 23.1 -> 19.4 / 39.9 -> 35.7, fp8 12288 x 6144 19.7 -> 16.5 / 34.3 -> 30.2; without the 10 %, one block
-// of fp8 28672 x 8192 at 1 row 38.3 -> 38.0 / 71 -> 79; of seven blocks, which deal 28672 columns evenly, fp8 gate + up at 12 rows
-// 80 -> 77 / 142 -> 146: not taken]
-int width_for(int M, int N, int split_k, bool fused) {
-  int best = 1;
-  int64_t least = INT64_MAX;
-  for (int width : {4, 3, 2, 1}) {
-    const int64_t groups = (int64_t)((N + 16 * width - 1) / (16 * width)) * split_k;
-    const int64_t most = ((groups + 255) / 256 + (2 * groups + 255) / 256) * ((fused ? 32 : 16) * width + (M + 15) / 16 * 16);
-    if ((width > 1 && groups < 160) || (least < INT64_MAX && 10 * most > 9 * least)) continue;
-    best = width;
-    least = most;
-  }
-  return best;
+int width_for(int N, int split_k) {
+  for (int width = 4; width > 1; width /= 2)
+    if ((int64_t)((N + 16 * width - 1) / (16 * width)) * split_k >= 160) return width;
+  return 1;
 }
 
 template <bool FP8, bool FUSED>
 int dispatch(const StreamArgs& p, hipStream_t stream) {
-  const int width = width_for(p.side[0].M, p.N, p.split_k, FUSED);
+  const int width = width_for(p.N, p.split_k);
   if constexpr (!FUSED && !FP8)
     if (p.split_k > 1) return launch_rows<FP8, FUSED, true>(p, width, stream);
   return launch_rows<FP8, FUSED, false>(p, width, stream);

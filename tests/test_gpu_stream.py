@@ -87,9 +87,9 @@ def test_tiles_of_64_rows(M, N, K):
     assert torch.equal(ops.linear_variant(few, w, 6), whole[0][:40])
 
 
-# 256 and 161 tiles of three blocks, the last one ragged, whole and in two parts
+# columns of which 256 compute units get uneven shares, the last tile ragged or not, whole and in two parts
 @pytest.mark.parametrize("M,N,K", [(1, 12280, 1024), (16, 12288, 1088), (32, 12264, 2048), (17, 6136, 4096), (24, 7720, 2112)])
-def test_tiles_of_three_blocks(M, N, K):
+def test_columns_dealt_unevenly(M, N, K):
     """Within the bound of the other few-row launches of the fp32 product, bf16 and fp8."""
     from dynaflow_amd import ops
     from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
@@ -107,3 +107,29 @@ def test_tiles_of_three_blocks(M, N, K):
         y = ops.linear_fp8(xq, wq, xs, ws)
         want = (xq.float() * xs) @ (wq.float() * ws[:, None]).t()
         assert (y.float() - want).abs().max().item() <= 2.0 ** -6 * want.abs().max().item()
+
+
+# 18496 .. 20480 columns are between one and a half and two rounds of the compute units; 16 and 17 rows are one and two blocks
+@pytest.mark.parametrize("N,K", [(18944, 3584), (18496, 4096), (20480, 4096)])
+def test_the_order_of_sums_is_that_of_the_columns(N, K):
+    """Whatever the rows are and whether gate and up come in one launch: the fused launch has the bits of the separate ones,
+    and rows of a launch of 17 those of a launch of 16 and of one (bf16 throughout, fp8 where both are streamed).  Operands over
+    many binades, so that the order of the fp32 sums shows."""
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
+
+    spread = lambda shape, seed: randn(shape, seed) * torch.exp2(randn(shape, seed + 50, 4.0))
+    x, gate, up = spread((17, K), 1), spread((N, K), 2), spread((N, K), 3)
+    fused = {M: ops.gate_up_silu(x[:M], gate, up) for M in (1, 16, 17)}
+    for M, got in fused.items():
+        assert torch.equal(got, ops.silu_mul(ops.linear(x[:M], gate), ops.linear(x[:M], up), True)), M
+        assert torch.equal(got, fused[17][:M]), M
+    xq, xs = ops.quant_fp8(x)
+    (wq, ws), (uq, us) = quantize_weight_per_channel(gate), quantize_weight_per_channel(up)
+    y = {M: ops.linear_fp8(xq[:M], wq, xs, ws) for M in (1, 16, 17)}
+    for M in (1, 16, 17):
+        q, scale = ops.gate_up_silu_quant_fp8(xq[:M], wq, uq, xs, ws, us)
+        want_q, want_scale = ops.silu_mul_quant_fp8(y[M], ops.linear_fp8(xq[:M], uq, xs, us))
+        assert torch.equal(scale, want_scale) and torch.equal(q.view(torch.uint8), want_q.view(torch.uint8)), M
+        if K >= 4096:
+            assert torch.equal(y[M], y[17][:M]), M
