@@ -221,10 +221,17 @@ rope_bf16_kernel(const uint16_t* __restrict__ x, int64_t ld_x, uint16_t* __restr
   *reinterpret_cast<u32x4*>(out + (int64_t)row * ld_out + lo_off + half) = ohi;
 }
 
-__global__ void __launch_bounds__(256) fill_u32_kernel(uint32_t* dst, uint32_t value, int64_t count) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (int64_t)gridDim.x * 256)
-    dst[i] = value;
-}
+struct FillU32 {
+  static constexpr int THREADS = 256;
+  uint32_t* dst;
+  int64_t count;
+  uint32_t value;
+  DFHIP_DEVICE void run(unsigned block, unsigned blocks) const {
+    for (int64_t i = (int64_t)block * THREADS + threadIdx.x; i < count; i += (int64_t)blocks * THREADS) dst[i] = value;
+  }
+  bool beside(const FillU32& other) const { return dst != other.dst; }
+};
+__global__ void __launch_bounds__(256) fill_u32_kernel(const FillU32 p) { p.run(blockIdx.x, gridDim.x); }
 
 int check_rowwise(const void* gate, int64_t ld_gate, const void* up, int64_t ld_up, const void* out,
                   int64_t ld_out, int M, int D, int vec) {
@@ -305,8 +312,11 @@ extern "C" int dfhip_fill_u32(void* dst, uint32_t value, int64_t count, dfhip_st
   if (count < 1) return DFHIP_ERR_BAD_SHAPE;
   int64_t blocks = (count + 255) / 256;
   if (blocks > 1024) blocks = 1024;
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(fill_u32_kernel), dfhip_join_beside<FillU32>,
+                                            DFHIP_SHORT_BLOCKS), true);
+  (void)known;
   hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     static_cast<uint32_t*>(dst), value, count);
+                     FillU32{static_cast<uint32_t*>(dst), count, value});
   return dfhip_check_launch();
 }
 

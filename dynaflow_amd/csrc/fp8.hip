@@ -75,25 +75,6 @@ DFHIP_DEVICE uint32_t quant4(float a, float b, float c, float d, float scale) {
   return r;
 }
 
-// q = e4m3fn(x / scale), scale = max(amax, 1e-12) / 448; group = 8 values -> 8 bytes
-__global__ void __launch_bounds__(QT)
-quant_fp8_bf16_kernel(const uint16_t* __restrict__ x, int64_t ld, uint8_t* __restrict__ q, int64_t ld_q,
-                      uint32_t groups, uint32_t per_row, const float* __restrict__ amax,
-                      float* __restrict__ scale_out) {
-  const float scale = fmaxf(amax[0], 1e-12f) / FP8_MAX;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && scale_out != nullptr) scale_out[0] = scale;
-  for (uint32_t gi = blockIdx.x * QT + threadIdx.x; gi < groups; gi += gridDim.x * QT) {
-    const uint32_t row = gi / per_row, col = (gi - row * per_row) * 8;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(x + (int64_t)row * ld + col);
-    u32x2 o;
-    o[0] = quant4(bf16_bits_to_f32(v[0] & 0xffffu), __uint_as_float(v[0] & 0xffff0000u),
-                  bf16_bits_to_f32(v[1] & 0xffffu), __uint_as_float(v[1] & 0xffff0000u), scale);
-    o[1] = quant4(bf16_bits_to_f32(v[2] & 0xffffu), __uint_as_float(v[2] & 0xffff0000u),
-                  bf16_bits_to_f32(v[3] & 0xffffu), __uint_as_float(v[3] & 0xffff0000u), scale);
-    *reinterpret_cast<u32x2*>(q + (int64_t)row * ld_q + col) = o;
-  }
-}
-
 // out = bf16(silu(g) * u) (optional store) and amax over the rounded values
 __global__ void __launch_bounds__(QT)
 silu_mul_absmax_kernel(const uint16_t* __restrict__ gate, int64_t ld_gate, const uint16_t* __restrict__ up,
@@ -204,8 +185,8 @@ template <bool FLAT, bool SILU>
 __global__ void __launch_bounds__(QT) absmax_parts_kernel(const AbsmaxParts<FLAT, SILU> p) { p.run(blockIdx.x, gridDim.x); }
 
 // q = e4m3fn(x / scale), scale = max(amax, 1e-12) / 448.  PARTS: amax is the maximum of n_parts values; else `amax` is one
-// value, which the last block to have read it clears, with the count of those that have: the cells are zero again for the
-// launch that folds the next maximum into them.
+// value, and with `readers` the last block to have read it clears it and the count of those that have: the cells are zero
+// again for the launch that folds the next maximum into them.
 template <bool FLAT, bool PARTS>
 DFHIP_DEVICE void quant_after(unsigned block, unsigned blocks, const uint16_t* __restrict__ x, int64_t ld,
                               uint8_t* __restrict__ q, int64_t ld_q, uint32_t groups, uint32_t per_row,
@@ -234,7 +215,7 @@ DFHIP_DEVICE void quant_after(unsigned block, unsigned blocks, const uint16_t* _
     if (threadIdx.x == 0) cell = __hip_atomic_load(amax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     m = cell;
-    if (threadIdx.x == 0 && atomicAdd(readers, 1) == (int)blocks - 1) {
+    if (readers && threadIdx.x == 0 && atomicAdd(readers, 1) == (int)blocks - 1) {
       __hip_atomic_store(amax, 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(readers, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -1073,19 +1054,6 @@ extern "C" int dfhip_absmax_bf16(const void* x, int64_t ld, int M, int D, float*
   return dfhip_check_launch();
 }
 
-extern "C" int dfhip_quant_fp8_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D,
-                                    const float* amax, float* scale_out, dfhip_stream_t stream) {
-  if (int rc = check_q(x, ld, M, D)) return rc;
-  if (!q || !amax) return DFHIP_ERR_NULL_POINTER;
-  if (ld_q < D) return DFHIP_ERR_BAD_STRIDE;
-  if (ld_q % 8 || (reinterpret_cast<uintptr_t>(q) & 7u)) return DFHIP_ERR_BAD_ALIGNMENT;
-  const uint32_t per_row = D / 8, groups = (uint32_t)M * per_row;
-  hipLaunchKernelGGL(quant_fp8_bf16_kernel, dim3(grid_for(groups)), dim3(QT), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(x), ld, static_cast<uint8_t*>(q), ld_q, groups, per_row, amax,
-                     scale_out);
-  return dfhip_check_launch();
-}
-
 namespace {
 unsigned parts_for(uint32_t groups) {
   const uint32_t blocks = (groups + QT * QUNROLL - 1) / (QT * QUNROLL);
@@ -1117,6 +1085,15 @@ int launch_absmax_parts(const void* x, int64_t ld, const void* up, int64_t ld_up
                              parts_for(groups), stream);
 }
 }  // namespace
+
+extern "C" int dfhip_quant_fp8_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D,
+                                    const float* amax, float* scale_out, dfhip_stream_t stream) {
+  if (int rc = check_q(x, ld, M, D)) return rc;
+  if (!amax) return DFHIP_ERR_NULL_POINTER;
+  if (int rc = check_q_out(q, ld_q, D)) return rc;
+  return launch_quant_after<false>(x, ld, q, ld_q, M, D, const_cast<float*>(amax), 0, nullptr, scale_out,
+                                   static_cast<hipStream_t>(stream));
+}
 
 extern "C" int dfhip_quant_fp8_dynamic_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, float* parts,
                                             float* scale_out, dfhip_stream_t stream) {

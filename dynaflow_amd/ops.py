@@ -734,11 +734,6 @@ torch.library.register_fake(
 # --------------------------------------------------------------------- fp8
 #: DFHIP_FP8_PARTS: floats in which the blocks of a quantisation leave their maxima
 _FP8_PARTS = 1024
-#: cells that a fused launch folds max |act| into, and the count of blocks that have read it: zero between launches.
-#: Keyed like the split-K workspaces.
-_amax_cells: dict[tuple, torch.Tensor] = {}
-#: held from the launch that folds into a cell to the one that clears it again: threads that share a stream
-_amax_pair = threading.Lock()
 
 
 def _quant_fp8_impl(x: torch.Tensor):
@@ -797,22 +792,22 @@ def _gate_up_silu_quant_fp8_impl(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w
         wg, wu = wg.contiguous(), wu.contiguous()
         ldg = K
     act = torch.empty((M, I), dtype=torch.bfloat16, device=x_q.device)
-    scale = torch.empty(1, dtype=torch.float32, device=x_q.device)
+    # The scale, and the cell that the fused launch folds max |act| into: memory of this call (or of the graph that it is
+    # captured into), so that nothing else, on whatever stream, folds into it or clears it in between.
+    scale = torch.empty(2, dtype=torch.float32, device=x_q.device)
     q = torch.empty((M, I), dtype=FP8_DTYPE, device=x_q.device)
     if M > 0:
         gate_scale, up_scale, stream = w_gate_scale.contiguous(), w_up_scale.contiguous(), _stream()
-        with _amax_pair:
-            cells = _zeroed_workspace(_amax_cells, x_q.device, stream, 256, 256)
-            rc = lib.dfhip_gemm_fp8_gate_up_silu_absmax_shared(
-                a.data_ptr(), lda, wg.data_ptr(), wu.data_ptr(), ldg, act.data_ptr(), I, x_scale.data_ptr(),
-                gate_scale.data_ptr(), up_scale.data_ptr(), cells.data_ptr(), M, I, K, _side_by_side(), stream,
-            )
-            _cabi.check("dfhip_gemm_fp8_gate_up_silu_absmax_shared", rc)
-            rc = lib.dfhip_requant_fp8_bf16(act.data_ptr(), I, q.data_ptr(), I, M, I, cells.data_ptr(), scale.data_ptr(),
-                                            stream)
-            if rc != 0:
-                lib.dfhip_fill_u32(cells.data_ptr(), 0, 2, stream)
-            _cabi.check("dfhip_requant_fp8_bf16", rc)
+        amax = scale.data_ptr() + 4
+        _cabi.check("dfhip_fill_u32", lib.dfhip_fill_u32(amax, 0, 1, stream))
+        rc = lib.dfhip_gemm_fp8_gate_up_silu_absmax_shared(
+            a.data_ptr(), lda, wg.data_ptr(), wu.data_ptr(), ldg, act.data_ptr(), I, x_scale.data_ptr(),
+            gate_scale.data_ptr(), up_scale.data_ptr(), amax, M, I, K, _side_by_side(), stream,
+        )
+        _cabi.check("dfhip_gemm_fp8_gate_up_silu_absmax_shared", rc)
+        rc = lib.dfhip_quant_fp8_bf16(act.data_ptr(), I, q.data_ptr(), I, M, I, amax, scale.data_ptr(), stream)
+        _cabi.check("dfhip_quant_fp8_bf16", rc)
+    scale = scale[:1]
     return q.view(*x_q.shape[:-1], I), scale
 
 

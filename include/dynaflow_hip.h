@@ -442,8 +442,10 @@ int dfhip_silu_mul_absmax_bf16(const void* gate, int64_t ld_gate, const void* up
  * (DFHIP_FP8_PARTS floats, contents of no matter before and after).
  * The same codes and scale as the pairs of calls above.
  * dfhip_silu_mul_quant_fp8_bf16: act = bf16(silu(gate) * up) [M, D] is written on the way.
- * dfhip_requant_fp8_bf16: the launch behind dfhip_gemm_fp8_gate_up_silu_absmax; cells = the amax that one folded
- * its maximum into, followed by a 32-bit count; both zero before, and zero again when this launch is done. */
+ * dfhip_requant_fp8_bf16: the launch behind dfhip_gemm_fp8_gate_up_silu_absmax where that has no cell of its own to
+ * be cleared first; cells = the amax that one folded its maximum into, followed by a 32-bit count; both zero before,
+ * and zero again when this launch is done.  From the fold to the end of this launch they are nobody else's: launches on
+ * other streams, and graphs that may replay at the same time, need cells of their own. */
 #define DFHIP_FP8_PARTS 1024
 int dfhip_quant_fp8_dynamic_bf16(const void* x, int64_t ld, void* q, int64_t ld_q, int M, int D, float* parts,
                                  float* scale_out, dfhip_stream_t stream);
