@@ -49,7 +49,8 @@ def attend_and_append(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
     """Rotate q and k of the new tokens, append k and v to the caches, attend over the cache.
 
     Token t belongs to cache slot ``slots[t]``, sits at position ``lengths[t] - 1`` and attends to
-    positions ``0 .. lengths[t] - 1``.  qkv is ``[T, (q_heads + 2 kv_heads) * 128]``.
+    positions ``0 .. lengths[t] - 1``.  qkv is ``[T, (q_heads + 2 kv_heads) * 128]``.  The tokens of a forward,
+    over all its nano-batches, name distinct slots: their launches are not ordered among each other.
 
     Declared as an operator that mutates the two caches: a function that writes to its inputs must not
     be handed to dynamo as a plain in-graph function.

@@ -315,6 +315,16 @@ class DynaFlowManager:
             output = run_coroutine(self._forward_async(args, kwargs, split))
         return graph, output
 
+    def _schedules_plainly(self) -> bool:
+        """Whether the scheduler issues its operators, and nothing else, the way the shipped ones do: on the streams of
+        ``stream_policy``."""
+        from dynaflow_amd.schedulers import MLPOverlapScheduler, StaggeredScheduler
+
+        kind, own = type(self.scheduler), vars(self.scheduler)
+        return (issubclass(kind, StaggeredScheduler) and kind.schedule in (StaggeredScheduler.schedule, MLPOverlapScheduler.schedule)
+                and kind._issue is StaggeredScheduler._issue and kind._stream_for is StaggeredScheduler._stream_for
+                and not {"schedule", "_issue", "_stream_for"} & own.keys())
+
     def _capture_paired(self, args: tuple, kwargs: dict, split: SplitConfig, caller, origin, capture_on: dict) -> tuple:
         """The schedule with the launches of two nano-batches against the same weights as one: (graph, output, pairs);
         the graph is None where nothing is to be gained by pairs or it failed half-way.
@@ -327,10 +337,15 @@ class DynaFlowManager:
         assert self.config is not None and self.scheduler is not None
         policy = getattr(self.scheduler, "stream_policy", None)
         one_stream = getattr(self.scheduler, "comp_stream", None) is getattr(self.scheduler, "comm_stream", None)
+        kept = None if self._schedules_plainly() else type(self.scheduler).__name__
+        kept = kept or capture_plan.needs_its_order(self.graph_module)
         # (a collective looks like a short launch and waits for other ranks: what ran beside it stays beside it)
         several_ranks = torch.distributed.is_available() and torch.distributed.is_initialized() and \
             torch.distributed.get_world_size() > 1
         if not self.config.knob("pair_launches", True) or self.config.knob("cu_split", None) or one_stream or several_ranks:
+            return None, None, 0
+        if kept is not None:
+            log.info("launches are not paired: %s", kept)
             return None, None, 0
         if policy == "by_nano_batch":
             graph, output = self._capture(args, kwargs, split, capture_on)

@@ -381,7 +381,8 @@ int dfhip_causal_attention_ragged_bf16(const void* q, int64_t ld_q, const void* 
  *   nano-batch of a decode step, and no q_out buffer.
  * The tokens of one call (and of calls that run at the same time) name distinct slots: a decode
  *   step has one new token per sequence, and two tokens of one slot would append to and read one
- *   cache concurrently. */
+ *   cache concurrently.  The calls of a forward's nano-batches count as calls that run at the same
+ *   time whatever streams they are issued on: dfhip_graph_pair_launches joins them. */
 int dfhip_rope_kv_append_bf16(const void* qkv, int64_t ld_qkv, void* q_out, int64_t ld_q, void* k_cache,
                               void* v_cache, const int32_t* slots, const int32_t* lengths,
                               const float* cos_table, const float* sin_table, int T, int q_heads, int kv_heads,

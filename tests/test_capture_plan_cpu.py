@@ -111,3 +111,97 @@ def test_multi_layer_schedule_by_kind_is_captured_from_its_main_stream(host_devi
 def test_multi_layer_schedule_by_nano_batch(host_device):
     log = decode_log(host_device, streams="by_nano_batch")
     assert plan.choose_origin(log, "default") == "default"
+
+
+# ------------------------------------------------------------ which schedules may be put in another order
+class Scratch(torch.nn.Module):
+    """Both nano-batches write to one buffer and read it again."""
+
+    def __init__(self):
+        super().__init__()
+        self.weight = torch.nn.Parameter(torch.ones(8, 8))
+        self.register_buffer("last", torch.zeros(8))
+
+    def forward(self, x):
+        self.last.copy_(x[0])
+        return torch.nn.functional.silu(x) + self.last
+
+
+def split_graph_of(fn, lowered=False):
+    """A split graph as the manager leaves it: its sub-graph calls run what stands in their backends."""
+    from types import SimpleNamespace
+
+    from dynaflow_amd.executor.hip_lowering import lower_to_hip
+
+    inner = fn if isinstance(fn, torch.fx.GraphModule) else torch.fx.symbolic_trace(fn)
+    if lowered:
+        inner = lower_to_hip(inner)[0]
+    graph = torch.fx.Graph()
+    x = graph.placeholder("x")
+    graph.output(graph.call_module("submod_0", (x,)))
+    outer = torch.fx.GraphModule({"submod_0": torch.nn.Identity()}, graph)
+    del outer._modules["submod_0"]
+    outer.__dict__["submod_0"] = SimpleNamespace(callable_dynamic=inner, callables_per_size={})
+    return outer
+
+
+@pytest.mark.parametrize("fn,kept", [
+    (lambda x: torch.nn.functional.rms_norm(x, (8,)) + x.view(2, 4).reshape(8) * 2, False),
+    (lambda x: torch.cat([x.split(4, -1)[0], x.float()], dim=-1), False),
+    (lambda x: torch.nn.functional.embedding(x, x), False),
+    (lambda x: torch.nn.functional.embedding(x, x, None, 1.0), True),            # renormalises the table in place
+    (lambda x: torch.nn.functional.embedding(x, x, max_norm=1.0), True),
+    (lambda x: torch.nn.functional.silu(x, True), True),
+    (lambda x: torch.add(x, 1, out=x), True),
+    (lambda x: x.mul_(2), True),
+    (lambda x: torch.relu_(x), True),
+    (lambda x: torch.sort(x)[0], True),                                          # a launch of unknown length
+    (lambda x: torch.nn.functional.linear(x, x), True),
+    (lambda x: torch.nn.functional.dropout(x), True),
+    (Scratch(), True),
+])
+def test_what_needs_its_order(fn, kept):
+    assert (plan.needs_its_order(split_graph_of(fn)) is not None) == kept
+
+
+def test_in_place_operators_and_opaque_callables_keep_their_order():
+    import operator
+    from types import SimpleNamespace
+
+    for target in (operator.iadd, operator.setitem, lambda x: x):
+        graph = torch.fx.Graph()
+        x = graph.placeholder("x")
+        graph.output(graph.call_function(target, (x, x, x)))
+        assert plan.needs_its_order(split_graph_of(torch.fx.GraphModule({}, graph))) is not None
+    outer = split_graph_of(lambda x: x + 1)
+    outer.__dict__["submod_0"] = SimpleNamespace(callable_dynamic=lambda x: x, callables_per_size={})
+    assert plan.needs_its_order(outer) is not None
+    # a callable for one size, and what a graph wrapper runs
+    outer.__dict__["submod_0"] = SimpleNamespace(callable_dynamic=torch.fx.symbolic_trace(lambda x: x + 1),
+                                                 callables_per_size={4: torch.fx.symbolic_trace(lambda x: x.mul_(2))})
+    assert plan.needs_its_order(outer) is not None
+    outer.__dict__["submod_0"] = SimpleNamespace(
+        callable_dynamic=SimpleNamespace(runnable=torch.fx.symbolic_trace(lambda x: x + 1)), callables_per_size={})
+    assert plan.needs_its_order(outer) is None
+
+
+def test_lowered_models_do_not_need_their_order():
+    """The decode model: embedding, norms, projections, the attention that writes to the slots of its tokens."""
+    from dynaflow_amd.decode import DecodeModel
+
+    captured = {}
+    model = DecodeModel(layers=2, vocab=100, hidden=512, heads=4, kv_heads=2, inter=256, slots=6, capacity=64, dtype=torch.bfloat16)
+    model.init_weights()
+    inputs = [torch.arange(6), torch.arange(6).int(), torch.full((6,), 5).int()]
+
+    def backend(gm, example_inputs):
+        captured["gm"] = gm
+        return gm
+
+    torch._dynamo.reset()
+    for t in inputs:
+        torch._dynamo.mark_dynamic(t, 0)
+    torch.compile(model, backend=backend, fullgraph=True)(*inputs)
+    assert plan.needs_its_order(split_graph_of(captured["gm"], lowered=True)) is None
+    # the same on torch's own kernels
+    assert plan.needs_its_order(split_graph_of(captured["gm"])) is not None

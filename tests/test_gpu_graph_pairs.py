@@ -11,6 +11,7 @@ from dynaflow_amd.config import CUDAGraphConfig, DynaFlowConfig, InductorConfig
 from dynaflow_amd.fp8_mlp import Fp8SwiGLU
 from dynaflow_amd.manager import DynaFlowManager
 from dynaflow_amd.mlp import SwiGLUMLP
+from dynaflow_amd.schedulers import MLPOverlapScheduler
 
 
 def test_arguments():
@@ -24,9 +25,9 @@ def randn(shape, seed, std=1.0):
     return (torch.randn(shape, generator=g, device="cuda") * std).bfloat16()
 
 
-def program(model, tokens, **knobs):
+def program(model, tokens, scheduler="dynaflow_amd.schedulers:MLPOverlapScheduler", **knobs):
     manager = DynaFlowManager()
-    cfg = DynaFlowConfig("dynaflow_amd.schedulers:MLPOverlapScheduler", 4, InductorConfig(enabled=True),
+    cfg = DynaFlowConfig(scheduler, 4, InductorConfig(enabled=True),
                          CUDAGraphConfig(enabled=False, capture_sizes=[tokens]),
                          {"min_nano_split_tokens": 1, "num_nano_batches": 2, "dump_graph": False, "whole_graph": True,
                           "streams": "by_nano_batch", "fuse_silu_epilogue": True, **knobs})
@@ -117,4 +118,50 @@ def test_other_schedules_stay_as_they_are(tokens, knobs):
     want = forward(manager, compiled, x, False).clone()
     for _ in range(3):
         assert torch.equal(forward(manager, compiled, x, True), want)
+    assert list(manager.paired_launches.values()) == [0]
+
+
+class WritesBetween(SwiGLUMLP):
+    """Each nano-batch leaves its first row in one buffer and adds it to its result."""
+
+    def __init__(self, hidden, inter):
+        super().__init__(hidden, inter, dtype=torch.bfloat16, device="cuda")
+        self.hidden = hidden
+        self.register_buffer("first", torch.zeros(hidden, dtype=torch.bfloat16, device="cuda"))
+
+    def forward(self, x):
+        y = super().forward(x)
+        self.first.copy_(x[0])
+        return y + self.first
+
+
+@pytest.mark.gpu
+def test_a_buffer_of_both_nano_batches_keeps_the_order_of_the_schedule():
+    """Streams by kind run the two writers one after the other, each in front of its reader; so does the captured schedule."""
+    model = WritesBetween(2048, 5632)
+    with torch.no_grad():
+        for p, (shape, seed) in zip(model.parameters(), (((5632, 2048), 2), ((5632, 2048), 3), ((2048, 5632), 4))):
+            assert tuple(p.shape) == shape
+            p.copy_(randn(shape, seed, 0.03))
+    manager, compiled = program(model, 64, streams="by_kind")
+    for seed in (5, 6):
+        x = randn((64, 2048), seed)
+        want = forward(manager, compiled, x, False).clone()
+        for _ in range(3):
+            assert torch.equal(forward(manager, compiled, x, True), want)
+    assert list(manager.paired_launches.values()) == [0]
+
+
+class OwnSchedule(MLPOverlapScheduler):
+    async def schedule(self, context):
+        await super().schedule(context)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("streams", ["by_kind", "by_nano_batch"])
+def test_a_scheduler_of_its_own_keeps_its_schedule(streams):
+    manager, compiled = program(mlp("bf16", 2048, 5632), 64, "test_gpu_graph_pairs:OwnSchedule", streams=streams)
+    x = randn((64, 2048), 5)
+    want = forward(manager, compiled, x, False).clone()
+    assert torch.equal(forward(manager, compiled, x, True), want)
     assert list(manager.paired_launches.values()) == [0]
