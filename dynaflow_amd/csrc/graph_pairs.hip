@@ -150,9 +150,11 @@ extern "C" int dfhip_graph_pair_launches(void* graph, int side_by_side, int* pai
       b.pair = (int)i;
       found += a.known.in_line == 0;
     }
-    // a launch that would lose its company
-    if (blocks_of(a) > a.known.in_line && (a.pair < 0 || (side_by_side && a.known.in_line > 0))) return DFHIP_OK;
   }
+  // launches that would lose their company
+  for (const Node& node : nodes)
+    if (node.kernel && blocks_of(node) > node.known.in_line && (node.pair < 0 || (side_by_side && node.known.in_line > 0)))
+      return DFHIP_OK;
   if (!found) return DFHIP_OK;
   const std::vector<int> order = order_of(nodes, edges);
   if (order.empty()) return DFHIP_OK;                                 // two pairs that wait for each other crosswise

@@ -8,6 +8,7 @@ import torch
 from dynaflow_amd import _cabi
 from dynaflow_amd.backend import make_backend
 from dynaflow_amd.config import CUDAGraphConfig, DynaFlowConfig, InductorConfig
+from dynaflow_amd.decode import DecodeModel
 from dynaflow_amd.fp8_mlp import Fp8SwiGLU
 from dynaflow_amd.manager import DynaFlowManager
 from dynaflow_amd.mlp import SwiGLUMLP
@@ -165,3 +166,57 @@ def test_a_scheduler_of_its_own_keeps_its_schedule(streams):
     want = forward(manager, compiled, x, False).clone()
     assert torch.equal(forward(manager, compiled, x, True), want)
     assert list(manager.paired_launches.values()) == [0]
+
+
+# ------------------------------------------------------------------------------------------------ decode steps
+def decode_program(T, capacity, streams, hidden=4096, heads=32, kv_heads=8, inter=4096, layers=2):
+    model = DecodeModel(layers=layers, vocab=512, hidden=hidden, heads=heads, kv_heads=kv_heads, inter=inter, slots=T + 3,
+                        capacity=capacity, dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad():
+        for seed, p in enumerate(model.parameters()):
+            if p.dim() > 1:
+                p.copy_(randn(p.shape, 20 + seed, 1.0 if p is model.embed else 0.03))
+        for block in model.attn:
+            block.k_cache.copy_(randn(block.k_cache.shape, 60))
+            block.v_cache.copy_(randn(block.v_cache.shape, 61))
+    manager = DynaFlowManager()
+    cfg = DynaFlowConfig("dynaflow_amd.schedulers:DecoderOverlapScheduler", 2, InductorConfig(enabled=True),
+                         CUDAGraphConfig(enabled=False, capture_sizes=[T // 2, T - T // 2, T]),
+                         {"min_nano_split_tokens": 1, "dump_graph": False, "whole_graph": True, "streams": streams,
+                          "fuse_silu_epilogue": True})
+    step = step_inputs(T, capacity, 1)
+    torch._dynamo.reset()
+    for t in step:
+        torch._dynamo.mark_dynamic(t, 0)
+    compiled = torch.compile(model, backend=make_backend(manager, cfg), fullgraph=True)
+    with torch.no_grad():
+        manager.prepare(T, [1] * T)
+        compiled(*step)
+    return model, manager, compiled
+
+
+def step_inputs(T, capacity, seed):
+    """Sequences of 1 to `capacity` positions, the shortest and the longest among them, in slots of any order."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    lengths = torch.randint(1, capacity + 1, (T,), generator=g, device="cuda").int()
+    lengths[T // 3], lengths[-1] = 1, capacity
+    return [torch.randint(0, 512, (T,), generator=g, device="cuda"),
+            torch.randperm(T + 3, generator=g, device="cuda")[:T].int(), lengths]
+
+
+def step(manager, compiled, inputs, graph):
+    with torch.no_grad():
+        manager.prepare(len(inputs[0]), [1] * len(inputs[0]), use_cudagraph=graph)
+        return compiled(*inputs).clone()
+
+
+# 26 sequences with 20 kv heads are 520 workgroups of attention, the other 25 of 51 are 500
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,joined", [(50, True), (51, False), (52, False)])
+def test_long_attention_of_either_side_keeps_a_schedule_with_a_stream_per_nano_batch(T, joined):
+    model, manager, compiled = decode_program(T, 128, "by_nano_batch", hidden=2048, heads=20, kv_heads=20, inter=2048)
+    inputs = step_inputs(T, 128, 2)
+    want = step(manager, compiled, inputs, False)
+    for _ in range(2):
+        assert torch.equal(step(manager, compiled, inputs, True), want)
+    assert [n > 0 for n in manager.paired_launches.values()] == [joined]
