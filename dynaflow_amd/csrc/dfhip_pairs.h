@@ -53,6 +53,12 @@ typedef bool (*DfhipJoin)(const void* a, const void* b, dim3 ga, dim3 gb, void* 
 constexpr size_t DFHIP_PAIR_MAX_ARGS = 512;
 constexpr unsigned DFHIP_SHORT_BLOCKS = 512;     // also that of a kernel that is not known
 void dfhip_pairable(const void* kernel, DfhipJoin join, unsigned in_line = 0);
+// A long kernel of which there is no launch of two: a graph that holds one stays as it is.
+#define DFHIP_NOT_IN_LINE(kernel) \
+  do { \
+    static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), nullptr), true); \
+    (void)known; \
+  } while (0)
 inline bool dfhip_same(dim3 a, dim3 b) { return a.x == b.x && a.y == b.y && a.z == b.z; }
 
 // A launch without weights is K::run(workgroup) of K::THREADS threads; two of them sit one behind the other.

@@ -689,6 +689,7 @@ int launch_fp8_ring(const void* A, int64_t lda, const void* W, int64_t ldw, void
   auto kernel = gemm_fp8_ring_kernel<false, TM, SPLIT>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), F8_RING_LDS, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(kernel);
   const int tiles_m = (M + 32 * TM - 1) / (32 * TM), tiles_n = (N + 255) / 256;
   float* partials = nullptr;
   if (SPLIT) {
@@ -710,6 +711,7 @@ int launch_fp8_ring_fused(const void* A, int64_t lda, const void* Wg, const void
   auto kernel = gemm_fp8_ring_kernel<true, TM, false>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), F8_RING_LDS, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(kernel);
   const int tiles_m = (M + 32 * TM - 1) / (32 * TM), tiles_n = (I + 127) / 128;
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(256), F8_RING_LDS, stream,
                      static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(Wg), static_cast<const uint8_t*>(Wu),
@@ -896,6 +898,7 @@ int launch_fp8_ring224(const void* A, int64_t lda, const void* W, int64_t ldw, v
                        const float* a_scale, const float* w_scale, int M, int N, int K, hipStream_t stream) {
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(gemm_fp8_ring224_kernel), F8_RING_LDS, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(gemm_fp8_ring224_kernel);
   const int tiles_m = (M + 255) / 256, tiles_n = (N + F8_TBN - 1) / F8_TBN;
   hipLaunchKernelGGL(gemm_fp8_ring224_kernel, dim3(tiles_m * tiles_n), dim3(256), F8_RING_LDS, stream,
                      static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(W), static_cast<uint16_t*>(C),
@@ -910,6 +913,7 @@ int launch_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, 
   auto kernel = gemm_fp8_nt_kernel<BM, BN>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), LDS_BYTES, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(kernel);
   const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(256), LDS_BYTES, stream, static_cast<const uint8_t*>(A),
                      static_cast<const uint8_t*>(W), static_cast<uint16_t*>(C), a_scale, w_scale, M, N, K, lda, ldw,

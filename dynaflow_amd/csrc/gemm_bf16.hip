@@ -579,6 +579,7 @@ int launch_ring(const void* A, int64_t lda, const void* W, const void* W2, int64
   auto kernel = gemm_bf16_ring_kernel<FUSED>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), RING_LDS, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(kernel);
   const int tiles_m = (M + RBM - 1) / RBM;
   const int tiles_n = FUSED ? (N + 127) / 128 : (N + RBN - 1) / RBN;
   int* arrivals = static_cast<int*>(workspace);
@@ -836,6 +837,7 @@ int launch_ring224(const void* A, int64_t lda, const void* W, const void* W2, in
   auto kernel = gemm_bf16_ring224_kernel<FUSED, TN, TM>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), RING_LDS, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(kernel);
   constexpr int OUT_N = FUSED ? TN / 2 : TN;
   const int tiles_m = (M + TM - 1) / TM;
   const int tiles_n = (N + OUT_N - 1) / OUT_N;
@@ -1150,6 +1152,7 @@ int launch_walk(const void* A, int64_t lda, const void* W, const void* W2, int64
   auto kernel = gemm_bf16_gate_up_silu_walk_kernel;
   static std::atomic<uint64_t> lds_opted_in{0};
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), RING_LDS, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(kernel);
   const int tiles_m = M / RBM, tiles_n = N / (TBN / 2);
   int grid = compute_units_of_current_device() / 8 * 8;   // one workgroup per compute unit, a multiple of the XCDs
   if (grid < 8) return DFHIP_ERR_NO_DEVICE;
@@ -1703,6 +1706,7 @@ int launch(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int6
   auto kernel = gemm_bf16_nt_kernel<BM, BN, WAVES_M, WAVES_N>;
   static std::atomic<uint64_t> lds_opted_in{0};   // per instantiation, one bit per device
   if (int rc = dfhip_opt_in_lds(reinterpret_cast<const void*>(kernel), S::LDS_BYTES, lds_opted_in)) return rc;
+  DFHIP_NOT_IN_LINE(kernel);
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = (N + BN - 1) / BN;
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(S::THREADS), S::LDS_BYTES, stream,

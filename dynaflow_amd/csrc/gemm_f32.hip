@@ -7,7 +7,7 @@
 // gemm_f32_nt_kernel (v_mfma_f32_32x32x2_f32, any K that is a multiple of 4; many rows with a K up to about 3000): a
 //   128x128 tile per workgroup, K walked in slabs of 16 through one LDS buffer.  LDS rows hold 16 floats padded to 17 so
 //   that the 32 lanes of a fragment read (one float each, rows 17 words apart) hit 32 different banks.
-#include "dfhip_common.h"
+#include "dfhip_pairs.h"
 
 namespace {
 
@@ -200,7 +200,9 @@ int64_t split_tiles(const F32Args& p, int mb, int nb) {
 
 template <int MB, int NB, int DEPTH>
 int launch_split(const F32Args& p, hipStream_t stream) {
-  hipLaunchKernelGGL((gemm_f32_split_kernel<MB, NB, DEPTH>), dim3((unsigned)split_tiles(p, MB, NB)), dim3(SWAVES * 64), 0,
+  const auto kernel = gemm_f32_split_kernel<MB, NB, DEPTH>;
+  DFHIP_NOT_IN_LINE(kernel);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)split_tiles(p, MB, NB)), dim3(SWAVES * 64), 0,
                      stream, p.A, p.W, p.C, p.M, p.N, p.K / 32, p.lda, p.ldw, p.ldc, (p.M + 16 * MB - 1) / (16 * MB));
   return dfhip_check_launch();
 }
@@ -218,6 +220,7 @@ constexpr int SPLIT_MIN_K = 32 * SWAVES * 2;
 
 int launch_tile128(const F32Args& p, hipStream_t stream) {
   dim3 grid((p.N + FBN - 1) / FBN, (p.M + FBM - 1) / FBM);
+  DFHIP_NOT_IN_LINE(gemm_f32_nt_kernel);
   hipLaunchKernelGGL(gemm_f32_nt_kernel, grid, dim3(FTHREADS), 0, stream, p.A, p.W, p.C, p.M, p.N, p.K, p.lda, p.ldw, p.ldc);
   return dfhip_check_launch();
 }

@@ -391,6 +391,8 @@ int launch(const StreamArgs& p, hipStream_t stream) {
   if constexpr (MB <= 2) {
     static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), join_stream<FP8, MB, WIDTH, FUSED, SPLIT>), true);
     (void)known;
+  } else {
+    DFHIP_NOT_IN_LINE(kernel);
   }
   constexpr int COLS = 16 * WIDTH;
   hipLaunchKernelGGL(kernel, dim3((p.N + COLS - 1) / COLS * p.split_k), dim3(WAVES * 64),

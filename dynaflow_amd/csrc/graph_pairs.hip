@@ -11,7 +11,9 @@
 // fp8 254 / 170]
 //
 // Where every launch of a graph is one of a pair or short, nothing is left that gains from running side by side: the graph
-// becomes a chain, which saves the meetings of two queues (6 - 10 us each).  Any other graph stays as it is.  Short launches and
+// becomes a chain, which saves the meetings of two queues (6 - 10 us each).  Any other graph stays as it is: also one with a
+// GEMM that has no launch of two, however few its workgroups are; of kernels that are not of this library, those of up to 512
+// workgroups count as short, and the caller vouches for what they are.  Short launches and
 // attention over a cache pair as well (their workgroups side by side: one launch's gap less, and of attention one tail).
 // A schedule with a stream per nano-batch (`side_by_side`) runs long attention of one beside the projections of the other, which
 // is worth as much from 512 workgroups on: it stays.  [us of a decode step of 4 layers, sequences of 1/4 .. 1 of 4096 positions,

@@ -467,8 +467,9 @@ int dfhip_fill_u32(void* dst, uint32_t value, int64_t count, dfhip_stream_t stre
  * attention over a cache, each two become one launch (of projections, one whose workgroups read a weight together), and
  * the graph a chain of what is left, in an order that its edges allow.  Any other graph stays as it is, and with
  * side_by_side != 0 (two nano-batches run attention beside projections) also one with attention of more than 512
- * workgroups on either side.  *pairs: how many projections were joined.  Same results.  A negative status: the graph is of no use any
- * more. */
+ * workgroups on either side.  A GEMM of this library is never short; a kernel that is not of this library is where it has
+ * up to 512 workgroups, so the caller sees to it that no such kernel is long or waits for anything.  *pairs: how many projections
+ * were joined.  Same results.  A negative status: the graph is of no use any more. */
 int dfhip_graph_pair_launches(void* graph, int side_by_side, int* pairs);
 
 #ifdef __cplusplus

@@ -220,3 +220,42 @@ def test_long_attention_of_either_side_keeps_a_schedule_with_a_stream_per_nano_b
     for _ in range(2):
         assert torch.equal(step(manager, compiled, inputs, True), want)
     assert [n > 0 for n in manager.paired_launches.values()] == [joined]
+
+
+# ------------------------------------------------------------------------------------- graphs that a program captured itself
+def captured(first, second):
+    """`first` and `second` (lists of calls) on two streams of one graph: its handle, to be replayed after the pairing."""
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for s, calls in zip(streams, (first, second)):           # workspaces are made outside of the capture
+        with torch.cuda.stream(s):
+            for call in calls:
+                call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        start = torch.cuda.current_stream().record_event()
+        for s, calls in zip(streams, (first, second)):
+            with torch.cuda.stream(s):
+                s.wait_event(start)
+                for call in calls:
+                    call()
+                end = s.record_event()
+            torch.cuda.current_stream().wait_event(end)
+    pairs = ctypes.c_int(-1)
+    assert _cabi.load().dfhip_graph_pair_launches(graph.raw_cuda_graph(), 0, ctypes.byref(pairs)) == 0
+    graph.instantiate()
+    return graph, pairs.value
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("between", ["ring", "fp32"])
+def test_a_gemm_without_a_launch_of_two_keeps_the_graph(between):
+    """However few its workgroups are."""
+    from dynaflow_amd import ops
+
+    w, x = randn((1024, 1024), 1, 0.03), [randn((8, 1024), 3 + i) for i in range(2)]
+    other = (lambda: ops.linear_variant(x[0], w, 0)) if between == "ring" else (lambda: ops.linear(x[0].float(), w.float()))
+    kept = []
+    calls = [[lambda i=i: kept.append(ops.linear_variant(x[i], w, 8))] for i in range(2)]
+    assert captured(*calls)[1] == 1
+    assert captured(calls[0] + [lambda: kept.append(other())], calls[1])[1] == 0
