@@ -1,6 +1,7 @@
 """Launches of two nano-batches against the same weights as one, in a schedule captured as one graph: every replay has the bits
 of the eager schedule, and a schedule that is not all of such launches is left as it is."""
 import ctypes
+import re
 
 import pytest
 import torch
@@ -210,6 +211,42 @@ def step(manager, compiled, inputs, graph):
         return compiled(*inputs).clone()
 
 
+def launches(manager, tmp_path):
+    """The kernels of the one captured schedule, by name."""
+    (entry,) = manager._schedule_graphs.values()
+    entry.graph.debug_dump(str(tmp_path / "graph.dot"))
+    return (tmp_path / "graph.dot").read_text()
+
+
+# attention uncut on both sides; cut on both, in 8 and 7 parts (8 and 9 tokens) and in 3 and 4 (21 and 22 tokens: o and down
+# projections of both sides with their residuals and K in parts, as one launch); 64 rows on tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,capacity,cut", [(43, 512, False), (17, 2048, True), (43, 4096, True), (2, 2048, True), (128, 256, False)])
+@pytest.mark.parametrize("streams", ["by_kind", "by_nano_batch"])
+def test_decode_steps_in_pairs(T, capacity, cut, streams, tmp_path):
+    """Results and caches of every replay are those of the eager schedule: projections, norms and attention of the two
+    nano-batches in one launch each."""
+    model, manager, compiled = decode_program(T, capacity, streams)
+    caches = [c for block in model.attn for c in (block.k_cache, block.v_cache)]
+    step(manager, compiled, step_inputs(T, capacity, 2), True)
+    assert list(manager.paired_launches.values()) == [4 * 2], manager.paired_launches
+    names = launches(manager, tmp_path)
+    assert names.count(f"DecodeAttentionOfILb1ELb{int(cut)}E") == 2 and len(re.findall(r"beside_kernel\w+7RmsNorm", names)) == 4
+    if T == 43:          # K in parts and the rows of both sides: q/k/v, o and down of both layers
+        assert len(re.findall(r"gemm_stream_kernelILb0ELi\dELi\dELi\dELb0ELb1ELb1E", names)) >= 4
+    for seed in (3, 4):
+        inputs = step_inputs(T, capacity, seed)
+        before = [c.clone() for c in caches]
+        want = step(manager, compiled, inputs, False)
+        after = [c.clone() for c in caches]
+        for _ in range(2):
+            for c, b in zip(caches, before):
+                c.copy_(b)
+            got = step(manager, compiled, inputs, True)
+            assert torch.equal(got, want)
+            assert all(torch.equal(c, a) for c, a in zip(caches, after))
+
+
 # 26 sequences with 20 kv heads are 520 workgroups of attention, the other 25 of 51 are 500
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,joined", [(50, True), (51, False), (52, False)])
@@ -245,6 +282,34 @@ def captured(first, second):
     assert _cabi.load().dfhip_graph_pair_launches(graph.raw_cuda_graph(), 0, ctypes.byref(pairs)) == 0
     graph.instantiate()
     return graph, pairs.value
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order,found", [((0, 1), 2), ((1, 0), 0)])
+def test_pairs_that_wait_for_each_other_crosswise_stay(order, found):
+    """Two chains through the same two weights: in the same order they pair, in opposite orders no order of two joined launches
+    exists."""
+    from dynaflow_amd import ops
+
+    w = [randn((1024, 1024), 1 + i, 0.03) for i in range(2)]
+    x = [randn((8, 1024), 3 + i) for i in range(2)]
+    got = [torch.empty((8, 1024), dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    kept = [[], []]
+
+    def chain(i, way):
+        return [lambda: kept[i].append(ops.linear_variant(x[i], w[way[0]], 8)),
+                lambda: kept[i].append(ops.linear_variant(kept[i][-1], w[way[1]], 8)),
+                lambda: torch.mul(kept[i][-1], 1, out=got[i])]
+
+    want = [ops.linear_variant(ops.linear_variant(x[i], w[way[0]], 8), w[way[1]], 8) for i, way in enumerate(((0, 1), order))]
+    graph, pairs = captured(chain(0, (0, 1)), chain(1, order))
+    assert pairs == found
+    for _ in range(3):
+        for g in got:
+            g.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
 @pytest.mark.gpu
