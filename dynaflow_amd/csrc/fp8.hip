@@ -921,19 +921,6 @@ int launch_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, 
   return dfhip_check_launch();
 }
 
-// Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip); with 16 rows and more from K = 4096
-// on, as for bf16 rows of the same bytes.  From 33 rows on every workgroup re-reads the activations four times as wide as
-// up to 16, and two such launches side by side are bound by that; the ring tiles share what they read.  A pair of more
-// than 2^27 weights takes those, and one cut along K from 2^25 on.  [us a pair at 33 / 64 rows, streamed / ring: 28672 x
-// 8192 97 / 82 and 112 / 83, with gate + up + SiLU*mul 185 / 170 and 200 / 169; 8192 x 28672 118 / 91 and 155 / 91, 4096
-// x 14336 48 / 46 and 66 / 46; but 14336 x 4096 30 / 38 and 35 / 39, 1536 x 7168 24 / 28 and 28 / 29.  Alone 28672 x 8192
-// 53 / 71 and 64 / 72, 8192 x 28672 62 / 77 and 80 / 77]
-bool stream_planned(int M, int N, int K, int share, bool may_split) {
-  if (!dfhip_stream_fits(M, N, K, 1) || (M >= 16 && K < 4096)) return false;
-  const int64_t most = may_split && K > N ? 1 << 25 : 1 << 27;
-  return M <= 32 || share == 1 || (int64_t)N * K <= most;
-}
-
 constexpr int F8_MAX_SPLIT = 16;
 
 // 16-row blocks per wave of a ring tile (256 columns), 0 for the other kernels
@@ -997,13 +984,14 @@ DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share,
   return best.cost < cube * cube * now ? best : DfhipRing3Plan{-1, 1, 0.0};
 }
 
-// Up to 64 rows, what the streaming kernel of the 128-row tiles' plan (stream_planned) leaves to the 128 x 128 tile: launches
-// of 33 rows and more, unless they are alone and their weights few.  [us at 33 / 64 rows, streamed or on 128-row tiles against
-// 128 x 128: alone 28672 x 8192 53 / 63 against 55 / 56, with gate + up + SiLU*mul 103 / 110 against 91 / 94, 14336 x 4096
-// 17 / 19 against 23 / 22, with gate + up 35 / 37 against 33 / 33; in pairs 28672 x 8192 81 / 84 against 76 / 78, 14336 x 4096
-// 30 / 35 against 25 / 26.]  A product that may be cut along K goes there alone from 33 rows on, in pairs from 17, or 9 where its
-// weights are many.  [8192 x 28672 at 17 / 24 / 33 / 64 rows: in pairs 91 / 97 / 92 / 92 against 77 / 78 / 79 / 82, alone
-// 44 / 48 / 59 / 79 against 50 / 49 / 50 / 52; 4096 x 14336 in pairs 34 / 38 / 45 / 45 against 31 / 32 / 31 / 32, alone
+// Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip); with 16 rows and more from K = 4096
+// on, as for bf16 rows of the same bytes.  From 33 rows on every workgroup re-reads the activations four times as wide as
+// up to 16, which a tile shares: there the 128 x 128 tiles take over, unless the launch is alone and its weights few.  [us at 33 / 64
+// rows, streamed or on 128-row tiles against 128 x 128: alone 28672 x 8192 53 / 63 against 55 / 56, with gate + up + SiLU*mul 103 /
+// 110 against 91 / 94, 14336 x 4096 17 / 19 against 23 / 22, with gate + up 35 / 37 against 33 / 33; in pairs 28672 x 8192 81 / 84
+// against 76 / 78, 14336 x 4096 30 / 35 against 25 / 26.]  A product that may be cut along K goes there alone from 33 rows on, in
+// pairs from 17, or 9 where its weights are many.  [8192 x 28672 at 17 / 24 / 33 / 64 rows: in pairs 91 / 97 / 92 / 92 against 77 / 78 /
+// 79 / 82, alone 44 / 48 / 59 / 79 against 50 / 49 / 50 / 52; 4096 x 14336 in pairs 34 / 38 / 45 / 45 against 31 / 32 / 31 / 32, alone
 // 19 / 21 / 25 / 34 against 24; at 12 rows in pairs 8192 x 28672 82 against 79, 4096 x 14336 30 against 32.  Fewer than 2^25 weights
 // stay: 1536 x 7168 alone at 40 rows 15 against 18, in pairs at 12 rows 17 against 23.]
 bool few_rows_streamed(int M, int N, int K, int share, bool may_split) {
@@ -1190,7 +1178,7 @@ extern "C" int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* v
   if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
   *variant = -1;
   *split_k = 1;
-  if (stream_planned(M, N, K, share, true)) return DFHIP_OK;
+  if (few_rows_streamed(M, N, K, share, true)) return DFHIP_OK;
   const TilePlan plan = plan_tile(M, N, K, share, true);
   *variant = plan.variant;
   *split_k = plan.split_k;

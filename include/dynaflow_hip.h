@@ -256,7 +256,9 @@ int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* W, int64_t 
  * dfhip_gemm_fp8_nt_shared).  For the projection back to the model width: K is only cut where K > N, and the
  * projections in front of it, which keep the order of sums of dfhip_gemm_fp8_gate_up_silu_absmax, are launched without a
  * split whatever their widths are.
- * dfhip_gemm_fp8_plan_tiles: the same among all tiles, 11, 12 and 15 (those of dfhip_gemm_bf16_nt_variant) included. */
+ * dfhip_gemm_fp8_plan_tiles: the same among all tiles, 11, 12 and 15 (those of dfhip_gemm_bf16_nt_variant) included: what
+ * dfhip_gemm_fp8_nt_shared launches where may_split is 0.  Both plans leave the same launches of few rows to the
+ * streaming kernel (variant < 0). */
 int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
 int dfhip_gemm_fp8_plan_tiles(int M, int N, int K, int share, int may_split, int* variant, int* split_k);
 size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k);

@@ -137,15 +137,39 @@ def test_fused_fp8_launch_with_an_intermediate_width_below_the_model_width(M, I,
     assert torch.equal(*outs)
 
 
-def test_fp8_launches_side_by_side_are_planned_as_such():
-    """From 33 rows on a pair of large launches takes the ring tiles, a lone one the streaming kernel; a pair of narrower
-    ones and up to 32 rows stay with it, and a projection that is not cut along K never is."""
+# 2^25 weights are 2048 x 16384, 2^27 are 8192 x 16384
+@pytest.mark.parametrize("M,N,K,share,may_split,streamed", [
+    # whole K: up to 32 rows; alone up to 64 while the weights are fewer than 2^27
+    (32, 28672, 8192, 1, 0, True), (33, 28672, 8192, 1, 0, False), (32, 28672, 8192, 2, 0, True), (33, 28672, 8192, 2, 0, False),
+    (64, 16376, 8192, 1, 0, True), (64, 16384, 8192, 1, 0, False), (64, 14336, 4096, 1, 0, True), (65, 14336, 4096, 1, 0, False),
+    (33, 14336, 4096, 2, 0, False), (64, 4096, 14336, 1, 0, True),
+    # K that may be cut, but is not where the output is as wide
+    (64, 14336, 4096, 1, 1, True), (32, 8192, 8192, 2, 1, True), (33, 8192, 8192, 2, 1, False),
+    # K that is cut: alone up to 32 rows, in pairs up to 16, or 8 from 2^27 weights on; few weights up to 32, alone up to 64
+    (32, 8192, 28672, 1, 1, True), (33, 8192, 28672, 1, 1, False), (8, 8192, 28672, 2, 1, True), (9, 8192, 28672, 2, 1, False),
+    (8, 8192, 16384, 2, 1, True), (9, 8192, 16384, 2, 1, False), (16, 8184, 16384, 2, 1, True), (17, 8184, 16384, 2, 1, False),
+    (16, 4096, 14336, 2, 1, True), (17, 4096, 14336, 2, 1, False), (32, 2040, 16384, 2, 1, True), (33, 2040, 16384, 2, 1, False),
+    (64, 2040, 16384, 1, 1, True), (17, 2048, 16384, 2, 1, False), (64, 1536, 7168, 1, 1, True),
+    # a short K from 16 rows on
+    (15, 8192, 3968, 1, 0, True), (16, 8192, 3968, 1, 0, False), (16, 8192, 4096, 1, 0, True)])
+def test_few_rows_are_streamed(M, N, K, share, may_split, streamed):
+    """Both sides of every boundary, in the plan that is launched and in the one without the three-slab tiles."""
     lib, v, s = _cabi.load(), ctypes.c_int(), ctypes.c_int()
-    for M, N, K, share, streamed in ((48, 28672, 8192, 1, True), (48, 28672, 8192, 2, False), (64, 8192, 28672, 2, False),
-                                     (33, 4096, 14336, 2, False), (32, 28672, 8192, 2, True), (64, 14336, 4096, 2, True),
-                                     (64, 1536, 7168, 2, True), (65, 14336, 4096, 1, False)):
+    assert lib.dfhip_gemm_fp8_plan_tiles(M, N, K, share, may_split, ctypes.byref(v), ctypes.byref(s)) == 0
+    assert (v.value < 0) == streamed
+    if may_split:
         assert lib.dfhip_gemm_fp8_plan_shared(M, N, K, share, ctypes.byref(v), ctypes.byref(s)) == 0
-        assert (v.value < 0) == streamed, (M, N, K, share)
+        assert (v.value < 0) == streamed
+
+
+def test_fp8_launches_side_by_side_are_planned_as_such():
+    """A pair of large launches takes tiles where a lone one streams its weights, and the other way round nowhere."""
+    lib, v, s = _cabi.load(), ctypes.c_int(), ctypes.c_int()
+    for M, N, K, alone, paired in ((24, 8192, 28672, True, False), (12, 8192, 28672, True, False), (40, 14336, 4096, True, False),
+                                   (20, 4096, 14336, True, False), (32, 28672, 8192, True, True), (40, 28672, 8192, False, False)):
+        for share, streamed in ((1, alone), (2, paired)):
+            assert lib.dfhip_gemm_fp8_plan_tiles(M, N, K, share, K > N, ctypes.byref(v), ctypes.byref(s)) == 0
+            assert (v.value < 0) == streamed, (M, N, K, share)
     args = (16, 1024, 16, 1024, 16, 8, 16, 16, 1, 8, 1024)
     assert lib.dfhip_gemm_fp8_nt_shared(*args, 0, None) == -7 and lib.dfhip_gemm_fp8_nt_shared(*args, 17, None) == -7
 
