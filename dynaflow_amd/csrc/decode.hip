@@ -500,14 +500,16 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
 
 // Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), with at least 256 positions of
 // a full cache each (two chunks per wave).  The lengths are on the device: the launch is sized for full caches and each
-// sequence takes its share of it (sequence_parts).  A launch with fewer than MIN_PARTS of them, from 171 pairs on, cuts
-// nothing.  [us, uncut / cut: 2 sequences of 8192 positions 111 / 20.8 (their bytes at 6.7 TB/s: 10), 8 of 2048 33 / 16.8
+// sequence takes its share of it (sequence_parts).  A launch with fewer than MIN_PARTS of them, from 171 pairs on but for those
+// below, cuts nothing.  [us, uncut / cut: 2 sequences of 8192 positions 111 / 20.8 (their bytes at 6.7 TB/s: 10), 8 of 2048 33 / 16.8
 // (10), 20 of 4096 69 / 58 (50); in two parts, not taken: 32 of 512, 2048 and 4096 14.6 / 16.5, 42.9 / 46.0, 79 / 84]
 // A compute unit takes in no more than 29 GB/s, so a few pairs more than units take twice the time: 257 .. 384 of them are cut
 // in four where the cache has room for 2048 positions, and so are 171 .. 192, which leave a quarter of the units idle, where it
-// has room for 4096.  [us, uncut / four parts, all full / of 1/4 .. 1 of the capacity, 8 kv heads: 34 sequences of 2048 70 / 58,
-// 42 / 47; 36 of 4096 139 / 109, 94 / 83; 40 of 8192 275 / 213, 223 / 167; 48 of 2048 80 / 76, 62 / 60; 24 of 4096 75 / 71, 68 / 65, of
-// 8192 142 / 130, 129 / 109; not taken: 36 of 1024 38.5 / 38, 26 of 4096 78 / 85, 69 / 66, 54 of 2048 80 / 85, 68 / 68]
+// has room for 4096.  [us, uncut / four parts, 8 kv heads, all full: 34 sequences of 2048 69 / 55, 48 of 2048 73 / 70, 36 of 4096 134 / 102,
+// 40 of 8192 268 / 204, 24 of 4096 69 / 66, of 8192 134 / 123; of 1/4 .. 1 of the capacity the uncut launch depends on which sequences
+// meet on a unit, so over ten orders: 33 of 2048 41 .. 52 / 41 .. 44 (mean 46 / 43), 34 of 2048 44 .. 62 / 43 .. 45, 48 of 2048 57 .. 64 /
+// 56 .. 58, 36 of 4096 85 .. 120 / 78 .. 82, 24 of 4096 63 .. 64 / 58 .. 62, of 8192 122 / 102 .. 115; not taken: 36 of 1024 38.5 / 38, 26 of 4096
+// 78 / 85, 69 / 66, 54 of 2048 80 / 85, 68 / 68]
 constexpr int MIN_PARTS = 3;
 static int attention_parts(int T, int kv_heads, int capacity) {
   const int64_t pairs = (int64_t)T * kv_heads;

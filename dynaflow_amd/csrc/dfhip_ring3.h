@@ -8,9 +8,11 @@
 // kernels.  `share` launches of one shape side by side take their
 // rounds of 256 workgroups together.  A round costs a start and an end and, per slab of K, a time that grows with the share of
 // the compute units at work (the clock falls with the power they draw); parts of K cost their meeting; and the weights do
-// not come in faster than `intake` (MB per us, i.e. TB/s).  Fitted to some 3000 timings of the tiles below and of the kernels
+// not come in faster than `intake` (MB per us, i.e. TB/s).  Fitted to timings of the tiles below and of the kernels
 // beside them at 17 .. 4096 rows, alone and in pairs, on fp8 weights 28672 x 8192, 14336 x 4096 and transposed, bf16 ones
-// also 6144 x 4096, 4096 x 4096, 5632 x 2048: right to 5 % on average and to 12 % for nine in ten.
+// also 6144 x 4096, 4096 x 4096, 5632 x 2048.  Timed again, alone, on these and on 11264 x 2048 and fp8 16384 x 4096 and transposed: of the 767 timings
+// within 25 % of the fastest of their shape 9 % off on average and 18 % for nine in ten; two launches in step on two streams take
+// 5 - 30 % less than priced (they read their weights together).  What the choices by it give stands at three_slabs_cheaper.
 struct DfhipPrice { double slab, slab_full, round, parts, part, intake; };
 inline double dfhip_price(const DfhipPrice& p, int64_t tiles, int share, double slabs, int split_k, double weight_mb) {
   const int64_t work = tiles * split_k * share;

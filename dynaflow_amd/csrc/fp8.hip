@@ -965,10 +965,10 @@ constexpr DfhipPrice F8_RING224_PRICE = {0.861, 0.401, 8.58, 0.0, 0.0, 6.0};
 
 // Whether a three-slab tile takes the place of the planned kernel, and which: where it is 4 % cheaper, 7 % above 256 rows and
 // for gate + up, whose pairs above 128 rows need 15 % (192 rows of 2 x 28672 x 8192 in pairs, priced 8 % lower, took 228 us
-// on 224 x 192 tiles where the 192-row ones take 195).  Over 190 timed shapes
-// (those of dfhip_price) this takes 9.4 % off the mean, 9.8 % being what the best choice for each would; the worst loss is
-// 6 % (350 x 4096 x 16384 alone: 42 -> 45 us), the best gains 63 % (96 x 4096 x 14336 alone: 41 -> 25) and 44 % (96 x 8192 x 28672
-// alone: 78 -> 55).
+// on 224 x 192 tiles where the 192-row ones take 195).  At 25 counts of rows of six
+// weights (those of dfhip_price), alone and in pairs, 136 launches change their kernel: 19 % less on the geometric mean, at best 49 %
+// (33 x 4096 x 14336 alone: 40 -> 20.5 us), at worst 7 % more (350 x 4096 x 16384 alone: 42 -> 45), the only one that stays above 3 %
+// in every run.
 DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share, int variant, int split_k, bool may_split) {
   const int tm = ring_blocks(variant);
   const int rows = tm ? 32 * tm : 256, cols = !tm ? F8_TBN : gate_up ? 128 : 256;
@@ -977,7 +977,10 @@ DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share,
   const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
   const double now = dfhip_price(price, tiles, share, K / FBK, split_k, (double)N * K * (gate_up ? 2e-6 : 1e-6));
   const DfhipRing3Plan best = dfhip_ring3_plan(true, gate_up, M, N, K, share, may_split);
-  // (side by side and up to 128 rows also where it costs 5 % more: two of these launches can become one, dfhip_pairs.h)
+  // (side by side and up to 128 rows also where it is priced 5 % higher, which only gate + up is: two of these launches can become
+  // one, dfhip_pairs.h, and where they do not it is faster or within 1 %.  [us a pair on two streams at 33 / 64 / 100 / 128 rows against the
+  // 128-row ring: 28672 x 8192 152 / 153 / 160 / 168 and 154 / 154 / 158 / 166, 14336 x 4096 40.9 / 42.1 / 44.6 / 45.5 and 42.7 / 43.1 /
+  // 44.4 / 45.1, 13824 x 5120 50 / 52 / 55 / 57 and 58 / 59 / 59 / 60])
   const double clearly = share > 1 && M <= DFHIP_PAIR_MAX_M ? 1.05
                          : gate_up && share > 1 ? 0.85 : M > 256 || gate_up ? 0.93 : 0.96;
   const double cube = clearly * clearly * clearly;

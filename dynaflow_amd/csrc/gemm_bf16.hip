@@ -1765,9 +1765,10 @@ constexpr DfhipPrice RING_PRICE = {0.764, 0.703, 4.67, 1.82, 4.25, 5.0}, RING224
 
 // Whether a three-slab tile takes the place of the planned kernel (`variant`, K in `split_k` parts), and which.  It has to be
 // clearly cheaper: 4 %, and more where the prices are the least sure: 13 % against weight-streaming tiles that split K (20 % up
-// to 256 rows), in pairs 8 % for gate + up and 15 % against 192-row tiles.  Over 279 timed shapes (those of dfhip_price above 128 rows) this takes 5 % off the mean, 7 % being what
-// the best choice for each would; the worst loss is 7 % (200 x 28672 x 4096 alone: 71 -> 76 us), the best gains 48 % (1100 x
-// 2048 x 5632 alone: 58 -> 39) and 44 % (300 x 4096 x 14336 in pairs: 119 -> 83).
+// to 256 rows), in pairs 8 % for gate + up and 15 % against 192-row tiles.  At 25 counts of rows of seven weights (those of dfhip_price), alone and in
+// pairs, 97 launches change their kernel: 12 % less on the geometric mean, at best 37 % (1100 x 2048 x 5632 alone: 66 -> 42 us; 300
+// x 4096 x 14336 in pairs 119 -> 80), at worst 5 % more (160 x 28672 x 4096 alone: 69 -> 72), the only one that stays above 3 % in
+// every run.  Gate + up of 14336 x 4096 and 5632 x 2048: 2 % less over all.
 DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share, int variant, int split_k, bool may_split) {
   struct Kernel { int rows, cols; DfhipPrice price; } k;
   switch (variant) {
