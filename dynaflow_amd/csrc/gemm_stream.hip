@@ -8,7 +8,8 @@
 //     128-byte slabs of the rows in turn (wave w: slabs w, w + 4, ...) and up to four slabs per wave are in flight;
 //   * weights and activations go straight from memory to registers, no LDS and no barrier inside the loop.  A load
 //     takes eight whole 128-byte lines (half a block of 16 rows), which is what lets the weights be loaded
-//     non-temporally; lanes eight apart then exchange a piece each (DPP), which gives the MFMA operand layout;
+//     non-temporally; neighbouring lanes, which share 32 bytes, then exchange a piece each (DPP), which gives the MFMA
+//     operand layout;
 //   * the activation rows are re-read by every workgroup from its XCD's L2; the rows of a matrix lie a multiple of
 //     4 KiB apart and so on one L2 channel, hence the workgroups start at different slabs;
 //   * at the end the four partial sums meet in LDS and are added in wave order.  Where K is cut into parts (a
@@ -77,15 +78,20 @@ gemm_stream_kernel(const StreamArgs p) {
   const int slab0 = SPLIT ? (int)((int64_t)p.slabs * part / p.split_k) : 0;
   const int slabs = SPLIT ? (int)((int64_t)p.slabs * (part + 1) / p.split_k) - slab0 : p.slabs;
 
-  // load h of a slab takes rows 8 h .. 8 h + 7 of a block, whole 128-byte lines (lane: row lane % 8, chunk lane / 8)
-  const int lrow = lane & 7, lchunk = lane >> 3;
+  // load h of a slab takes rows h, 2 + h .. 14 + h of a block, whole 128-byte lines (lane: row 2 (lane / 2 % 8) + h, chunk
+  // 2 (lane / 16) + lane % 2).  Neighbouring lanes share 32 bytes: with one row per lane (row lane % 8, chunk lane / 8) a
+  // compute unit takes in 34 GB/s at most, from its L2 too and whatever is in flight, with pairs of lanes 66 (with eight
+  // lanes to a line 114, but then the exchange has three stages).  [us: decode step of 40 x 4096 positions, 4 layers
+  // 819 -> 771, fp8 layer 8192 x 28672 of 2 x 12 tokens 174 -> 166]
+  const int lrow = lane & 14, lchunk = 2 * (lane >> 4) + (lane & 1);
+  const bool odd = lane & 1;
   const uint8_t* w_ptr[NB][2];
   const uint8_t* a_ptr[MB][2];
 #pragma unroll
   for (int j = 0; j < NB; ++j)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      int n = n0 + 16 * (FUSED ? j % OB : j) + 8 * h + lrow;
+      int n = n0 + 16 * (FUSED ? j % OB : j) + lrow + h;
       n = n < p.N ? n : p.N - 1;                   // columns past the edge re-read the last one; never stored
       w_ptr[j][h] = (FUSED && j >= OB ? p.W2 : p.W) + (int64_t)n * p.ldw + (slab0 + wave) * 128 + lchunk * 16;
     }
@@ -93,7 +99,7 @@ gemm_stream_kernel(const StreamArgs p) {
   for (int i = 0; i < MB; ++i) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      int m = 16 * i + 8 * h + lrow;
+      int m = 16 * i + lrow + h;
       const bool other = MERGED && m >= second;
       m -= other ? second : 0;
       const int M = other ? p.side[1].M : p.side[0].M;
@@ -127,14 +133,17 @@ gemm_stream_kernel(const StreamArgs p) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) af[d][i][h] = *reinterpret_cast<const u32x4*>(a_ptr[i][h] + off);
   };
-  // the two loads of a block -> its two MFMA fragments (lane: row lane % 16, chunks 2 (lane / 16) and + 1): lanes
-  // eight apart exchange one of their two pieces
+  // the two loads of a block -> its two MFMA fragments (lane: row lane % 16, chunks 2 (lane / 16) and + 1):
+  // neighbouring lanes exchange one of their two pieces
   auto deal = [&](u32x4 (&v)[2]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int x = (int)v[0][e], y = (int)v[1][e];
-      v[0][e] = (uint32_t)__builtin_amdgcn_update_dpp(x, y, 0x128, 0xF, 0xC, false);   // row_ror:8 into lanes 8 .. 15
-      v[1][e] = (uint32_t)__builtin_amdgcn_update_dpp(y, x, 0x128, 0xF, 0x3, false);   // ... into lanes 0 .. 7
+      constexpr int SWAP = 0xB1;                 // quad_perm [1, 0, 3, 2]
+      const int from_x = __builtin_amdgcn_update_dpp(x, x, SWAP, 0xF, 0xF, true);
+      const int from_y = __builtin_amdgcn_update_dpp(y, y, SWAP, 0xF, 0xF, true);
+      v[0][e] = (uint32_t)(odd ? from_y : x);
+      v[1][e] = (uint32_t)(odd ? y : from_x);
     }
   };
   auto multiply = [&](int d) {
