@@ -123,8 +123,13 @@ DFHIP_DEVICE void decode_attention(int pair, const uint16_t* __restrict__ q, int
       for (int e = 0; e < 8; ++e) qf[ks][e] = static_cast<bf16_t>(0.0f);
     }
   }
-  const int krow = 8 * (hq >> 2) + (hq & 3);
-  const uint16_t* k_lane = kbase + (int64_t)krow * HD + 8 * g;
+  // SPLIT: a K load takes eight whole 128-byte lines, two neighbouring lanes 32 bytes of one; bits 0, 5, 4 of the lane are the
+  // 16-byte chunk of the line, 1, 2, 3 bits 1, 3, 4 of the row, and load (a, s, half) gives bits 0 and 2 of it and the half.
+  // With a row per lane, as the fragments have it, a compute unit takes in 34 GB/s of keys at most, which is what few
+  // workgroups with a part each wait for [us, 2 x 20 sequences of 1/4 .. 1 of 4096 positions: 92 -> 83].  Whole sequences keep
+  // every unit busy at the rate of the memory, and are 1 % slower that way (2 x 128 of 2048).
+  const int krow = 8 * (hq >> 2) + (hq & (SPLIT ? 2 : 3));
+  const uint16_t* k_lane = kbase + (int64_t)krow * HD + 8 * (SPLIT ? (lane & 1) + 4 * (g & 1) + 2 * (g >> 1) : g);
   const uint16_t* v_lane = vbase + ((int64_t)g * HD + hq) * 8;
 
   // every cached element is read once per step and by nobody else: non-temporal loads, which do not displace
@@ -136,9 +141,28 @@ DFHIP_DEVICE void decode_attention(int pair, const uint16_t* __restrict__ q, int
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
-        f.k[s][ks] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kp + s * 4 * HD + 32 * ks));
+        f.k[s][ks] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(
+            SPLIT ? kp + (4 * s + (ks & 1)) * HD + 64 * (ks >> 1) : kp + s * 4 * HD + 32 * ks));
 #pragma unroll
     for (int nb = 0; nb < 8; ++nb) f.v[nb] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(vp + nb * 16 * 8));
+  };
+
+  // SPLIT: two loads -> two fragments (lane: row hq, chunk 4 ks + g): neighbouring lanes exchange one of their two pieces, then
+  // lanes 16 apart
+  auto deal = [&](bf16x8& first, bf16x8& second) {
+    u32x4 x = __builtin_bit_cast(u32x4, first), y = __builtin_bit_cast(u32x4, second);
+    const bool odd = lane & 1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      constexpr int SWAP = 0xB1;                 // quad_perm [1, 0, 3, 2]
+      const int from_x = __builtin_amdgcn_update_dpp((int)x[e], (int)x[e], SWAP, 0xF, 0xF, true);
+      const int from_y = __builtin_amdgcn_update_dpp((int)y[e], (int)y[e], SWAP, 0xF, 0xF, true);
+      const auto both = __builtin_amdgcn_permlane16_swap(odd ? (uint32_t)from_y : x[e], odd ? y[e] : (uint32_t)from_x, false, false);
+      x[e] = both[0];
+      y[e] = both[1];
+    }
+    first = __builtin_bit_cast(bf16x8, x);
+    second = __builtin_bit_cast(bf16x8, y);
   };
 
   float m = -INFINITY, l = 0.0f;
@@ -147,6 +171,11 @@ DFHIP_DEVICE void decode_attention(int pair, const uint16_t* __restrict__ q, int
   for (int nb = 0; nb < 8; ++nb) o[nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   auto step = [&](KVFrags& f, int c) {
+    if constexpr (SPLIT)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int ks = 0; ks < 4; ks += 2) deal(f.k[s][ks], f.k[s][ks + 1]);
     if (APPEND && append && c == pos / CHUNK) {
       // the chunk of the new token: its key row and value column come from LDS, whatever the loads returned
       const int krow_pos = c * CHUNK + 8 * (hq >> 2) + (hq & 3);
