@@ -16,6 +16,7 @@ namespace {
 constexpr int HD = 128;           // head dim
 constexpr int DEC_THREADS = 256;  // 4 waves
 constexpr int CHUNK = 32;         // positions per softmax step of a wave
+constexpr int COMPUTE_UNITS = 256;
 constexpr int MAX_GROUP = 16;     // query heads per kv head (rows of the MFMA tile)
 
 DFHIP_DEVICE f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -56,6 +57,81 @@ DFHIP_DEVICE int sequence_parts(int len, int parts) {
   return len / 256 < parts ? len / 256 : parts;
 }
 
+// What a workgroup is to work on.
+struct Share { int token, kvh, part, slot, len; };
+
+// Workgroup `block` of a launch.  Of more workgroups than compute units the longest sequences come first (ties in the order of the
+// tokens), all parts of one before the next sequence, so that what runs at the end is short and what shares a unit differs.
+// A wave ranks the sequences by itself: the length of the `rank`-th longest is the largest that more than `rank` tokens reach,
+// found bit by bit, then the token is counted off among those of that length.  Up to 64 J tokens.
+// Sequences of one length, launches of few workgroups and of many tokens (whose workgroups even out by themselves) keep the order
+// of the tokens, and the first parts of all tokens come before the second ones, so that the parts that every sequence uses lie
+// on all XCDs; so do those whose number of kv heads is no multiple of the XCDs.  (The parts of a token first, the only
+// workgroups with work of 8 short sequences are every eighth one, on one XCD: 512 positions 20.2 us, so 12.2.)
+// [us, order of the tokens -> longest first, sequences of 1/4 .. 1 of the capacity in any order: 20 of 4096 positions 47 -> 43, 36
+// of 4096 72 -> 70, 24 of 4096 55 -> 51, 16 of 8192 67 -> 63; whole ones: 40 of 4096 79 -> 76, 64 of 2048 67 -> 62, 128 of 2048 125 -> 107,
+// 100 of 1024 59 -> 50; all of one length, level (200 of 1024 140 -> 142).  Ranked with fewer workgroups than units: 12 of 512
+// 11.9 -> 12.8; the first parts of all tokens first, ranked: 16 of 8192 68, 24 of 4096 54]
+template <bool SPLIT, int J>
+DFHIP_DEVICE Share share_of(int block, const int32_t* __restrict__ slots, const int32_t* __restrict__ lengths, int tokens,
+                            int kv_heads, int parts, int capacity) {
+  const int lane = threadIdx.x & 63;
+  int own[J], own_slot[J], len[J];
+  bool same = true;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int t = 64 * j + lane < tokens ? 64 * j + lane : 0;
+    own[j] = lengths[t];
+    own_slot[j] = slots[t];
+  }
+  const int first = __builtin_amdgcn_readfirstlane(own[0]);
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    same &= own[j] == first;
+    len[j] = 64 * j + lane >= tokens ? -1 : own[j] < 0 ? 0 : own[j] < capacity ? own[j] : capacity;
+  }
+  same = __all(same);
+  const bool together = SPLIT && !same && kv_heads % 8 == 0;    // the parts of a token
+  const int per_part = together ? kv_heads : tokens * kv_heads;
+  int rank = 0;
+  if (together) {
+    rank = block / (kv_heads * parts);
+    block -= rank * kv_heads * parts;
+  }
+  const int part = SPLIT ? block / per_part : 0;
+  block -= part * per_part;
+  if (!together) rank = block / kv_heads;
+  const int kvh = together ? block : block - rank * kv_heads;
+  int token = rank;
+  if (!same) {
+    auto reach = [&](int least) {              // tokens of at least this length
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < J; ++j) n += __popcll(__ballot(len[j] >= least));
+      return n;
+    };
+    int length = 0;
+    for (int bit = 31 - __clz(capacity); bit >= 0; --bit)
+      if (reach(length | 1 << bit) > rank) length |= 1 << bit;
+    int before = rank - reach(length + 1);     // tokens of this length that come first
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const uint64_t equal = __ballot(len[j] == length);
+      const int n = __popcll(equal);
+      const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(equal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)equal, 0));
+      const uint64_t found = __ballot(len[j] == length && at == before);
+      if (before >= 0 && before < n) token = 64 * j + __builtin_ctzll(found);
+      before -= n;
+    }
+    token = __builtin_amdgcn_readfirstlane(token);
+  }
+  int slot_of = own_slot[0], len_of = own[0];
+#pragma unroll
+  for (int j = 1; j < J; ++j)
+    if (token >= 64 * j) slot_of = own_slot[j], len_of = own[j];
+  return {token, kvh, part, __builtin_amdgcn_readlane(slot_of, token & 63), __builtin_amdgcn_readlane(len_of, token & 63)};
+}
+
 // One workgroup per (token, kv head).  Wave w takes the chunks w, w+4, ... of 32 positions.
 // MFMA row i of a score tile is mapped to position 8*(i/4) + i%4 (+4 for the second tile of the
 // chunk), so that after the two tiles lane (head = lane%16, g = lane/16) holds the scores of its
@@ -74,7 +150,7 @@ DFHIP_DEVICE int sequence_parts(int len, int parts) {
 // its unnormalised sums, maximum and sum of exponentials in `partials` ([pair][part][part_block(group)] words of 16
 // bytes), counts itself in and is done; the part that arrives last combines them, in the same order whoever that is.
 template <bool APPEND, bool SPLIT>
-DFHIP_DEVICE void decode_attention(int pair, const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* __restrict__ kc,
+DFHIP_DEVICE void decode_attention(int block, bool ordered, int tokens, const uint16_t* __restrict__ q, int64_t ld_q, uint16_t* __restrict__ kc,
                                    uint16_t* __restrict__ vc, const int32_t* __restrict__ slots,
                                    const int32_t* __restrict__ lengths, uint16_t* __restrict__ out, int64_t ld_out,
                                    int kv_heads, int group, int num_slots, int capacity, float scale_log2,
@@ -86,14 +162,24 @@ DFHIP_DEVICE void decode_attention(int pair, const uint16_t* __restrict__ q, int
   float* const o_lds = combine_lds;                       // [4][group][HD]
   float* const m_lds = combine_lds + 4 * group * HD;      // [4][group]
   float* const l_lds = m_lds + 4 * group;                 // [4][group]
-  // Part-major: the parts that every sequence uses are dispatched first and lie on all XCDs.  (Pair-major, the only
-  // workgroups with work of 8 short sequences are every eighth one, on one XCD: 512 positions 20.2 us, so 12.2.)
-  const int part = SPLIT ? blockIdx.y : 0;
-  const int t = pair / kv_heads, kvh = pair - t * kv_heads;
+  Share my;
+  if (ordered && tokens > 1 && tokens <= 64) {
+    my = share_of<SPLIT, 1>(block, slots, lengths, tokens, kv_heads, parts, capacity);
+  } else if (ordered && tokens > 1 && tokens <= 256) {
+    my = share_of<SPLIT, 4>(block, slots, lengths, tokens, kv_heads, parts, capacity);
+  } else {
+    my.part = SPLIT ? block / (tokens * kv_heads) : 0;
+    block -= my.part * tokens * kv_heads;
+    my.token = block / kv_heads;
+    my.kvh = block - my.token * kv_heads;
+    my.slot = slots[my.token];
+    my.len = lengths[my.token];
+  }
+  const int part = my.part, t = my.token, kvh = my.kvh, pair = t * kv_heads + kvh;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hq = lane & 15, g = lane >> 4;
-  const int slot = slots[t];
-  int len = lengths[t];
+  const int slot = my.slot;
+  int len = my.len;
   uint16_t* out_row = out + (int64_t)t * ld_out + (int64_t)kvh * group * HD;
   if (slot < 0 || slot >= num_slots || len < 1) {   // nothing to attend to: defined output, no access
     if (part == 0)
@@ -419,14 +505,15 @@ struct DecodeAttention {
   float* partials;
   int* arrivals;
   int64_t ld_q, ld_out;
-  int kv_heads, group, num_slots, capacity, table_rows, parts;
+  int tokens, kv_heads, group, num_slots, capacity, table_rows, parts;
   float scale_log2;
 };
 template <bool APPEND, bool SPLIT>
 struct DecodeAttentionOf : DecodeAttention {
   static constexpr int THREADS = DEC_THREADS;
-  DFHIP_DEVICE void run(unsigned block, unsigned) const {
-    decode_attention<APPEND, SPLIT>(block, q, ld_q, kc, vc, slots, lengths, out, ld_out, kv_heads, group, num_slots, capacity,
+  __host__ __device__ int blocks() const { return tokens * kv_heads * parts; }
+  DFHIP_DEVICE void run(int block, bool ordered) const {
+    decode_attention<APPEND, SPLIT>(block, ordered, tokens, q, ld_q, kc, vc, slots, lengths, out, ld_out, kv_heads, group, num_slots, capacity,
                                     scale_log2, cos_t, sin_t, table_rows, parts, partials, arrivals);
   }
   bool beside(const DecodeAttentionOf& other) const {
@@ -435,15 +522,32 @@ struct DecodeAttentionOf : DecodeAttention {
 };
 template <bool APPEND, bool SPLIT>
 __global__ void __launch_bounds__(DEC_THREADS) decode_attention_kernel(const DecodeAttentionOf<APPEND, SPLIT> p) {
-  p.run(blockIdx.x, gridDim.x);
+  p.run(blockIdx.y * gridDim.x + blockIdx.x, p.blocks() > COMPUTE_UNITS);
+}
+// The launches of two nano-batches as one: eight workgroups of each in turn, so that the long sequences of both come first.
+template <class K>
+__global__ void __launch_bounds__(DEC_THREADS) decode_attention_pair_kernel(const DfhipBoth<K> p) {
+  const int block = blockIdx.y * gridDim.x + blockIdx.x;
+  const int first = p.side[0].blocks(), second = p.side[1].blocks(), both = (first < second ? first : second) & ~7;
+  int side = (block >> 3) & 1, own = (block >> 4) * 8 + (block & 7);
+  if (block >= 2 * both) {
+    own = block - both;                        // what the longer launch has left
+    side = own >= first;
+    if (side) own -= first - both;
+  }
+  if (own < (side ? second : first)) p.side[side].run(own, first + second > COMPUTE_UNITS);
+}
+template <class K>
+bool join_attention(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
+  return dfhip_join_as<K>(reinterpret_cast<const void*>(decode_attention_pair_kernel<K>), a, b, ga, gb, both, joined);
 }
 template <bool APPEND, bool SPLIT>
-int launch_attention(const DecodeAttention& args, int pairs, size_t lds_bytes, hipStream_t stream) {
+int launch_attention(const DecodeAttention& args, size_t lds_bytes, hipStream_t stream) {
   using K = DecodeAttentionOf<APPEND, SPLIT>;
   const auto kernel = decode_attention_kernel<APPEND, SPLIT>;
-  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), dfhip_join_beside<K>, DFHIP_SHORT_BLOCKS), true);
+  static const bool known = (dfhip_pairable(reinterpret_cast<const void*>(kernel), join_attention<K>, DFHIP_SHORT_BLOCKS), true);
   (void)known;
-  hipLaunchKernelGGL(kernel, dim3(pairs, args.parts), dim3(DEC_THREADS), lds_bytes, stream, K{args});
+  hipLaunchKernelGGL(kernel, dim3(args.tokens * args.kv_heads, args.parts), dim3(DEC_THREADS), lds_bytes, stream, K{args});
   return dfhip_check_launch();
 }
 
@@ -522,9 +626,9 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
   const size_t combine_bytes = (size_t)4 * group * (HD + 2) * sizeof(float);
   const DecodeAttention args{static_cast<const uint16_t*>(q), static_cast<uint16_t*>(const_cast<void*>(k_cache)),
                              static_cast<uint16_t*>(const_cast<void*>(v_cache)), slots, lengths, static_cast<uint16_t*>(out),
-                             nullptr, nullptr, nullptr, nullptr, ld_q, ld_out, kv_heads, group, num_slots, capacity, 1, 1,
+                             nullptr, nullptr, nullptr, nullptr, ld_q, ld_out, T, kv_heads, group, num_slots, capacity, 1, 1,
                              scale_log2};
-  return launch_attention<false, false>(args, T * kv_heads, combine_bytes, static_cast<hipStream_t>(stream));
+  return launch_attention<false, false>(args, combine_bytes, static_cast<hipStream_t>(stream));
 }
 
 // Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), with at least 256 positions of
@@ -534,11 +638,10 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
 // (10), 20 of 4096 69 / 58 (50); in two parts, not taken: 32 of 512, 2048 and 4096 14.6 / 16.5, 42.9 / 46.0, 79 / 84]
 // A compute unit takes in no more than 29 GB/s, so a few pairs more than units take twice the time: 257 .. 384 of them are cut
 // in four where the cache has room for 2048 positions, and so are 171 .. 192, which leave a quarter of the units idle, where it
-// has room for 4096.  [us, uncut / four parts, 8 kv heads, all full: 34 sequences of 2048 69 / 55, 48 of 2048 73 / 70, 36 of 4096 134 / 102,
-// 40 of 8192 268 / 204, 24 of 4096 69 / 66, of 8192 134 / 123; of 1/4 .. 1 of the capacity the uncut launch depends on which sequences
-// meet on a unit, so over ten orders: 33 of 2048 41 .. 52 / 41 .. 44 (mean 46 / 43), 34 of 2048 44 .. 62 / 43 .. 45, 48 of 2048 57 .. 64 /
-// 56 .. 58, 36 of 4096 85 .. 120 / 78 .. 82, 24 of 4096 63 .. 64 / 58 .. 62, of 8192 122 / 102 .. 115; not taken: 36 of 1024 38.5 / 38, 26 of 4096
-// 78 / 85, 69 / 66, 54 of 2048 80 / 85, 68 / 68]
+// has room for 4096.  [us, uncut / four parts, 8 kv heads, all full: 33 sequences of 2048 68 / 53, 48 of 2048 73 / 69, 36 of 4096 133 / 100,
+// 36 of 8192 266 / 190, 24 of 4096 70 / 65, of 8192 134 / 126; of 1/4 .. 1 of the capacity, longest first: 33 of 2048 45 / 41, 48 of 2048
+// 56 / 57, 36 of 4096 90 / 71, 48 of 4096 106 / 91, 24 of 4096 65 / 51, of 8192 124 / 90; not taken, for the sake of full caches: 32 of
+// 4096 79 / 86, 69 / 62, 64 of 4096 160 / 169, 121 / 117, 56 of 2048 77 / 80, 61 / 66]
 constexpr int MIN_PARTS = 3;
 static int attention_parts(int T, int kv_heads, int capacity) {
   const int64_t pairs = (int64_t)T * kv_heads;
@@ -572,10 +675,10 @@ static int decode_attention_append(const void* qkv, int64_t ld_qkv, void* k_cach
   float* partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + ATTENTION_COUNTER_BYTES);
   const DecodeAttention args{static_cast<const uint16_t*>(qkv), static_cast<uint16_t*>(k_cache), static_cast<uint16_t*>(v_cache),
                              slots, lengths, static_cast<uint16_t*>(out), cos_table, sin_table, parts > 1 ? partials : nullptr,
-                             static_cast<int*>(workspace), ld_qkv, ld_out, kv_heads, group, num_slots, capacity, table_rows,
+                             static_cast<int*>(workspace), ld_qkv, ld_out, T, kv_heads, group, num_slots, capacity, table_rows,
                              parts, scale * 1.4426950408889634f};
   const auto launch = parts > 1 ? launch_attention<true, true> : launch_attention<true, false>;
-  return launch(args, T * kv_heads, lds_bytes, static_cast<hipStream_t>(stream));
+  return launch(args, lds_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int dfhip_decode_attention_append_bf16(const void* qkv, int64_t ld_qkv, void* k_cache, void* v_cache,

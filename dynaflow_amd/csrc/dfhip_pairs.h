@@ -70,10 +70,14 @@ __global__ void __launch_bounds__(K::THREADS) dfhip_beside_kernel(const DfhipBot
   p.side[second].run(blockIdx.x - (second ? p.blocks : 0), second ? gridDim.x - p.blocks : p.blocks);
 }
 template <class K>
-bool dfhip_join_beside(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
+bool dfhip_join_as(const void* kernel, const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
   static_assert(sizeof(DfhipBoth<K>) <= DFHIP_PAIR_MAX_ARGS);
   const K &x = *static_cast<const K*>(a), &y = *static_cast<const K*>(b);
-  *joined = {reinterpret_cast<const void*>(dfhip_beside_kernel<K>), joined->lds, dim3(ga.x + gb.x, ga.y > gb.y ? ga.y : gb.y)};
+  *joined = {kernel, joined->lds, dim3(ga.x + gb.x, ga.y > gb.y ? ga.y : gb.y)};
   *static_cast<DfhipBoth<K>*>(both) = {{x, y}, ga.x};
   return x.beside(y);
+}
+template <class K>
+bool dfhip_join_beside(const void* a, const void* b, dim3 ga, dim3 gb, void* both, DfhipJoined* joined) {
+  return dfhip_join_as<K>(reinterpret_cast<const void*>(dfhip_beside_kernel<K>), a, b, ga, gb, both, joined);
 }

@@ -224,6 +224,46 @@ def test_decode_attention_cut_in_four(ops, heads, kv_heads, capacity, lengths):
     test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, lengths)
 
 
+@pytest.mark.parametrize("T,kv_heads,capacity", [
+    (33, 8, 64), (64, 8, 64), (65, 4, 96), (256, 2, 32),       # longest first: one and four lengths a lane
+    (257, 2, 32),                                             # the order of the tokens
+    (20, 8, 4096), (36, 8, 2048), (86, 3, 2048),              # in parts: of eight heads together, of three one after the other
+])
+def test_decode_attention_in_any_order_of_the_sequences(ops, T, kv_heads, capacity):
+    """More workgroups than compute units start with the longest sequences: every token gets its own result, wherever it stands
+    in the batch, with many sequences of one length, some that are empty or longer than the cache, and slots that do not exist."""
+    from dynaflow_amd.decode import pack_v_cache
+    from dynaflow_amd.decoder import rope_tables
+
+    g = torch.Generator().manual_seed(T + capacity)
+    lens = torch.randint(1, capacity + 1, (T,), generator=g)
+    lens[: T // 3] = lens[0]
+    lens[T // 2], lens[T - 1], lens[T - 2], lens[1] = capacity, capacity + 5, 0, 1
+    slots = torch.randperm(T, generator=g).int()
+    slots[T // 4] = -1
+    k_cache = torch.randn(T, kv_heads, capacity, D, generator=g).bfloat16().cuda()
+    v_cache = pack_v_cache(torch.randn(T, kv_heads, capacity, D, generator=g).bfloat16()).cuda()
+    qkv = torch.randn(T, 3 * kv_heads * D, generator=g).bfloat16()
+    cos, sin = (t.cuda() for t in rope_tables(capacity, D, 500000.0))
+    lens = lens.int()
+
+    def run(order):
+        return ops.decode_attention(qkv[order].cuda(), k_cache, v_cache, slots[order].cuda(), lens[order].cuda(), cos, sin,
+                                    kv_heads, kv_heads)
+
+    straight, order = torch.arange(T), torch.randperm(T, generator=g)
+    out = run(straight)
+    assert torch.equal(run(order), out[order.cuda()])          # (the second launch appends what the first one did)
+    kc, vc = (t.cuda() for t in natural(k_cache, v_cache))
+    pos = (lens.long() - 1).clamp(0, capacity - 1)
+    q = ref.rope_at(qkv[:, : kv_heads * D].double().view(T, kv_heads, D), pos, 500000.0).cuda()
+    for t in range(T):
+        s, L = int(slots[t]), min(int(lens[t]), capacity)
+        want = ref.attend(q[t], kc[s, :L], vc[s, :L]).reshape(-1) if s >= 0 and L > 0 else torch.zeros(kv_heads * D)
+        if int(lens[t]) <= capacity:                           # (beyond it the rotation is by the last angle of the table)
+            assert rel_err(out[t].float(), want) < TOL_BF16, (t, L)
+
+
 @pytest.mark.parametrize("T,capacity,lengths", [(2, 8192, [1, 33, 512, 767]), (8, 1024, [64, 767]), (32, 2048, [2048, 700])])
 def test_decode_attention_stays_whole_where_parts_do_not_pay(ops, T, capacity, lengths):
     """Sequences too short for three parts of 256 positions, and launches with room for two parts only: the bits of the
