@@ -10,13 +10,13 @@ bool dfhip_stream_fits(int M, int N, int64_t k_bytes, int split_k);
 // The parts K should be cut into by a caller with a workspace.
 int dfhip_stream_split(int M, int N, int64_t k_bytes);
 
-// split_k > 1: `partials` holds ceil(N / 64) * 64 * split_k * 64 floats, `arrivals` one zero per 16 columns (left zero).
+// split_k > 1 (up to 32 rows): `partials` holds ceil(N / 64) * 64 * split_k * 64 floats, `arrivals` one zero per 16 columns (left zero).
 int dfhip_stream_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const void* R, void* C, int64_t ldc, int M,
                       int N, int K, int split_k, void* partials, int* arrivals, hipStream_t stream);
 int dfhip_stream_bf16_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                               int M, int N, int K, hipStream_t stream);
 int dfhip_stream_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
-                     const float* w_scale, int M, int N, int K, hipStream_t stream);
+                     const float* w_scale, int M, int N, int K, int split_k, void* partials, int* arrivals, hipStream_t stream);
 int dfhip_stream_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
                              const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, int M, int N,
                              int K, hipStream_t stream);

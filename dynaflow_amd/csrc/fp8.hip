@@ -922,6 +922,7 @@ int launch_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, 
 }
 
 constexpr int F8_MAX_SPLIT = 16;
+constexpr int F8_STREAM = 8;          // the streaming kernel with K in parts, as a variant (up to 32 rows)
 
 // 16-row blocks per wave of a ring tile (256 columns), 0 for the other kernels
 int ring_blocks(int variant) { return variant == 0 ? 8 : variant == 3 ? 6 : variant == 4 ? 4 : 0; }
@@ -1005,9 +1006,27 @@ bool few_rows_streamed(int M, int N, int K, int share, bool may_split) {
   return M <= (share == 1 ? 32 : weights < (int64_t)1 << 27 ? 16 : 8);
 }
 
-// The plan of a launch: -1 for the streaming kernel, else a tile and the parts of K.
+// Parts of K for 9 .. 32 rows beside as many of another nano-batch, where K may be cut (down to the model width): the fewest that give
+// 160 workgroups of 32 columns and more, as a whole K does with fewer columns each, for which the activations are read again.
+// Two such launches in a captured schedule become one, whose workgroups take each weight once for the rows of both; on
+// 128 x 128 tiles they read it twice, and 128 rows of activations with it.  [us a pair in one launch, whole K up to 16 (8192 x 28672:
+// 8) rows or 128 x 128 tiles -> in parts, at 12 / 17 / 24 / 32 rows: 8192 x 28672 60 / 62 / 64 / 64 -> 40 / 42 / 45 / 49, 4096 x 14336
+// 15.4 / 21.4 / 21.5 / 21.9 -> 14.3 / 16.3 / 17.6 / 19.8, 2048 x 16384 14.4 / 17.0 / 17.3 / 17.4 -> 10.0 / 11.3 / 12.1 / 13.5, 8192 x 16384 39
+// / 41 / 39 / 40 -> 31 / 33 / 33 / 35; at 2 rows 4096 x 14336 11.9 -> 13.5; layer 8192 x 28672 of 2 x 12 tokens 163 -> 142.
+// A pair that stays two launches on two streams: 73 / 72 / 76 / 76 -> 72 / 76 / 78 / 81, 22 / 25 / 26 / 26 -> 23 / 23 / 25 / 26, 17 / 19 / 19 / 20
+// -> 14 / 15 / 15 / 16, 45 / 46 / 47 / 48 -> 53 / 53 / 54 / 53]
+int few_rows_parts(int M, int N, int K, int share, bool may_split) {
+  if (!may_split || share < 2 || K <= N || M < 9 || M > 32) return 1;
+  for (int s = 2; s <= 8; s *= 2)
+    if ((int64_t)((N + 31) / 32) * s >= 160) return dfhip_stream_fits(M, N, K, s) ? s : 1;
+  return 1;
+}
+
+// The plan of a launch: -1 for the streaming kernel (F8_STREAM for counts of rows that have a tile as well), or a tile, and the parts of K.
 TilePlan plan_launch(int M, int N, int K, int share, bool may_split) {
-  if (few_rows_streamed(M, N, K, share, may_split)) return {-1, 1, 0.0};
+  const bool streamed = few_rows_streamed(M, N, K, share, may_split);
+  const int parts = few_rows_parts(M, N, K, share, may_split);
+  if (streamed || parts > 1) return {streamed ? -1 : F8_STREAM, parts, 0.0};
   const TilePlan plan = plan_tile(M, N, K, share, may_split);
   const DfhipRing3Plan tiles = three_slabs_cheaper(false, M, N, K, share, plan.variant, plan.split_k, may_split && K > N);
   return tiles.tile < 0 ? plan : TilePlan{DFHIP_RING3_VARIANT + tiles.tile, tiles.split_k, tiles.cost};
@@ -1171,7 +1190,7 @@ extern "C" int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* 
   if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
   const TilePlan plan = plan_launch(M, N, K, share, false);
   if (plan.variant < 0)
-    return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, static_cast<hipStream_t>(stream));
+    return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, 1, nullptr, nullptr, static_cast<hipStream_t>(stream));
   return dfhip_gemm_fp8_nt_variant(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, plan.variant, stream);
 }
 
@@ -1200,6 +1219,8 @@ extern "C" int dfhip_gemm_fp8_plan_tiles(int M, int N, int K, int share, int may
 
 extern "C" size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k) {
   const int tm = ring_blocks(variant);
+  if (M >= 1 && N >= 1 && (variant < 0 || variant == F8_STREAM) && split_k >= 2 && split_k <= F8_MAX_SPLIT)
+    return DFHIP_COMMON_COUNTERS + (size_t)((N + 63) / 64) * 64 * split_k * 64 * sizeof(float);
   if (M >= 1 && N >= 1 && split_k >= 2 && split_k <= DFHIP_RING3_MAX_SPLIT && dfhip_ring3_variant(variant, true))
     return dfhip_ring3_workspace_bytes(M, N, variant - DFHIP_RING3_VARIANT, split_k);
   if (M < 1 || N < 1 || split_k < 2 || split_k > F8_MAX_SPLIT || !tm) return 0;
@@ -1212,12 +1233,16 @@ extern "C" int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* 
                                         int split_k, void* workspace, size_t workspace_bytes, dfhip_stream_t stream) {
   if (int rc = check_gemm(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K)) return rc;
   const int tm = ring_blocks(variant);
-  const bool three_slabs = dfhip_ring3_variant(variant, true);
-  if ((!tm && !three_slabs) || split_k < 2 || split_k > F8_MAX_SPLIT || K / FBK < 2 * split_k) return DFHIP_ERR_BAD_ARGUMENT;
+  const bool three_slabs = dfhip_ring3_variant(variant, true), streamed = variant < 0 || variant == F8_STREAM;
+  if (streamed && (M > 32 || split_k < 2 || !dfhip_stream_fits(M, N, K, split_k))) return DFHIP_ERR_BAD_ARGUMENT;
+  if ((!tm && !three_slabs && !streamed) || split_k < 2 || split_k > F8_MAX_SPLIT || K / FBK < 2 * split_k) return DFHIP_ERR_BAD_ARGUMENT;
   if (!workspace) return DFHIP_ERR_NULL_POINTER;
   if (!dfhip_aligned16(workspace)) return DFHIP_ERR_BAD_ALIGNMENT;
   if (workspace_bytes < dfhip_gemm_fp8_splitk_workspace_bytes(M, N, variant, split_k)) return DFHIP_ERR_BAD_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (streamed)
+    return dfhip_stream_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, split_k,
+                            static_cast<uint8_t*>(workspace) + DFHIP_COMMON_COUNTERS, static_cast<int*>(workspace), s);
   if (three_slabs)
     return dfhip_ring3_fp8(A, lda, W, ldw, C, ldc, a_scale, w_scale, M, N, K, variant - DFHIP_RING3_VARIANT, split_k,
                            workspace, s);

@@ -425,7 +425,7 @@ template <bool FP8, bool FUSED, bool SPLIT>
 int launch_rows(const StreamArgs& p, int width, hipStream_t stream) {
   if (p.side[0].M <= 16) return launch_width<FP8, 1, FUSED, SPLIT>(p, width, stream);
   if (p.side[0].M <= 32) return launch_width<FP8, 2, FUSED, SPLIT>(p, width, stream);
-  if constexpr (!FP8 && (FUSED || SPLIT)) return DFHIP_ERR_BAD_SHAPE;   // bf16: whole K alone, by variant
+  if constexpr (SPLIT || (!FP8 && FUSED)) return DFHIP_ERR_BAD_SHAPE;   // bf16: whole K alone, by variant
   else return launch_width<FP8, 4, FUSED, SPLIT>(p, width, stream);
 }
 
@@ -443,7 +443,7 @@ int width_for(int N, int split_k) {
 template <bool FP8, bool FUSED>
 int dispatch(const StreamArgs& p, hipStream_t stream) {
   const int width = width_for(p.N, p.split_k);
-  if constexpr (!FUSED && !FP8)
+  if constexpr (!FUSED)
     if (p.split_k > 1) return launch_rows<FP8, FUSED, true>(p, width, stream);
   return launch_rows<FP8, FUSED, false>(p, width, stream);
 }
@@ -490,9 +490,9 @@ int dfhip_stream_bf16_gate_up(const void* A, int64_t lda, const void* W, const v
   return dispatch<false, true>(p, stream);
 }
 int dfhip_stream_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
-                     const float* w_scale, int M, int N, int K, hipStream_t stream) {
-  const StreamArgs p{static_cast<const uint8_t*>(W), nullptr, w_scale, nullptr, N, K / 128, 1, ldw,
-                     {{A, nullptr, C, a_scale, nullptr, nullptr, nullptr, lda, ldc, M}, {}}};
+                     const float* w_scale, int M, int N, int K, int split_k, void* partials, int* arrivals, hipStream_t stream) {
+  const StreamArgs p{static_cast<const uint8_t*>(W), nullptr, w_scale, nullptr, N, K / 128, split_k, ldw,
+                     {{A, nullptr, C, a_scale, nullptr, static_cast<float*>(partials), arrivals, lda, ldc, M}, {}}};
   return dispatch<true, false>(p, stream);
 }
 int dfhip_stream_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,

@@ -249,7 +249,8 @@ int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* W, int64_t 
                              const float* a_scale, const float* w_scale, int M, int N, int K, int share,
                              dfhip_stream_t stream);
 /* The same with K cut into split_k parts (2 .. 16, at least two slabs of 128 each), for outputs of too few tiles to
- * fill the GPU; variant 0, 3, 4, 11, 12 or 15.  workspace: dfhip_gemm_fp8_splitk_workspace_bytes bytes, 16-byte aligned, whose
+ * fill the GPU; variant 0, 3, 4, 11, 12 or 15, or up to 32 rows 8 or negative: the streaming kernel (parts of 16 slabs and
+ * more, N <= 16384).  workspace: dfhip_gemm_fp8_splitk_workspace_bytes bytes, 16-byte aligned, whose
  * arrival counters (4 bytes a tile at its start) are zero; they are left zero.  Launches that may overlap need one
  * each.  The parts are added in part order: the same bits in every run.
  * dfhip_gemm_fp8_plan_shared: the variant and split for `share` launches of this shape side by side (variant < 0:
@@ -258,7 +259,7 @@ int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* W, int64_t 
  * split whatever their widths are.
  * dfhip_gemm_fp8_plan_tiles: the same among all tiles, 11, 12 and 15 (those of dfhip_gemm_bf16_nt_variant) included: what
  * dfhip_gemm_fp8_nt_shared launches where may_split is 0.  Both plans leave the same launches of few rows to the
- * streaming kernel (variant < 0). */
+ * streaming kernel (variant < 0); this one cuts K in some of them, and in more launches of up to 32 rows (variant 8). */
 int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
 int dfhip_gemm_fp8_plan_tiles(int M, int N, int K, int share, int may_split, int* variant, int* split_k);
 size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k);

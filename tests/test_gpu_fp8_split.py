@@ -260,3 +260,50 @@ def test_split_launches_of_more_tiles_than_the_common_counters_share_a_workspace
                                              128 * 1030, 1024, 2, workspace.data_ptr(), nbytes, stream) == 0
         want = x.float() @ w.float().t()
         assert (out.float() - want).abs().max().item() <= 2.0 ** -7 * want.abs().max().item()
+
+
+# side by side and cut from 9 to 32 rows: whole K on either side of them, parts of 16 slabs, more parts for narrow outputs, K too short
+@pytest.mark.parametrize("M,N,K,share,parts", [
+    (8, 8192, 28672, 2, 1), (9, 8192, 28672, 2, 2), (32, 8192, 28672, 2, 2), (33, 8192, 28672, 2, 1), (9, 8192, 28672, 1, 1),
+    (12, 4096, 14336, 2, 2), (24, 4096, 4224, 2, 2), (24, 2560, 4096, 2, 2), (24, 2528, 8192, 2, 4), (24, 2048, 4096, 2, 1),
+    (24, 1280, 16384, 4, 4), (24, 1248, 16384, 2, 8), (24, 608, 65536, 2, 1), (24, 16384, 16512, 2, 2), (24, 16392, 28672, 2, 1)])
+def test_few_rows_in_parts(M, N, K, share, parts):
+    lib, v, s = _cabi.load(), ctypes.c_int(), ctypes.c_int()
+    assert lib.dfhip_gemm_fp8_plan_tiles(M, N, K, share, 1, ctypes.byref(v), ctypes.byref(s)) == 0
+    streamed = v.value < 0 or v.value == 8
+    assert s.value == parts if streamed else parts == 1
+    if parts > 1:
+        assert streamed and lib.dfhip_gemm_fp8_splitk_workspace_bytes(M, N, v.value, parts) > 0
+    args = (16, 65536, 16, 65536, 16, 16392, 16, 16)
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 33, 8192, 28672, 8, 2, 16, 1 << 30, None) == -7     # more than 32 rows
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 9, 8192, 3968, 8, 2, 16, 1 << 30, None) == -7       # fewer than 16 slabs a part
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 9, 16392, 28672, 8, 2, 16, 1 << 30, None) == -7     # more tiles than counters
+    assert lib.dfhip_gemm_fp8_nt_splitk(*args, 9, 8192, 28672, 8, 2, 16, 4096, None) == -7         # no room for the parts
+
+
+# one and two row blocks; tiles of 16, 32 and 64 columns, ragged ones; parts of 16 slabs, of uneven lengths, 16 of them
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,split", [(1, 8, 4096, 2), (16, 1032, 4224, 2), (17, 1032, 8320, 4), (32, 2568, 4224, 2), (9, 5128, 4224, 2),
+                                         (31, 264, 33024, 16), (12, 16384, 4096, 2)])
+def test_fp8_streamed_in_parts(M, N, K, split):
+    """Against the product in float64: half an ulp of the bf16 result (2^-8 of it) and the fp32 sums.  A sum goes through an instruction
+    of 128 products, as many of those as a part has slabs, the four waves' sums and those of the parts: at most 128 + K / 128 + 4 +
+    `split` roundings, each off by no more than 2^-24 of a partial sum, and none of those larger than the sum of the magnitudes.  The
+    same bits in every run."""
+    lib = _cabi.load()
+    xq, wq, ws, xs = operands(M, N, K)
+    want = ((xq.double() * xs.double()) @ (wq.double() * ws.double()[:, None]).t())
+    nbytes = lib.dfhip_gemm_fp8_splitk_workspace_bytes(M, N, 8, split)
+    workspace = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+    runs = []
+    for variant in (8, -1, 8):
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert lib.dfhip_gemm_fp8_nt_splitk(
+            xq.data_ptr(), K, wq.data_ptr(), K, out.data_ptr(), N, xs.data_ptr(), ws.data_ptr(), M, N, K, variant, split,
+            workspace.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream) == 0
+        runs.append(out)
+    size = (xq.double().abs() * xs.double()) @ (wq.double().abs() * ws.double()[:, None]).t()
+    off = (runs[0].double() - want).abs()
+    assert (off <= 2.0 ** -8 * want.abs() + (132 + K // 128 + split) * 2.0 ** -24 * size).all()
+    assert torch.equal(runs[0], runs[1]) and torch.equal(runs[0], runs[2])
+    assert not workspace[:4096].any()
