@@ -174,14 +174,19 @@ gemm_ring3_kernel(const Ring3Args p) {
     wait_vmcnt<(U - 2) * D>();
     workgroup_barrier();
     const int next = u == U - 1 ? 0 : u + 1;
-    constexpr int DQ = (MQ + 2) / 3, RQ = (MQ * 3 + 3) / 4;
+    // The loads are spread over the whole slab, the reads over three quarters of it.  A compute unit has 32 KiB of loads in flight
+    // whatever is asked for, so loads asked for early only make the waves wait, and what they put into LDS keeps the reads from it; half a
+    // slab later is early enough.  [us, first third of a slab -> all of it, alone with weights from memory / in the memory-side cache: 670 x
+    // 28672 x 4096 132 / 120 -> 128 / 113, 777 x 4096 x 14336 uncut 186 / 179 -> 183 / 156, 1554 x 28672 x 4096 300 / 294 -> 288 / 277; all at
+    // the head of a slab 144 / 134, 220 / 219, 336 / 333; weights before activations 143 / 121, 211 / 176, 320 / 298]
+    constexpr int RQ = (MQ * 3 + 3) / 4;
 #pragma unroll
     for (int q = 0; q < MQ; ++q) {
       multiply(q, slot);
 #pragma unroll
       for (int r = q * READS / RQ; r < (q + 1) * READS / RQ && r < READS; ++r) read(r, slot ^ 1, next);
 #pragma unroll
-      for (int t = q * D / DQ; t < (q + 1) * D / DQ && t < D; ++t) dma(t, kt + U, u);
+      for (int t = q * D / MQ; t < (q + 1) * D / MQ; ++t) dma(t, kt + U, u);
       DFHIP_PIN;
     }
     u = next;
