@@ -1477,6 +1477,9 @@ gemm_bf16_skinny_kernel(const SkinnyArgs p) {
 // a unit of the ring is A 16 KiB | W 32 KiB and three of them fit, so a slab's first fragments are read after the
 // barrier that follows its landing (no read ahead across slabs) and two slabs are in flight meanwhile.  For two
 // launches that share the GPU (2 x 112 workgroups at 14336 outputs: one round together) and for 129 .. 256 rows.
+// The loads of a slab are asked for a quarter at each k-step: a compute unit has 32 KiB of them in flight whatever is asked for, and the
+// waves wait for the rest.  [us, all at the head of a slab -> spread: 256 rows alone 78.5 -> 75.2, in pairs on two streams 138 -> 131, 100 / 128
+// rows in pairs 83.5 / 86.5 -> 80.8 / 84.5, joined 76.8 / 78.4 -> 74.4 / 75.8; gemm_bf16_skinny_kernel, whose slabs are shorter, is level]
 // Same instruction and same order of K as gemm_bf16_skinny_kernel<true>: the same bits.
 constexpr int SKW_BN = 128, SKW_UNIT = 49152, SKW_UNITS = 3, SKW_LDS = SKW_UNITS * SKW_UNIT;
 
@@ -1518,12 +1521,13 @@ gemm_bf16_skinny_wide_kernel(const SkinnyArgs p) {
     wr = wr < N ? wr : N - 1;
     w_src[t] = reinterpret_cast<const uint8_t*>((((row >> 6) & 1) ? W2 : W) + (int64_t)wr * ldw + chunk * 8);
   }
-  auto issue = [&](int slab, int unit) {
+  auto issue = [&](int slab, int unit, int quarter) {       // a quarter of a slab's loads
     const int64_t off = (int64_t)(slab < KT ? slab : KT - 1) * (BK * 2);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) dma16(unit * SKW_UNIT + (wave * 4 + t) * 1024, a_src[t] + off);
-#pragma unroll
-    for (int t = 0; t < 8; ++t) dma16(unit * SKW_UNIT + 16384 + (wave * 8 + t) * 1024, w_src[t] + off);
+    for (int t = 3 * quarter; t < 3 * quarter + 3; ++t) {
+      if (t < 4) dma16(unit * SKW_UNIT + (wave * 4 + t) * 1024, a_src[t] + off);
+      else dma16(unit * SKW_UNIT + 16384 + (wave * 8 + t - 4) * 1024, w_src[t - 4] + off);
+    }
   };
 
   const int frow = lane & 31, fhalf = lane >> 5, fswz = (frow >> 1) & 7;
@@ -1548,18 +1552,18 @@ gemm_bf16_skinny_wide_kernel(const SkinnyArgs p) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) fw[slot][j] = *reinterpret_cast<const bf16x8*>(u + w_lane + j * 4096 + koff[ks]);
   };
-  issue(0, 0);
-  issue(1, 1);
+#pragma unroll
+  for (int h = 0; h < 8; ++h) issue(h / 4, h / 4, h % 4);
   wait_vmcnt<12>();          // slab 0 has landed
   workgroup_barrier();
   int unit = 0;
   for (int kt = 0; kt < KT; ++kt) {
     read_frags(unit, 0, 0);
     const int free_unit = unit == 0 ? SKW_UNITS - 1 : unit - 1;   // slab kt-1: everybody passed the barrier after it
-    issue(kt + 2, free_unit);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const int slot = ks & 1;
+      issue(kt + 2, free_unit, ks);
       if (ks < 3) read_frags(unit, ks + 1, slot ^ 1);
       DFHIP_PIN;
 #pragma unroll
