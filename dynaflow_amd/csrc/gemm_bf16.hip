@@ -1287,13 +1287,21 @@ gemm_bf16_skinny_kernel(const SkinnyArgs p) {
       w_src[t] = reinterpret_cast<const uint8_t*>(W + (int64_t)wr * ldw + chunk * 8);
     }
   }
+  // A launch for both nano-batches is the only one that reads a weight (two workgroups of an XCD do so together): non-temporally.  [us,
+  // 2 x 40 / 48 / 64 rows: gate + up 2 x 14336 x 4096 55.6 / 56.5 / 58.3 -> 52.8 / 53.3 / 54.3, 14336 x 4096 36.7 / 37.6 / 39.5 -> 34.4 / 35.0 /
+  // 36.9; of a launch for one of them the other finds the weights in the memory-side cache, 75 -> 85 at 48 rows; K in parts, whose rows are
+  // pieces of 2 KiB and more, 2048 x 5632 16.4 -> 17.9, 4096 x 4096 16.2 -> 17.9]
+  const bool once = PAIRED != DFHIP_ALONE && split_k == 1;
   auto issue = [&](int slab, int unit) {
     const int64_t off = (int64_t)(slab0 + (slab < KT ? slab : KT - 1)) * (BK * 2);
 #pragma unroll
     for (int t = 0; t < T::A_DMA; ++t) dma16(unit * T::UNIT_BYTES + (wave * T::A_DMA + t) * 1024, a_src[t] + off);
 #pragma unroll
-    for (int t = 0; t < T::W_DMA; ++t)
-      dma16(unit * T::UNIT_BYTES + T::A_BYTES + (wave * T::W_DMA + t) * 1024, w_src[t] + off);
+    for (int t = 0; t < T::W_DMA; ++t) {
+      const uint32_t at = unit * T::UNIT_BYTES + T::A_BYTES + (wave * T::W_DMA + t) * 1024;
+      if (once) dma16_once(at, w_src[t] + off);
+      else dma16(at, w_src[t] + off);
+    }
   };
 
   const int frow = lane & 31, fhalf = lane >> 5, fswz = (frow >> 1) & 7;
