@@ -105,6 +105,8 @@ SIGNATURES: dict[str, tuple] = {
     ),
     "dfhip_gemm_fp8_gate_up_silu_absmax": (c_int, [_P, c_int64, _P, _P, c_int64, _P, c_int64, _P, _P, _P, _P, c_int,
                                                      c_int, c_int, _P]),
+    "dfhip_gemm_fp8_gate_up_silu_quant_shared": (c_int, [_P, c_int64, _P, _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, _P, _P,
+                                                         c_int, c_int, c_int, c_int, _P]),
     "dfhip_gemm_fp8_gate_up_silu_absmax_shared": (c_int, [_P, c_int64, _P, _P, c_int64, _P, c_int64, _P, _P, _P, _P,
                                                             c_int, c_int, c_int, c_int, _P]),
     "dfhip_silu_mul_bf16": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P]),

@@ -57,5 +57,7 @@ int dfhip_ring3_bf16_gate_up(const void* A, int64_t lda, const void* W, const vo
 int dfhip_ring3_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
                     const float* w_scale, int M, int N, int K, int tile, int split_k, void* workspace, hipStream_t stream);
 int dfhip_ring3_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
-                            const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, int M, int N,
-                            int K, int tile, hipStream_t stream);
+                            const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, bool amax_apart,
+                            int M, int N, int K, int tile, hipStream_t stream);
+// Workgroups of the latter; with `amax_apart` each leaves four maxima.
+int dfhip_ring3_gate_up_blocks(int M, int N, int tile);

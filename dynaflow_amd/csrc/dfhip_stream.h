@@ -18,5 +18,7 @@ int dfhip_stream_bf16_gate_up(const void* A, int64_t lda, const void* W, const v
 int dfhip_stream_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const float* a_scale,
                      const float* w_scale, int M, int N, int K, int split_k, void* partials, int* arrivals, hipStream_t stream);
 int dfhip_stream_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
-                             const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, int M, int N,
-                             int K, hipStream_t stream);
+                             const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, bool amax_apart,
+                             int M, int N, int K, hipStream_t stream);
+// Workgroups of a launch with whole K; with `amax_apart` each leaves four maxima.
+int dfhip_stream_blocks(int N);

@@ -206,9 +206,10 @@ DFHIP_DEVICE void quant_after(unsigned block, unsigned blocks, const uint16_t* _
   load();
   float m = 0.0f;
   if (PARTS) {
+    for (int p0 = threadIdx.x; p0 < n_parts; p0 += QPARTS)
 #pragma unroll
-    for (int p = 0; p < QPARTS / QT; ++p)
-      if (p * QT + (int)threadIdx.x < n_parts) m = fmaxf(m, amax[p * QT + threadIdx.x]);
+      for (int p = 0; p < QPARTS / QT; ++p)
+        if (p0 + p * QT < n_parts) m = fmaxf(m, amax[p0 + p * QT]);
     m = block_max<QT>(m);
   } else {
     __shared__ float cell;
@@ -1253,24 +1254,11 @@ extern "C" int dfhip_gemm_fp8_nt_splitk(const void* A, int64_t lda, const void* 
   }
 }
 
-extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t lda, const void* W_gate,
-                                                         const void* W_up, int64_t ldw, void* act, int64_t ld_act,
-                                                         const float* a_scale, const float* w_gate_scale,
-                                                         const float* w_up_scale, float* amax, int M, int I, int K,
-                                                         int share, dfhip_stream_t stream) {
-  if (!A || !W_gate || !W_up || !act || !a_scale || !w_gate_scale || !w_up_scale || !amax)
-    return DFHIP_ERR_NULL_POINTER;
-  if (M < 1 || I < 8 || K < 1 || K % FBK != 0 || I % 8 != 0) return DFHIP_ERR_BAD_SHAPE;
-  if (lda < K || ldw < K || ld_act < I) return DFHIP_ERR_BAD_STRIDE;
-  if (lda >= (1 << 23) || ldw >= (1 << 23)) return DFHIP_ERR_BAD_STRIDE;
-  if (lda % 16 || ldw % 16 || ld_act % 8 || !dfhip_aligned16(A) || !dfhip_aligned16(W_gate) ||
-      !dfhip_aligned16(W_up) || !dfhip_aligned16(act) || !dfhip_aligned16(w_gate_scale) ||
-      !dfhip_aligned16(w_up_scale))
-    return DFHIP_ERR_BAD_ALIGNMENT;
-  if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
-  if (few_rows_streamed(M, I, K, share, false))
-    return dfhip_stream_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I,
-                                    K, static_cast<hipStream_t>(stream));
+namespace {
+// The kernel of a gate + up + SiLU*mul launch: a three-slab tile, the streaming kernel (both -1), or a ring tile of 32 `tm` rows.
+struct GateUpPlan { int three_slabs, tm; };
+GateUpPlan plan_gate_up(int M, int I, int K, int share) {
+  if (few_rows_streamed(M, I, K, share, false)) return {-1, -1};
   // the height of the tile that costs least in rounds (see tile_cost); every height adds in the same order.  A pair of
   // 2 x 14336 x 4096 at 192 / 256 rows: one round of 192 and 256-row tiles 53 / 59 us, two of 128-row ones 66 / 68.  (Of a
   // pair the last round runs beside the other launch, and can cost less than it is priced at: 2 x 12288 x 6144 at 700
@@ -1282,12 +1270,33 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t 
     const double cost = tile_cost(tiles, 1, share, K, r.per_slab, r.tm);
     if (&r == &F8_RINGS[0] || cost < least) { ring = &r; least = cost; }
   }
-  hipStream_t s = static_cast<hipStream_t>(stream);
   const DfhipRing3Plan three = three_slabs_cheaper(true, M, I, K, share, ring->variant, 1, false);
-  if (three.tile >= 0)
-    return dfhip_ring3_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I, K,
-                                   three.tile, s);
-  switch (ring->tm) {
+  return three.tile >= 0 ? GateUpPlan{three.tile, 0} : GateUpPlan{-1, ring->tm};
+}
+int check_gate_up(const void* A, int64_t lda, const void* W_gate, const void* W_up, int64_t ldw, const void* act, int64_t ld_act,
+                  const float* a_scale, const float* w_gate_scale, const float* w_up_scale, const float* amax, int M, int I, int K,
+                  int share) {
+  if (!A || !W_gate || !W_up || !act || !a_scale || !w_gate_scale || !w_up_scale || !amax)
+    return DFHIP_ERR_NULL_POINTER;
+  if (M < 1 || I < 8 || K < 1 || K % FBK != 0 || I % 8 != 0) return DFHIP_ERR_BAD_SHAPE;
+  if (lda < K || ldw < K || ld_act < I) return DFHIP_ERR_BAD_STRIDE;
+  if (lda >= (1 << 23) || ldw >= (1 << 23)) return DFHIP_ERR_BAD_STRIDE;
+  if (lda % 16 || ldw % 16 || ld_act % 8 || !dfhip_aligned16(A) || !dfhip_aligned16(W_gate) ||
+      !dfhip_aligned16(W_up) || !dfhip_aligned16(act) || !dfhip_aligned16(w_gate_scale) ||
+      !dfhip_aligned16(w_up_scale))
+    return DFHIP_ERR_BAD_ALIGNMENT;
+  if (share < 1 || share > 16) return DFHIP_ERR_BAD_ARGUMENT;
+  return DFHIP_OK;
+}
+int launch_gate_up(const GateUpPlan& plan, const void* A, int64_t lda, const void* W_gate, const void* W_up, int64_t ldw, void* act,
+                   int64_t ld_act, const float* a_scale, const float* w_gate_scale, const float* w_up_scale, float* amax,
+                   bool amax_apart, int M, int I, int K, hipStream_t s) {
+  if (plan.three_slabs >= 0)
+    return dfhip_ring3_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, amax_apart, M, I,
+                                   K, plan.three_slabs, s);
+  switch (plan.tm) {
+    case -1: return dfhip_stream_fp8_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax,
+                                             amax_apart, M, I, K, s);
     case 8: return launch_fp8_ring_fused<8>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax,
                                             M, I, K, s);
     case 6: return launch_fp8_ring_fused<6>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax,
@@ -1295,6 +1304,37 @@ extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t 
     default: return launch_fp8_ring_fused<4>(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale,
                                              amax, M, I, K, s);
   }
+}
+}  // namespace
+
+extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t lda, const void* W_gate,
+                                                         const void* W_up, int64_t ldw, void* act, int64_t ld_act,
+                                                         const float* a_scale, const float* w_gate_scale,
+                                                         const float* w_up_scale, float* amax, int M, int I, int K,
+                                                         int share, dfhip_stream_t stream) {
+  if (int rc = check_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax, M, I, K, share)) return rc;
+  return launch_gate_up(plan_gate_up(M, I, K, share), A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, amax,
+                        false, M, I, K, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int dfhip_gemm_fp8_gate_up_silu_quant_shared(const void* A, int64_t lda, const void* W_gate, const void* W_up, int64_t ldw,
+                                                        void* act, int64_t ld_act, void* q, int64_t ld_q, const float* a_scale,
+                                                        const float* w_gate_scale, const float* w_up_scale, float* parts,
+                                                        float* scale_out, int M, int I, int K, int share, dfhip_stream_t stream) {
+  if (int rc = check_gate_up(A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, parts, M, I, K, share)) return rc;
+  if (int rc = check_q(act, ld_act, M, I)) return rc;
+  if (int rc = check_q_out(q, ld_q, I)) return rc;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const GateUpPlan plan = plan_gate_up(M, I, K, share);
+  const int64_t blocks = plan.three_slabs >= 0 ? dfhip_ring3_gate_up_blocks(M, I, plan.three_slabs)
+                                               : plan.tm < 0 ? dfhip_stream_blocks(I) : DFHIP_FP8_GEMM_PARTS;
+  const bool apart = 4 * blocks <= DFHIP_FP8_GEMM_PARTS;
+  if (!apart)
+    if (int rc = dfhip_fill_u32(parts, 0u, 1, stream)) return rc;
+  if (int rc = launch_gate_up(plan, A, lda, W_gate, W_up, ldw, act, ld_act, a_scale, w_gate_scale, w_up_scale, parts, apart, M, I, K, s))
+    return rc;
+  return apart ? launch_quant_after<true>(act, ld_act, q, ld_q, M, I, parts, 4 * (int)blocks, nullptr, scale_out, s)
+               : launch_quant_after<false>(act, ld_act, q, ld_q, M, I, parts, 0, nullptr, scale_out, s);
 }
 
 extern "C" int dfhip_gemm_fp8_gate_up_silu_absmax(const void* A, int64_t lda, const void* W_gate, const void* W_up,

@@ -316,9 +316,7 @@ gemm_ring3_kernel(const Ring3Args p) {
       if (FP8) *at = o; else __builtin_nontemporal_store(o, at);
     }
     if constexpr (FP8) {
-      vmax = wave_max(vmax);
-      // non-negative floats order like their bit patterns
-      if (lane == 0 && vmax > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(my.amax), __float_as_uint(vmax));
+      fold_amax(my, block, wave, wave_max(vmax));
     }
   } else {
     const int m_base = m0 + wave_m * (16 * IB), n_base = n0 + wave_n * (16 * JB);
@@ -427,9 +425,13 @@ int dfhip_ring3_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, void
                      : launch_tile<true, false, false>(p, tile, nullptr, stream);
 }
 int dfhip_ring3_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
-                            const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, int M, int N,
-                            int K, int tile, hipStream_t stream) {
+                            const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, bool amax_apart,
+                            int M, int N, int K, int tile, hipStream_t stream) {
   const Ring3Args p{static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), w_scale, w2_scale, N, K / 128, 0, 0, 1,
-                    ldw, {{A, nullptr, C, a_scale, amax, nullptr, nullptr, lda, ldc, M}, {}}};
+                    ldw, {{A, nullptr, C, a_scale, amax, nullptr, nullptr, lda, ldc, M, amax_apart}, {}}};
   return launch_tile<true, true, false>(p, tile, nullptr, stream);
+}
+int dfhip_ring3_gate_up_blocks(int M, int N, int tile) {
+  const DfhipRing3Tile& t = DFHIP_RING3[tile];
+  return ((M + t.rows - 1) / t.rows) * ((N + t.cols / 2 - 1) / (t.cols / 2));
 }

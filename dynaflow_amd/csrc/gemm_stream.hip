@@ -352,12 +352,8 @@ gemm_stream_kernel(const StreamArgs p) {
     if (i0 + RI < MB) __syncthreads();
   }
   if constexpr (FP8 && FUSED) {
-    // non-negative floats order like their bit patterns
 #pragma unroll
-    for (int c = 0; c <= MERGED; ++c) {
-      const float top = wave_max(vmax[c]);
-      if (lane == 0 && top > 0.0f) atomicMax(reinterpret_cast<unsigned int*>(p.side[c].amax), __float_as_uint(top));
-    }
+    for (int c = 0; c <= MERGED; ++c) fold_amax(p.side[c], tile, wave, wave_max(vmax[c]));
   }
 }
 
@@ -496,9 +492,13 @@ int dfhip_stream_fp8(const void* A, int64_t lda, const void* W, int64_t ldw, voi
   return dispatch<true, false>(p, stream);
 }
 int dfhip_stream_fp8_gate_up(const void* A, int64_t lda, const void* W, const void* W2, int64_t ldw, void* C, int64_t ldc,
-                             const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, int M, int N,
-                             int K, hipStream_t stream) {
+                             const float* a_scale, const float* w_scale, const float* w2_scale, float* amax, bool amax_apart,
+                             int M, int N, int K, hipStream_t stream) {
   const StreamArgs p{static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(W2), w_scale, w2_scale, N, K / 128, 1, ldw,
-                     {{A, nullptr, C, a_scale, amax, nullptr, nullptr, lda, ldc, M}, {}}};
+                     {{A, nullptr, C, a_scale, amax, nullptr, nullptr, lda, ldc, M, amax_apart}, {}}};
   return dispatch<true, true>(p, stream);
+}
+int dfhip_stream_blocks(int N) {
+  const int cols = 16 * width_for(N, 1);
+  return (N + cols - 1) / cols;
 }

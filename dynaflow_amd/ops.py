@@ -734,6 +734,8 @@ torch.library.register_fake(
 # --------------------------------------------------------------------- fp8
 #: DFHIP_FP8_PARTS: floats in which the blocks of a quantisation leave their maxima
 _FP8_PARTS = 1024
+#: DFHIP_FP8_GEMM_PARTS, and the rows up to which a gate + up launch is short enough for the clearing of a cell to show
+_FP8_GEMM_PARTS, _FP8_ONE_CALL_ROWS = 4096, 128
 
 
 def _quant_fp8_impl(x: torch.Tensor):
@@ -792,6 +794,16 @@ def _gate_up_silu_quant_fp8_impl(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w
         wg, wu = wg.contiguous(), wu.contiguous()
         ldg = K
     act = torch.empty((M, I), dtype=torch.bfloat16, device=x_q.device)
+    if 0 < M <= _FP8_ONE_CALL_ROWS and K >= 2048:
+        # the waves leave their maxima side by side: no cell to clear in front of a launch that is short itself
+        scale = torch.empty(1 + _FP8_GEMM_PARTS, dtype=torch.float32, device=x_q.device)
+        q = torch.empty((M, I), dtype=FP8_DTYPE, device=x_q.device)
+        gate_scale, up_scale = w_gate_scale.contiguous(), w_up_scale.contiguous()
+        rc = lib.dfhip_gemm_fp8_gate_up_silu_quant_shared(
+            a.data_ptr(), lda, wg.data_ptr(), wu.data_ptr(), ldg, act.data_ptr(), I, q.data_ptr(), I, x_scale.data_ptr(),
+            gate_scale.data_ptr(), up_scale.data_ptr(), scale.data_ptr() + 4, scale.data_ptr(), M, I, K, _side_by_side(), _stream())
+        _cabi.check("dfhip_gemm_fp8_gate_up_silu_quant_shared", rc)
+        return q.view(*x_q.shape[:-1], I), scale[:1]
     # The scale, and the cell that the fused launch folds max |act| into: memory of this call (or of the graph that it is
     # captured into), so that nothing else, on whatever stream, folds into it or clears it in between.
     scale = torch.empty(2, dtype=torch.float32, device=x_q.device)

@@ -283,6 +283,13 @@ int dfhip_gemm_fp8_gate_up_silu_absmax_shared(const void* A, int64_t lda, const 
                                               int64_t ldw, void* act, int64_t ld_act, const float* a_scale,
                                               const float* w_gate_scale, const float* w_up_scale, float* amax, int M,
                                               int I, int K, int share, dfhip_stream_t stream);
+/* That launch and the quantisation of act behind it: the codes q [M, I] and the scale that dfhip_quant_fp8_bf16 gives.  Nothing has to
+ * be cleared: the maxima meet in `parts` (DFHIP_FP8_GEMM_PARTS floats, contents of no matter before and after). */
+#define DFHIP_FP8_GEMM_PARTS 4096
+int dfhip_gemm_fp8_gate_up_silu_quant_shared(const void* A, int64_t lda, const void* W_gate, const void* W_up, int64_t ldw,
+                                             void* act, int64_t ld_act, void* q, int64_t ld_q, const float* a_scale,
+                                             const float* w_gate_scale, const float* w_up_scale, float* parts, float* scale_out,
+                                             int M, int I, int K, int share, dfhip_stream_t stream);
 
 /* ------------------------------------------------------------ elementwise
  *

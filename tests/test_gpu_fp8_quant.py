@@ -95,3 +95,31 @@ def test_fused_launches_of_two_threads_on_one_stream():
         assert len(got[i]) == 40
         for q, scale in got[i]:
             assert torch.equal(scale, want[i][1]) and torch.equal(q.view(torch.uint8), want[i][0].view(torch.uint8))
+
+
+# streamed in 16, 32 and 64 columns a workgroup, ragged; three-slab tiles; more workgroups than parts have room for; a ring tile
+@pytest.mark.parametrize("M,I,K,share", [(1, 136, 2048, 1), (17, 5120, 4096, 2), (32, 16392, 4096, 1), (128, 14336, 4096, 1), (40, 7176, 4096, 2),
+                                         (16, 65544, 2048, 1), (128, 1032, 2048, 16)])
+def test_gate_up_with_maxima_side_by_side(M, I, K, share):
+    """The codes and the scale of the launch that folds into a cell and the quantisation behind it; parts that hold infinities before."""
+    lib, s = _cabi.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(M + I)
+    x, wg, wu = ((torch.randn(shape, generator=g, device="cuda") * 20).to(torch.float8_e4m3fn) for shape in ((M, K), (I, K), (I, K)))
+    xs, ws = torch.full((1,), 0.01, device="cuda"), torch.rand(I, generator=g, device="cuda") * 0.01
+    act, amax, scale = torch.empty((M, I), dtype=torch.bfloat16, device="cuda"), torch.zeros(1, device="cuda"), torch.empty(1, device="cuda")
+    want, q = (torch.zeros((M, I), dtype=torch.uint8, device="cuda") for _ in range(2))
+    weights = (wg.data_ptr(), wu.data_ptr(), K, act.data_ptr(), I)
+    scales = (xs.data_ptr(), ws.data_ptr(), ws.data_ptr())
+    assert lib.dfhip_gemm_fp8_gate_up_silu_absmax_shared(x.data_ptr(), K, *weights, *scales, amax.data_ptr(), M, I, K, share, s) == 0
+    assert lib.dfhip_quant_fp8_bf16(act.data_ptr(), I, want.data_ptr(), I, M, I, amax.data_ptr(), scale.data_ptr(), s) == 0
+    want_act, want_scale = act.clone(), scale.clone()
+    parts = torch.full((4096,), float("inf"), device="cuda")
+    for _ in range(2):
+        act.zero_(), scale.zero_()
+        assert lib.dfhip_gemm_fp8_gate_up_silu_quant_shared(x.data_ptr(), K, *weights, q.data_ptr(), I, *scales, parts.data_ptr(),
+                                                            scale.data_ptr(), M, I, K, share, s) == 0
+        assert torch.equal(act, want_act) and torch.equal(scale, want_scale) and torch.equal(q, want)
+    assert lib.dfhip_gemm_fp8_gate_up_silu_quant_shared(x.data_ptr(), K, *weights, None, I, *scales, parts.data_ptr(), scale.data_ptr(),
+                                                        M, I, K, share, s) == -1
+    assert lib.dfhip_gemm_fp8_gate_up_silu_quant_shared(x.data_ptr(), K, *weights, q.data_ptr(), I, *scales, None, scale.data_ptr(),
+                                                        M, I, K, share, s) == -1
