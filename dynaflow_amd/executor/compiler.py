@@ -84,8 +84,11 @@ class SubgraphBackend:
                 )
                 fn = self.callables_per_size[size] = self.compile(list(args), size)
             return fn(*args, **kwargs)
-        assert self.callable_dynamic is not None
-        return self.callable_dynamic(*args, **kwargs)
+        fn = self.callable_dynamic
+        assert fn is not None
+        if isinstance(fn, fx.GraphModule) and not (fn._forward_hooks or fn._forward_pre_hooks):
+            return fn.forward(*args, **kwargs)           # (3 us less than through Module.__call__)
+        return fn(*args, **kwargs)
 
 
 class SubgraphCompiler(fx.Interpreter):

@@ -39,7 +39,7 @@ from dynaflow_amd.matching import split_graph, tag_graph
 from dynaflow_amd.runtime import capture_plan
 from dynaflow_amd.runtime.device import get_device, stream_key
 from dynaflow_amd.runtime.engine import DynaFlowEngine
-from dynaflow_amd.runtime.loop import run_coroutine
+from dynaflow_amd.runtime.loop import run_coroutine, run_without_loop
 
 log = logging.getLogger("dynaflow")
 if os.environ.get("DYNAFLOW_VERBOSE"):
@@ -238,7 +238,8 @@ class DynaFlowManager:
                     return self.engine.execute_single_batch(split, args, kwargs)
                 if self._wants_whole_graph(split):
                     return self._forward_whole_graph(split, args, kwargs)
-                return run_coroutine(self._forward_async(args, kwargs, split))
+                run = run_without_loop if self._schedules_plainly() else run_coroutine
+                return run(self._forward_async(args, kwargs, split))
             finally:
                 self.cached_config = None
 
@@ -259,7 +260,7 @@ class DynaFlowManager:
                 await self.scheduler.schedule(ExecutionContext(split, forward=forward))
                 results, events = await forward.completed()
         # the caller's stream continues only after every nano-batch's last launch
-        for event in events:
+        for event in get_device().tails(events):
             event.wait()
         return join_results(results, len(results), getattr(self.engine, "shared_output_buffer", None))
 

@@ -14,6 +14,7 @@ All streams are created at the default priority.
 from __future__ import annotations
 
 import contextlib
+import itertools
 import threading
 from typing import Any
 
@@ -75,6 +76,15 @@ class HostDevice:
     def new_event(self) -> HostEvent:
         return HostEvent(self.log)
 
+    def starts(self, lanes: int) -> list[HostEvent]:
+        events = [self.new_event() for _ in range(lanes)]
+        for event in events:
+            event.record()
+        return events
+
+    def tails(self, events: list) -> list:
+        return events
+
     def new_stream(self, name: str | None = None, cu_mask: "list[int] | None" = None) -> HostStream:
         self._stream_count += 1
         stream = HostStream(name or f"stream{self._stream_count}")
@@ -122,6 +132,11 @@ def current_stream() -> "torch.cuda.Stream":
     return stream
 
 
+def _make_current(stream: "torch.cuda.Stream") -> None:
+    """``torch.cuda.set_stream`` for a stream that is one."""
+    torch._C._cuda_setStream(stream_id=stream.stream_id, device_index=stream.device_index, device_type=stream.device_type)
+
+
 class _CurrentStream:
     """``torch.cuda.stream`` for a stream of the current device."""
 
@@ -132,11 +147,11 @@ class _CurrentStream:
 
     def __enter__(self) -> "torch.cuda.Stream":
         self._previous = current_stream()
-        torch.cuda.set_stream(self._stream)
+        _make_current(self._stream)
         return self._stream
 
     def __exit__(self, *exc) -> None:
-        torch.cuda.set_stream(self._previous)
+        _make_current(self._previous)
 
 
 class _Range:
@@ -156,12 +171,14 @@ class HipEvent:
     """A HIP event that knows the stream it was recorded on.
 
     ``wait`` on that very stream issues nothing: stream order already gives the edge, and under stream capture
-    such a wait would make the stream its own child in the runtime's books (see ``capture_plan``).  While the
+    such a wait would make the stream its own child in the runtime's books (see ``capture_plan``).  Nor does a second
+    wait of one stream (a wait for work that is still running costs the host 8 us).  While the
     device's ``trace`` is a list, every ``record`` / ``wait`` is logged there in the recording seam's format.
     """
 
-    __slots__ = ("_owner", "_event", "_recorded_on", "uid")
+    __slots__ = ("_owner", "_event", "_recorded_on", "_order", "_waited", "uid")
     _counter = 0
+    _records = itertools.count(1)
 
     def __init__(self, owner: "HipDevice") -> None:
         HipEvent._counter += 1
@@ -169,20 +186,26 @@ class HipEvent:
         self._owner = owner
         self._event = torch.cuda.Event()
         self._recorded_on: tuple[int, int] | None = None
+        self._order = 0                                         # of the last record among those of all events
+        self._waited: tuple[tuple[int, int], ...] = ()          # streams that wait for it already
 
     def record(self, stream: "torch.cuda.Stream | None" = None) -> None:
-        stream = stream if stream is not None else current_stream()
-        self._recorded_on = stream_key(stream)
-        self._owner.note(("record", self.uid, self._recorded_on), stream)
+        if stream is None:
+            stream = current_stream()
+        self._recorded_on = key = (stream.device_index, stream.cuda_stream)
+        if self._owner.trace is not None:
+            self._owner.note(("record", self.uid, key), stream)
         self._event.record(stream)
+        self._order, self._waited = next(HipEvent._records), ()
 
     def wait(self, stream: "torch.cuda.Stream | None" = None) -> None:
-        key = stream_key(stream) if stream is not None else current_stream_key()
+        key = (stream.device_index, stream.cuda_stream) if stream is not None else current_stream_key()
         if self._owner.trace is not None:
             self._owner.note(("wait", self.uid, key), stream if stream is not None else current_stream())
-        if self._recorded_on is None or key == self._recorded_on:
+        if self._recorded_on is None or key == self._recorded_on or key in self._waited:
             return
         self._event.wait(stream if stream is not None else current_stream())
+        self._waited += (key,)
 
     def synchronize(self) -> None:
         self._event.synchronize()
@@ -241,6 +264,22 @@ class HipDevice:
 
     def new_event(self) -> HipEvent:
         return HipEvent(self)
+
+    def starts(self, lanes: int) -> "list[HipEvent]":
+        """The event, recorded now, that each of ``lanes`` nano-batches starts behind."""
+        start = self.new_event()
+        start.record()
+        return [start] * lanes
+
+    def tails(self, events: "list[HipEvent]") -> "list[HipEvent]":
+        """Those of ``events``, recorded by the forward that asks, behind which lies the work of all of them: the last on
+        each stream."""
+        last = {}
+        for event in events:
+            other = last.get(event._recorded_on)
+            if other is None or other._order < event._order:
+                last[event._recorded_on] = event
+        return list(last.values())
 
     def new_stream(self, name: str | None = None, cu_mask: "list[int] | None" = None) -> "torch.cuda.Stream":
         """A stream at the default priority.  ``cu_mask`` (32-bit words, bit i = compute unit i may run this

@@ -36,7 +36,7 @@ import torch.fx
 from dynaflow_amd.config import DynaFlowConfig
 from dynaflow_amd.interface import OperatorHandle, SplitConfig
 from dynaflow_amd.runtime.device import get_device
-from dynaflow_amd.runtime.env import ExecutionEnvironment, set_op_handle
+from dynaflow_amd.runtime.env import ExecutionEnvironment, set_op_handle, swap_op_handle
 from dynaflow_amd.runtime.loop import may_have_other_tasks
 
 _DEFAULT_MAX_TOKENS = 16384
@@ -134,6 +134,17 @@ class DynaFlowEngine:
         self.placeholder_node_to_idx: dict[torch.fx.Node, int] = {
             node: i for i, node in enumerate(self.placeholder_nodes)
         }
+        #: inputs that every nano-batch gets whole (tensors whose dim 0 is no number of tokens: weights)
+        self._whole_inputs: set[torch.fx.Node] = {
+            node for node in self.placeholder_nodes
+            if isinstance(example := node.meta.get("example_value", None), torch.Tensor) and example.dim() > 0
+            and not _is_symbolic(example.shape[0])
+        }
+        #: of a sub-graph call: the node-valued positional inputs, which are the ones that are forwarded (engine.py:304-310)
+        self._node_inputs: dict[torch.fx.Node, list[torch.fx.Node]] = {
+            node: [a for a in node.args if isinstance(a, torch.fx.Node)] for node in self.nodes if node.op == "call_module"
+        }
+        self._returning_module: "tuple[str | None] | None" = None     # of _output_module, once it is known
         #: (module name, nano-batch) of every launch of the last ``execute``
         self.issue_trace: list[tuple[str, int]] = []
         self.last_env: ExecutionEnvironment | None = None
@@ -167,6 +178,9 @@ class DynaFlowEngine:
         (engine.py:441-477).
         """
         idx = self.placeholder_node_to_idx[node]
+        if node in self._whole_inputs:
+            env.put(batch_idx, node, args[idx])
+            return
         example = node.meta.get("example_value", None)
         if isinstance(example, torch.Tensor):
             if not _is_symbolic(example.shape[0]):
@@ -281,7 +295,9 @@ class DynaFlowEngine:
             return None
         if list(split_config.num_tokens_padded) != list(split_config.num_tokens):
             return None
-        module = self._output_module()
+        if self._returning_module is None:
+            self._returning_module = (self._output_module(),)
+        (module,) = self._returning_module
         return None if module is None else _SharedOutput(module, split_config, device)
 
     # ------------------------------------------------------------------ dry-run
@@ -442,7 +458,6 @@ class ScheduledForward:
         engine.last_env = self.env
         engine.issue_trace = []
         self.results: dict[int, Any] = {}
-        self.tail_events = [self.device.new_event() for _ in range(lanes)]
         self.finished = [False] * lanes
         self.ready: list[deque[OperatorHandle]] = [deque() for _ in range(lanes)]
         # operators handed out and not yet executed, per nano-batch
@@ -450,10 +465,10 @@ class ScheduledForward:
         self._next = [0] * lanes                       # index of each nano-batch's next node
         self._waiting: list[asyncio.Event] = []        # of coroutines that wait for an operator
         self.shared_output = engine._shared_output_for(split_config, self.device)
-        # Inputs of every nano-batch are bound up front, on the caller's stream.
+        # Inputs of every nano-batch are bound up front, on the caller's stream; all start behind that.
         for b in range(lanes):
             self._run_inline(b)
-            self.tail_events[b].record()
+        self.tail_events = self.device.starts(lanes)
         for b in range(lanes):
             self._advance(b)
 
@@ -508,8 +523,61 @@ class ScheduledForward:
 
     def launch(self, operators: "OperatorHandle | tuple[OperatorHandle, ...]", func: Callable | None = None) -> None:
         """Enqueue operators on the current stream, behind the previous work of their nano-batches."""
+        if not isinstance(operators, OperatorHandle) and len(operators) == 1:
+            operators = operators[0]
         if isinstance(operators, OperatorHandle):
-            operators = (operators,)
+            self._launch_one(operators, func)
+        else:
+            self._launch_several(operators, func)
+        for b in range(len(self.finished)):
+            if not self.finished[b]:
+                self._advance(b)
+        waiting, self._waiting = self._waiting, []
+        for moved in waiting:
+            moved.set()
+
+    def _launch_one(self, op: OperatorHandle, func: Callable | None) -> None:
+        engine, device, env, b = self.engine, self.device, self.env, op.batch_idx
+        node = engine.module_name_to_node[op.module_name]
+        current = device.current_stream()
+        # chain: this launch starts after the nano-batch's previous work
+        self.tail_events[b].wait(current)
+        self.tail_events[b] = tail = device.new_event()
+        pos = [env.get(b, a) for a in engine._node_inputs[node]]
+        kw = {k: engine._load(env, b, v) for k, v in node.kwargs.items()}
+        if device.is_gpu:
+            for value in pos:
+                _record_use(value, current)
+        if func is not None:
+            with set_op_handle(op):
+                value = func(*pos, **kw)
+        else:
+            with device.range(f"op_{op.module_name}_{b}"):
+                shared = self.shared_output
+                before = swap_op_handle(op)
+                offered = False
+                try:
+                    module = getattr(engine.graph_module, op.module_name)
+                    offered = shared is not None and shared.offer(op)
+                    value = module(*pos, **kw)
+                finally:
+                    if offered:
+                        shared.withdraw()
+                    swap_op_handle(before)
+        tail.record()                    # (on the stream that is current now: a sub-graph may leave another one)
+        self._launched(op, node, value)
+
+    def _launched(self, op: OperatorHandle, node: torch.fx.Node, value: Any) -> None:
+        b = op.batch_idx
+        self.env.put(b, node, value)
+        # per-nano-batch FIFO: the executed handle is the oldest published one
+        assert self._outstanding[b] and op is self._outstanding[b][0], (
+            f"{op.module_name} of nano-batch {b} executed out of order"
+        )
+        self._outstanding[b].popleft()
+        self.engine.issue_trace.append((op.module_name, b))
+
+    def _launch_several(self, operators: tuple[OperatorHandle, ...], func: Callable | None) -> None:
         engine, device, env = self.engine, self.device, self.env
         call_pos: list[list[Any]] = []
         call_kw: list[dict[str, Any]] = []
@@ -519,8 +587,7 @@ class ScheduledForward:
             # chain: this launch starts after the nano-batch's previous work
             self.tail_events[b].wait()
             self.tail_events[b] = device.new_event()
-            # only node-valued positional inputs are forwarded (engine.py:304-310)
-            pos = [env.get(b, a) for a in node.args if isinstance(a, torch.fx.Node)]
+            pos = [env.get(b, a) for a in engine._node_inputs[node]]
             kw = {k: engine._load(env, b, v) for k, v in node.kwargs.items()}
             if device.is_gpu:
                 current = device.current_stream()
@@ -530,41 +597,21 @@ class ScheduledForward:
             call_kw.append(kw)
 
         outputs: list[Any] = []
-        if func is not None:
-            if len(operators) != 1:
-                raise NotImplementedError("Operator batching is not implemented")
-            with set_op_handle(operators[0]):
-                outputs.append(func(*call_pos[0], **call_kw[0]))
-        elif len(operators) != 1 and all(op.module_name == operators[0].module_name for op in operators):
+        if func is not None or all(op.module_name == operators[0].module_name for op in operators):
             raise NotImplementedError("Operator batching is not implemented")
-        else:
-            for i, op in enumerate(operators):
-                with device.range(f"op_{op.module_name}_{op.batch_idx}"), set_op_handle(op):
-                    module = getattr(engine.graph_module, op.module_name)
-                    offered = self.shared_output.offer(op) if self.shared_output is not None else False
-                    try:
-                        outputs.append(module(*call_pos[i], **call_kw[i]))
-                    finally:
-                        if offered:
-                            self.shared_output.withdraw()
+        for i, op in enumerate(operators):
+            with device.range(f"op_{op.module_name}_{op.batch_idx}"), set_op_handle(op):
+                module = getattr(engine.graph_module, op.module_name)
+                offered = self.shared_output.offer(op) if self.shared_output is not None else False
+                try:
+                    outputs.append(module(*call_pos[i], **call_kw[i]))
+                finally:
+                    if offered:
+                        self.shared_output.withdraw()
 
         for op, value in zip(operators, outputs):
-            b = op.batch_idx
-            self.tail_events[b].record()
-            env.put(b, engine.module_name_to_node[op.module_name], value)
-            # per-nano-batch FIFO: the executed handle is the oldest published one
-            assert self._outstanding[b] and op is self._outstanding[b][0], (
-                f"{op.module_name} of nano-batch {b} executed out of order"
-            )
-            self._outstanding[b].popleft()
-            engine.issue_trace.append((op.module_name, b))
-
-        for b in range(len(self.finished)):
-            if not self.finished[b]:
-                self._advance(b)
-        waiting, self._waiting = self._waiting, []
-        for moved in waiting:
-            moved.set()
+            self.tail_events[op.batch_idx].record()
+            self._launched(op, engine.module_name_to_node[op.module_name], value)
 
     async def completed(self) -> tuple[dict[int, Any], list[Any]]:
         """The per-nano-batch results and tail events once every nano-batch has produced its output (tasks that the

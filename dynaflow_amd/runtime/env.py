@@ -77,14 +77,21 @@ def peek_op_handle() -> OperatorHandle | tuple[OperatorHandle, ...] | None:
     return _current_op_handle
 
 
+def swap_op_handle(
+    handle: OperatorHandle | tuple[OperatorHandle, ...] | None,
+) -> OperatorHandle | tuple[OperatorHandle, ...] | None:
+    """Make ``handle`` the current one; returns the one before."""
+    global _current_op_handle
+    saved, _current_op_handle = _current_op_handle, handle
+    return saved
+
+
 @contextmanager
 def set_op_handle(
     handle: OperatorHandle | tuple[OperatorHandle, ...],
 ) -> Generator[None, None, None]:
-    global _current_op_handle
-    saved = _current_op_handle
-    _current_op_handle = handle
+    saved = swap_op_handle(handle)
     try:
         yield
     finally:
-        _current_op_handle = saved
+        swap_op_handle(saved)

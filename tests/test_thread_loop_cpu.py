@@ -12,7 +12,7 @@ import warnings
 
 import pytest
 
-from dynaflow_amd.runtime.loop import run_coroutine
+from dynaflow_amd.runtime.loop import run_coroutine, run_without_loop
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -121,3 +121,35 @@ def test_a_left_over_task_that_fails_while_it_is_cancelled_is_reported(caplog):
     with caplog.at_level(logging.ERROR, "asyncio"):
         run_coroutine(leaves_it())
     assert any(r.exc_info and "lost work" in str(r.exc_info[1]) for r in caplog.records)
+
+
+def test_a_forward_that_waits_for_nothing_needs_no_loop(monkeypatch):
+    made = []
+    monkeypatch.setattr(asyncio, "new_event_loop", lambda: made.append(1))
+    assert run_without_loop(nothing()) == 7 and not made
+
+    async def fails():
+        raise KeyError("its own")
+
+    with pytest.raises(KeyError, match="its own"):
+        run_without_loop(fails())
+    closed = []
+
+    async def waits():
+        try:
+            await asyncio.sleep(0)
+        finally:
+            closed.append(1)
+
+    with pytest.raises(RuntimeError, match="waits"):
+        run_without_loop(waits())
+    assert closed == [1]
+
+
+def test_a_forward_without_a_loop_is_refused_inside_one():
+    async def inside():
+        with pytest.raises(RuntimeError, match="running event loop"):
+            run_without_loop(nothing())
+        return 3
+
+    assert run_coroutine(inside()) == 3
