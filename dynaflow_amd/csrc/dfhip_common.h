@@ -98,6 +98,30 @@ DFHIP_DEVICE float wave_max(float v) {
   return v;
 }
 
+// Two loads of 16 rows of 128 bytes, in which neighbouring lanes share 32 bytes of a row (load h, lane: row 2 (lane / 2 % 8) + h, chunk
+// 2 (lane / 16) + lane % 2 of 16 bytes) -> two MFMA fragments (lane: row lane % 16, chunks 2 (lane / 16) and + 1): neighbours
+// exchange one of their two pieces.
+// Written out: a selection whose one operand comes from the neighbour is one instruction, of which the compiler makes two.  The wait
+// states are those between a write of a register and its read by another lane.
+DFHIP_DEVICE void deal_neighbours(u32x4& first, u32x4& second) {
+  uint32_t a0, a1, a2, a3, b0, b1, b2, b3;
+  asm("s_mov_b32 vcc_lo, 0x55555555\n\ts_mov_b32 vcc_hi, 0x55555555\n\ts_nop 1\n\t"       // even lanes keep their own
+      "v_cndmask_b32_dpp %0, %12, %8, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %1, %13, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %2, %14, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %15, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"                                                            // odd ones
+      "v_cndmask_b32_dpp %4, %8, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %5, %9, %13, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %6, %10, %14, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %7, %11, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3), "=&v"(b0), "=&v"(b1), "=&v"(b2), "=&v"(b3)
+      : "v"(first[0]), "v"(first[1]), "v"(first[2]), "v"(first[3]), "v"(second[0]), "v"(second[1]), "v"(second[2]), "v"(second[3])
+      : "vcc", "scc");
+  first = u32x4{a0, a1, a2, a3};
+  second = u32x4{b0, b1, b2, b3};
+}
+
 // The 8 XCDs of the chip take workgroups round-robin (workgroup i runs on XCD
 // i % 8) and each XCD has a private L2.  remap_xcd turns the launch index into
 // a tile index such that every XCD walks one contiguous range of tiles, so the

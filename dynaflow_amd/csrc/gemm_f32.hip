@@ -86,31 +86,41 @@ gemm_f32_nt_kernel(const float* __restrict__ A, const float* __restrict__ W, flo
   }
 }
 
-// A tile of MB x NB blocks of 16 x 16.  A lane loads 16 bytes of a row, k = 4 (lane / 16) + e of the 16 floats of half a
-// slab; the e-th MFMA takes element e of both operands, so four MFMAs cover the 16 floats (each sums its own quarter of
-// them: the same order of k for both operands is all that matters).
+// A tile of MB x NB blocks of 16 x 16.  A lane multiplies eight floats of a row's slab of 32, four of each load; an MFMA takes element e
+// of load h of both operands, so eight MFMAs cover the slab (each sums its own four of the floats: the same order of k for both
+// operands is all that matters).
+// PAIRS: neighbouring lanes load 32 bytes of a row and exchange pieces (deal_neighbours: floats 8 (lane / 16) + 4 h + e).  With a row per lane
+// (floats 16 h + 4 (lane / 16) + e) a compute unit takes in 34 GB/s, which was the time of most launches; with pairs of lanes 66.  The
+// exchange costs as much as a tenth of the products of 4 x 4 blocks, and registers: several workgroups on a compute unit hide the
+// loads anyway.  [us, a row per lane -> pairs, alone / in pairs: 128 x 1024 x 2816 17.3 / 30.2 -> 13.7 / 20.1, 128 x 2816 x 1024 12.6 / 20.0 -> 12.1
+// / 17.9, 64 x 2048 x 5632 31.7 / 59.0 -> 24.2 / 37.6, 256 x 2816 x 1024 18.1 / 37.9 -> 18.1 / 29.9; one round of 4 x 4 and 4 x 3 blocks, not taken alone: 512 x 2048
+// x 5632 87 / 274 -> 98 / 196, 128 x 5632 x 2048 30.5 / 69.5 -> 31.6 / 57.0; four slabs in flight, not taken: 1000 x 2048 x 5632 178 / 353 -> 202 / 400, 256 x 5632 x 2048 62 / 116 -> 64 / 117]
 constexpr int SWAVES = 4;
 
-template <int MB, int NB, int SDEPTH>
+template <int MB, int NB, int SDEPTH, bool PAIRS>
 __global__ void __launch_bounds__(SWAVES * 64)
 gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C, int M, int N,
                       int slabs, int64_t lda, int64_t ldw, int64_t ldc, int tiles_m) {
   __shared__ f32x4 sums[SWAVES * MB * NB * 64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int row = lane & 15, quad = lane >> 4;
+  const int row = lane & (PAIRS ? 14 : 15), chunk = PAIRS ? 2 * (lane >> 4) + (lane & 1) : lane >> 4;
+  constexpr int ROW_H = PAIRS ? 1 : 0, CHUNK_H = PAIRS ? 0 : 4;  // of load 1 behind load 0
   const int m0 = (int)(blockIdx.x % tiles_m) * (16 * MB), n0 = (int)(blockIdx.x / tiles_m) * (16 * NB);
-  const float* a_ptr[MB];
-  const float* w_ptr[NB];
+  const float* a_ptr[MB][2];
+  const float* w_ptr[NB][2];
 #pragma unroll
-  for (int i = 0; i < MB; ++i) {
-    int m = m0 + 16 * i + row; m = m < M ? m : M - 1;        // rows past the edge re-read the last one; never stored
-    a_ptr[i] = A + (int64_t)m * lda + wave * 32 + quad * 4;
-  }
+  for (int h = 0; h < 2; ++h) {
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    int n = n0 + 16 * j + row; n = n < N ? n : N - 1;
-    w_ptr[j] = W + (int64_t)n * ldw + wave * 32 + quad * 4;
+    for (int i = 0; i < MB; ++i) {
+      int m = m0 + 16 * i + row + ROW_H * h; m = m < M ? m : M - 1;  // rows past the edge re-read the last one; never stored
+      a_ptr[i][h] = A + (int64_t)m * lda + wave * 32 + (chunk + CHUNK_H * h) * 4;
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      int n = n0 + 16 * j + row + ROW_H * h; n = n < N ? n : N - 1;
+      w_ptr[j][h] = W + (int64_t)n * ldw + wave * 32 + (chunk + CHUNK_H * h) * 4;
+    }
   }
   const int n_slabs = (slabs - wave + SWAVES - 1) / SWAVES;   // >= SDEPTH (checked by the launch)
 
@@ -119,18 +129,24 @@ gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, 
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  f32x4 af[SDEPTH][MB][2], wf[SDEPTH][NB][2];
+  u32x4 af[SDEPTH][MB][2], wf[SDEPTH][NB][2];
   auto load = [&](int d, int s) {
     const int off = s * (SWAVES * 32);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
-      for (int i = 0; i < MB; ++i) af[d][i][h] = *reinterpret_cast<const f32x4*>(a_ptr[i] + off + h * 16);
+      for (int i = 0; i < MB; ++i) af[d][i][h] = *reinterpret_cast<const u32x4*>(a_ptr[i][h] + off);
 #pragma unroll
-      for (int j = 0; j < NB; ++j) wf[d][j][h] = *reinterpret_cast<const f32x4*>(w_ptr[j] + off + h * 16);
+      for (int j = 0; j < NB; ++j) wf[d][j][h] = *reinterpret_cast<const u32x4*>(w_ptr[j][h] + off);
     }
   };
   auto multiply = [&](int d) {
+    if constexpr (PAIRS) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) deal_neighbours(af[d][i][0], af[d][i][1]);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) deal_neighbours(wf[d][j][0], wf[d][j][1]);
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -139,7 +155,8 @@ gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, 
         for (int i = 0; i < MB; ++i)
 #pragma unroll
           for (int j = 0; j < NB; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[d][j][h][e], af[d][i][h][e], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wf[d][j][h][e]), __uint_as_float(af[d][i][h][e]),
+                                                             acc[i][j], 0, 0, 0);
   };
 #pragma unroll
   for (int d = 0; d < SDEPTH; ++d) load(d, d);
@@ -198,9 +215,9 @@ int64_t split_tiles(const F32Args& p, int mb, int nb) {
   return (int64_t)((p.M + 16 * mb - 1) / (16 * mb)) * ((p.N + 16 * nb - 1) / (16 * nb));
 }
 
-template <int MB, int NB, int DEPTH>
+template <int MB, int NB, int DEPTH, bool PAIRS>
 int launch_split(const F32Args& p, hipStream_t stream) {
-  const auto kernel = gemm_f32_split_kernel<MB, NB, DEPTH>;
+  const auto kernel = gemm_f32_split_kernel<MB, NB, DEPTH, PAIRS>;
   DFHIP_NOT_IN_LINE(kernel);
   hipLaunchKernelGGL(kernel, dim3((unsigned)split_tiles(p, MB, NB)), dim3(SWAVES * 64), 0,
                      stream, p.A, p.W, p.C, p.M, p.N, p.K / 32, p.lda, p.ldw, p.ldc, (p.M + 16 * MB - 1) / (16 * MB));
@@ -210,9 +227,10 @@ int launch_split(const F32Args& p, hipStream_t stream) {
 // each other on a compute unit and their loads cost more than their registers: 256 x 5632 x 2048 77 -> 62 us, 1024 x 2048
 // x 5632 264 -> 178, but 256 x 2816 x 1024, one round, 18 -> 20).
 template <int MB, int NB>
-int launch_deep(const F32Args& p, hipStream_t stream) {
-  if (p.K >= 512 && split_tiles(p, MB, NB) > 256) return launch_split<MB, NB, 4>(p, stream);
-  return launch_split<MB, NB, 2>(p, stream);
+int launch_deep(const F32Args& p, int share, hipStream_t stream) {
+  if (p.K >= 512 && split_tiles(p, MB, NB) > 256) return launch_split<MB, NB, 4, false>(p, stream);
+  if (MB * NB >= 12 && share == 1) return launch_split<MB, NB, 2, false>(p, stream);
+  return launch_split<MB, NB, 2, true>(p, stream);
 }
 
 // Smallest tile for which a wave's share of K has two slabs in flight.
@@ -227,7 +245,7 @@ int launch_tile128(const F32Args& p, hipStream_t stream) {
 
 // The split tile that takes the least: one round of 256 workgroups costs its blocks and about 1.5 blocks' worth of start,
 // loads and meeting; of several rounds, whose workgroups overlap, each costs 0.6 of its blocks and of seven more for the
-// operands (per round at K = 2048: 4 x 4 blocks 37 us, 4 x 3 31, 4 x 2 25).  [us at [128 x 1024] x [2816 x 1024]^T / [128 x
+// operands (per round at K = 2048: 4 x 4 blocks 37 us, 4 x 3 31, 4 x 2 25).  [us with a row per lane, at [128 x 1024] x [2816 x 1024]^T / [128 x
 // 2816] x [1024 x 2816]^T, with the workgroups in parentheses: 2 x 3 blocks 12.4 (236) / 27.5 (88), 4 x 2 14.9 (176) /
 // 32.7 (64), 2 x 2 17.2 (352) / 22.2 (128), 2 x 1 18.4 (704) / 16.9 (256); the 128 x 128 tiles 105 (22) / 274 (8).  Floor at
 // the fp32 rate: 4.9.]
@@ -253,14 +271,14 @@ int launch_f32(const F32Args& p, int share, hipStream_t stream) {
   if (fits && k * (45.0 + 58.0 * rounds128) + 8.0 * rounds128 < 1.06 * share * least * (0.52 + 1.06 * k))
     return launch_tile128(p, stream);
   switch (best) {
-    case 0: return launch_deep<4, 4>(p, stream);
-    case 1: return launch_deep<4, 3>(p, stream);
-    case 2: return launch_deep<4, 2>(p, stream);
-    case 3: return launch_split<2, 3, 2>(p, stream);
-    case 4: return launch_split<2, 2, 2>(p, stream);
-    case 5: return launch_split<2, 1, 2>(p, stream);
-    case 6: return launch_split<1, 2, 2>(p, stream);
-    default: return launch_split<1, 1, 2>(p, stream);
+    case 0: return launch_deep<4, 4>(p, share, stream);
+    case 1: return launch_deep<4, 3>(p, share, stream);
+    case 2: return launch_deep<4, 2>(p, share, stream);
+    case 3: return launch_split<2, 3, 2, true>(p, stream);
+    case 4: return launch_split<2, 2, 2, true>(p, stream);
+    case 5: return launch_split<2, 1, 2, true>(p, stream);
+    case 6: return launch_split<1, 2, 2, true>(p, stream);
+    default: return launch_split<1, 1, 2, true>(p, stream);
   }
 }
 

@@ -84,7 +84,6 @@ gemm_stream_kernel(const StreamArgs p) {
   // lanes to a line 114, but then the exchange has three stages).  [us: decode step of 40 x 4096 positions, 4 layers
   // 819 -> 771, fp8 layer 8192 x 28672 of 2 x 12 tokens 174 -> 166]
   const int lrow = lane & 14, lchunk = 2 * (lane >> 4) + (lane & 1);
-  const bool odd = lane & 1;
   const uint8_t* w_ptr[NB][2];
   const uint8_t* a_ptr[MB][2];
 #pragma unroll
@@ -133,24 +132,11 @@ gemm_stream_kernel(const StreamArgs p) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) af[d][i][h] = *reinterpret_cast<const u32x4*>(a_ptr[i][h] + off);
   };
-  // the two loads of a block -> its two MFMA fragments (lane: row lane % 16, chunks 2 (lane / 16) and + 1):
-  // neighbouring lanes exchange one of their two pieces
-  auto deal = [&](u32x4 (&v)[2]) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int x = (int)v[0][e], y = (int)v[1][e];
-      constexpr int SWAP = 0xB1;                 // quad_perm [1, 0, 3, 2]
-      const int from_x = __builtin_amdgcn_update_dpp(x, x, SWAP, 0xF, 0xF, true);
-      const int from_y = __builtin_amdgcn_update_dpp(y, y, SWAP, 0xF, 0xF, true);
-      v[0][e] = (uint32_t)(odd ? from_y : x);
-      v[1][e] = (uint32_t)(odd ? y : from_x);
-    }
-  };
   auto multiply = [&](int d) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) deal(wf[d][j]);
+    for (int j = 0; j < NB; ++j) deal_neighbours(wf[d][j][0], wf[d][j][1]);
 #pragma unroll
-    for (int i = 0; i < MB; ++i) deal(af[d][i]);
+    for (int i = 0; i < MB; ++i) deal_neighbours(af[d][i][0], af[d][i][1]);
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll

@@ -44,3 +44,21 @@ def test_gemm_f32_of_many_rows(M, N, K, share, tile128):
     assert bool(((got[::97].double() - a[::97].double() @ w.double().t()).abs() <= bound).all())
     padded = ops.linear(*(torch.nn.functional.pad(t, (0, 4)) for t in (a, w)))
     assert torch.equal(got, padded) == tile128
+
+
+# one round of each tile, ragged in both directions, with the shortest K, an uneven share of the waves, and rows that are not contiguous
+@pytest.mark.parametrize("share", [1, 2, 16])
+@pytest.mark.parametrize("M,N,K", [(1, 9, 256), (17, 1409, 512), (33, 2817, 1056), (100, 1030, 2816), (130, 520, 288), (200, 2810, 1024),
+                                   (250, 4090, 800), (515, 2040, 544)])
+def test_gemm_f32_lanes_in_pairs(M, N, K, share):
+    """Against the product in float64: a wave sums K / 4 products (and up to a slab more than the others) and the four sums meet, each
+    rounding off by no more than 2^-24 of a partial sum of the magnitudes."""
+    from dynaflow_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, K + 4), generator=g, device="cuda")[:, :K]
+    w = torch.randn((N, K + 8), generator=g, device="cuda")[:, :K]
+    with ops.launch_options(share):
+        got = ops.linear(x, w)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert ((got.double() - want).abs() <= (K // 4 + 36) * 2.0 ** -24 * size).all()
