@@ -21,11 +21,18 @@ from typing import Any
 
 import torch
 import torch.fx as fx
+from torch.nn.modules.module import _has_any_global_hook as has_any_global_hook
 
 from dynaflow_amd.config import CUDAGraphConfig, DynaFlowConfig, InductorConfig
 from dynaflow_amd.executor.hipgraph import CUDAGraphWrapper
 from dynaflow_amd.interface import OperatorHandle
 from dynaflow_amd.runtime.env import get_op_handle
+
+
+def _is_hooked(module: torch.nn.Module) -> bool:
+    """Whether ``Module.__call__`` does more than call ``forward``: hooks of this module or of all modules, or tracing."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or has_any_global_hook() or torch._C._get_tracing_state())
 
 
 class SubgraphBackend:
@@ -86,7 +93,7 @@ class SubgraphBackend:
             return fn(*args, **kwargs)
         fn = self.callable_dynamic
         assert fn is not None
-        if isinstance(fn, fx.GraphModule) and not (fn._forward_hooks or fn._forward_pre_hooks):
+        if isinstance(fn, fx.GraphModule) and not _is_hooked(fn):
             return fn.forward(*args, **kwargs)           # (3 us less than through Module.__call__)
         return fn(*args, **kwargs)
 

@@ -8,6 +8,7 @@ import torch
 
 from dynaflow_amd.backend import make_backend
 from dynaflow_amd.config import CUDAGraphConfig, DynaFlowConfig, InductorConfig
+from dynaflow_amd.executor.compiler import SubgraphBackend
 from dynaflow_amd.interface import ExecutionContext, OpSchedulerBase, SplitConfig
 from dynaflow_amd.manager import DynaFlowManager
 from dynaflow_amd.mlp import SwiGLUMLP
@@ -562,3 +563,28 @@ def test_a_coroutine_per_nano_batch_is_launched_in_turn(host_device, lanes):
     assert manager.engine.issue_trace == [(name, b) for _, name in subgraphs for b in range(lanes)]
     assert [e[2] for e in host_device.log if e[0] == "range"] == [f"lane{b}" for _ in subgraphs for b in range(lanes)]
     assert host_device.current_stream().name == "default"
+
+
+@pytest.mark.parametrize("register", [
+    lambda module, hook: module.register_forward_hook(hook),
+    lambda module, hook: module.register_forward_pre_hook(hook),
+    lambda module, hook: torch.nn.modules.module.register_module_forward_hook(hook),
+    lambda module, hook: torch.nn.modules.module.register_module_forward_pre_hook(hook),
+], ids=["forward", "forward_pre", "all_modules_forward", "all_modules_forward_pre"])
+def test_hooks_see_a_subgraph_that_is_called_past_module_call(register):
+    class Twice(torch.nn.Module):
+        def forward(self, tokens, x):
+            return x * 2
+
+    gm = torch.fx.symbolic_trace(Twice())
+    backend = SubgraphBackend(gm, 0, InductorConfig(enabled=False), CUDAGraphConfig(enabled=False, capture_sizes=[]),
+                              use_inductor=False, use_cudagraph=False)
+    backend.callable_dynamic = gm
+    seen = []
+    handle = register(gm, lambda module, *rest: seen.append(module))
+    try:
+        backend(3, torch.ones(3))
+    finally:
+        handle.remove()
+    assert any(module is gm for module in seen)
+    assert torch.equal(backend(3, torch.ones(3)), torch.full((3,), 2.0)) and len(seen) == 1
