@@ -994,11 +994,11 @@ DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share,
 // up to 16, which a tile shares: there the 128 x 128 tiles take over, unless the launch is alone and its weights few.  [us at 33 / 64
 // rows, streamed or on 128-row tiles against 128 x 128: alone 28672 x 8192 53 / 63 against 55 / 56, with gate + up + SiLU*mul 103 /
 // 110 against 91 / 94, 14336 x 4096 17 / 19 against 23 / 22, with gate + up 35 / 37 against 33 / 33; in pairs 28672 x 8192 81 / 84
-// against 76 / 78, 14336 x 4096 30 / 35 against 25 / 26.]  A product that may be cut along K goes there alone from 33 rows on, in
-// pairs from 17, or 9 where its weights are many.  [8192 x 28672 at 17 / 24 / 33 / 64 rows: in pairs 91 / 97 / 92 / 92 against 77 / 78 /
-// 79 / 82, alone 44 / 48 / 59 / 79 against 50 / 49 / 50 / 52; 4096 x 14336 in pairs 34 / 38 / 45 / 45 against 31 / 32 / 31 / 32, alone
-// 19 / 21 / 25 / 34 against 24; at 12 rows in pairs 8192 x 28672 82 against 79, 4096 x 14336 30 against 32.  Fewer than 2^25 weights
-// stay: 1536 x 7168 alone at 40 rows 15 against 18, in pairs at 12 rows 17 against 23.]
+// against 76 / 78, 14336 x 4096 30 / 35 against 25 / 26.]  A product that may be cut along K goes there alone from 33 rows on;
+// in pairs it is streamed in parts of K from 9 to 32 rows (few_rows_parts) and goes there above.  [8192 x 28672 alone at 17 / 24 / 33 /
+// 64 rows: 44 / 48 / 59 / 79 against 50 / 49 / 50 / 52, in pairs at 33 / 64 92 / 92 against 79 / 82; 4096 x 14336 alone 19 / 21 / 25 / 34
+// against 24, in pairs at 33 / 64 45 / 45 against 31 / 32.  Fewer than 2^25 weights stay: 1536 x 7168 alone at 40 rows 15 against 18,
+// in pairs at 12 rows 17 against 23.]
 bool few_rows_streamed(int M, int N, int K, int share, bool may_split) {
   if (!dfhip_stream_fits(M, N, K, 1) || (M >= 16 && K < 4096)) return false;
   const int64_t weights = (int64_t)N * K;

@@ -1,6 +1,6 @@
 // Weight-streaming GEMMs for a handful of activation rows (M <= 64), bf16 and fp8 e4m3:
 //   C[M,N] = A[M,K] W[N,K]^T          bf16: optional residual [M,N] added in the epilogue
-//   C[M,N] = silu(A W^T) * (A W2^T)   gate and up projection in one launch (fp8: with max |C| folded into a cell)
+//   C[M,N] = silu(A W^T) * (A W2^T)   gate and up projection in one launch (fp8: max |C| beside it, a float a tile or one cell)
 //
 // Bound: HBM.  Every weight is read once and used for at most 64 rows, so the kernel is a load loop with a few
 // MFMAs in it.  What it is built for is many loads in flight and nothing that makes them wait for each other:
@@ -20,8 +20,8 @@
 // Measured (weights from HBM, us; M = 2 / 16 / 32 rows, against the 128-row tiles used before): gate + up + SiLU*mul
 // 2 x 14336 x 4096 (235 MB) 39 / 39 / 43, before 51; down 4096 x 14336 23 / 24 / 27, before 207 / 36 / 36; q/k/v
 // 6144 x 4096 12 / 15 / 18, before 62 / 22 / 22; o 4096 x 4096 8 / 10 / 13, before 61 / 21 / 21.  At 8 / 16 / 32 / 64
-// rows fp8 down 8192 x 28672 (235 MB) 37 / 42 / 54 / 79, before 240; fp8 gate + up 2 x 28672 x 8192 (470 MB)
-// 80 / 82 / 92 / 112, before 113 - 117.
+// rows fp8 down 8192 x 28672 (235 MB) 37 / 42 / 54 / 79, before 240 (two of 12 / 32 rows in one launch, K in parts: 40 / 49);
+// fp8 gate + up 2 x 28672 x 8192 (470 MB) 80 / 82 / 92 / 112, before 113 - 117.
 #include "dfhip_pairs.h"
 #include "dfhip_stream.h"
 
