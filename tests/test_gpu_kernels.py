@@ -156,7 +156,7 @@ def test_silu_mul_f32(ops):
     assert rel_err(got, want) < TOL["fp32"]
 
 
-@pytest.mark.parametrize("M,H", [(1, 8), (5, 512), (64, 4096), (3, 16384)])
+@pytest.mark.parametrize("M,H", [(1, 8), (5, 512), (64, 4096), (3, 16384), (2, 2056), (3, 4104), (2, 8192), (3, 8200)])
 def test_rms_norm(ops, M, H):
     x = randn((M, H), 13).bfloat16()
     w = (1 + 0.1 * randn((H,), 14)).bfloat16()
