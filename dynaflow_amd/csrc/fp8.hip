@@ -186,7 +186,8 @@ __global__ void __launch_bounds__(QT) absmax_parts_kernel(const AbsmaxParts<FLAT
 
 // q = e4m3fn(x / scale), scale = max(amax, 1e-12) / 448.  PARTS: amax is the maximum of n_parts values; else `amax` is one
 // value, and with `readers` the last block to have read it clears it and the count of those that have: the cells are zero
-// again for the launch that folds the next maximum into them.
+// again for the launch that folds the next maximum into them.  The parts of a turn are asked for together.  [us, both launches, one load
+// of a part after the other / together: 12 x 8192 5.7 / 5.6, 350 x 8192 7.7 / 7.3, 700 x 8192 9.5 / 8.9]
 template <bool FLAT, bool PARTS>
 DFHIP_DEVICE void quant_after(unsigned block, unsigned blocks, const uint16_t* __restrict__ x, int64_t ld,
                               uint8_t* __restrict__ q, int64_t ld_q, uint32_t groups, uint32_t per_row,
@@ -206,10 +207,14 @@ DFHIP_DEVICE void quant_after(unsigned block, unsigned blocks, const uint16_t* _
   load();
   float m = 0.0f;
   if (PARTS) {
-    for (int p0 = threadIdx.x; p0 < n_parts; p0 += QPARTS)
+    for (int p0 = threadIdx.x; p0 < n_parts; p0 += QPARTS) {
+      float part[QPARTS / QT];
 #pragma unroll
-      for (int p = 0; p < QPARTS / QT; ++p)
-        if (p0 + p * QT < n_parts) m = fmaxf(m, amax[p0 + p * QT]);
+      for (int p = 0; p < QPARTS / QT; ++p) part[p] = amax[p0 + p * QT < n_parts ? p0 + p * QT : p0];
+      DFHIP_PIN;
+#pragma unroll
+      for (int p = 0; p < QPARTS / QT; ++p) m = fmaxf(m, part[p]);
+    }
     m = block_max<QT>(m);
   } else {
     __shared__ float cell;
