@@ -631,16 +631,15 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
   return launch_attention<false, false>(args, combine_bytes, static_cast<hipStream_t>(stream));
 }
 
-// Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), one up to 32 pairs of 16384 positions,
-// where a share is short and the last part's reading of the others' sums counts, with at least 256 positions of a full cache each
-// (two chunks per wave).  The lengths are on the device: the launch is sized for full caches and each sequence takes its share of
-// it (sequence_parts).  A launch with fewer than MIN_PARTS of them, from 171 pairs on but for those below, cuts nothing.  [us, two
-// to a unit / one, full caches then 1/4 .. 1 of them, 8 kv heads: 2 sequences of 8192 positions 21.5 / 18.8 (uncut 111; their bytes
-// at 6.7 TB/s: 10), 18.6 / 16.8, 3 of 8192 24.7 / 23.7, 21.8 / 21.5, 4 of 8192 28.5 / 27.2, 23.5 / 23.5, 4 of 4096 18.2 / 17.1,
-// 16.7 / 15.7, 4 of 16384 47.7 / 46.6, 39.2 / 39.1; not taken: 4 of 32768 86.9 / 85.8, 68.5 / 71.7, of more pairs 8 of 8192
-// 47.0 / 45.9, 36.4 / 37.7.  At most 16 parts instead of 32, not taken: 1 of 8192 15.2 / 14.4, but 1 of 32768 28.5 / 32.1, with one
-// kv head 20.2 / 29.4.  Uncut / cut: 8 of 2048 33 / 16.8 (10), 20 of 4096 69 / 57 (50); in two parts, not taken: 32 of 512, 2048
-// and 4096 14.6 / 16.5, 42.9 / 46.0, 79 / 84]
+// Workgroups per (token, kv head) pair: two to a compute unit in all (what fits at once), with at least 256 positions of a full
+// cache each (two chunks per wave).  The lengths are on the device: the launch is sized for full caches and each sequence takes
+// its share of it (sequence_parts).  A launch with fewer than MIN_PARTS of them, from 171 pairs on but for those below, cuts
+// nothing.  [us, uncut / cut, 8 kv heads, all full: 2 sequences of 8192 positions 111 / 21.5 (their bytes at 6.7 TB/s: 10), 8 of 2048
+// 33 / 16.8 (10), 20 of 4096 69 / 57 (50); in two parts, not taken: 32 of 512, 2048 and 4096 14.6 / 16.5, 42.9 / 46.0, 79 / 84]
+// One workgroup to a unit up to 32 pairs, not taken: 2 of 8192 21.5 -> 18.8, 3 of 8192 24.7 -> 23.7, 4 of 4096 18.2 -> 17.1, 4 of
+// 16384 47.7 -> 46.6, but further from float64.  A probability is rounded to bf16 relative to its wave's largest, which is exact:
+// half as many waves round more of the large ones.  [distance, 2-norm, mean of 16 draws, 2 of 8192 2.650e-3 -> 2.672e-3, 4 of 8192
+// 2.682e-3 -> 2.713e-3, 4 of 16384 2.706e-3 -> 2.738e-3, each +- 0.15 %]
 // A compute unit takes in no more than 29 GB/s, so a few pairs more than units take twice the time: 257 .. 384 of them are cut
 // in four where the cache has room for 2048 positions, and so are 171 .. 192, which leave a quarter of the units idle, where it
 // has room for 4096.  [us, uncut / four parts, 8 kv heads, all full: 33 sequences of 2048 68 / 53, 48 of 2048 73 / 69, 36 of 4096 133 / 100,
@@ -651,7 +650,7 @@ constexpr int MIN_PARTS = 3;
 static int attention_parts(int T, int kv_heads, int capacity) {
   const int64_t pairs = (int64_t)T * kv_heads;
   if ((pairs > 256 && pairs <= 384 && capacity >= 2048) || (pairs > 170 && pairs <= 192 && capacity >= 4096)) return 4;
-  int64_t parts = (pairs <= 32 && capacity <= 16384 ? 256 : 512) / pairs;
+  int64_t parts = 512 / pairs;
   if (parts > capacity / 256) parts = capacity / 256;
   if (parts > 32) parts = 32;
   return parts < 1 ? 1 : (int)parts;

@@ -171,8 +171,8 @@ def test_one_launch_decode_attention_has_the_bits_of_the_two_launches(heads, kv_
     (32, 8, 2048, [2048 - 31 * i for i in range(32)]),   # two parts again
     (32, 8, 2048, [2048 - 64 * i for i in range(21)]),   # the most pairs that are still cut: three parts each
     (8, 2, 4096, [767, 768, 1023, 1024, 1025, 4096]),    # around the lengths that take one, three and four parts
-    (32, 8, 4096, [4096, 1, 2500, 255]),             # 32 pairs: one workgroup to a compute unit, eight parts each
-    (3, 3, 4096, [4096 - 370 * i for i in range(11)]),   # 33: two, fifteen parts each
+    (32, 8, 4096, [4096, 1, 2500, 255]),             # 16 parts for the longest, nine, and two whole
+    (3, 3, 4096, [4096 - 370 * i for i in range(11)]),   # fifteen parts and fewer
 ])
 def test_decode_attention_cut_over_positions(ops, heads, kv_heads, capacity, lengths):
     """Few (token, kv head) pairs: several workgroups share a token's positions and the last to arrive combines them.
