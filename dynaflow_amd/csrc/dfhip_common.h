@@ -101,8 +101,10 @@ DFHIP_DEVICE float wave_max(float v) {
 // Two loads of 16 rows of 128 bytes, in which neighbouring lanes share 32 bytes of a row (load h, lane: row 2 (lane / 2 % 8) + h, chunk
 // 2 (lane / 16) + lane % 2 of 16 bytes) -> two MFMA fragments (lane: row lane % 16, chunks 2 (lane / 16) and + 1): neighbours
 // exchange one of their two pieces.
-// Written out: a selection whose one operand comes from the neighbour is one instruction, of which the compiler makes two.  The wait
-// states are those between a write of a register and its read by another lane.
+// Written out: a selection whose one operand comes from the neighbour is one instruction, of which the compiler makes two.  It does
+// not see the registers being read and written in here, so the block waits for them itself, two states each: in front between the
+// write of a register and its read by another lane, behind between the last write and an MFMA that reads it (an fp8 one reads all
+// eight registers at once).
 DFHIP_DEVICE void deal_neighbours(u32x4& first, u32x4& second) {
   uint32_t a0, a1, a2, a3, b0, b1, b2, b3;
   asm("s_mov_b32 vcc_lo, 0x55555555\n\ts_mov_b32 vcc_hi, 0x55555555\n\ts_nop 1\n\t"       // even lanes keep their own
@@ -114,7 +116,8 @@ DFHIP_DEVICE void deal_neighbours(u32x4& first, u32x4& second) {
       "v_cndmask_b32_dpp %4, %8, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
       "v_cndmask_b32_dpp %5, %9, %13, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
       "v_cndmask_b32_dpp %6, %10, %14, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-      "v_cndmask_b32_dpp %7, %11, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      "v_cndmask_b32_dpp %7, %11, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1"
       : "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3), "=&v"(b0), "=&v"(b1), "=&v"(b2), "=&v"(b3)
       : "v"(first[0]), "v"(first[1]), "v"(first[2]), "v"(first[3]), "v"(second[0]), "v"(second[1]), "v"(second[2]), "v"(second[3])
       : "vcc", "scc");
