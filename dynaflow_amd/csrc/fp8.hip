@@ -1019,19 +1019,29 @@ bool few_rows_streamed(int M, int N, int K, int share, bool may_split) {
 // 8) rows or 128 x 128 tiles -> in parts, at 12 / 17 / 24 / 32 rows: 8192 x 28672 60 / 62 / 64 / 64 -> 40 / 42 / 45 / 49, 4096 x 14336
 // 15.4 / 21.4 / 21.5 / 21.9 -> 14.3 / 16.3 / 17.6 / 19.8, 2048 x 16384 14.4 / 17.0 / 17.3 / 17.4 -> 10.0 / 11.3 / 12.1 / 13.5, 8192 x 16384 39
 // / 41 / 39 / 40 -> 31 / 33 / 33 / 35; at 2 rows 4096 x 14336 11.9 -> 13.5; layer 8192 x 28672 of 2 x 12 tokens 163 -> 142.
-// A pair that stays two launches on two streams: 73 / 72 / 76 / 76 -> 72 / 76 / 78 / 81, 22 / 25 / 26 / 26 -> 23 / 23 / 25 / 26, 17 / 19 / 19 / 20
-// -> 14 / 15 / 15 / 16, 45 / 46 / 47 / 48 -> 53 / 53 / 54 / 53]
-int few_rows_parts(int M, int N, int K, int share, bool may_split) {
+// Launches that stay two (DFHIP_SPLIT_APART) read their weights twice either way.  They take four parts and more, which fill the chip,
+// and two where whole K would be streamed with fewer than 160 workgroups; two parts of anything wider, or instead of tiles, are
+// slower.  [us a pair on two streams in a graph, without parts -> in parts, at 9 / 12 / 16 / 17 / 24 / 32 rows: taken 1280 x 16384 25.8 / 27.4 / 29.4
+// / 31.3 / 33.9 / 36.9 -> 20.1 / 20.3 / 20.4 / 21.8 / 22.1 / 23.0, 2048 x 16384 27.1 / 27.4 / 29.0 / 26.0 / 26.2 / 26.3 -> 21.9 / 21.9 / 22.0 / 23.1 /
+// 22.9 / 24.2, from 12 rows 3072 x 8192 20.1 / 20.8 / 22.0 / 23.2 / 24.4 / 26.2 -> 20.9 / 20.8 / 21.6 / 22.1 / 23.3 / 23.7, at 12 and 16 4096 x 14336
+// 29.2 / 30.4 / 32.9 / 31.0 / 31.4 / 31.5 -> 29.9 / 30.2 / 30.6 / 31.1 / 32.6 / 33.5, 4608 x 18432 50 / 46 / 49 / 39 / 39 / 40 -> 43 / 44 / 45 / 46 / 48
+// / 50; not taken 5120 x 25600 64 / 64 / 67 / 52 / 52 / 53 -> 64 / 63 / 64 / 65 / 67 / 70, 6144 x 16384 47 / 48 / 48 / 45 / 45 / 46 -> 50 / 50 / 50 / 51 / 51
+// / 52, 8192 x 16384 50 / 51 / 50 / 51 / 52 / 52 -> 59 / 59 / 59 / 60 / 61 / 61, 8192 x 28672 78 / 76 / 76 / 77 / 77 / 78 -> 84 / 82 / 82 / 84 / 85 / 88]
+int few_rows_parts(int M, int N, int K, int share, int may_split, bool streamed) {
   if (!may_split || share < 2 || K <= N || M < 9 || M > 32) return 1;
-  for (int s = 2; s <= 8; s *= 2)
-    if ((int64_t)((N + 31) / 32) * s >= 160) return dfhip_stream_fits(M, N, K, s) ? s : 1;
+  const int64_t tiles = (N + 31) / 32;
+  for (int s = 2; s <= 8; s *= 2) {
+    if (tiles * s < 160) continue;
+    if (may_split == DFHIP_SPLIT_APART && s < 4 && !(streamed && M >= 12 && tiles < 160)) return 1;
+    return dfhip_stream_fits(M, N, K, s) ? s : 1;
+  }
   return 1;
 }
 
 // The plan of a launch: -1 for the streaming kernel (F8_STREAM for counts of rows that have a tile as well), or a tile, and the parts of K.
-TilePlan plan_launch(int M, int N, int K, int share, bool may_split) {
+TilePlan plan_launch(int M, int N, int K, int share, int may_split) {
   const bool streamed = few_rows_streamed(M, N, K, share, may_split);
-  const int parts = few_rows_parts(M, N, K, share, may_split);
+  const int parts = few_rows_parts(M, N, K, share, may_split, streamed);
   if (streamed || parts > 1) return {streamed ? -1 : F8_STREAM, parts, 0.0};
   const TilePlan plan = plan_tile(M, N, K, share, may_split);
   const DfhipRing3Plan tiles = three_slabs_cheaper(false, M, N, K, share, plan.variant, plan.split_k, may_split && K > N);

@@ -146,6 +146,8 @@ class DynaFlowManager:
         self._side_by_side: int | None = None     # instead of launches_side_by_side while a schedule is captured in pairs
         #: per captured schedule: how many pairs of launches against the same weights became one launch
         self.paired_launches: dict[tuple, int] = {}
+        #: splits (their ``split_indices``) whose capture had no pairs although ``launches_join``
+        self._unpaired: set[tuple] = set()
 
     # ------------------------------------------------------------ set-up
     def initialize(
@@ -196,6 +198,7 @@ class DynaFlowManager:
         self.engine = DynaFlowEngine(self.graph_module, config)
         self.scheduler = scheduler
         self._schedule_graphs = {}
+        self._unpaired = set()
 
     # ----------------------------------------------------- split selection
     def prepare(
@@ -252,7 +255,8 @@ class DynaFlowManager:
         assert split is not None
         from dynaflow_amd import ops
 
-        with ops.launch_options(side_by_side=self._side_by_side or self.launches_side_by_side(split)):
+        with ops.launch_options(side_by_side=self._side_by_side or self.launches_side_by_side(split)), \
+                ops.launches_join(self.launches_join(split)):
             if split.is_dryrun:
                 results, events = self.engine.dryrun(args, kwargs, split)
             else:
@@ -298,6 +302,32 @@ class DynaFlowManager:
                 'use streams="by_nano_batch"')
         return asked
 
+    def launches_join(self, split: SplitConfig) -> bool:
+        """Whether two launches side by side, of few rows against the same weights, become one in the graph of this schedule, which
+        some are planned for (``ops.launches_join``).  It says the same for an eager forward of such a manager: that has the bits
+        of the replays."""
+        assert self.config is not None and self.scheduler is not None
+        return (bool(self.config.knob("whole_graph", False)) and not split.is_dryrun
+                and getattr(self.scheduler, "stream_policy", None) == "by_nano_batch"
+                and split.num_nano_batches % 2 == 0 and max(split.num_tokens) <= PAIR_MAX_ROWS
+                and tuple(split.split_indices) not in self._unpaired and self._kept_apart() is None)
+
+    def _kept_apart(self) -> str | None:
+        """Why a captured schedule of this manager keeps every launch as it is, if it does."""
+        assert self.config is not None and self.scheduler is not None
+        if not self.config.knob("pair_launches", True):
+            return "pair_launches is off"
+        if self.config.knob("cu_split", None):
+            return "the streams have compute units of their own"
+        if getattr(self.scheduler, "comp_stream", None) is getattr(self.scheduler, "comm_stream", None):
+            return "one stream"
+        # (a collective looks like a short launch and waits for other ranks: what ran beside it stays beside it)
+        if torch.distributed.is_available() and torch.distributed.is_initialized() and torch.distributed.get_world_size() > 1:
+            return "several ranks"
+        if not self._schedules_plainly():
+            return type(self.scheduler).__name__
+        return capture_plan.needs_its_order(self.graph_module)
+
     # ------------------------------------------------- whole-schedule graphs
     def _logged_pass(self, args: tuple, kwargs: dict, split: SplitConfig) -> list:
         """An eager pass before a capture: lazy one-time set-up (kernel attributes, allocator growth) must not happen
@@ -337,14 +367,7 @@ class DynaFlowManager:
         2 x 50 tokens 363 / 241]"""
         assert self.config is not None and self.scheduler is not None
         policy = getattr(self.scheduler, "stream_policy", None)
-        one_stream = getattr(self.scheduler, "comp_stream", None) is getattr(self.scheduler, "comm_stream", None)
-        kept = None if self._schedules_plainly() else type(self.scheduler).__name__
-        kept = kept or capture_plan.needs_its_order(self.graph_module)
-        # (a collective looks like a short launch and waits for other ranks: what ran beside it stays beside it)
-        several_ranks = torch.distributed.is_available() and torch.distributed.is_initialized() and \
-            torch.distributed.get_world_size() > 1
-        if not self.config.knob("pair_launches", True) or self.config.knob("cu_split", None) or one_stream or several_ranks:
-            return None, None, 0
+        kept = self._kept_apart()
         if kept is not None:
             log.info("launches are not paired: %s", kept)
             return None, None, 0
@@ -366,8 +389,14 @@ class DynaFlowManager:
             pairs = _pair_launches(graph, policy == "by_nano_batch")
         except KernelError as error:     # the graph may be half changed
             log.warning("captured launches were not paired: %s", error)
-            return None, None, 0
-        return (graph, output, pairs) if pairs or policy == "by_nano_batch" else (None, None, 0)
+            graph, pairs = None, 0
+        if not pairs and self.launches_join(split):
+            # planned for launches of two, of which there are none: again as launches that stay apart
+            self._unpaired.add(tuple(split.split_indices))
+            self._logged_pass(args, kwargs, split)
+            torch.cuda.current_stream().synchronize()
+            graph = None
+        return (graph, output, pairs) if graph is not None and (pairs or policy == "by_nano_batch") else (None, None, 0)
 
     def _wants_whole_graph(self, split: SplitConfig) -> bool:
         assert self.config is not None

@@ -131,6 +131,22 @@ def _side_by_side() -> int:
     return getattr(_launch_options, "side_by_side", 1)
 
 
+@contextlib.contextmanager
+def launches_join(join: bool):
+    """``join``: of the launches issued inside the block, two of nano-batches side by side become one (``dfhip_graph_pair_launches``),
+    which a few rows against many weights are planned for (fp8, K in parts).  Outside, and by default, they stay two."""
+    previous = _join()
+    _launch_options.join = bool(join)
+    try:
+        yield
+    finally:
+        _launch_options.join = previous
+
+
+def _join() -> bool:
+    return getattr(_launch_options, "join", False)
+
+
 def _zeroed_workspace(cache: dict, device: torch.device, stream: int, nbytes: int, clear: int = 65536) -> torch.Tensor:
     """A scratch buffer whose first ``clear`` bytes are zero at first use, kept for the life of the process.
 
@@ -175,7 +191,7 @@ _FIRST_TILE_VARIANT = 10
 
 
 @functools.lru_cache(maxsize=4096)
-def _plan_tiles(entry: str, M: int, N: int, K: int, share: int, may_split: bool) -> tuple[int, int]:
+def _plan_tiles(entry: str, M: int, N: int, K: int, share: int, may_split: int) -> tuple[int, int]:
     variant, split_k = ctypes.c_int(0), ctypes.c_int(1)
     _cabi.check(entry, getattr(_cabi.load(), entry)(M, N, K, share, may_split, ctypes.byref(variant), ctypes.byref(split_k)))
     return variant.value, split_k.value
@@ -734,6 +750,8 @@ torch.library.register_fake(
 # --------------------------------------------------------------------- fp8
 #: DFHIP_FP8_PARTS: floats in which the blocks of a quantisation leave their maxima
 _FP8_PARTS = 1024
+#: DFHIP_SPLIT_APART
+_SPLIT_APART = 2
 #: DFHIP_FP8_GEMM_PARTS, and the rows up to which a gate + up launch is short enough for the clearing of a cell to show
 _FP8_GEMM_PARTS, _FP8_ONE_CALL_ROWS = 4096, 128
 
@@ -840,7 +858,8 @@ def _linear_fp8_impl(x_q, w_q, x_scale, w_scale, variant: int = -1, to_output: b
     if M > 0:
         stream, split_k = _stream(), 1
         if cut_k and SPLIT_K_ENABLED:
-            variant, split_k = _plan_tiles("dfhip_gemm_fp8_plan_tiles", M, N, K, _side_by_side(), True)
+            may_split = 1 if _join() else _SPLIT_APART
+            variant, split_k = _plan_tiles("dfhip_gemm_fp8_plan_tiles", M, N, K, _side_by_side(), may_split)
         scale = w_scale.contiguous()
         gemm = (a.data_ptr(), lda, w.data_ptr(), ldw, out.data_ptr(), N, x_scale.data_ptr(), scale.data_ptr(), M, N, K)
         if split_k > 1:

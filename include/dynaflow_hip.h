@@ -259,7 +259,9 @@ int dfhip_gemm_fp8_nt_shared(const void* A, int64_t lda, const void* W, int64_t 
  * split whatever their widths are.
  * dfhip_gemm_fp8_plan_tiles: the same among all tiles, 11, 12 and 15 (those of dfhip_gemm_bf16_nt_variant) included: what
  * dfhip_gemm_fp8_nt_shared launches where may_split is 0.  Both plans leave the same launches of few rows to the
- * streaming kernel (variant < 0); this one cuts K in some of them, and in more launches of up to 32 rows (variant 8). */
+ * streaming kernel (variant < 0); this one cuts K in some of them, and in more launches of up to 32 rows (variant 8), as pays
+ * where dfhip_graph_pair_launches makes one of two launches.  may_split = DFHIP_SPLIT_APART: they stay two, and fewer are cut. */
+#define DFHIP_SPLIT_APART 2
 int dfhip_gemm_fp8_plan_shared(int M, int N, int K, int share, int* variant, int* split_k);
 int dfhip_gemm_fp8_plan_tiles(int M, int N, int K, int share, int may_split, int* variant, int* split_k);
 size_t dfhip_gemm_fp8_splitk_workspace_bytes(int M, int N, int variant, int split_k);

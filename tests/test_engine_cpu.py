@@ -460,6 +460,37 @@ def test_kernel_plans_follow_the_schedule_not_a_promise(host_device, monkeypatch
         assert manager.launches_side_by_side(single) == 1
 
 
+@pytest.mark.parametrize("knobs,splits,ranks,tokens,join", [
+    ({"streams": "by_nano_batch", "whole_graph": True}, 2, 1, 96, True),
+    ({"streams": "by_nano_batch", "whole_graph": True}, 4, 1, 96, True),
+    ({"streams": "by_nano_batch", "whole_graph": True}, 2, 1, 258, False),     # more rows than two launches of one take
+    ({"streams": "by_nano_batch", "whole_graph": True}, 3, 1, 96, False),      # one without a partner
+    ({"streams": "by_nano_batch", "whole_graph": True}, 2, 2, 96, False),
+    ({"streams": "by_nano_batch", "whole_graph": True, "pair_launches": False}, 2, 1, 96, False),
+    ({"streams": "by_nano_batch", "whole_graph": True, "serialize": True}, 2, 1, 96, False),
+    ({"streams": "by_nano_batch"}, 2, 1, 96, False),                           # launched one by one, or a graph a sub-graph
+    ({"streams": "by_kind", "whole_graph": True}, 2, 1, 96, False),            # captured in pairs, but planned as lone launches
+])
+def test_kernel_plans_know_which_launches_become_one(host_device, monkeypatch, knobs, splits, ranks, tokens, join):
+    """A kernel that pays where two launches become one is not planned where they stay two; an eager forward has the plans of
+    the graph of its manager."""
+    from dynaflow_amd import ops
+
+    monkeypatch.setattr(torch.distributed, "is_initialized", lambda: ranks > 1)
+    monkeypatch.setattr(torch.distributed, "get_world_size", lambda: ranks)
+    cfg = make_config(splits, num_nano_batches=splits, **knobs)
+    model, manager, compiled, x = compile_mlp(cfg, tokens=tokens)
+    monkeypatch.setattr("dynaflow_amd.runtime.capture_plan.needs_its_order", lambda graph: None)   # (not lowered here)
+    split, seen = manager.prepare(tokens, [1] * tokens), []
+    assert split.num_nano_batches == splits and manager.launches_join(split) == join
+    manager.engine.graph_module.submod_0.callable_dynamic.register_forward_pre_hook(lambda *_: seen.append(ops._join()))
+    with torch.no_grad():
+        compiled(x)
+    assert seen == [join] * splits and not ops._join()
+    monkeypatch.setattr("dynaflow_amd.runtime.capture_plan.needs_its_order", lambda graph: "something")
+    assert not manager.launches_join(split)
+
+
 @pytest.mark.parametrize("knobs", [{"streams": "by_kind", "side_by_side": 2},
                                    {"streams": "by_nano_batch", "side_by_side": 3},
                                    {"streams": "by_nano_batch", "side_by_side": 0}])

@@ -281,6 +281,29 @@ def test_few_rows_in_parts(M, N, K, share, parts):
     assert lib.dfhip_gemm_fp8_nt_splitk(*args, 9, 8192, 28672, 8, 2, 16, 4096, None) == -7         # no room for the parts
 
 
+# rows whose launches are streamed in parts although they stay two: four parts and more all of them, two where whole K would be
+# streamed in fewer than 160 workgroups of 32 columns
+@pytest.mark.parametrize("N,K,rows", [(8192, 28672, ()), (8192, 16384, ()), (5120, 25600, ()), (5088, 25600, (12, 16)),
+                                      (4096, 14336, (12, 16)), (3072, 8192, (12, 16, 17, 24, 32)), (3072, 24576, (12, 16)),
+                                      (2048, 16384, (9, 12, 16, 17, 24, 32)), (1280, 16384, (9, 12, 16, 17, 24, 32))])
+def test_launches_that_stay_two_are_streamed_in_parts_where_that_pays(N, K, rows):
+    """All other plans are those of launches that may become one."""
+    lib, v, s = _cabi.load(), ctypes.c_int(), ctypes.c_int()
+
+    def plan(M, share, may_split):
+        assert lib.dfhip_gemm_fp8_plan_tiles(M, N, K, share, may_split, ctypes.byref(v), ctypes.byref(s)) == 0
+        return v.value, s.value
+
+    for M in (8, 9, 12, 16, 17, 24, 32, 33, 64, 350):
+        for share in (1, 2, 4):
+            variant, parts = plan(M, share, 2)
+            assert ((variant < 0 or variant == 8) and parts > 1) == (share > 1 and M in rows)
+            if not (share > 1 and 9 <= M <= 32) or M in rows:
+                assert (variant, parts) == plan(M, share, 1)
+            else:
+                assert plan(M, share, 1)[0] in (-1, 8) and plan(M, share, 1)[1] > 1
+
+
 # one and two row blocks; tiles of 16, 32 and 64 columns, ragged ones; parts of 16 slabs, of uneven lengths, 16 of them
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,split", [(1, 8, 4096, 2), (16, 1032, 4224, 2), (17, 1032, 8320, 4), (32, 2568, 4224, 2), (9, 5128, 4224, 2),

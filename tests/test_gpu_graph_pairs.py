@@ -97,6 +97,32 @@ def test_paired_replays_have_the_bits_of_the_eager_schedule(kind, tokens, hidden
             assert torch.equal(got, want)
 
 
+class LongBeside(torch.nn.Module):
+    """An fp8 layer beside a kernel of many workgroups that has no launch of two."""
+
+    def __init__(self, hidden, inter):
+        super().__init__()
+        self.layer, self.hidden = mlp("fp8", hidden, inter), hidden
+        self.register_buffer("table", randn((4096, hidden), 9).float())
+
+    def forward(self, x):
+        return self.layer(x) + (self.table * 2)[7].bfloat16()
+
+
+@pytest.mark.gpu
+def test_launches_that_turn_out_to_stay_two_are_planned_as_such():
+    """The first capture finds no pairs: the schedule is captured again with the plans of launches that stay apart."""
+    manager, compiled = program(LongBeside(4096, 14336), 24)
+    x = randn((24, 4096), 5)
+    split = manager.prepare(24, [1] * 24)
+    assert manager.launches_join(split)
+    forward(manager, compiled, x, True)
+    assert list(manager.paired_launches.values()) == [0] and not manager.launches_join(split)
+    want = forward(manager, compiled, x, False).clone()
+    for _ in range(3):
+        assert torch.equal(forward(manager, compiled, x, True), want)
+
+
 @pytest.mark.gpu
 def test_ranks_keep_their_schedule(monkeypatch):
     """Collectives are kernels of few workgroups: with several ranks nothing is put in line."""
