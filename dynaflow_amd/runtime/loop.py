@@ -79,8 +79,8 @@ def may_have_other_tasks() -> bool:
     """False if the coroutine of ``run_coroutine`` that runs now is the only one: it has started no task.  (Half a
     microsecond where a turn of the loop takes three.)"""
     kept = getattr(_thread, "kept", None)
-    loop = asyncio._get_running_loop()
-    if loop is None:
+    loop = asyncio.get_running_loop()
+    if loop is _on_demand:
         return False                                   # run_without_loop
     if kept is None or kept.loop is not loop or loop.get_task_factory() is not kept.tasks:
         return True
@@ -93,14 +93,47 @@ def _refuse_running_loop(coroutine: Coroutine) -> None:
         raise RuntimeError("a forward cannot be called from a running event loop")
 
 
+class _LoopOnDemand(asyncio.AbstractEventLoop):
+    """The running loop while a coroutine is run without one: what looks for a running loop finds one (another forward and
+    ``asyncio.run`` refuse to start inside it), and what uses it uses the thread's."""
+
+    def __getattribute__(self, name: str) -> Any:
+        return getattr(_kept_loop().loop, name)
+
+
+_on_demand = _LoopOnDemand()
+
+
+def _cancel_left(loop: asyncio.AbstractEventLoop) -> None:
+    left = asyncio.all_tasks(loop)
+    if left:
+        for task in left:
+            task.cancel()
+        loop.run_until_complete(asyncio.gather(*left, return_exceptions=True))
+        for task in left:
+            if not task.cancelled() and task.exception() is not None:
+                loop.call_exception_handler({"message": "a task that outlived its forward failed while it was cancelled",
+                                             "exception": task.exception(), "task": task})
+
+
 def run_without_loop(coroutine: Coroutine) -> Any:
     """Run a coroutine that waits for nothing (a forward under a scheduler that issues one operator after the other) to its end.
-    A turn of the loop and the task around the coroutine cost 30 us of a forward's 400."""
+    A turn of the loop and the task around the coroutine cost 30 us of a forward's 400.  Tasks that something inside it starts are
+    cancelled at its end."""
     _refuse_running_loop(coroutine)
+    before = getattr(_thread, "kept", None)
+    if before is not None:
+        before.tasks.made = 0
+    asyncio._set_running_loop(_on_demand)
     try:
         coroutine.send(None)
     except StopIteration as done:
         return done.value
+    finally:
+        asyncio._set_running_loop(None)
+        kept = getattr(_thread, "kept", None)
+        if kept is not None and kept.tasks.made and not kept.loop.is_closed():
+            _cancel_left(kept.loop)
     coroutine.close()
     raise RuntimeError("a schedule that was taken to wait for nothing waits")
 
@@ -113,12 +146,4 @@ def run_coroutine(coroutine: Coroutine) -> Any:
     try:
         return loop.run_until_complete(coroutine)
     finally:
-        left = asyncio.all_tasks(loop)
-        if left:
-            for task in left:
-                task.cancel()
-            loop.run_until_complete(asyncio.gather(*left, return_exceptions=True))
-            for task in left:
-                if not task.cancelled() and task.exception() is not None:
-                    loop.call_exception_handler({"message": "a task that outlived its forward failed while it was cancelled",
-                                                 "exception": task.exception(), "task": task})
+        _cancel_left(loop)

@@ -596,6 +596,34 @@ def test_a_coroutine_per_nano_batch_is_launched_in_turn(host_device, lanes):
     assert host_device.current_stream().name == "default"
 
 
+@pytest.mark.parametrize("policy", ["dynaflow_amd.schedulers:MLPOverlapScheduler", "test_engine_cpu:OwnWay"])
+def test_a_forward_inside_an_operator_is_refused(host_device, policy):
+    """Under every scheduler: a nested forward would take over the engine's state in the middle of the outer one."""
+    cfg = make_config(2)
+    cfg.scheduler_path = policy
+    model, manager, compiled, x = compile_mlp(cfg)
+    refused = []
+
+    def operator(*_):
+        manager.prepare(64, [64])
+        with pytest.raises(RuntimeError, match="running event loop"):
+            compiled(x)
+        refused.append(1)
+
+    hook = manager.engine.graph_module.submod_0.callable_dynamic.register_forward_pre_hook(operator)
+    for _ in range(2):
+        manager.prepare(64, [64])
+        with torch.no_grad():
+            torch.testing.assert_close(compiled(x), model(x), rtol=0, atol=0)
+    hook.remove()
+    assert len(refused) == 4
+
+
+class OwnWay(MLPOverlapScheduler):
+    async def schedule(self, context):
+        await super().schedule(context)
+
+
 @pytest.mark.parametrize("register", [
     lambda module, hook: module.register_forward_hook(hook),
     lambda module, hook: module.register_forward_pre_hook(hook),

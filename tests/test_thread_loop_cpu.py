@@ -153,3 +153,37 @@ def test_a_forward_without_a_loop_is_refused_inside_one():
         return 3
 
     assert run_coroutine(inside()) == 3
+
+
+@pytest.mark.parametrize("inner", [run_without_loop, run_coroutine, asyncio.run])
+def test_a_forward_without_a_loop_refuses_what_one_with_a_loop_refuses(inner):
+    """An operator cannot start another forward, or a loop of its own, in the middle of a schedule."""
+    async def operator():
+        coroutine = nothing()
+        with pytest.raises(RuntimeError, match="running event loop"):
+            inner(coroutine)
+        coroutine.close()
+        return 3
+
+    assert run_without_loop(operator()) == run_coroutine(operator()) == 3
+    assert run_without_loop(nothing()) == asyncio.run(nothing()) == 7
+
+
+def test_an_operator_finds_a_running_loop_without_one():
+    ended = []
+
+    async def other():
+        try:
+            await asyncio.sleep(60)
+        finally:
+            ended.append(asyncio.current_task().get_loop())
+
+    async def operator():
+        task = asyncio.get_running_loop().create_task(other())
+        task.get_loop().call_soon(ended.append, "called")
+        return task
+
+    task = run_without_loop(operator())
+    assert task.cancelled() and ended == ["called"]
+    assert asyncio._get_running_loop() is None
+    assert run_coroutine(nothing()) == 7
