@@ -347,14 +347,11 @@ class DynaFlowManager:
         return graph, output
 
     def _schedules_plainly(self) -> bool:
-        """Whether the scheduler issues its operators, and nothing else, the way the shipped ones do: on the streams of
-        ``stream_policy``."""
-        from dynaflow_amd.schedulers import MLPOverlapScheduler, StaggeredScheduler
+        """Whether the scheduler issues its operators, and nothing else, the way the staggered ones that are shipped do: on the
+        streams of ``stream_policy``."""
+        from dynaflow_amd.schedulers import issues_as_shipped
 
-        kind, own = type(self.scheduler), vars(self.scheduler)
-        return (issubclass(kind, StaggeredScheduler) and kind.schedule in (StaggeredScheduler.schedule, MLPOverlapScheduler.schedule)
-                and kind._issue is StaggeredScheduler._issue and kind._stream_for is StaggeredScheduler._stream_for
-                and not {"schedule", "_issue", "_stream_for"} & own.keys())
+        return issues_as_shipped(self.scheduler)
 
     def _capture_paired(self, args: tuple, kwargs: dict, split: SplitConfig, caller, origin, capture_on: dict) -> tuple:
         """The schedule with the launches of two nano-batches against the same weights as one: (graph, output, pairs);

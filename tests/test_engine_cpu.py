@@ -12,7 +12,7 @@ from dynaflow_amd.executor.compiler import SubgraphBackend
 from dynaflow_amd.interface import ExecutionContext, OpSchedulerBase, SplitConfig
 from dynaflow_amd.manager import DynaFlowManager
 from dynaflow_amd.mlp import SwiGLUMLP
-from dynaflow_amd.schedulers import MLPOverlapScheduler
+from dynaflow_amd.schedulers import MLPOverlapScheduler, NanoFlowScheduler, StaggeredScheduler
 from dynaflow_amd.schedulers.mlp_overlap import mlp_split_rules, mlp_tag_rules
 from oracle import schedule_trace as ref
 
@@ -622,6 +622,48 @@ def test_a_forward_inside_an_operator_is_refused(host_device, policy):
 class OwnWay(MLPOverlapScheduler):
     async def schedule(self, context):
         await super().schedule(context)
+
+
+class Waits(StaggeredScheduler):
+    async def schedule(self, context):
+        await asyncio.sleep(0)
+        await super().schedule(context)
+
+
+class WaitsBehindTheShippedOne(MLPOverlapScheduler, Waits):
+    pass
+
+
+def plain(patch):
+    return MLPOverlapScheduler
+
+
+def patched(home):
+    async def schedule(self, context):
+        await asyncio.sleep(0)
+        await shipped(self, context)
+
+    shipped = home.schedule
+
+    def patch(monkeypatch):
+        monkeypatch.setattr(home, "schedule", schedule)
+        return MLPOverlapScheduler
+
+    return patch
+
+
+@pytest.mark.parametrize("kind,order,as_shipped", [
+    (plain, "staggered", True), (plain, "round_robin", True), (lambda patch: WaitsBehindTheShippedOne, "staggered", False),
+    (patched(StaggeredScheduler), "staggered", False), (patched(MLPOverlapScheduler), "staggered", False),
+    (patched(NanoFlowScheduler), "round_robin", False)])
+def test_a_schedule_that_waits_gets_a_loop(host_device, monkeypatch, kind, order, as_shipped):
+    """Whichever class on the way to the shipped schedule waits, and whoever has put it there."""
+    cfg = make_config(2, schedule=order)
+    model, manager, compiled, x = compile_mlp(cfg, scheduler=kind(monkeypatch)(cfg))
+    assert manager._schedules_plainly() == as_shipped
+    manager.prepare(64, [64])
+    with torch.no_grad():
+        torch.testing.assert_close(compiled(x), model(x), rtol=0, atol=0)
 
 
 @pytest.mark.parametrize("register", [
