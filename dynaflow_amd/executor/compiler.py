@@ -29,10 +29,15 @@ from dynaflow_amd.interface import OperatorHandle
 from dynaflow_amd.runtime.env import get_op_handle
 
 
+_module_call = torch.nn.Module.__call__
+
+
 def _is_hooked(module: torch.nn.Module) -> bool:
-    """Whether ``Module.__call__`` does more than call ``forward``: hooks of this module or of all modules, or tracing."""
+    """Whether ``Module.__call__`` does more than call ``forward``: hooks of this module or of all modules, tracing, a module that
+    was compiled in place (``Module.compile``), or another ``__call__`` in the place of torch's."""
     return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
-                or has_any_global_hook() or torch._C._get_tracing_state())
+                or has_any_global_hook() or torch._C._get_tracing_state() or module._compiled_call_impl is not None
+                or torch.nn.Module.__call__ is not _module_call)
 
 
 class SubgraphBackend:

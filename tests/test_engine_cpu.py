@@ -689,3 +689,32 @@ def test_hooks_see_a_subgraph_that_is_called_past_module_call(register):
         handle.remove()
     assert any(module is gm for module in seen)
     assert torch.equal(backend(3, torch.ones(3)), torch.full((3,), 2.0)) and len(seen) == 1
+
+
+@pytest.mark.parametrize("how", ["compiled in place", "another __call__"])
+def test_a_subgraph_module_that_is_called_otherwise_is_not_called_past_that(monkeypatch, how):
+    class Twice(torch.nn.Module):
+        def forward(self, tokens, x):
+            return x * 2
+
+    gm, seen = torch.fx.symbolic_trace(Twice()), []
+    backend = SubgraphBackend(gm, 0, InductorConfig(enabled=False), CUDAGraphConfig(enabled=False, capture_sizes=[]),
+                              use_inductor=False, use_cudagraph=False)
+    backend.callable_dynamic = gm
+    if how == "compiled in place":
+        def compiler(graph, inputs):
+            seen.append(gm)
+            return graph.forward
+
+        torch._dynamo.reset()
+        gm.compile(backend=compiler)
+    else:
+        call = torch.nn.Module.__call__
+
+        def watched(module, *args, **kwargs):
+            seen.append(module)
+            return call(module, *args, **kwargs)
+
+        monkeypatch.setattr(torch.nn.Module, "__call__", watched)
+    assert torch.equal(backend(3, torch.ones(3)), torch.full((3,), 2.0))
+    assert any(module is gm for module in seen)
