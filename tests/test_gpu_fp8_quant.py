@@ -97,6 +97,24 @@ def test_fused_launches_of_two_threads_on_one_stream():
             assert torch.equal(scale, want[i][1]) and torch.equal(q.view(torch.uint8), want[i][0].view(torch.uint8))
 
 
+# one slab of K and few, where no wave of the launch leaves its maximum apart, and the shortest K where they do
+@pytest.mark.parametrize("M,I,K", [(1, 8, 128), (64, 264, 256), (128, 2816, 512), (24, 1408, 1024), (128, 4104, 1152)])
+def test_gate_up_of_few_rows_and_a_short_k(M, I, K):
+    """One call as for a long K: the codes and scale of the separate operators, and the entry point by itself."""
+    from dynaflow_amd import ops
+    from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
+
+    def randn(shape, seed):
+        return torch.randn(shape, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda").bfloat16()
+
+    xq, xs = ops.quant_fp8(randn((M, K), 1))
+    (wq, ws), (uq, us) = (quantize_weight_per_channel(randn((I, K), seed)) for seed in (2, 3))
+    q, scale = ops.gate_up_silu_quant_fp8(xq, wq, uq, xs, ws, us)
+    want_q, want_scale = ops.silu_mul_quant_fp8(ops.linear_fp8(xq, wq, xs, ws), ops.linear_fp8(xq, uq, xs, us))
+    assert torch.equal(scale, want_scale) and torch.equal(q.view(torch.uint8), want_q.view(torch.uint8))
+    test_gate_up_with_maxima_side_by_side(M, I, K, 1)
+
+
 # streamed in 16, 32 and 64 columns a workgroup, ragged; three-slab tiles; more workgroups than parts have room for; a ring tile
 @pytest.mark.parametrize("M,I,K,share", [(1, 136, 2048, 1), (17, 5120, 4096, 2), (32, 16392, 4096, 1), (128, 14336, 4096, 1), (40, 7176, 4096, 2),
                                          (16, 65544, 2048, 1), (128, 1032, 2048, 16)])
