@@ -640,8 +640,8 @@ extern "C" int dfhip_decode_attention_bf16(const void* q, int64_t ld_q, const vo
 // 16384 47.7 -> 46.6, but further from float64.  A probability is rounded to bf16 relative to its wave's largest, which is exact:
 // half as many waves round more of the large ones.  [distance, 2-norm, mean of 16 draws, 2 of 8192 2.650e-3 -> 2.672e-3, 4 of 8192
 // 2.682e-3 -> 2.713e-3, 4 of 16384 2.706e-3 -> 2.738e-3, each +- 0.15 %]
-// A compute unit takes in no more than 29 GB/s, so a few pairs more than units take twice the time: 257 .. 384 of them are cut
-// in four where the cache has room for 2048 positions, and so are 171 .. 192, which leave a quarter of the units idle, where it
+// While every compute unit loads, each gets 26 GB/s, its share of what the memory gives (one by itself takes in 50 and more), so a few
+// pairs more than units take up to twice the time, most units idle in the second half: 257 .. 384 of them are cut in four where the cache has room for 2048 positions, and so are 171 .. 192, which leave a quarter of the units idle, where it
 // has room for 4096.  [us, uncut / four parts, 8 kv heads, all full: 33 sequences of 2048 68 / 53, 48 of 2048 73 / 69, 36 of 4096 133 / 100,
 // 36 of 8192 266 / 190, 24 of 4096 70 / 65, of 8192 134 / 126; of 1/4 .. 1 of the capacity, longest first: 33 of 2048 45 / 41, 48 of 2048
 // 56 / 57, 36 of 4096 90 / 71, 48 of 4096 106 / 91, 24 of 4096 65 / 51, of 8192 124 / 90; not taken, for the sake of full caches: 32 of

@@ -12,7 +12,10 @@
 // beside them at 17 .. 4096 rows, alone and in pairs, on fp8 weights 28672 x 8192, 14336 x 4096 and transposed, bf16 ones
 // also 6144 x 4096, 4096 x 4096, 5632 x 2048.  Timed again, alone, on these and on 11264 x 2048 and fp8 16384 x 4096 and transposed: of the 767 timings
 // within 25 % of the fastest of their shape 9 % off on average and 18 % for nine in ten; two launches in step on two streams take
-// 5 - 30 % less than priced (they read their weights together).  What the choices by it give stands at three_slabs_cheaper.
+// 5 - 30 % less than priced (they read their weights together).  That was before a slab's loads were spread over all of it.  With them
+// spread the bf16 prices of 428 such timings are 6 % too high on average alone and level in pairs, 9 and 7 % off, 15 % for nine in ten,
+// and the tile chosen takes 0.1 % more than the fastest of these alone (3.6 % at worst) and 1.5 % in pairs (10.5 %: 1100 x 2048 x 5632).  What the choices
+// by it give stands at three_slabs_cheaper.
 struct DfhipPrice { double slab, slab_full, round, parts, part, intake; };
 inline double dfhip_price(const DfhipPrice& p, int64_t tiles, int share, double slabs, int split_k, double weight_mb) {
   const int64_t work = tiles * split_k * share;

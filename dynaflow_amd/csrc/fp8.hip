@@ -997,13 +997,13 @@ DfhipRing3Plan three_slabs_cheaper(bool gate_up, int M, int N, int K, int share,
 // Activations of a few rows: the kernel that streams W past LDS (gemm_stream.hip); with 16 rows and more from K = 4096
 // on, as for bf16 rows of the same bytes.  From 33 rows on every workgroup re-reads the activations four times as wide as
 // up to 16, which a tile shares: there the 128 x 128 tiles take over, unless the launch is alone and its weights few.  [us at 33 / 64
-// rows, streamed or on 128-row tiles against 128 x 128: alone 28672 x 8192 53 / 63 against 55 / 56, with gate + up + SiLU*mul 103 /
-// 110 against 91 / 94, 14336 x 4096 17 / 19 against 23 / 22, with gate + up 35 / 37 against 33 / 33; in pairs 28672 x 8192 81 / 84
-// against 76 / 78, 14336 x 4096 30 / 35 against 25 / 26.]  A product that may be cut along K goes there alone from 33 rows on;
-// in pairs it is streamed in parts of K from 9 to 32 rows (few_rows_parts) and goes there above.  [8192 x 28672 alone at 17 / 24 / 33 /
-// 64 rows: 44 / 48 / 59 / 79 against 50 / 49 / 50 / 52, in pairs at 33 / 64 92 / 92 against 79 / 82; 4096 x 14336 alone 19 / 21 / 25 / 34
-// against 24, in pairs at 33 / 64 45 / 45 against 31 / 32.  Fewer than 2^25 weights stay: 1536 x 7168 alone at 40 rows 15 against 18,
-// in pairs at 12 rows 17 against 23.]
+// rows, streamed against 128 x 128: alone 28672 x 8192 47 / 52 against 52 / 54, with gate + up + SiLU*mul 96 / 96 against 91 / 90,
+// 14336 x 4096 15 / 16 against 24 / 25, with gate + up 34 / 35 against 33 / 34; in pairs 28672 x 8192 94 / 110 against 89 / 92,
+// 14336 x 4096 34 / 37 against 30 / 30.  The first goes with its gate + up.]  A product that may be cut along K goes there alone from 33
+// rows on; in pairs it is streamed in parts of K from 9 to 32 rows (few_rows_parts) and goes there above.  [8192 x 28672 alone at 17 / 24
+// / 33 / 64 rows: 38 / 41 / 47 / 58 against 46 / 46 / 48 / 50, in pairs at 33 / 64 100 / 122 against 80 / 84; 4096 x 14336 alone 13 / 14 / 18
+// / 23 against 19 / 19 / 20 / 22, in pairs at 33 / 64 42 / 53 against 32 / 35.  Fewer than 2^25 weights stay: 1536 x 7168 alone at 40
+// rows 10 against 13, in pairs at 12 rows level.]
 bool few_rows_streamed(int M, int N, int K, int share, bool may_split) {
   if (!dfhip_stream_fits(M, N, K, 1) || (M >= 16 && K < 4096)) return false;
   const int64_t weights = (int64_t)N * K;

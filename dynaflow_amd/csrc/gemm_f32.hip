@@ -245,10 +245,13 @@ int launch_tile128(const F32Args& p, hipStream_t stream) {
 
 // The split tile that takes the least: one round of 256 workgroups costs its blocks and about 1.5 blocks' worth of start,
 // loads and meeting; of several rounds, whose workgroups overlap, each costs 0.6 of its blocks and of seven more for the
-// operands (per round at K = 2048: 4 x 4 blocks 37 us, 4 x 3 31, 4 x 2 25).  [us with a row per lane, at [128 x 1024] x [2816 x 1024]^T / [128 x
-// 2816] x [1024 x 2816]^T, with the workgroups in parentheses: 2 x 3 blocks 12.4 (236) / 27.5 (88), 4 x 2 14.9 (176) /
+// operands (per round at K = 2048: 4 x 4 blocks 37 us, 4 x 3 31, 4 x 2 25).  [us with a row per lane, at [128 x 1024] x [2816 x 1024]^T /
+// [128 x 2816] x [1024 x 2816]^T, with the workgroups in parentheses: 2 x 3 blocks 12.4 (236) / 27.5 (88), 4 x 2 14.9 (176) /
 // 32.7 (64), 2 x 2 17.2 (352) / 22.2 (128), 2 x 1 18.4 (704) / 16.9 (256); the 128 x 128 tiles 105 (22) / 274 (8).  Floor at
-// the fp32 rate: 4.9.]
+// the fp32 rate: 4.9.]  These prices and those below were fitted with a row per lane, and not again since lanes pair up: of 54 launches
+// (16 .. 1000 rows of six weights) the one chosen takes 1.7 % more than the fastest, of 54 pairs 3.9 %; it is 5 % off and more in 20 of
+// these, most of several rounds, where 4 x 3 and 4 x 4 blocks are taken and 2 x 2 would be faster (1000 x 2816 x 1024 69 / 60, pairs of
+// 1000 x 1408 x 512 56 / 44), and in a pair of 1000 x 5632 x 2048, on 128 x 128 tiles 581 / 422.
 // Many rows and a K up to about 3000 keep the 128 x 128 tiles, which read their operands half as often: both are priced
 // in us, fitted to about 190 launches (0.5 * 10^9 .. 10^12 flops, K = 288 .. 14336, alone and in pairs), the 128 x 128
 // tiles by their rounds (of all launches side by side: they fill each other's units).  [us, 128 x 128 / split: 8192 x 2816

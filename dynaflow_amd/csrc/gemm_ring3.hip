@@ -8,8 +8,8 @@
 // its use.  Here
 //   * the tile decides: LDS holds as many whole slabs as fit, three of 224 + 192 rows up to five of 128 + 128;
 //   * the fragments of a slab move to registers while the slab before it is multiplied (two sets, 208 registers for the
-//     largest tiles), so its LDS is free for DMA as soon as its own products start: with three slabs a fetch has 1.7 to 2
-//     slabs of time, with five 3.7 to 4; one barrier a slab;
+//     largest tiles), so its LDS is free for DMA as soon as its own products start: with three slabs a fetch has 1 to 2 slabs
+//     of time (the loads of a slab are spread over all of it), with five 3 to 4; one barrier a slab;
 //   * the two 32-byte halves of a fragment are read from LDS slots that lie in different banks for both types;
 //   * parts of K end without a wait: the part that comes last adds the blocks of all in part order, four of them in flight.
 // Every tile adds in the order of K of the other kernels of its type: the same bits.

@@ -18,10 +18,10 @@
 // slab its waves start: a row of W can sum in another order in a matrix of another N, or at another place in it.  The
 // fused launch has the bits of the separate, uncut ones because N, and with it the tiles, are the same.
 // Measured (weights from HBM, us; M = 2 / 16 / 32 rows, against the 128-row tiles used before): gate + up + SiLU*mul
-// 2 x 14336 x 4096 (235 MB) 39 / 39 / 43, before 51; down 4096 x 14336 23 / 24 / 27, before 207 / 36 / 36; q/k/v
-// 6144 x 4096 12 / 15 / 18, before 62 / 22 / 22; o 4096 x 4096 8 / 10 / 13, before 61 / 21 / 21.  At 8 / 16 / 32 / 64
-// rows fp8 down 8192 x 28672 (235 MB) 37 / 42 / 54 / 79, before 240 (two of 12 / 32 rows in one launch, K in parts: 40 / 49);
-// fp8 gate + up 2 x 28672 x 8192 (470 MB) 80 / 82 / 92 / 112, before 113 - 117.
+// 2 x 14336 x 4096 (235 MB) 38 / 38 / 39, before 51; down 4096 x 14336 22 / 22 / 24, before 207 / 36 / 36; q/k/v
+// 6144 x 4096 11 / 12 / 16, before 62 / 22 / 22; o 4096 x 4096 8 / 10 / 11, before 61 / 21 / 21.  At 8 / 16 / 32 / 64
+// rows fp8 down 8192 x 28672 (235 MB) 36 / 37 / 44 / 58, before 240 (two of 12 / 32 rows in one launch, K in parts: 40 / 49);
+// fp8 gate + up 2 x 28672 x 8192 (470 MB) 77 / 76 / 84 / 96, before 113 - 117.
 #include "dfhip_pairs.h"
 #include "dfhip_stream.h"
 
