@@ -752,10 +752,11 @@ torch.library.register_fake(
 _FP8_PARTS = 1024
 #: DFHIP_SPLIT_APART
 _SPLIT_APART = 2
-#: DFHIP_FP8_GEMM_PARTS, and the rows up to which a gate + up launch is short enough for the clearing of a cell to show, whatever its
-#: K is.  [us in a graph, cleared cell / one call, at 12 and 128 rows: 2816 x 256 11.4 / 11.1 and 13.0 / 13.0 (no maxima apart: the same
-#: launches), 2816 x 1024 12.2 / 10.8 and 14.6 / 11.9, 14336 x 4096 32.9 / 24.3 and 42.9 / 35.8, 28672 x 8192 80 / 70 and 104 / 97]
-_FP8_GEMM_PARTS, _FP8_ONE_CALL_ROWS = 4096, 128
+#: DFHIP_FP8_GEMM_PARTS, and the rows up to which and the K from which a gate + up launch is short enough for the clearing of a cell
+#: to show, and planned on kernels whose waves can leave their maxima apart.  [us in a graph, cleared cell / one call, at 12 and 128
+#: rows: 2816 x 768 13.9 / 13.9 and 15.3 / 15.3 (the same launches), 2816 x 896 11.8 / 10.3 and 14.3 / 11.6, 2816 x 1024 12.2 / 10.8 and 14.6 /
+#: 11.9, 14336 x 4096 32.9 / 24.3 and 42.9 / 35.8, 28672 x 8192 80 / 70 and 104 / 97]
+_FP8_GEMM_PARTS, _FP8_ONE_CALL_ROWS, _FP8_ONE_CALL_K = 4096, 128, 896
 
 
 def _quant_fp8_impl(x: torch.Tensor):
@@ -814,7 +815,7 @@ def _gate_up_silu_quant_fp8_impl(x_q, w_gate_q, w_up_q, x_scale, w_gate_scale, w
         wg, wu = wg.contiguous(), wu.contiguous()
         ldg = K
     act = torch.empty((M, I), dtype=torch.bfloat16, device=x_q.device)
-    if 0 < M <= _FP8_ONE_CALL_ROWS:
+    if 0 < M <= _FP8_ONE_CALL_ROWS and K >= _FP8_ONE_CALL_K:
         # the waves leave their maxima side by side: no cell to clear in front of a launch that is short itself
         scale = torch.empty(1 + _FP8_GEMM_PARTS, dtype=torch.float32, device=x_q.device)
         q = torch.empty((M, I), dtype=FP8_DTYPE, device=x_q.device)

@@ -98,9 +98,9 @@ def test_fused_launches_of_two_threads_on_one_stream():
 
 
 # one slab of K and few, where no wave of the launch leaves its maximum apart, and the shortest K where they do
-@pytest.mark.parametrize("M,I,K", [(1, 8, 128), (64, 264, 256), (128, 2816, 512), (24, 1408, 1024), (128, 4104, 1152)])
+@pytest.mark.parametrize("M,I,K", [(1, 8, 128), (64, 264, 256), (128, 2816, 768), (12, 2816, 896), (24, 1408, 1024), (128, 4104, 1152)])
 def test_gate_up_of_few_rows_and_a_short_k(M, I, K):
-    """One call as for a long K: the codes and scale of the separate operators, and the entry point by itself."""
+    """On both sides of the K from which it is one call: the codes and scale of the separate operators, and the entry point by itself."""
     from dynaflow_amd import ops
     from dynaflow_amd.fp8_mlp import quantize_weight_per_channel
 
