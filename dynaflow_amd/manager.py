@@ -21,6 +21,7 @@ scheduler and all launches.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import logging
 import os
@@ -105,6 +106,8 @@ def join_results(results: dict[int, Any], num_nano_batches: int, shared_buffer: 
         return tuple(fields)
     return first
 
+
+_AS_IT_IS = contextlib.nullcontext()
 
 #: Rows of a nano-batch up to which two of its launches may become one (DFHIP_PAIR_MAX_M).
 PAIR_MAX_ROWS = 128
@@ -255,8 +258,9 @@ class DynaFlowManager:
         assert split is not None
         from dynaflow_amd import ops
 
+        join = self.launches_join(split)
         with ops.launch_options(side_by_side=self._side_by_side or self.launches_side_by_side(split)), \
-                ops.launches_join(self.launches_join(split)):
+                ops.launches_join(join) if join != ops._join() else _AS_IT_IS:
             if split.is_dryrun:
                 results, events = self.engine.dryrun(args, kwargs, split)
             else:

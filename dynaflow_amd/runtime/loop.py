@@ -78,10 +78,10 @@ def _kept_loop() -> _KeptLoop:
 def may_have_other_tasks() -> bool:
     """False if the coroutine of ``run_coroutine`` that runs now is the only one: it has started no task.  (Half a
     microsecond where a turn of the loop takes three.)"""
-    kept = getattr(_thread, "kept", None)
     loop = asyncio.get_running_loop()
     if loop is _on_demand:
         return False                                   # run_without_loop
+    kept = getattr(_thread, "kept", None)
     if kept is None or kept.loop is not loop or loop.get_task_factory() is not kept.tasks:
         return True
     return kept.tasks.made > 1
@@ -121,9 +121,9 @@ def run_without_loop(coroutine: Coroutine) -> Any:
     A turn of the loop and the task around the coroutine cost 30 us of a forward's 400.  Tasks that something inside it starts are
     cancelled at its end."""
     _refuse_running_loop(coroutine)
-    before = getattr(_thread, "kept", None)
-    if before is not None:
-        before.tasks.made = 0
+    kept = getattr(_thread, "kept", None)
+    if kept is not None:
+        kept.tasks.made = 0
     asyncio._set_running_loop(_on_demand)
     try:
         coroutine.send(None)

@@ -5,10 +5,15 @@ from dynaflow_amd.schedulers.staggered import StaggeredScheduler  # noqa: F401
 from dynaflow_amd.schedulers.mlp_overlap import MLPOverlapScheduler  # noqa: F401
 from dynaflow_amd.schedulers.decoder_overlap import DecoderOverlapScheduler  # noqa: F401
 
-_PARTS = ("schedule", "_issue", "_stream_for")
-#: How the staggered policies issue their operators, as they are shipped: what each class on the way has of that.
-_SHIPPED = {home: [(name, vars(home).get(name)) for name in _PARTS]
-            for home in (StaggeredScheduler, MLPOverlapScheduler, DecoderOverlapScheduler, OpSchedulerBase)}
+def _parts(home: type) -> tuple:
+    """What a class itself has of how operators are issued."""
+    own = home.__dict__
+    return own.get("schedule"), own.get("_issue"), own.get("_stream_for")
+
+
+#: The staggered policies' as they are shipped; any other class has none of it.
+_SHIPPED = {home: _parts(home) for home in (StaggeredScheduler, MLPOverlapScheduler, OpSchedulerBase)}
+_NOTHING = (None, None, None)
 _ROUND_ROBIN = NanoFlowScheduler.schedule
 
 
@@ -18,13 +23,9 @@ def issues_as_shipped(scheduler: OpSchedulerBase) -> bool:
     put something else in the place of what does that."""
     staggered = False
     for home in type(scheduler).__mro__:
-        parts, shipped = home.__dict__, _SHIPPED.get(home)
-        if shipped is None:
-            if "schedule" in parts or "_issue" in parts or "_stream_for" in parts:
-                return False
-            continue
+        if _parts(home) != _SHIPPED.get(home, _NOTHING):
+            return False
         staggered |= home is StaggeredScheduler
-        for name, function in shipped:
-            if parts.get(name) is not function:
-                return False
-    return staggered and NanoFlowScheduler.schedule is _ROUND_ROBIN and not any(name in scheduler.__dict__ for name in _PARTS)
+    own = scheduler.__dict__
+    return staggered and NanoFlowScheduler.schedule is _ROUND_ROBIN and not (
+        "schedule" in own or "_issue" in own or "_stream_for" in own)
